@@ -235,3 +235,32 @@ def test_trained_warm_start_gain(pbf, scenes):
     assert res["learned"][1] >= res["plain"][1]
     assert res["learned"][0] * 1.5 <= res["plain"][0]
     assert res["learned"][0] <= 1.05 * res["previous"][0]
+
+
+@pytest.mark.parametrize("count", [1, 17, 2048, 2049, 16385])
+def test_batch_sums_at_row_edges(pbf, count):
+    """The gradient's sum over training blocks at 1, 2, 128, 129 and 1,024
+    rows (16 samples a row up to 1,024), and the same sums followed by Adam in
+    a one-batch training epoch: an Adam update from zero moments moves a
+    parameter by learning_rate * g / (|g| + eps), so a gradient whose sum
+    order differs by rounding (1e-4 relative here) gives the same move to
+    1e-3 * learning_rate wherever |g| is well above both eps and that rounding."""
+    X, y = _data(count, 5)
+    m = pbf.WarmModel(count)
+    m.init(3)
+    p = m.params()
+    m.add_samples(X, y)
+    g, loss = m.gradient(0, count)
+    gref, lref = M.gradient(p, X, y, rounding=True)
+    assert np.linalg.norm(g - gref) <= 1e-2 * np.linalg.norm(gref)
+    assert abs(loss - lref) <= 1e-3 * abs(lref)
+    m.adam_step(g, 1e-3)
+    stepped = m.params()
+    m.set_params(p)
+    trained_loss = m.train(1, count, 1e-3, 9)
+    trained = m.params()
+    big = np.abs(g) > 1e-2 * np.abs(g).max()
+    assert big.any()
+    assert np.abs(trained - stepped)[big].max() <= 1e-3 * 1e-3 + 2 * np.spacing(np.abs(p).max())
+    assert abs(trained_loss - loss) <= 1e-5 * abs(loss) + 1e-9
+    m.close()

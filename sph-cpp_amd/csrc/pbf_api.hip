@@ -169,6 +169,9 @@ static int compute_kparams(const pbf_params& P, KParams& K, uint64_t dims[3]) {
   K.gamma = P.gamma;
   K.vthr = 0.000001 * (double)P.max_speed;         // particles.h:380
   K.st_rmin = (double)P.smoothing_radius * 0.000001;  // particles.h:420
+  K.st_rmin_float = (float)K.st_rmin;
+  if ((double)K.st_rmin_float < K.st_rmin)
+    K.st_rmin_float = std::nextafter(K.st_rmin_float, std::numeric_limits<float>::infinity());
   for (int i = 0; i < 3; ++i) {
     K.bmin[i] = P.boundary_min[i];
     K.bmax[i] = P.boundary_max[i];
@@ -199,6 +202,7 @@ static int compute_kparams(const pbf_params& P, KParams& K, uint64_t dims[3]) {
   K.batched = 0;
   K.scenes = nullptr;
   K.sid = nullptr;
+  K.pad = (uint32_t)P.max_particles_local;
   K.heavy_budget = 768u;
   return PBF_OK;
 }
@@ -290,7 +294,7 @@ __global__ void k_compact_perm(uint32_t n, const uint32_t* __restrict__ oid, uin
 }
 
 // neighbour search body shared by pbf_find_neighbors and pbf_step
-static void find_neighbors_impl(pbf_context* c, uint64_t bin_end, uint64_t fb, uint64_t fe, bool skin = false);
+static void find_neighbors_impl(pbf_context* c, uint64_t bin_end, uint64_t fb, uint64_t fe, bool fused);
 
 void drop_graph(pbf_context* c) {
   if (c->graph_exec) hipGraphExecDestroy(c->graph_exec);
@@ -400,11 +404,11 @@ int pbf_create(const pbf_params* params, pbf_context** out) {
   if ((rc = dalloc(&c->x, NP)) || (rc = dalloc(&c->xs, NP)) || (rc = dalloc(&c->v, NP)) ||
       (rc = dalloc(&c->xa, NP)) || (rc = dalloc(&c->xsa, NP)) || (rc = dalloc(&c->va, NP)) ||
       (rc = dalloc(&c->xt, NP)) ||
-      (rc = dalloc(&c->scr, N)) || (rc = dalloc(&c->scra, N)) || (rc = dalloc(&c->rho, N)) ||
-      (rc = dalloc(&c->lam, N)) || (rc = dalloc(&c->rhoa, N)) || (rc = dalloc(&c->lama, N)) ||
+      (rc = dalloc(&c->scr, NP)) || (rc = dalloc(&c->scra, NP)) || (rc = dalloc(&c->rho, NP)) ||
+      (rc = dalloc(&c->lam, NP)) || (rc = dalloc(&c->rhoa, NP)) || (rc = dalloc(&c->lama, NP)) ||
       (rc = dalloc(&c->oid, N)) || (rc = dalloc(&c->oida, N)) || (rc = dalloc(&c->key, N)) ||
       (rc = dalloc(&c->keya, N)) || (rc = dalloc(&c->slot, N)) || (rc = dalloc(&c->tmp, N + 1)) ||
-      (rc = dalloc(&c->tmpo, N + 1)) || (rc = dalloc(&c->nbr, (N + 63) / 64 * 64 * (uint64_t)c->K.stride)) ||
+      (rc = dalloc(&c->tmpo, N + 1)) || (rc = dalloc(&c->nbr, list_size(N, c->K.stride))) ||
       (rc = dalloc(&c->nbr_count, N)) || (rc = dalloc(&c->counters, (uint64_t)C_NUM)) ||
       (rc = dalloc(&c->stage, 4 * N)) || (rc = dalloc(&c->stage64, N + 1)) || (rc = alloc_grid(c)) ||
       (rc = dalloc(&c->sk[0], N + 1)) || (rc = dalloc(&c->sk[1], N + 1)) || (rc = dalloc(&c->sv[0], N + 1)) ||
@@ -412,8 +416,8 @@ int pbf_create(const pbf_params* params, pbf_context** out) {
       (rc = dalloc(&c->roffs, radix_hist_size(N) + 1)) ||
       (rc = dalloc(&c->rpart, scan_partials_size(radix_hist_size(N) + 1))) || (rc = dalloc(&c->heavy, N)) ||
       (rc = dalloc(&c->chbox, 2 * ((N + 63) / 64))) || (rc = dalloc(&c->wmask, 2 * N)) ||
-      (rc = dalloc(&c->cnb, (N + 63) / 64 * 64 * (uint64_t)c->K.stride)) || (rc = dalloc(&c->cnb_count, N)) ||
-      (rc = dalloc(&c->snb, (N + 63) / 64 * 64 * (uint64_t)c->K.stride)) || (rc = dalloc(&c->snb_count, N)) ||
+      (rc = dalloc(&c->cnb, list_size(N, c->K.stride))) || (rc = dalloc(&c->cnb_count, N)) ||
+      (rc = dalloc(&c->snb, list_size(N, c->K.stride))) || (rc = dalloc(&c->snb_count, N)) ||
       (rc = dalloc(&c->xs0, NP)) || (rc = dalloc(&c->skin_hint, 1)) ||
       (rc = dalloc(&c->moved, N)) || (rc = dalloc(&c->dirty, N)) || (rc = dalloc(&c->mflag, N)) ||
       (rc = dalloc(&c->ehist, (uint64_t)kMaxSolveSlots + 1)) || (rc = dalloc(&c->lsum, N)) ||
@@ -435,6 +439,8 @@ int pbf_create(const pbf_params* params, pbf_context** out) {
     return rc;
   }
   launch_fill_u64(c->counters, 0ull, C_NUM, c->stream);
+  // the far row of the position stars: +inf
+  for (float4* a : {c->xs, c->xsa, c->xt}) launch_fill_u32((uint32_t*)(a + N), 0x7F800000u, 4 * kRowPad, c->stream);
   launch_fill_u32((uint32_t*)c->nbr_count, 0u, N, c->stream);
   launch_fill_u32(c->dirty, 0u, N, c->stream);
   launch_fill_u32(c->mflag, 0u, N, c->stream);
@@ -506,6 +512,7 @@ int pbf_set_params(pbf_context* c, const pbf_params* params) {
   c->P = *params;
   c->K = K;
   c->cap = K.cap;
+  c->pass_skin = false;  // (the skin radius follows h)
   ++c->version;
   for (int i = 0; i < 3; ++i) c->dims[i] = dims[i];
   c->ncells = K.ncells;
@@ -675,7 +682,10 @@ int pbf_get_scratch(pbf_context* c, float* out) { return get_vec(c, c ? c->scr :
 int pbf_get_densities(pbf_context* c, float* out) { return get_scalar(c, c ? c->rho : nullptr, out); }
 int pbf_get_lambdas(pbf_context* c, float* out) { return get_scalar(c, c ? c->lam : nullptr, out); }
 int pbf_set_positions(pbf_context* c, const float* in) { return set_vec(c, c ? c->x : nullptr, in); }
-int pbf_set_position_stars(pbf_context* c, const float* in) { return set_vec(c, c ? c->xs : nullptr, in); }
+int pbf_set_position_stars(pbf_context* c, const float* in) {
+  if (c) c->pass_skin = false;
+  return set_vec(c, c ? c->xs : nullptr, in);
+}
 int pbf_set_velocities(pbf_context* c, const float* in) { return set_vec(c, c ? c->v : nullptr, in); }
 int pbf_set_scratch(pbf_context* c, const float* in) { return set_vec(c, c ? c->scr : nullptr, in); }
 int pbf_set_densities(pbf_context* c, const float* in) { return set_scalar(c, c ? c->rho : nullptr, in); }
@@ -699,6 +709,7 @@ int pbf_predict_positions(pbf_context* c, pbf_index_span s) {
   PBF_TRACE("pbf_predict_positions");
   PBF_CHECK_CTX_SPAN(c, s);
   launch_forces_predict(c, F_PREDICT, s.begin, s.end);
+  c->pass_skin = false;  // x* is no longer where its lists were built
   return check_hip(hipGetLastError(), "predict_positions");
 }
 
@@ -709,7 +720,8 @@ int pbf_find_neighbors(pbf_context* c, pbf_index_span bin_span, pbf_index_span f
   if (bin_span.begin != 0)
     return set_error(PBF_ERR_ARG, "bin span must start at 0: sort_bins sorts [0, count) (neighbors.h:130-132)");
   launch_fill_u64(c->counters, 0ull, 3, c->stream);  // overflow, outside, hacks
-  find_neighbors_impl(c, bin_span.end, fill_span.begin, fill_span.end);
+  find_neighbors_impl(c, bin_span.end, fill_span.begin, fill_span.end, false);
+  c->pass_skin = c->K.skin_mode != 0;
   return check_hip(hipGetLastError(), "find_neighbors");
 }
 
@@ -758,7 +770,7 @@ int pbf_apply_surface_tension(pbf_context* c, pbf_index_span cs, pbf_index_span 
   PBF_CHECK_CTX_SPAN(c, cs);
   PBF_CHECK_CTX_SPAN(c, ts);
   if (int rc = need_lists(c)) return rc;
-  launch_surface_tension(c, cs.begin, cs.end, ts.begin, ts.end);
+  launch_surface_tension(c, cs.begin, cs.end, ts.begin, ts.end, c->pass_skin);
   return check_hip(hipGetLastError(), "apply_surface_tension");
 }
 
@@ -766,7 +778,7 @@ int pbf_apply_viscosity(pbf_context* c, pbf_index_span s) {
   PBF_TRACE("pbf_apply_viscosity");
   PBF_CHECK_CTX_SPAN(c, s);
   if (int rc = need_lists(c)) return rc;
-  launch_viscosity(c, c->v, c->va, 0, s.begin, s.end);
+  launch_viscosity(c, c->v, c->va, s.begin, s.end);
   std::swap(c->v, c->va);
   return check_hip(hipGetLastError(), "apply_viscosity");
 }
@@ -797,7 +809,7 @@ int pbf_update_positions(pbf_context* c, pbf_index_span s) {
 // The part of the step after the pressure solve (Simulation/Source/main.cpp:108-124).
 static void step_tail(pbf_context* c) {
   const uint64_t n = c->n;
-  if (c->P.gamma != 0.f) launch_surface_tension(c, 0, n, 0, n);
+  if (c->P.gamma != 0.f) launch_surface_tension(c, 0, n, 0, n, c->K.skin_mode != 0);
   launch_viscosity_first(c);         // XSPH 1: v -> va, compact lists of the final positions
   launch_vorticity_masked(c);        // omega -> scr
   launch_apply_vorticity_masked(c);  // va += ...
@@ -891,6 +903,7 @@ int pbf_step_graph(pbf_context* c, uint32_t nsteps) {
     c->graph_sig = buffer_sig(c);
   }
   uint32_t st = 0;
+  if (nsteps) c->pass_skin = false;
   for (; st + 2 <= nsteps; st += 2)
     if ((rc = check_hip(hipGraphLaunch(c->graph_exec, c->stream), "hipGraphLaunch"))) return rc;
   if (st < nsteps) step_body(c);
@@ -1046,6 +1059,7 @@ int pbf_solve_graph(pbf_context* c, float tolerance, uint32_t max_iterations, in
     c->sgraph_gain = c->warm_gain;
   }
   uint32_t st = 0;
+  if (nsteps) c->pass_skin = false;
   for (; st + 2 <= nsteps; st += 2)  // nsteps >= 2: the graph is current
     if ((rc = check_hip(hipGraphLaunch(c->sgraph_exec, c->stream), "hipGraphLaunch"))) return rc;
   if (st < nsteps && (rc = solve_body(c, tolerance, max_iterations, warm_start, false))) return rc;
@@ -1332,7 +1346,7 @@ int pbf_autotune_layout(pbf_context* c, uint32_t steps, pbf_layout* best) {
     if ((rc = pbf_set_params(c, &P)) || (rc = S.restore())) break;
     launch_fill_u64(c->counters, 0ull, C_NUM, c->stream);
     launch_forces_predict(c, F_FORCES | F_PREDICT, 0, c->n);
-    find_neighbors_impl(c, c->n, 0, c->n);
+    find_neighbors_impl(c, c->n, 0, c->n, false);
     unsigned long long over = 0;
     uint32_t longest = 0;
     if ((rc = check_hip(hipMemcpyAsync(&over, c->counters + C_OVERFLOW, sizeof(over), hipMemcpyDeviceToHost,
@@ -1462,7 +1476,7 @@ int pbf_get_neighbor_lists(pbf_context* c, uint64_t* out, int32_t* counts) {
   std::vector<uint32_t> o, cnt, lists;
   if (int rc = download_u32(c, c->oid, n, o)) return rc;
   if (int rc = download_u32(c, (const uint32_t*)c->nbr_count, n, cnt)) return rc;
-  if (int rc = download_u32(c, (const uint32_t*)c->nbr, (n + 63) / 64 * 64 * c->K.stride, lists)) return rc;
+  if (int rc = download_u32(c, (const uint32_t*)c->nbr, (n + 63) / 64 * 64 * (uint64_t)c->K.stride, lists)) return rc;
   std::memset(out, 0, n * K * sizeof(uint64_t));
   for (uint64_t p = 0; p < n; ++p) {
     const uint64_t op = o[p];
@@ -1572,14 +1586,15 @@ int pbf_region_end(pbf_context* c, double* ms) {
 
 namespace pbf {
 
-static void find_neighbors_impl(pbf_context* c, uint64_t bin_end, uint64_t fb, uint64_t fe, bool skin) {
-  launch_bin(c, bin_end);  // (clears the list build's counters)
+static void find_neighbors_impl(pbf_context* c, uint64_t bin_end, uint64_t fb, uint64_t fe, bool fused) {
+  launch_bin(c, bin_end, fused);  // (clears the list build's counters)
   launch_sort(c);
   // a fused step recomputes densities, multipliers and the scratch vector
   // before reading them (with at least one Jacobi iteration): they stay unsorted
-  launch_reorder(c, !(skin && c->P.solve_step_count > 0));
-  launch_fill_neighbors(c, fb, fe, skin);
+  launch_reorder(c, !(fused && c->P.solve_step_count > 0));
+  launch_fill_neighbors(c, fb, fe);
   c->lists_valid = true;
+  c->pass_skin = false;
 }
 
 }  // namespace pbf

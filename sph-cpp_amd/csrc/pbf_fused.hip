@@ -5,20 +5,20 @@
 //
 //  * Latency: a neighbour walk is a chain of dependent loads (list entry, then
 //    the neighbour's data).  Neighbours are taken in batches of kBatch: the
-//    batch's list entries load first (entry k of a wavefront's 64 particles
-//    is one 256-byte row), then all gathers are issued, then the arithmetic
-//    runs in list order.  The density pass loads the next batch's entries
-//    while it works on the current one.
+//    batch's list entries load first (two 16-byte loads of a lane), then all
+//    gathers are issued, then the arithmetic runs in list order.  The density
+//    and pressure passes load the next batch's entries while they work on the
+//    current one.
 //  * Only about half of a particle's listed neighbours lie within h (the list
 //    radius is the 1.2 h bin spacing, neighbors.h:198); the others contribute
-//    exact zeros.  The density pass walks the whole list once, summing the
-//    entries within h as it goes, and records them in a bit mask per particle
-//    (one bit per list entry); the Jacobi iteration's dp pass, which sees the
-//    same positions, walks the list again but gathers and sums only the
-//    masked entries.  The first XSPH pass appends the entries within h of the
-//    final positions to a compact row (cnb), staged in LDS; vorticity,
-//    vorticity-apply and the second XSPH pass walk only that row, in the same
-//    order.
+//    exact zeros, and a test of their squared distance leaves them out (the
+//    single lanes' pressure update takes the density pass's verdicts from a
+//    bit mask instead, and does not gather the others).  The first XSPH pass
+//    appends the entries within h of the final positions to a compact row
+//    (cnb); vorticity, vorticity-apply and the second XSPH pass walk only that
+//    row, in the same order.
+//  * A particle is walked by one lane, or in small scenes by four (quad walks,
+//    below).
 //  * The density pass writes lambda into the w word of its x* output, so the
 //    dp pass gathers a neighbour's x* and lambda in one 16-byte load.
 //  * The near-coincidence fix of compute_densities (particles.h:303-305) moves
@@ -28,146 +28,149 @@
 //    back to plain walks for the particles next to a moved one.
 #include <hip/hip_cooperative_groups.h>
 
+#include <algorithm>
+
 #include "pbf_mlp_device.h"
+#include "pbf_walk.h"
 
 namespace pbf {
 
 constexpr int kBlock = 256;
-constexpr int kBatch = 8;
 static inline uint32_t nblocks(uint64_t n) { return (uint32_t)((n + kBlock - 1) / kBlock); }
-
-__device__ __forceinline__ f3 xyz(float4 t) { return {t.x, t.y, t.z}; }
-
-// Entries k0 .. k0+7 of particle p's list (tiled, list_at): for each entry,
-// the 64 lanes of a wavefront read one contiguous segment.  Entries at or
-// past cnt are replaced by p, which keeps every gather in bounds.
-__device__ __forceinline__ void load_batch(const int32_t* __restrict__ list, uint32_t stride, int k0, int cnt,
-                                           uint32_t p, uint32_t (&q)[kBatch]) {
-#pragma unroll
-  for (int u = 0; u < kBatch; ++u) q[u] = (k0 + u < cnt) ? (uint32_t)list[list_at(k0 + u, p, stride)] : p;
-}
-
-// The pass that builds the compact lists (the first XSPH pass) runs one
-// wavefront per block and stages each lane's entries in its own LDS column
-// (entry k of the 64 lanes contiguous): its second loop reads them from LDS,
-// and the global copy is written at the end with entry k of the 64 lanes in
-// one contiguous store.
-constexpr int kStageBlock = 64;
-
-__device__ __forceinline__ void load_batch_lds(const int32_t* __restrict__ s_list, uint32_t lane, int k0, int cnt,
-                                               uint32_t p, uint32_t (&q)[kBatch]) {
-#pragma unroll
-  for (int u = 0; u < kBatch; ++u) q[u] = (k0 + u < cnt) ? (uint32_t)s_list[(k0 + u) * kStageBlock + lane] : p;
-}
-
-__device__ __forceinline__ void flush_compact(const int32_t* __restrict__ s_list, uint32_t lane, int nc,
-                                              int32_t* __restrict__ cnb, uint32_t stride, uint32_t p) {
-  for (int k = 0; k < nc; ++k) cnb[list_at(k, p, stride)] = s_list[k * kStageBlock + lane];
-}
-
-// Skin lists (built with the lists, pbf_grid.hip): the entries within
-// 1.1 h of the positions the lists were built from (x*_0), in list order,
-// each slot packed with its place in the full list (slot | place << 25).  A
-// pass may walk the skin list instead of the full one while no particle has
-// moved 0.045 h or more from x*_0: an entry outside the skin list was at
-// least 1.1 h away, so it is still farther than 1.01 h, well past h and any
-// rounding of the within-h test, and adds nothing to any sum.  The entries
-// within h come in the same order, so the sums are the same bit for bit.
-// Every position a pressure update writes is checked against that move; a
-// larger one (or a NaN position) sets a flag: C_DISP by iteration parity
-// (read by the next iteration's passes) and C_DISP_ALL for the rest of the
-// step.  The flags are written only when a move is too large, so a step at
-// rest issues no atomics.
-constexpr uint32_t kSkinSlotBits = 25;
-constexpr uint32_t kSkinSlotMask = (1u << kSkinSlotBits) - 1u;
-
-__device__ __forceinline__ bool skin_usable(const unsigned long long* __restrict__ counters, int flag) {
-  return counters[C_SKIN] != 0ull && counters[flag] == 0ull;
-}
-
-// the squared move of a new position star from x*_0
-__device__ __forceinline__ float move2(f3 nw, float4 x0) { return magsq3(sub3(nw, xyz(x0))); }
-
-// Sets counters[a] and counters[C_DISP_ALL] when a lane's squared move m is
-// not below the limit (NaN included); every lane of the wavefront calls it.
-__device__ __forceinline__ void record_move(float m, unsigned long long* __restrict__ counters, int a,
-                                            const KParams& K) {
-  const uint64_t over = __ballot(!(m < K.disp_lim2));
-  if (over != 0ull && (threadIdx.x & 63) == 0) {
-    if (counters[a] == 0ull) atomicExch(&counters[a], 1ull);
-    if (counters[C_DISP_ALL] == 0ull) atomicExch(&counters[C_DISP_ALL], 1ull);
-  }
-}
 
 // x limited to [lo, hi] (NaN gives lo)
 __device__ __forceinline__ float clampf(float x, float lo, float hi) { return x > lo ? (x < hi ? x : hi) : lo; }
 
 // ---------------------------------------------------------------------------
 // compute_densities (particles.h:292-313) + compute_pressure_lambdas (:318-342)
-// xs -> xt (x* with lambda in w), rho, lam, and the particle's within-h mask
-// (bit k of wmask[p], of wmask[n + p] for k >= 64: list entry k lies within h
-// and is in the sums; not read for a particle the density fix moved).  With FEAT, also the learned warm start's features of
-// the particle (FeatCtl).
-// Returns the particle's density error max(rho/rho0 - 1, 0).
+// xs -> xt (x* with lambda in w), rho, lam.  With FEAT, also the learned warm
+// start's features of the particle (FeatCtl).
+struct DensitySums {
+  float density, sum_C;
+  f3 sg;
+  float dy, div;  // FEAT
+  int within;     // FEAT
+};
+__device__ __forceinline__ DensitySums density_start(const KParams& K) {
+  return DensitySums{K.mass_W0, 0.0f, {0.f, 0.f, 0.f}, 0.0f, 0.0f, 0};
+}
+
+// particles.h:304-305: a plain walk over the full list from its first entry,
+// in list order, moves x*_p at each near-coincident entry
+template <bool FEAT, bool FAST>
+__device__ __forceinline__ DensitySums density_plain(uint32_t p, f3& xp, f3 vp, const KParams& K,
+                                                     const float4* __restrict__ xs, const float4* __restrict__ v,
+                                                     const int32_t* __restrict__ nbr,
+                                                     const int32_t* __restrict__ nbr_count, uint32_t& hacks) {
+  DensitySums s = density_start(K);
+  const int full = nbr_count[p];
+  for (int k0 = 0; k0 < full; k0 += kBatch) {
+    // a batch's positions load together; the entries are taken in order
+    uint32_t q[kBatch];
+    load_batch(nbr, K.stride, k0, full, p, q);
+    f3 t[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) t[u] = ld3(xs, q[u]);
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      f3 d = sub3(xp, t[u]);
+      float d2 = magsq3(d);
+      if (k0 + u >= full || !within_h(d2, K)) continue;
+      if (d2 < K.T_hack) {
+        dec3(xp, div3(mul3(ld3(v, p), K.dt), 50.0f));
+        ++hacks;
+        d = sub3(xp, t[u]);
+        d2 = magsq3(d);
+        if (!within_h(d2, K)) continue;
+      }
+      const float r = nb_sqrt<FAST>(d2);
+      s.density += K.mass * poly6_in(r, K);
+      const f3 grad = smul3(K.neg_inv_rho0, nb_spiky<FAST>(d, r, K));
+      dec3(s.sg, grad);
+      s.sum_C += magsq3(grad);
+      if (FEAT) {
+        ++s.within;
+        s.dy -= d.y;
+        const f3 dv = sub3(vp, ld3(v, q[u]));
+        s.div -= (dv.x * grad.x + dv.y * grad.y) + dv.z * grad.z;
+      }
+    }
+  }
+  return s;
+}
+
+// rho, lambda and x* of the particle from its sums; returns the density error
+// max(rho/rho0 - 1, 0).
+__device__ __forceinline__ float density_finish(uint32_t p, const DensitySums& s, f3 xp, const KParams& K,
+                                                float4* __restrict__ xt, float* __restrict__ rho,
+                                                float* __restrict__ lam, float& sum_C, float& lp) {
+  rho[p] = s.density;
+  sum_C = s.sum_C + magsq3(s.sg);
+  const float constraint = s.density / K.rho0 - 1.0f;
+  const float C_p = ((double)constraint < 0.0) ? 0.0f : constraint;
+  lp = -C_p / (sum_C + K.eps);
+  lam[p] = lp;
+  xt[p] = make_float4(xp.x, xp.y, xp.z, lp);  // the dp pass gathers x* and lambda in one load
+  return constraint;
+}
+
+// By one lane; also the particle's within-h mask (bit k of wmask[p], of
+// wmask[n + p] for k >= 64: entry k of the walked list lies within h; not
+// read for a particle the density fix moved).
 template <bool FEAT, bool FAST, bool SR>
-__device__ __forceinline__ float density_lambda_one(uint32_t p, uint32_t n, int it, const KParams& K,
-                                                    const float4* __restrict__ xs, const float4* __restrict__ v,
-                                                    float4* __restrict__ xt, float* __restrict__ rho,
-                                                    float* __restrict__ lam, const int32_t* __restrict__ nbr,
+__device__ __forceinline__ float density_lambda_one(uint32_t p, uint32_t n, const KParams& K, const float4* __restrict__ xs,
+                                                    const float4* __restrict__ v, float4* __restrict__ xt,
+                                                    float* __restrict__ rho, float* __restrict__ lam,
+                                                    const int32_t* __restrict__ nbr,
                                                     const int32_t* __restrict__ nbr_count,
                                                     uint64_t* __restrict__ wmask, const FeatCtl& F,
-                                                    uint32_t& hacks_out, float (&fo)[8],
-                                                    const int32_t* __restrict__ snb,
+                                                    uint32_t& hacks, float (&fo)[8], const int32_t* __restrict__ snb,
                                                     const int32_t* __restrict__ snb_count, bool skin) {
   f3 xp = ld3(xs, p);
   // the walk goes over the skin list when it may (skin lists, above); the
   // plain walk after a density fix always takes the full list
   const int32_t* __restrict__ walk = skin ? snb : nbr;
   const int cnt = skin ? snb_count[p] : nbr_count[p];
-  float density = K.mass_W0;
-  float sum_C = 0.0f;
-  f3 sg = {0.f, 0.f, 0.f};
-  uint32_t hacks = 0;
-  float dy_sum = 0.0f, div = 0.0f;
+  DensitySums s = density_start(K);
   const f3 vp = FEAT ? ld3(v, p) : f3{0.f, 0.f, 0.f};
   // one walk over the list: the entries within h go into the sums, in list
-  // order, and into the mask.  A near-coincident entry ends the walk after
-  // its batch, and the plain walk below redoes the particle; the mask of such
-  // a particle is not read (the pressure update walks a moved particle's
-  // full list with the test).
-  uint64_t m0 = 0, m1 = 0;
+  // order (padding entries read the far row and are never within h).  A
+  // near-coincident entry (particles.h:304) ends the walk after its batch, and
+  // the plain walk below redoes the particle with fresh sums.
   bool hack = false;
-  const uint32_t qmask = skin ? kSkinSlotMask : ~0u;  // the slot of a walked entry
-  uint32_t qn[kBatch];  // skin entries keep their place in the full list in the top bits
-  load_batch(walk, K.stride, 0, cnt, p, qn);
+  uint64_t m0 = 0, m1 = 0;
+  const int4* __restrict__ row = list_row(walk, p, K.stride);
+  uint32_t q[kBatch];
+  load_row(row, 0, q);
   for (int k0 = 0; k0 < cnt && !hack; k0 += kBatch) {
-    uint32_t q[kBatch];
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) q[u] = qn[u];
-    float4 t[kBatch];
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) t[u] = gather4(xs, q[u] & qmask);
-    load_batch(walk, K.stride, k0 + kBatch, cnt, p, qn);  // the next batch's entries load under this one's work
     uint32_t bits = 0;
+    float4 t[kBatch];
+    f3 vq[FEAT ? kBatch : 1];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) t[u] = gather4(xs, q[u]);
+    if (FEAT) {
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) vq[u] = xyz(gather4(v, q[u]));
+    }
+    load_row(row, k0 + kBatch, q);  // the next batch's entries load under this one's work
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
       const f3 d = sub3(xp, xyz(t[u]));
       const float d2 = magsq3(d);
-      const bool w = (k0 + u < cnt) & within_h(d2, K);
-      const bool hk = w & (d2 < K.T_hack);  // particles.h:304: handled by the plain walk below
-      const bool acc = w & !hk;
-      bits |= (uint32_t)acc << u;
-      hack |= hk;
-      if (acc) {
+      const bool in = within_h(d2, K);
+      hack |= d2 < K.T_hack;
+      bits |= (uint32_t)in << u;
+      if (in) {
         const float r = nb_sqrt<FAST, SR>(d2);
-        density += K.mass * poly6_in(r, K);
+        s.density += K.mass * poly6_in(r, K);
         const f3 grad = smul3(K.neg_inv_rho0, nb_spiky<FAST, SR>(d, r, K));
-        dec3(sg, grad);
-        sum_C += magsq3(grad);
+        dec3(s.sg, grad);
+        s.sum_C += magsq3(grad);
         if (FEAT) {  // (feature passes walk the full lists)
-          dy_sum -= d.y;
-          const f3 dv = sub3(vp, ld3(v, q[u]));
-          div -= (dv.x * grad.x + dv.y * grad.y) + dv.z * grad.z;
+          ++s.within;
+          s.dy -= d.y;
+          const f3 dv = sub3(vp, vq[u]);
+          s.div -= (dv.x * grad.x + dv.y * grad.y) + dv.z * grad.z;
         }
       }
     }
@@ -177,72 +180,74 @@ __device__ __forceinline__ float density_lambda_one(uint32_t p, uint32_t n, int 
     else
       m1 |= (uint64_t)bits << (k0 - 64);
   }
-  wmask[p] = m0;
-  if (K.cap > 64) wmask[n + p] = m1;
-  int within = __popcll(m0) + __popcll(m1);
-  if (hack) {
-    // particles.h:304-305: a plain walk over the full list from its first
-    // entry, in list order, moves x*_p at each near-coincident entry
-    density = K.mass_W0;
-    sum_C = 0.0f;
-    sg = {0.f, 0.f, 0.f};
-    dy_sum = 0.0f;
-    div = 0.0f;
-    within = 0;
-    const int full = nbr_count[p];
-    for (int k0 = 0; k0 < full; k0 += kBatch) {
-      // a batch's positions load together; the entries are taken in order
-      uint32_t q[kBatch];
-      load_batch(nbr, K.stride, k0, full, p, q);
-      f3 t[kBatch];
-#pragma unroll
-      for (int u = 0; u < kBatch; ++u) t[u] = ld3(xs, q[u]);
-#pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        f3 d = sub3(xp, t[u]);
-        float d2 = magsq3(d);
-        if (k0 + u >= full || !within_h(d2, K)) continue;
-        if (d2 < K.T_hack) {
-          dec3(xp, div3(mul3(ld3(v, p), K.dt), 50.0f));
-          ++hacks;
-          d = sub3(xp, t[u]);
-          d2 = magsq3(d);
-          if (!within_h(d2, K)) continue;
-        }
-        const float r = nb_sqrt<FAST>(d2);
-        density += K.mass * poly6_in(r, K);
-        const f3 grad = smul3(K.neg_inv_rho0, nb_spiky<FAST>(d, r, K));
-        dec3(sg, grad);
-        sum_C += magsq3(grad);
-        if (FEAT) {
-          ++within;
-          dy_sum -= d.y;
-          const f3 dv = sub3(vp, ld3(v, q[u]));
-          div -= (dv.x * grad.x + dv.y * grad.y) + dv.z * grad.z;
-        }
-      }
-    }
+  if (!FEAT) {
+    wmask[p] = m0;
+    if (K.cap > 64) wmask[n + p] = m1;
   }
-  rho[p] = density;
-  sum_C += magsq3(sg);
-  const float constraint = density / K.rho0 - 1.0f;
-  const float C_p = ((double)constraint < 0.0) ? 0.0f : constraint;
-  const float lp = -C_p / (sum_C + K.eps);
-  lam[p] = lp;
-  xt[p] = make_float4(xp.x, xp.y, xp.z, lp);  // the dp pass gathers x* and lambda in one load
-  hacks_out = hacks;
+  if (hack) s = density_plain<FEAT, FAST>(p, xp, vp, K, xs, v, nbr, nbr_count, hacks);
+  float sum_C, lp;
+  const float constraint = density_finish(p, s, xp, K, xt, rho, lam, sum_C, lp);
   if (FEAT) {
     const float inv_s = 1.0f / kWarmLambdaScale;
-    const float dyn = dy_sum / (float)(within > 0 ? within : 1);
+    const float dyn = s.dy / (float)(s.within > 0 ? s.within : 1);
     fo[0] = clampf(constraint, -1.0f, 4.0f);
     fo[1] = clampf(lp * inv_s, -64.0f, 0.0f);
     fo[2] = clampf(F.lprev[p] * inv_s, -64.0f, 0.0f);
     fo[3] = clampf(sum_C * 1e-5f, 0.0f, 8.0f);
-    fo[4] = clampf((float)within / 32.0f, 0.0f, 4.0f);
+    fo[4] = clampf((float)s.within / 32.0f, 0.0f, 4.0f);
     fo[5] = clampf(vp.y * K.dt / K.h, -4.0f, 4.0f);
     fo[6] = clampf(dyn / K.h, -2.0f, 2.0f);
-    fo[7] = clampf(div * K.mass * K.dt, -4.0f, 4.0f);
+    fo[7] = clampf(s.div * K.mass * K.dt, -4.0f, 4.0f);
   }
+  return constraint > 0.0f ? constraint : 0.0f;
+}
+
+// The same by a quad (no features); lane 0 writes, counts the fixes and
+// returns the error, the other lanes return 0.
+template <bool FAST, bool SR>
+__device__ __forceinline__ float density_lambda_quad(uint32_t p, const KParams& K, const float4* __restrict__ xs,
+                                                     const float4* __restrict__ v, float4* __restrict__ xt,
+                                                     float* __restrict__ rho, float* __restrict__ lam,
+                                                     const int32_t* __restrict__ nbr,
+                                                     const int32_t* __restrict__ nbr_count, uint32_t& hacks,
+                                                     const int32_t* __restrict__ snb,
+                                                     const int32_t* __restrict__ snb_count, bool skin) {
+  f3 xp = ld3(xs, p);
+  const int cnt = skin ? snb_count[p] : nbr_count[p];
+  DensitySums s = density_start(K);
+  bool hack = false;
+  const uint32_t* __restrict__ row = quad_row(skin ? snb : nbr, p, K.stride);
+  uint32_t q[2] = {row[0], row[256]};
+  for (int k0 = 0; k0 < cnt && !hack; k0 += kBatch) {
+    const float4 t[2] = {gather4(xs, q[0]), gather4(xs, q[1])};
+    row += kBatch * 64;
+    q[0] = row[0], q[1] = row[256];  // the next batch
+    bool near = false;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const f3 d = sub3(xp, xyz(t[j]));
+      const float d2 = magsq3(d);
+      near |= d2 < K.T_hack;
+      float dens = 0.0f, c2 = 0.0f;
+      f3 grad = {0.f, 0.f, 0.f};
+      if (within_h(d2, K)) {
+        const float r = nb_sqrt<FAST, SR>(d2);
+        dens = K.mass * poly6_in(r, K);
+        grad = smul3(K.neg_inv_rho0, nb_spiky<FAST, SR>(d, r, K));
+        c2 = magsq3(grad);
+      }
+      quad_add(s.density, dens);
+      quad_sub(s.sg.x, grad.x);
+      quad_sub(s.sg.y, grad.y);
+      quad_sub(s.sg.z, grad.z);
+      quad_add(s.sum_C, c2);
+    }
+    hack = quad_any(near);
+  }
+  if ((threadIdx.x & 3u) != 0u) return 0.0f;
+  if (hack) s = density_plain<false, FAST>(p, xp, f3{0.f, 0.f, 0.f}, K, xs, v, nbr, nbr_count, hacks);
+  float sum_C, lp;
+  const float constraint = density_finish(p, s, xp, K, xt, rho, lam, sum_C, lp);
   return constraint > 0.0f ? constraint : 0.0f;
 }
 
@@ -302,7 +307,8 @@ __device__ __forceinline__ void warm_network(const FeatCtl& F, uint32_t wave_fir
 // calling thread is the one that clears the pass's flags (first): the same
 // bodies run as their own kernels (vb from xcd_block()) and inside the
 // persistent Jacobi kernel (vb from the calling block's share).
-template <int FM, bool FAST, bool SR>
+// QUAD: by quads, a block of vb holding a quarter as many particles.
+template <int FM, bool FAST, bool SR, bool QUAD>
 __device__ __forceinline__ void density_pass(uint32_t vb, bool first, uint32_t n, int it, int eslot,
                                              const SolveCtl& S, const FeatCtl& F,
                                              const KParams& K, const float4* __restrict__ xs,
@@ -317,14 +323,20 @@ __device__ __forceinline__ void density_pass(uint32_t vb, bool first, uint32_t n
                                              const int32_t* __restrict__ snb,
                                              const int32_t* __restrict__ snb_count) {
   if (S.tol >= 0.0f && counters[C_DONE] != 0ull) return;
-  const uint32_t p = vb * blockDim.x + threadIdx.x;
+  const uint32_t p = QUAD ? (vb * blockDim.x + threadIdx.x) >> 2 : vb * blockDim.x + threadIdx.x;
   // this iteration's pressure update records its moves in the other slot
   const bool skin = FM == 0 && skin_usable(counters, C_DISP + (it & 1));
   if (first) counters[C_DISP + ((it + 1) & 1)] = 0ull;
   float e = 0.0f;
   uint32_t hacks = 0;
   float fo[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if (p < n) e = density_lambda_one<FM != 0, FAST, SR>(p, n, it, K, xs, v, xt, rho, lam, nbr, nbr_count, wmask, F, hacks, fo, snb, snb_count, skin);
+  if (p < n) {
+    if constexpr (QUAD)
+      e = density_lambda_quad<FAST, SR>(p, K, xs, v, xt, rho, lam, nbr, nbr_count, hacks, snb, snb_count, skin);
+    else
+      e = density_lambda_one<FM != 0, FAST, SR>(p, n, K, xs, v, xt, rho, lam, nbr, nbr_count, wmask, F, hacks, fo,
+                                                snb, snb_count, skin);
+  }
   if (FM != 0 && F.feat && p < n) {
     float4* o = reinterpret_cast<float4*>(F.feat + (uint64_t)p * 8);
     o[0] = make_float4(fo[0], fo[1], fo[2], fo[3]);
@@ -363,7 +375,7 @@ __device__ __forceinline__ void density_pass(uint32_t vb, bool first, uint32_t n
 }
 
 // (the exact and fast instances of the plain pass fit 64 registers: 8 wavefronts per SIMD)
-template <int FM, bool FAST, bool SR>
+template <int FM, bool FAST, bool SR, bool QUAD>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu((FM == 0 && (SR || FAST)) ? 8 : 1)))
 k_density_lambda_c(uint32_t n, int it, int eslot, SolveCtl S, FeatCtl F,
                    KParams K, const float4* __restrict__ xs,
@@ -377,7 +389,7 @@ k_density_lambda_c(uint32_t n, int it, int eslot, SolveCtl S, FeatCtl F,
                    unsigned long long* __restrict__ counters,
                    const int32_t* __restrict__ snb,
                    const int32_t* __restrict__ snb_count) {
-  density_pass<FM, FAST, SR>(xcd_block(), blockIdx.x == 0 && threadIdx.x == 0, n, it, eslot, S, F, K, xs, v, xt, rho,
+  density_pass<FM, FAST, SR, QUAD>(xcd_block(), blockIdx.x == 0 && threadIdx.x == 0, n, it, eslot, S, F, K, xs, v, xt, rho,
                          lam, nbr, nbr_count, wmask, moved, stamp, mflag, counters, snb, snb_count);
 }
 
@@ -534,30 +546,56 @@ __device__ __forceinline__ float mean_error(unsigned long long sum, uint32_t n) 
   return (float)((double)sum / 4294967296.0 / (double)n);
 }
 
-// The pressure update's sum over one particle's list (particles.h:355-366):
-// the entries under the within-h mask, or with plain every entry within h.
+// The pressure update's sum over the entries of one particle's list within h
+// (particles.h:355-366), by one lane: under the density pass's mask (entries
+// outside h then gather the particle itself), or with plain every entry of
+// the list tested.
 template <bool FAST, bool SR>
-__device__ __forceinline__ f3 dp_walk(const int32_t* __restrict__ walk, int cnt, bool skin, bool plain, uint64_t m0,
-                                      uint64_t m1, uint32_t p, f3 xp, float lp, const KParams& K,
+__device__ __forceinline__ f3 dp_walk(const int32_t* __restrict__ walk, int cnt, bool plain, uint64_t m0, uint64_t m1,
+                                      uint32_t p, f3 xp, float lp, const KParams& K,
                                       const float4* __restrict__ xt) {
   f3 dp = {0.f, 0.f, 0.f};
-  const uint32_t qmask = skin ? kSkinSlotMask : ~0u;  // the slot of a walked entry
+  const int4* __restrict__ row = list_row(walk, p, K.stride);
+  uint32_t q[kBatch];
   for (int k0 = 0; k0 < cnt; k0 += kBatch) {
-    uint32_t q[kBatch];
-    load_batch(walk, K.stride, k0, cnt, p, q);
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) q[u] &= qmask;
+    load_row(row, k0, q);
     const uint32_t bits = (uint32_t)((k0 < 64 ? m0 >> k0 : m1 >> (k0 - 64)) & 0xFFu);
     float4 t[kBatch];
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) t[u] = gather4(xt, (bits >> u) & 1u ? q[u] : p);  // masked entries read p itself
+    for (int u = 0; u < kBatch; ++u) t[u] = gather4(xt, (bits >> u) & 1u ? q[u] : p);
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
       const f3 d = sub3(xp, xyz(t[u]));
       const float d2 = magsq3(d);
-      if (k0 + u >= cnt || !((bits >> u) & 1u) || (plain && !within_h(d2, K))) continue;
+      if (!((bits >> u) & 1u) || (plain && !within_h(d2, K))) continue;
       const float r = nb_sqrt<FAST, SR>(d2);
       acc3(dp, smul3(lp + t[u].w, nb_spiky<FAST, SR>(d, r, K)));
+    }
+  }
+  return dp;
+}
+
+// The same by a quad.
+template <bool FAST, bool SR>
+__device__ __forceinline__ f3 dp_walk_quad(const int32_t* __restrict__ walk, int cnt, uint32_t p, f3 xp, float lp,
+                                           const KParams& K, const float4* __restrict__ xt) {
+  f3 dp = {0.f, 0.f, 0.f};
+  const uint32_t* __restrict__ row = quad_row(walk, p, K.stride);
+  uint32_t q[2] = {row[0], row[256]};
+  for (int k0 = 0; k0 < cnt; k0 += kBatch) {
+    const float4 t[2] = {gather4(xt, q[0]), gather4(xt, q[1])};
+    row += kBatch * 64;
+    q[0] = row[0], q[1] = row[256];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const f3 d = sub3(xp, xyz(t[j]));
+      const float d2 = magsq3(d);
+      f3 term = {0.f, 0.f, 0.f};
+      if (within_h(d2, K)) {
+        const float r = nb_sqrt<FAST, SR>(d2);
+        term = smul3(lp + t[j].w, nb_spiky<FAST, SR>(d, r, K));
+      }
+      quad_add3(dp, term);
     }
   }
   return dp;
@@ -570,7 +608,7 @@ __device__ __forceinline__ f3 dp_walk(const int32_t* __restrict__ walk, int cnt,
 // before the warm start; with the retry, also slot 1's after the damped
 // start) restores xsave; an error <= tol ends the solve with x* = xt.
 // Neither applies an update.
-template <bool FAST, bool SR>
+template <bool FAST, bool SR, bool QUAD>
 __device__ __forceinline__ void dp_pass(uint32_t vb, bool first, uint32_t n, int it, int last, uint32_t stamp,
                                         const SolveCtl& S,
                                         const KParams& K, const float4* __restrict__ xt,
@@ -597,7 +635,9 @@ __device__ __forceinline__ void dp_pass(uint32_t vb, bool first, uint32_t n, int
     counters[C_MOVED_N + ((it + 1) & 1)] = 0ull;
     counters[C_MOVED_ALL + ((it + 1) & 1)] = 0ull;
   }
-  const uint32_t p = vb * blockDim.x + threadIdx.x;
+  const uint32_t p = QUAD ? (vb * blockDim.x + threadIdx.x) >> 2 : vb * blockDim.x + threadIdx.x;
+  // (every lane of a quad computes the particle's new state; lane 0 writes it)
+  const bool writes = !QUAD || (threadIdx.x & 3u) == 0u;
   // what this slot does, the same for every thread: 0 the update, 1 the
   // rejected warm start's restore, 2 the end of the solve (x* = xt)
   int mode = 0;
@@ -632,20 +672,20 @@ __device__ __forceinline__ void dp_pass(uint32_t vb, bool first, uint32_t n, int
       }
     }
   }
-  const bool track = K.skin_mode && n < (1u << kSkinSlotBits);  // x*_0 is kept: check the moves
+  const bool track = K.skin_mode;  // x*_0 is kept: check the moves
   float mv = 0.0f;
   if (p < n && mode == 1) {
     const float4 sv = S.xsave[p];
-    xs[p] = sv;
+    if (writes) xs[p] = sv;
     if (track) mv = move2(xyz(sv), xs0[p]);
   } else if (p < n && mode == 2) {
     const float4 t = xt[p];
-    xs[p] = t;
+    if (writes) xs[p] = t;
     if (track) mv = move2(xyz(t), xs0[p]);
   } else if (p < n) {
     // a dirty particle (moved by the density fix, or next to one) walks its
-    // whole list with the test; the others walk the list the density pass
-    // walked (the skin list when it could) under its within-h mask
+    // whole list; the others walk the list the density pass walked (the skin
+    // list when it could)
     const bool plain = counters[C_HACK_FLAG + (it & 1)] != 0ull && dirty[p] == stamp;
     const bool skin = !plain && skin_usable(counters, C_DISP + (it & 1));
     const int32_t* __restrict__ walk = skin ? snb : nbr;
@@ -654,19 +694,25 @@ __device__ __forceinline__ void dp_pass(uint32_t vb, bool first, uint32_t n, int
     const f3 xp = xyz(xp4);
     const float lp = xp4.w;
     const int cnt = skin ? snb_count[p] : nbr_count[p];
-    const uint64_t m0 = plain ? ~0ull : wmask[p];
-    const uint64_t m1 = (plain || K.cap <= 64) ? ~0ull : wmask[n + p];
-    // with no dirty lane in the wavefront every pair the walk takes is one
-    // the density pass accepted at the same positions (static ranges)
-    const f3 dp = (SR && __ballot(plain) == 0ull)
-                      ? dp_walk<FAST, SR>(walk, cnt, skin, false, m0, m1, p, xp, lp, K, xt)
-                      : dp_walk<FAST, false>(walk, cnt, skin, plain, m0, m1, p, xp, lp, K, xt);
+    // with no dirty lane in the wavefront every pair within h is one the
+    // density pass accepted at the same positions (static ranges); the quads
+    // find them by the same test, the single lanes by the mask it left
+    f3 dp;
+    if constexpr (QUAD)
+      dp = (SR && __ballot(plain) == 0ull) ? dp_walk_quad<FAST, SR>(walk, cnt, p, xp, lp, K, xt)
+                                           : dp_walk_quad<FAST, false>(walk, cnt, p, xp, lp, K, xt);
+    else {
+      const uint64_t m0 = plain ? ~0ull : wmask[p];
+      const uint64_t m1 = (plain || K.cap <= 64) ? ~0ull : wmask[n + p];
+      dp = (SR && __ballot(plain) == 0ull) ? dp_walk<FAST, SR>(walk, cnt, false, m0, m1, p, xp, lp, K, xt)
+                                           : dp_walk<FAST, false>(walk, cnt, plain, m0, m1, p, xp, lp, K, xt);
+    }
     f3 nw = add3(xp, smul3(K.inv_rho0, dp));
     boundary(nw, K, p);
-    st3(xs, p, nw);
+    if (writes) st3(xs, p, nw);
     if (track) mv = move2(nw, xs0[p]);
-    if (S.lsum) S.lsum[p] += lp;
-    if (last) {  // the density rides in v.w for the XSPH passes' gathers
+    if (S.lsum && writes) S.lsum[p] += lp;
+    if (last && writes) {  // the density rides in v.w for the XSPH passes' gathers
       f3 vel = div3(sub3(nw, ld3(x, p)), K.dt);
       if ((double)magsq3(vel) < K.vthr) vel = {0.f, 0.f, 0.f};
       v[p] = make_float4(vel.x, vel.y, vel.z, rho[p]);
@@ -675,20 +721,20 @@ __device__ __forceinline__ void dp_pass(uint32_t vb, bool first, uint32_t n, int
   if (track) record_move(mv, counters, C_DISP + ((it + 1) & 1), K);
 }
 
-template <bool FAST, bool SR>
+template <bool FAST, bool SR, bool QUAD>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) k_dp_update_c(uint32_t n, int it, int last, uint32_t stamp, SolveCtl S,
                                                         KParams K, const float4* __restrict__ xt,
                                                         const float4* __restrict__ x, float4* __restrict__ xs,
                                                         float4* __restrict__ v, const int32_t* __restrict__ nbr,
                                                         const int32_t* __restrict__ nbr_count,
                                                         const uint64_t* __restrict__ wmask,
-                                                        const uint32_t* __restrict__ dirty,
+                                                                        const uint32_t* __restrict__ dirty,
                                                         unsigned long long* __restrict__ counters,
                                                         const int32_t* __restrict__ snb,
                                                         const int32_t* __restrict__ snb_count,
                                                         const float4* __restrict__ xs0,
                                                         const float* __restrict__ rho) {
-  dp_pass<FAST, SR>(xcd_block(), blockIdx.x == 0 && threadIdx.x == 0, n, it, last, stamp, S, K, xt, x, xs, v, nbr,
+  dp_pass<FAST, SR, QUAD>(xcd_block(), blockIdx.x == 0 && threadIdx.x == 0, n, it, last, stamp, S, K, xt, x, xs, v, nbr,
                 nbr_count, wmask, dirty, counters, snb, snb_count, xs0, rho);
 }
 
@@ -706,7 +752,7 @@ __global__ void __launch_bounds__(kBlock) k_warm_dp(uint32_t n, KParams K, const
                                                     unsigned long long* __restrict__ counters,
                                                     const float4* __restrict__ xs0) {
   const uint32_t p = xcd_block() * blockDim.x + threadIdx.x;
-  const bool track = K.skin_mode && n < (1u << kSkinSlotBits);
+  const bool track = K.skin_mode;
   float mv = 0.0f;
   if (p < n) {
     const float4 xp4 = xt[p];
@@ -768,7 +814,7 @@ __global__ void __launch_bounds__(kBlock) k_warm_retry(uint32_t n, KParams K, co
                                                        const float4* __restrict__ xs0) {
   if (counters[C_RETRY] == 0ull) return;
   const uint32_t p = xcd_block() * blockDim.x + threadIdx.x;
-  const bool track = K.skin_mode && n < (1u << kSkinSlotBits);
+  const bool track = K.skin_mode;
   float mv = 0.0f;
   if (p < n) {
     const f3 xp = ld3(xsave, p);
@@ -803,39 +849,26 @@ __global__ void __launch_bounds__(kBlock) k_warm_retry(uint32_t n, KParams K, co
   if (track) record_move(mv, counters, C_DISP + 1, K);
 }
 
-// XSPH sum (particles.h:441-444) over a compact row, from global memory
-// (FROM_LDS = false: cnb, tiled like the lists) or from the lane's LDS column
-template <bool FROM_LDS>
-__device__ __forceinline__ f3 xsph_sum(const int32_t* __restrict__ list, uint32_t n, uint32_t lane, int nc,
-                                       uint32_t p, f3 xp, f3 vp, const KParams& K, const float4* __restrict__ xs,
-                                       const float4* __restrict__ vin) {
-  f3 dv = {0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < nc; k0 += kBatch) {
-    uint32_t q[kBatch];
-    if (FROM_LDS)
-      load_batch_lds(list, lane, k0, nc, p, q);
-    else
-      load_batch(list, K.stride, k0, nc, p, q);
-    float4 t[kBatch], vq[kBatch];  // vq.w: the neighbour's density
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      t[u] = gather4(xs, q[u]);
-      vq[u] = gather4(vin, q[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      if (k0 + u >= nc) continue;
-      const float r = sqrt_cr(magsq3(sub3(xp, xyz(t[u]))));
-      acc3(dv, div3(mul3(sub3(xyz(vq[u]), vp), poly6_in(r, K)), vq[u].w));
-    }
-  }
-  return dv;
+// ---------------------------------------------------------------------------
+// The passes after the pressure solve, by quads.  A compact row (cnb) holds
+// the entries within h of the final positions as byte offsets into the
+// particle arrays.
+__device__ __forceinline__ float4 gather_at(const float4* __restrict__ a, uint32_t offset) {
+  return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(a) + offset);
 }
 
-// ---------------------------------------------------------------------------
-// apply_viscosity (particles.h:436-447), first call: walks the whole list and
-// leaves the compact rows of the final positions for the passes that follow.
-__global__ void __launch_bounds__(kStageBlock) k_viscosity_first(uint32_t n, KParams K, const float4* __restrict__ xs,
+// the XSPH term of one pair within h (particles.h:441-444); vq.w: the
+// neighbour's density
+__device__ __forceinline__ f3 xsph_term(f3 xp, f3 vp, float4 t, float4 vq, const KParams& K) {
+  const float r = sqrt_cr(magsq3(sub3(xp, xyz(t))));
+  return div3_shared(mul3(sub3(xyz(vq), vp), poly6_in(r, K)), vq.w);
+}
+
+// apply_viscosity (particles.h:436-447), first call: walks the skin or full
+// list and leaves the compact rows of the final positions for the passes that
+// follow.  An accepted entry's place in the row is the number accepted before
+// it: the quad's four verdicts come from one ballot.
+__global__ void __launch_bounds__(kBlock) k_viscosity_first(uint32_t n, KParams K, const float4* __restrict__ xs,
                                                             const float4* __restrict__ vin,
                                                             float4* __restrict__ vout,
                                                             const int32_t* __restrict__ nbr,
@@ -846,55 +879,126 @@ __global__ void __launch_bounds__(kStageBlock) k_viscosity_first(uint32_t n, KPa
                                                             const int32_t* __restrict__ snb,
                                                             const int32_t* __restrict__ snb_count,
                                                             unsigned long long* __restrict__ skin_hint) {
-  extern __shared__ int32_t s_list[];  // [cap + 1][kStageBlock]
-  const uint32_t lane = threadIdx.x;
-  const uint32_t p = xcd_block() * blockDim.x + threadIdx.x;
+  const uint32_t p = (xcd_block() * blockDim.x + threadIdx.x) >> 2;
+  const uint32_t u = threadIdx.x & 3u;
   // the next step builds skin lists only if this one's moves kept them usable to the end
-  if (K.skin_mode && blockIdx.x == 0 && lane == 0) *skin_hint = counters[C_DISP_ALL] == 0ull ? 1ull : 0ull;
+  if (K.skin_mode && blockIdx.x == 0 && threadIdx.x == 0) *skin_hint = counters[C_DISP_ALL] == 0ull ? 1ull : 0ull;
   if (p >= n) return;
   const f3 xp = ld3(xs, p);
-  const f3 vp = ld3(vin, p);
+  const float4 v4 = vin[p];
+  const f3 vp = xyz(v4);
   // the skin list holds every entry within h while no particle has moved
   // 0.045 h over the step (skin lists, above)
   const bool skin = skin_usable(counters, C_DISP_ALL);
-  const int32_t* __restrict__ walk = skin ? snb : nbr;
   const int cnt = skin ? snb_count[p] : nbr_count[p];
-  const uint32_t qmask = skin ? kSkinSlotMask : ~0u;  // the slot of a walked entry
-  int nc = 0;
+  const uint32_t* __restrict__ row = quad_row(skin ? snb : nbr, p, K.stride);
+  int32_t* __restrict__ out = cnb + list_at(0, p, K.stride);
+  const uint32_t shift = threadIdx.x & 60u, before = (1u << u) - 1u;
+  f3 dv = {0.f, 0.f, 0.f};
+  uint32_t nc = 0;
+  uint32_t q[2] = {row[0], row[256]};
   for (int k0 = 0; k0 < cnt; k0 += kBatch) {
-    uint32_t q[kBatch];
-    load_batch(walk, K.stride, k0, cnt, p, q);
+    const uint32_t at[2] = {q[0] << 4, q[1] << 4};
+    const float4 t[2] = {gather_at(xs, at[0]), gather_at(xs, at[1])};
+    const float4 vq[2] = {gather_at(vin, at[0]), gather_at(vin, at[1])};
+    row += kBatch * 64;
+    q[0] = row[0], q[1] = row[256];
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) q[u] &= qmask;
-    float4 t[kBatch];
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) t[u] = gather4(xs, q[u]);
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const float d2 = magsq3(sub3(xp, xyz(t[u])));
-      const bool acc = (k0 + u < cnt) & within_h(d2, K);
-      s_list[nc * kStageBlock + lane] = (int32_t)q[u];  // a rejected entry is overwritten by the next accepted one
-      nc += acc ? 1 : 0;
+    for (int j = 0; j < 2; ++j) {
+      const bool in = within_h(magsq3(sub3(xp, xyz(t[j]))), K);
+      const uint32_t bits = (uint32_t)(__ballot(in) >> shift) & 15u;
+      f3 term = {0.f, 0.f, 0.f};
+      if (in) {
+        const uint32_t k = nc + (uint32_t)__popc(bits & before);
+        out[(k & ~3u) * 64u + (k & 3u)] = (int32_t)at[j];
+        term = xsph_term(xp, vp, t[j], vq[j], K);
+      }
+      nc += (uint32_t)__popc(bits);
+      quad_add3(dv, term);
     }
   }
-  cnb_count[p] = nc;
-  flush_compact(s_list, lane, nc, cnb, K.stride, p);
-  const f3 dv = xsph_sum<true>(s_list, n, lane, nc, p, xp, vp, K, xs, vin);
+  if (u != 0u) return;
+  cnb_count[p] = (int32_t)nc;
   f3 nv = vp;
   acc3(nv, smul3(K.visc, dv));
-  vout[p] = make_float4(nv.x, nv.y, nv.z, vin[p].w);  // the density stays in w
+  vout[p] = make_float4(nv.x, nv.y, nv.z, v4.w);  // the density stays in w
 }
 
+// A quad's walk over a compact row: TERM(offset) gives the three terms of an
+// entry, which enter `sum` in list order.  Lanes past the row's end gather
+// the particle itself and add +0.
+template <class Load, class Term>
+__device__ __forceinline__ void quad_walk_compact(const int32_t* __restrict__ cnb, int cnt, uint32_t p,
+                                                  const KParams& K, f3& sum, Load load, Term term) {
+  const uint32_t* __restrict__ row = quad_row(cnb, p, K.stride);
+  const int u = (int)(threadIdx.x & 3u);
+  uint32_t q[2] = {row[0], row[256]};
+  for (int k0 = 0; k0 < cnt; k0 += kBatch) {
+    const bool on[2] = {k0 + u < cnt, k0 + 4 + u < cnt};
+    const uint32_t at[2] = {on[0] ? q[0] : p << 4, on[1] ? q[1] : p << 4};
+    const auto a = load(at[0]);
+    const auto b = load(at[1]);
+    row += kBatch * 64;
+    q[0] = row[0], q[1] = row[256];
+    f3 t = {0.f, 0.f, 0.f};
+    if (on[0]) t = term(a);
+    quad_add3(sum, t);
+    t = f3{0.f, 0.f, 0.f};
+    if (on[1]) t = term(b);
+    quad_add3(sum, t);
+  }
+}
+struct Pair2 {  // a neighbour's position and its velocity or vorticity
+  float4 t, w;
+};
+
+// The same by one lane: entries k0 .. k0+7 of a compact row; entries at or past cnt are the
+// particle itself.
+__device__ __forceinline__ void load_compact(const int4* __restrict__ row, int k0, int cnt, uint32_t p,
+                                             uint32_t (&at)[kBatch]) {
+  load_row(row, k0, at);
+#pragma unroll
+  for (int u = 0; u < kBatch; ++u) at[u] = k0 + u < cnt ? at[u] : p << 4;
+}
+template <class Load, class Term>
+__device__ __forceinline__ void lane_walk_compact(const int32_t* __restrict__ cnb, int cnt, uint32_t p,
+                                                  const KParams& K, f3& sum, Load load, Term term) {
+  const int4* __restrict__ row = list_row(cnb, p, K.stride);
+  for (int k0 = 0; k0 < cnt; k0 += kBatch) {
+    uint32_t at[kBatch];
+    load_compact(row, k0, cnt, p, at);
+    Pair2 q[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) q[u] = load(at[u]);
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+      if (k0 + u < cnt) acc3(sum, term(q[u]));
+  }
+}
+
+template <bool QUAD, class Load, class Term>
+__device__ __forceinline__ void walk_compact(const int32_t* __restrict__ cnb, int cnt, uint32_t p, const KParams& K,
+                                             f3& sum, Load load, Term term) {
+  if constexpr (QUAD)
+    quad_walk_compact(cnb, cnt, p, K, sum, load, term);
+  else
+    lane_walk_compact(cnb, cnt, p, K, sum, load, term);
+}
 // apply_viscosity, second call, fused with update_positions (particles.h:390-394)
+template <bool QUAD>
 __global__ void __launch_bounds__(kBlock) k_viscosity_last(uint32_t n, KParams K, const float4* __restrict__ xs,
                                                            const float4* __restrict__ vin, float4* __restrict__ vout,
                                                            float4* __restrict__ x, const int32_t* __restrict__ cnb,
                                                            const int32_t* __restrict__ cnb_count) {
-  const uint32_t p = xcd_block() * blockDim.x + threadIdx.x;
+  const uint32_t p = particle_of<QUAD>();
   if (p >= n) return;
   const f3 xp = ld3(xs, p);
   const f3 vp = ld3(vin, p);
-  const f3 dv = xsph_sum<false>(cnb, n, 0, cnb_count[p], p, xp, vp, K, xs, vin);
+  f3 dv = {0.f, 0.f, 0.f};
+  walk_compact<QUAD>(
+      cnb, cnb_count[p], p, K, dv, [&](uint32_t at) { return Pair2{gather_at(xs, at), gather_at(vin, at)}; },
+      [&](const Pair2& q) { return xsph_term(xp, vp, q.t, q.w, K); });
+  if (QUAD && (threadIdx.x & 3u) != 0u) return;
   f3 nv = vp;
   acc3(nv, smul3(K.visc, dv));
   st3(vout, p, nv);
@@ -902,72 +1006,107 @@ __global__ void __launch_bounds__(kBlock) k_viscosity_last(uint32_t n, KParams K
 }
 
 // compute_vorticity (particles.h:452-466) -> scr (omega, and |omega| in w)
-template <bool SR>
+template <bool SR, bool QUAD>
 __global__ void __launch_bounds__(kBlock) k_vorticity_c(uint32_t n, KParams K, const float4* __restrict__ xs,
                                                         const float4* __restrict__ vin, float4* __restrict__ scr,
                                                         const int32_t* __restrict__ cnb,
                                                         const int32_t* __restrict__ cnb_count) {
-  const uint32_t p = xcd_block() * blockDim.x + threadIdx.x;
+  const uint32_t p = particle_of<QUAD>();
   if (p >= n) return;
   const f3 xp = ld3(xs, p);
   const f3 vp = ld3(vin, p);
-  const int cnt = cnb_count[p];
   f3 w = {0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < cnt; k0 += kBatch) {
-    uint32_t q[kBatch];
-    load_batch(cnb, K.stride, k0, cnt, p, q);
-    float4 t[kBatch], vq[kBatch];
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      t[u] = gather4(xs, q[u]);
-      vq[u] = gather4(vin, q[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      if (k0 + u >= cnt) continue;
-      const f3 d = sub3(xp, xyz(t[u]));
-      const float r = sqrtf(magsq3(d));
-      acc3(w, cross3(sub3(xyz(vq[u]), vp), nb_spiky<false, SR>(d, r, K)));
-    }
-  }
+  walk_compact<QUAD>(
+      cnb, cnb_count[p], p, K, w, [&](uint32_t at) { return Pair2{gather_at(xs, at), gather_at(vin, at)}; },
+      [&](const Pair2& q) {
+        const f3 d = sub3(xp, xyz(q.t));
+        const float r = sqrt_cr(magsq3(d));
+        return cross3(sub3(xyz(q.w), vp), nb_spiky<false, SR>(d, r, K));
+      });
+  if (QUAD && (threadIdx.x & 3u) != 0u) return;
   scr[p] = make_float4(w.x, w.y, w.z, sqrtf(magsq3(w)));  // |omega| for apply_vorticity's gathers
 }
 
 // apply_vorticity (particles.h:471-487), v in place (own particle only)
-template <bool SR>
+template <bool SR, bool QUAD>
 __global__ void __launch_bounds__(kBlock) k_apply_vorticity_c(uint32_t n, KParams K, const float4* __restrict__ xs,
                                                               const float4* __restrict__ scr,
                                                               float4* __restrict__ v,
                                                               const int32_t* __restrict__ cnb,
                                                               const int32_t* __restrict__ cnb_count) {
-  const uint32_t p = xcd_block() * blockDim.x + threadIdx.x;
+  const uint32_t p = particle_of<QUAD>();
   if (p >= n) return;
   const f3 xp = ld3(xs, p);
-  const int cnt = cnb_count[p];
   f3 eta = {0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < cnt; k0 += kBatch) {
-    uint32_t q[kBatch];
-    load_batch(cnb, K.stride, k0, cnt, p, q);
-    float4 t[kBatch], wq[kBatch];
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      t[u] = gather4(xs, q[u]);
-      wq[u] = gather4(scr, q[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      if (k0 + u >= cnt) continue;
-      const f3 d = sub3(xp, xyz(t[u]));
-      const float r = sqrtf(magsq3(d));
-      const float wm = wq[u].w;  // |omega_q|, computed by the vorticity pass
-      acc3(eta, smul3(wm, nb_spiky<false, SR>(d, r, K)));
-    }
-  }
+  walk_compact<QUAD>(
+      cnb, cnb_count[p], p, K, eta, [&](uint32_t at) { return Pair2{gather_at(xs, at), gather_at(scr, at)}; },
+      [&](const Pair2& q) {
+        const f3 d = sub3(xp, xyz(q.t));
+        const float r = sqrt_cr(magsq3(d));
+        return smul3(q.w.w, nb_spiky<false, SR>(d, r, K));  // |omega_q|, computed by the vorticity pass
+      });
+  if (QUAD && (threadIdx.x & 3u) != 0u) return;
   const f3 N = div3(eta, sqrtf(magsq3(eta)) + K.r_eps);
   const float4 v4 = v[p];
   f3 vp = xyz(v4);
   acc3(vp, mul3(mul3(cross3(N, ld3(scr, p)), K.vort), K.dt));
   v[p] = make_float4(vp.x, vp.y, vp.z, v4.w);  // the density stays in w for the second XSPH pass
+}
+
+// The first XSPH pass by single lanes.  It runs one wavefront per block and stages each lane's
+// compact row in its own LDS column (entry k of the 64 lanes contiguous): its
+// second loop reads it there, and it goes to memory four entries at a time.
+constexpr int kStageBlock = 64;
+__global__ void __launch_bounds__(kStageBlock) k_viscosity_first_lane(
+    uint32_t n, KParams K, const float4* __restrict__ xs, const float4* __restrict__ vin, float4* __restrict__ vout,
+    const int32_t* __restrict__ nbr, const int32_t* __restrict__ nbr_count, int32_t* __restrict__ cnb,
+    int32_t* __restrict__ cnb_count, const unsigned long long* __restrict__ counters,
+    const int32_t* __restrict__ snb, const int32_t* __restrict__ snb_count,
+    unsigned long long* __restrict__ skin_hint) {
+  extern __shared__ uint32_t s_list[];  // [max(cap + 1, stride)][kStageBlock]
+  const uint32_t lane = threadIdx.x;
+  const uint32_t p = xcd_block() * blockDim.x + threadIdx.x;
+  // the next step builds skin lists only if this one's moves kept them usable to the end
+  if (K.skin_mode && blockIdx.x == 0 && lane == 0) *skin_hint = counters[C_DISP_ALL] == 0ull ? 1ull : 0ull;
+  if (p >= n) return;
+  const f3 xp = ld3(xs, p);
+  const float4 v4 = vin[p];
+  const f3 vp = xyz(v4);
+  const bool skin = skin_usable(counters, C_DISP_ALL);
+  const int cnt = skin ? snb_count[p] : nbr_count[p];
+  const int4* __restrict__ row = list_row(skin ? snb : nbr, p, K.stride);
+  int nc = 0;
+  for (int k0 = 0; k0 < cnt; k0 += kBatch) {
+    uint32_t q[kBatch];
+    load_row(row, k0, q);
+    float4 t[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) t[u] = gather4(xs, q[u]);
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      s_list[nc * kStageBlock + lane] = q[u] << 4;  // a rejected entry is overwritten by the next accepted one
+      nc += within_h(magsq3(sub3(xp, xyz(t[u]))), K) ? 1 : 0;
+    }
+  }
+  cnb_count[p] = nc;
+  int4* out = reinterpret_cast<int4*>(cnb + list_at(0, p, K.stride));
+  f3 dv = {0.f, 0.f, 0.f};
+  for (int k0 = 0; k0 < nc; k0 += kBatch) {
+    uint32_t at[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) at[u] = k0 + u < nc ? s_list[(k0 + u) * kStageBlock + lane] : p << 4;
+    out[(k0 / 4) * 64] = make_int4((int)at[0], (int)at[1], (int)at[2], (int)at[3]);
+    out[(k0 / 4 + 1) * 64] = make_int4((int)at[4], (int)at[5], (int)at[6], (int)at[7]);
+    Pair2 q[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) q[u] = Pair2{gather_at(xs, at[u]), gather_at(vin, at[u])};
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+      if (k0 + u < nc) acc3(dv, xsph_term(xp, vp, q[u].t, q[u].w, K));
+  }
+  f3 nv = vp;
+  acc3(nv, smul3(K.visc, dv));
+  vout[p] = make_float4(nv.x, nv.y, nv.z, v4.w);  // the density stays in w
 }
 
 // ---- launchers ----
@@ -981,13 +1120,44 @@ __global__ void __launch_bounds__(kBlock) k_apply_vorticity_c(uint32_t n, KParam
     timer_end((c), t_);                                                                                   \
   } while (0)
 
+// Whether a pass goes by quads or by single lanes (same results).  Quads take
+// a quarter of the steps with four times the wavefronts and pay for their
+// ordered sums with twelve to twenty DPP additions per four pairs, so they win
+// while single lanes leave the chip short of wavefronts (524,288 lanes fill
+// it).  Measured, quads against lanes, us per launch on a dam break at rest:
+//   particles            32,768       131,072      262,144      1,048,576
+//   density              10.7 / 14.3  19.8 / 18.0  30.8 / 25.8  95 / 80
+//   pressure update       9.6 / 15.0  17.1 / 18.1  27.7 / 25.5  91 / 77
+//   first XSPH           11.5 / 18.0  22.5 / 26.8  36.6 / 44.5  188 / 164
+//   vorticity             8.8 / 13.1  15.9 / 17.8  25.8 / 27.1  111 / 96
+//   confinement           8.6 / 13.1  15.3 / 16.3  26.8 / 27.6  87 / 84
+//   second XSPH           9.1 / 15.0  15.3 / 17.1  26.0 / 27.4  86 / 83
+// (lanes overtake between 65,536 and 131,072 particles in the pressure solve,
+// and near 524,288 in the passes after it)
+constexpr uint64_t kQuadsPressure = 98304;
+constexpr uint64_t kQuadsTail = 524288;
+static bool pressure_quads(const pbf_context* c) { return c->n <= kQuadsPressure; }
+static bool tail_quads(const pbf_context* c) { return c->n <= kQuadsTail; }
+
+// four lanes per particle
+#define PBF_LAUNCH_QUADS(c, name, kern, ...)                                                              \
+  do {                                                                                                    \
+    const uint32_t n_ = (uint32_t)(c)->n;                                                                 \
+    if (!n_) return;                                                                                      \
+    KernelTimer* t_ = timer_begin((c), name);                                                             \
+    const uint32_t b_ = (c)->tune.block_size;                                                             \
+    hipLaunchKernelGGL(kern, dim3((n_ + b_ / 4 - 1) / (b_ / 4)), dim3(b_), 0, (c)->stream, n_, __VA_ARGS__); \
+    timer_end((c), t_);                                                                                   \
+  } while (0)
+
 #define PBF_LAUNCH_STAGED(c, name, kern, ...)                                                              \
   do {                                                                                                      \
     const uint32_t n_ = (uint32_t)(c)->n;                                                                   \
     if (!n_) return;                                                                                        \
     KernelTimer* t_ = timer_begin((c), name);                                                               \
     hipLaunchKernelGGL(kern, dim3((n_ + kStageBlock - 1) / kStageBlock), dim3(kStageBlock),                 \
-                       (uint32_t)(kStageBlock * ((c)->K.cap + 1) * sizeof(int32_t)), (c)->stream, n_, __VA_ARGS__); \
+                       (uint32_t)(kStageBlock * std::max((c)->K.cap + 1, (c)->K.stride) * sizeof(uint32_t)), \
+                       (c)->stream, n_, __VA_ARGS__);                                                       \
     timer_end((c), t_);                                                                                     \
   } while (0)
 
@@ -999,44 +1169,41 @@ __global__ void __launch_bounds__(kBlock) k_apply_vorticity_c(uint32_t n, KParam
     else                                                  \
       launch(c, name, (KT<false>), __VA_ARGS__);          \
   } while (0)
-// the same with the static-range instance of the exact arithmetic (KParams::static_ranges)
-#define PBF_LAUNCH_ARITH_SR(launch, c, name, KT, ...)     \
-  do {                                                    \
-    if ((c)->K.fast)                                      \
-      launch(c, name, (KT<true, false>), __VA_ARGS__);    \
-    else if ((c)->K.static_ranges)                        \
-      launch(c, name, (KT<false, true>), __VA_ARGS__);    \
-    else                                                  \
-      launch(c, name, (KT<false, false>), __VA_ARGS__);   \
-  } while (0)
 
-template <int FM>
-static void launch_density_fm(pbf_context* c, const char* name, int it, int eslot, const SolveCtl& S,
+template <int FM, bool FAST, bool SR, bool QUAD>
+static void launch_density_as(pbf_context* c, const char* name, int it, int eslot, const SolveCtl& S,
                               const FeatCtl& F) {
-  if (c->K.fast)
-    PBF_LAUNCH(c, name, (k_density_lambda_c<FM, true, false>), it, eslot, S, F, c->K, (const float4*)c->xs,
-               (const float4*)c->v, c->xt, c->rho, c->lam, (const int32_t*)c->nbr, (const int32_t*)c->nbr_count,
-               c->wmask, c->moved, c->dirty_stamp, c->mflag, c->counters, (const int32_t*)c->snb,
-               (const int32_t*)c->snb_count);
-  else if (c->K.static_ranges)
-    PBF_LAUNCH(c, name, (k_density_lambda_c<FM, false, true>), it, eslot, S, F, c->K, (const float4*)c->xs,
-               (const float4*)c->v, c->xt, c->rho, c->lam, (const int32_t*)c->nbr, (const int32_t*)c->nbr_count,
-               c->wmask, c->moved, c->dirty_stamp, c->mflag, c->counters, (const int32_t*)c->snb,
-               (const int32_t*)c->snb_count);
+  if constexpr (QUAD)
+    PBF_LAUNCH_QUADS(c, name, (k_density_lambda_c<FM, FAST, SR, true>), it, eslot, S, F, c->K, (const float4*)c->xs,
+                     (const float4*)c->v, c->xt, c->rho, c->lam, (const int32_t*)c->nbr,
+                     (const int32_t*)c->nbr_count, c->wmask, c->moved, c->dirty_stamp, c->mflag, c->counters,
+                     (const int32_t*)c->snb, (const int32_t*)c->snb_count);
   else
-    PBF_LAUNCH(c, name, (k_density_lambda_c<FM, false, false>), it, eslot, S, F, c->K, (const float4*)c->xs,
+    PBF_LAUNCH(c, name, (k_density_lambda_c<FM, FAST, SR, false>), it, eslot, S, F, c->K, (const float4*)c->xs,
                (const float4*)c->v, c->xt, c->rho, c->lam, (const int32_t*)c->nbr, (const int32_t*)c->nbr_count,
                c->wmask, c->moved, c->dirty_stamp, c->mflag, c->counters, (const int32_t*)c->snb,
                (const int32_t*)c->snb_count);
 }
 
+template <int FM, bool QUAD>
+static void launch_density_fm(pbf_context* c, const char* name, int it, int eslot, const SolveCtl& S,
+                              const FeatCtl& F) {
+  if (c->K.fast)
+    launch_density_as<FM, true, false, QUAD>(c, name, it, eslot, S, F);
+  else if (c->K.static_ranges)
+    launch_density_as<FM, false, true, QUAD>(c, name, it, eslot, S, F);
+  else
+    launch_density_as<FM, false, false, QUAD>(c, name, it, eslot, S, F);
+}
+
 void launch_density_lambda_masked(pbf_context* c, int it, int eslot, const SolveCtl& S, const FeatCtl& F) {
   if (F.wlam)
-    launch_density_fm<2>(c, "density_warm_network", it, eslot, S, F);
+    launch_density_fm<2, false>(c, "density_warm_network", it, eslot, S, F);
   else if (F.feat)
-    launch_density_fm<1>(c, "density_features", it, eslot, S, F);
+    launch_density_fm<1, false>(c, "density_features", it, eslot, S, F);
   else
-    launch_density_fm<0>(c, "density_lambda", it, eslot, S, F);
+    pressure_quads(c) ? launch_density_fm<0, true>(c, "density_lambda", it, eslot, S, F)
+                      : launch_density_fm<0, false>(c, "density_lambda", it, eslot, S, F);
 }
 
 void launch_mark_dirty(pbf_context* c, int it, const SolveCtl& S) {
@@ -1055,11 +1222,25 @@ void launch_lambda_repair(pbf_context* c, int it, const SolveCtl& S) {
              (const uint32_t*)c->mflag, c->dirty, (const unsigned long long*)c->counters);
 }
 
+#define PBF_DP_ARGS                                                                                              \
+  it, last, c->dirty_stamp, S, c->K, (const float4*)c->xt, (const float4*)c->x, c->xs, c->v, (const int32_t*)c->nbr, \
+      (const int32_t*)c->nbr_count, (const uint64_t*)c->wmask, (const uint32_t*)c->dirty, c->counters,             \
+      (const int32_t*)c->snb, (const int32_t*)c->snb_count, (const float4*)c->xs0, (const float*)c->rho
+template <bool FAST, bool SR>
+static void launch_dp_as(pbf_context* c, int it, int last, const SolveCtl& S) {
+  if (pressure_quads(c))
+    PBF_LAUNCH_QUADS(c, "dp_update", (k_dp_update_c<FAST, SR, true>), PBF_DP_ARGS);
+  else
+    PBF_LAUNCH(c, "dp_update", (k_dp_update_c<FAST, SR, false>), PBF_DP_ARGS);
+}
+
 void launch_dp_update_masked(pbf_context* c, int it, int last, const SolveCtl& S) {
-  PBF_LAUNCH_ARITH_SR(PBF_LAUNCH, c, "dp_update", k_dp_update_c, it, last, c->dirty_stamp, S, c->K, (const float4*)c->xt,
-             (const float4*)c->x, c->xs, c->v, (const int32_t*)c->nbr,
-             (const int32_t*)c->nbr_count, (const uint64_t*)c->wmask, (const uint32_t*)c->dirty, c->counters,
-             (const int32_t*)c->snb, (const int32_t*)c->snb_count, (const float4*)c->xs0, (const float*)c->rho);
+  if (c->K.fast)
+    launch_dp_as<true, false>(c, it, last, S);
+  else if (c->K.static_ranges)
+    launch_dp_as<false, true>(c, it, last, S);
+  else
+    launch_dp_as<false, false>(c, it, last, S);
 }
 
 void launch_warm_retry(pbf_context* c) {
@@ -1113,7 +1294,7 @@ __global__ void __launch_bounds__(kBlock) k_jacobi_persistent(JacobiArgs A) {
     const uint32_t stamp = A.stamp0 + it;
     const int eslot = A.solve ? (int)it + 1 : 0;
     for (uint32_t vb = vb0; vb < vb1; ++vb)
-      density_pass<0, FAST, SR>(vb, vb == 0 && threadIdx.x == 0, A.n, (int)it, eslot, A.S, F0, A.K, A.xs, A.v, A.xt,
+      density_pass<0, FAST, SR, false>(vb, vb == 0 && threadIdx.x == 0, A.n, (int)it, eslot, A.S, F0, A.K, A.xs, A.v, A.xt,
                             A.rho, A.lam, A.nbr, A.nbr_count, A.wmask, A.moved, stamp, A.mflag, A.counters, A.snb,
                             A.snb_count);
     grid.sync();
@@ -1126,7 +1307,7 @@ __global__ void __launch_bounds__(kBlock) k_jacobi_persistent(JacobiArgs A) {
     grid.sync();
     const int last = A.last_vel && it + 1 == A.iters;
     for (uint32_t vb = vb0; vb < vb1; ++vb)
-      dp_pass<FAST, SR>(vb, vb == 0 && threadIdx.x == 0, A.n, (int)it, last, stamp, A.S, A.K, A.xt, A.x, A.xs, A.v,
+      dp_pass<FAST, SR, false>(vb, vb == 0 && threadIdx.x == 0, A.n, (int)it, last, stamp, A.S, A.K, A.xt, A.x, A.xs, A.v,
                     A.nbr, A.nbr_count, A.wmask, A.dirty, A.counters, A.snb, A.snb_count, A.xs0, A.rho);
     grid.sync();
   }
@@ -1223,36 +1404,51 @@ void launch_add_warm(pbf_context* c) {
   PBF_LAUNCH(c, "add_warm", k_add_warm, (const float*)c->wlam, c->lsum, (const unsigned long long*)c->counters);
 }
 
+#define PBF_VISC_ARGS                                                                                          \
+  c->K, (const float4*)c->xs, (const float4*)c->v, c->va, (const int32_t*)c->nbr, (const int32_t*)c->nbr_count, \
+      c->cnb, c->cnb_count, (const unsigned long long*)c->counters, (const int32_t*)c->snb,                     \
+      (const int32_t*)c->snb_count, c->skin_hint
 void launch_viscosity_first(pbf_context* c) {
-  PBF_LAUNCH_STAGED(c, "viscosity", k_viscosity_first, c->K, (const float4*)c->xs,
-             (const float4*)c->v, c->va, (const int32_t*)c->nbr, (const int32_t*)c->nbr_count, c->cnb,
-             c->cnb_count, (const unsigned long long*)c->counters, (const int32_t*)c->snb,
-             (const int32_t*)c->snb_count, c->skin_hint);
+  if (tail_quads(c))
+    PBF_LAUNCH_QUADS(c, "viscosity", k_viscosity_first, PBF_VISC_ARGS);
+  else
+    PBF_LAUNCH_STAGED(c, "viscosity", k_viscosity_first_lane, PBF_VISC_ARGS);
 }
 
 // the vorticity passes stay exact in both arithmetic modes; the static-range
 // instance of the divide where KParams::static_ranges holds
-#define PBF_LAUNCH_SR(c, name, KT, ...)                                     \
+#define PBF_LAUNCH_SR(c, name, KT, Q, ...)                                  \
   do {                                                                      \
-    if ((c)->K.static_ranges)                                               \
-      PBF_LAUNCH(c, name, (KT<true>), __VA_ARGS__);                         \
-    else                                                                    \
-      PBF_LAUNCH(c, name, (KT<false>), __VA_ARGS__);                        \
+    if ((c)->K.static_ranges) {                                             \
+      if (Q)                                                                \
+        PBF_LAUNCH_QUADS(c, name, (KT<true, true>), __VA_ARGS__);           \
+      else                                                                  \
+        PBF_LAUNCH(c, name, (KT<true, false>), __VA_ARGS__);                \
+    } else {                                                                \
+      if (Q)                                                                \
+        PBF_LAUNCH_QUADS(c, name, (KT<false, true>), __VA_ARGS__);          \
+      else                                                                  \
+        PBF_LAUNCH(c, name, (KT<false, false>), __VA_ARGS__);               \
+    }                                                                       \
   } while (0)
 
 void launch_vorticity_masked(pbf_context* c) {
-  PBF_LAUNCH_SR(c, "vorticity", k_vorticity_c, c->K, (const float4*)c->xs, (const float4*)c->va, c->scr,
+  PBF_LAUNCH_SR(c, "vorticity", k_vorticity_c, tail_quads(c), c->K, (const float4*)c->xs, (const float4*)c->va, c->scr,
                 (const int32_t*)c->cnb, (const int32_t*)c->cnb_count);
 }
 
 void launch_apply_vorticity_masked(pbf_context* c) {
-  PBF_LAUNCH_SR(c, "apply_vorticity", k_apply_vorticity_c, c->K, (const float4*)c->xs, (const float4*)c->scr,
-                c->va, (const int32_t*)c->cnb, (const int32_t*)c->cnb_count);
+  PBF_LAUNCH_SR(c, "apply_vorticity", k_apply_vorticity_c, tail_quads(c), c->K, (const float4*)c->xs,
+                (const float4*)c->scr, c->va, (const int32_t*)c->cnb, (const int32_t*)c->cnb_count);
 }
 
+#define PBF_LAST_ARGS \
+  c->K, (const float4*)c->xs, (const float4*)c->va, c->v, c->x, (const int32_t*)c->cnb, (const int32_t*)c->cnb_count
 void launch_viscosity_last(pbf_context* c) {
-  PBF_LAUNCH(c, "viscosity_positions", k_viscosity_last, c->K, (const float4*)c->xs,
-             (const float4*)c->va, c->v, c->x, (const int32_t*)c->cnb, (const int32_t*)c->cnb_count);
+  if (tail_quads(c))
+    PBF_LAUNCH_QUADS(c, "viscosity_positions", k_viscosity_last<true>, PBF_LAST_ARGS);
+  else
+    PBF_LAUNCH(c, "viscosity_positions", k_viscosity_last<false>, PBF_LAST_ARGS);
 }
 
 }  // namespace pbf

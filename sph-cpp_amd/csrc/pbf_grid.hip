@@ -17,7 +17,7 @@
 //
 // Lists.  One lane per particle walks the 27 cells in the reference's order
 // and stages its entries in LDS, then writes them tiled by groups of 64
-// particles (list_at: entry k of a wavefront's 64 particles contiguous).  A
+// particles, four entries at a time (list_at).  A
 // particle with many candidates whose walk passes a budget is handed to a
 // list of heavy particles that one wavefront each finishes with
 // ballot-compacted appends, so that collapsed cells do not serialise a
@@ -148,11 +148,17 @@ __global__ void __launch_bounds__(kBlock) k_bin(const float4* __restrict__ xs, u
                                                 KParams K, const uint32_t* __restrict__ oid,
                                                 uint32_t* __restrict__ key, uint32_t* __restrict__ inv,
                                                 unsigned long long* __restrict__ counters,
-                                                uint32_t* __restrict__ sk, uint32_t* __restrict__ sv) {
+                                                uint32_t* __restrict__ sk, uint32_t* __restrict__ sv,
+                                                unsigned long long* __restrict__ hint) {
   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p == 0) {  // counted by the list build that follows
     counters[C_HEAVY] = 0ull;
     counters[C_TILE] = 0ull;
+    if (hint) {  // per-pass: skin lists if the moves since the last build kept them usable
+      *hint = counters[C_DISP_ALL] == 0ull ? 1ull : 0ull;
+      counters[C_DISP_ALL] = 0ull;
+      counters[C_SKIN] = 0ull;
+    }
   }
   if (p >= n) return;
   const uint32_t o = oid[p];
@@ -168,13 +174,13 @@ __global__ void __launch_bounds__(kBlock) k_bin(const float4* __restrict__ xs, u
   sv[o] = p;
 }
 
-void launch_bin(pbf_context* c, uint64_t bin_end) {
+void launch_bin(pbf_context* c, uint64_t bin_end, bool fused) {
   const uint32_t n = (uint32_t)c->n;
   if (!n) return;
   KernelTimer* t = timer_begin(c, "bin");
   hipLaunchKernelGGL(k_bin, dim3(nblocks(n)), dim3(kBlock), 0, c->stream, (const float4*)c->xs, n,
                      (uint32_t)bin_end, c->K, (const uint32_t*)c->oid, c->key, c->slot, c->counters, c->sk[0],
-                     c->sv[0]);
+                     c->sv[0], fused ? nullptr : c->skin_hint);
   timer_end(c, t);
 }
 
@@ -480,8 +486,9 @@ __device__ __forceinline__ WalkCells walk_cells(f3 ps, float s) {
 
 // One wavefront per block; each lane stages its entries in its own LDS
 // column (entry k of the 64 lanes is contiguous) and writes them out at the
-// end, so that every global store of entry k covers the wavefront's 64
-// consecutive slots instead of 64 scattered 4-byte writes.  A staged entry is
+// end, four entries of a particle in one 16-byte store and those of the
+// wavefront's 64 particles one contiguous kilobyte (ListWriter), instead of
+// 64 scattered 4-byte writes per entry.  A staged entry is
 // 16 bits: the slot's offset in its cell (10 bits), the cell's place in the
 // 27-cell walk (c, 5 bits) and whether the candidate lies within the skin
 // radius (bit 15), which halves the staging and doubles the wavefronts the
@@ -490,14 +497,34 @@ __device__ __forceinline__ WalkCells walk_cells(f3 ps, float s) {
 // otherwise stops after a budget below it.
 //
 // Skin lists (with `skin`): the entries within 1.1 h (K.skin2) of the
-// positions the lists are built from, in list order, each slot packed with
-// its place in the full list (slot | place << 25; n < 2^25); x*_0 = x*.
+// positions the lists are built from, in list order; x*_0 = x*.
 // The Jacobi passes walk them instead of the full lists while no particle has
 // moved far enough for an entry outside them to come within h
 // (pbf_fused.hip).
 constexpr int kFillBlock = 64;
 constexpr uint32_t kMaxCellOffset = 1024u;
-constexpr uint32_t kSkinPlaceShift = 25;
+
+// Appends entries to particle p's list: four of them are one 16-byte store,
+// and close() fills the last batch of eight with the far row, so that a walk
+// loads whole batches without a test.
+struct ListWriter {
+  int4* row;
+  uint32_t pad, count = 0;
+  int4 e;
+  __device__ __forceinline__ ListWriter(int32_t* __restrict__ list, uint32_t p, const KParams& K)
+      : row(reinterpret_cast<int4*>(list + list_at(0, p, (uint32_t)K.stride))), pad(K.pad) {}
+  __device__ __forceinline__ void add(uint32_t slot) {
+    e = make_int4(e.y, e.z, e.w, (int)slot);
+    if ((++count & 3u) == 0u) row[(count / 4u - 1u) * 64u] = e;
+  }
+  __device__ __forceinline__ void close() {
+    uint32_t k = count;
+    while (k & 7u) {
+      e = make_int4(e.y, e.z, e.w, (int)pad);
+      if ((++k & 3u) == 0u) row[(k / 4u - 1u) * 64u] = e;
+    }
+  }
+};
 
 // The lane walk of particle p: writes its list and count and returns true,
 // or returns false when the particle goes to the wavefront builder.  ovf
@@ -578,7 +605,8 @@ done:
   nbr_count[p] = count;
   // staged entries come in walk order, so the cells' first slots are taken
   // from registers cell by cell
-  int k = 0, j = 0;
+  ListWriter full(nbr, p, K), near(snb, p, K);
+  int k = 0;
 #pragma unroll
   for (int c = 0; c < 27; ++c) {
     const uint32_t b = cb[c];
@@ -586,11 +614,15 @@ done:
       const uint32_t e16 = s_list[k * kFillBlock + lane];
       if (((e16 >> 10) & 31u) != (uint32_t)c) break;
       const uint32_t slot = b + (e16 & (kMaxCellOffset - 1u));
-      nbr[list_at(k, p, K.stride)] = (int32_t)slot;
-      if (SKIN && (e16 >> 15)) snb[list_at(j++, p, K.stride)] = (int32_t)(slot | ((uint32_t)k << kSkinPlaceShift));
+      full.add(slot);
+      if (SKIN && (e16 >> 15)) near.add(slot);
     }
   }
-  if (SKIN) snb_count[p] = j;
+  full.close();
+  if (SKIN) {
+    near.close();
+    snb_count[p] = (int32_t)near.count;
+  }
   return true;
 }
 
@@ -797,7 +829,7 @@ __device__ __forceinline__ bool tile_walk(uint32_t tb, uint32_t lane, uint32_t n
   nbr_count[p] = (int32_t)k;
   // flush: stream positions to slots, cell by cell
   uint32_t c = 0, co = 0, nxt = s_off[base + 1], cs = s_tab[base];
-  int js = 0;
+  ListWriter full(nbr, p, K), near(snb, p, K);
   for (uint32_t e = 0; e < k; ++e) {
     const uint32_t e16 = s_list[e * kFillBlock + lane];
     const uint32_t j = e16 & 1023u;
@@ -808,10 +840,14 @@ __device__ __forceinline__ bool tile_walk(uint32_t tb, uint32_t lane, uint32_t n
       nxt = s_off[base + c + 1];
     }
     const uint32_t slot = cs + (j - co);
-    nbr[list_at(e, p, K.stride)] = (int32_t)slot;
-    if (SKIN && (e16 >> 15)) snb[list_at(js++, p, K.stride)] = (int32_t)(slot | (e << kSkinPlaceShift));
+    full.add(slot);
+    if (SKIN && (e16 >> 15)) near.add(slot);
   }
-  if (SKIN) snb_count[p] = js;
+  full.close();
+  if (SKIN) {
+    near.close();
+    snb_count[p] = (int32_t)near.count;
+  }
   return true;
 }
 
@@ -901,7 +937,7 @@ __device__ __forceinline__ bool take_group(uint32_t q, bool valid, float4 t, f3 
     const bool in = acc && pos < cap && d2 < K.skin2;
     const uint64_t ms = __ballot(in);
     if (in)
-      snb[list_at(scount + (uint32_t)__popcll(ms & below), p, K.stride)] = (int32_t)(q | (pos << kSkinPlaceShift));
+      snb[list_at(scount + (uint32_t)__popcll(ms & below), p, K.stride)] = (int32_t)q;
     scount += (uint32_t)__popcll(ms);
   }
   count += (uint32_t)__popcll(m);
@@ -991,21 +1027,24 @@ __global__ void __launch_bounds__(kBlock) k_fill_heavy(uint32_t n, const float4*
       }
     }
   done:
+    // the last batch of eight is filled with the far row
+    const uint32_t kept = count < cap ? count : cap;
+    if (lane < (8u - (kept & 7u)) % 8u) nbr[list_at(kept + lane, p, K.stride)] = (int32_t)K.pad;
+    if (skin && lane < (8u - (scount & 7u)) % 8u) snb[list_at(scount + lane, p, K.stride)] = (int32_t)K.pad;
     if (lane == 0) {
-      nbr_count[p] = (int32_t)(count < cap ? count : cap);
+      nbr_count[p] = (int32_t)kept;
       if (skin) snb_count[p] = (int32_t)scount;
       if (count > cap && K.count_overflow) atomicAdd(&counters[C_OVERFLOW], (unsigned long long)(count - cap));
     }
   }
 }
 
-void launch_fill_neighbors(pbf_context* c, uint64_t fb, uint64_t fe, bool want_skin) {
+void launch_fill_neighbors(pbf_context* c, uint64_t fb, uint64_t fe) {
   const uint32_t n = (uint32_t)c->n;
   if (!n) return;
-  // skin lists for the fused step (their packed form needs slots below 2^25);
-  // x*_0 is kept whenever they may be used, the lists themselves when the
+  // x*_0 is kept whenever skin lists may be used, the lists themselves when the
   // previous step's moves stayed below their limit (c->skin_hint)
-  const int skin = want_skin && c->K.skin_mode && c->n < (1ull << kSkinPlaceShift);
+  const int skin = c->K.skin_mode;
   KernelTimer* t = timer_begin(c, "fill_neighbors");
   // the staging area holds a wavefront's lists, or the cell-tile walk's stream of slots
   const uint32_t stage = std::max<uint32_t>(kFillBlock * (c->K.cap + 1) * sizeof(uint16_t),

@@ -16,15 +16,17 @@
 //   cell_start       uint32[C+2] first sorted slot of every cell (C = the outside bucket)
 //   heavy            uint32[n]   particles whose 27 cells hold too many candidates
 //                                for one lane (built by a whole wavefront instead)
-//   nbr              int32[n/64][K][64] neighbour lists tiled by groups of 64 particles:
-//                                nbr[list_at(k, p, K)] (entry k of a wavefront's 64 particles
-//                                is one contiguous 256-byte read, its whole list one block)
+//   nbr              int32[n/64][K/4][64][4] neighbour lists tiled by groups of 64 particles:
+//                                nbr[list_at(k, p, K)] (entries 4j .. 4j+3 of a particle are one
+//                                16-byte load, a wavefront's one contiguous kilobyte, its whole
+//                                list one block); padded with the far row to a multiple of 8
 //   nbr_count        int32[n]
-//   cnb, cnb_count   int32[n/64][K][64], int32[n]  compact lists of the entries within h
-//                                (same tiling; built by the first XSPH pass)
-//   snb, snb_count   int32[n/64][K][64], int32[n]  skin lists: the entries within 1.1 h of the
-//                                positions the lists were built from (xs0), in list order, each
-//                                slot packed with its place in the full list (bits 25-31)
+//   cnb, cnb_count   compact lists of the entries within h (same tiling; built by the first
+//                                XSPH pass)
+//   snb, snb_count   skin lists: the entries within 1.1 h of the positions the lists were built
+//                                from (xs0), in list order (same tiling and padding)
+//   far row          row `capacity` of the position stars (xs, xsa, xt) holds +inf: a padding
+//                                entry of a list reads it and lies outside every radius
 //   counters         u64[16]     overflow, outside, hacks, hack flags, solve state, ...
 //   ehist            uint32[kMaxSolveSlots+1]  max density error per solve slot (float bits)
 //   lsum, lsuma      float[n]    multipliers summed over the updates of the last solve
@@ -66,6 +68,7 @@ struct KParams {
   float eps, visc, vort, gamma;
   double vthr;                   // 0.000001 * max_speed (particles.h:380), in double
   double st_rmin;                // h * 0.000001 (particles.h:420), in double
+  float st_rmin_float;           // smallest float r with (double)r >= st_rmin
   float bmin[3], bmax[3], mover[3];
   uint32_t dimx, dimy, dimz;
   uint32_t ncells;
@@ -79,6 +82,7 @@ struct KParams {
   int tile_lists;                // the cell-tile list walk (no PBF_OPT_LANE_LISTS)
   int fast;                      // PBF_OPT_FAST_MATH: hardware sqrt and reciprocal in the fused step
   int static_ranges;             // the exact sums' range tests hold for every accepted pair (nb_sqrt, nb_spiky)
+  uint32_t pad;                  // the far row (the capacity): what the lists are padded with
   uint32_t heavy_budget;         // candidates one lane scans before a wavefront takes over (see walk_list)
   // batched scenes: ncells is the total over the scenes, sid the scene of each slot
   int batched;
@@ -143,13 +147,18 @@ struct FeatCtl {
   float* wlam;          // null: no network in this pass
 };
 
-// Neighbour lists are tiled by groups of 64 particles: entry k of particle p
-// sits at ((p / 64) * stride + k) * 64 + p % 64.  Entry k of a wavefront's 64
-// particles is one 256-byte read, and a wavefront's whole list is one
-// contiguous block of stride * 256 bytes.
+// Neighbour lists are tiled by groups of 64 particles, four entries of a
+// particle together: entry k of particle p sits at
+// ((p / 64) * stride + k - k % 4) * 64 + (p % 64) * 4 + k % 4.  Four entries
+// are one 16-byte load, those of a wavefront's 64 particles one contiguous
+// kilobyte, and a wavefront's whole list one contiguous block of stride * 256
+// bytes.
 __host__ __device__ __forceinline__ uint64_t list_at(uint32_t k, uint32_t p, uint32_t stride) {
-  return ((uint64_t)(p >> 6) * stride + k) * 64u + (p & 63u);
+  return ((uint64_t)(p >> 6) * stride + (k & ~3u)) * 64u + (p & 63u) * 4u + (k & 3u);
 }
+// entries of the lists of `capacity` particles, with one more batch of eight
+// rows that a walk may load ahead
+inline uint64_t list_size(uint64_t capacity, uint64_t stride) { return ((capacity + 63) / 64 * stride + 8) * 64; }
 
 struct KernelTimer {
   std::string name;
@@ -200,8 +209,11 @@ struct pbf_context {
   int32_t *cnb = nullptr, *cnb_count = nullptr;
   int32_t *snb = nullptr, *snb_count = nullptr;  // skin lists (entries within 1.1 h when built)
   float4* xs0 = nullptr;                          // position stars the lists were built from
+  // the per-pass entry points may walk the skin lists: pbf_find_neighbors built
+  // them and only passes that check their moves have written x* since
+  bool pass_skin = false;
   unsigned long long* skin_hint = nullptr;  // 1: the last step's moves kept the skin lists usable
-  uint64_t* wmask = nullptr;  // [2][n] within-h masks of the last fused density pass
+  uint64_t* wmask = nullptr;  // [2][n] within-h masks of the last fused density pass by single lanes
   unsigned long long* counters = nullptr;
   uint32_t* ehist = nullptr;
   unsigned long long* esum = nullptr;
@@ -276,7 +288,8 @@ void launch_fill_u64(unsigned long long* p, unsigned long long value, uint64_t n
 // exclusive scan of in[0..n) into out[0..n]; out[n] = total.  partials needs scan_partials_size(n).
 uint64_t scan_partials_size(uint64_t n);
 void launch_exclusive_scan(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* partials, hipStream_t s);
-void launch_bin(pbf_context* c, uint64_t bin_end);  // key, inverse permutation, keys by original index
+// fused: part of a fused step (its counters are clear and its hint set)
+void launch_bin(pbf_context* c, uint64_t bin_end, bool fused);  // key, inverse permutation, keys by original index
 void launch_sort(pbf_context* c);            // radix sort -> perm, cell_start
 void launch_cell_box(pbf_context* c);        // bounding box of each cell's particles
 // gather state by perm (without all_fields: densities, multipliers and the
@@ -285,7 +298,7 @@ void launch_reorder(pbf_context* c, bool all_fields = true);
 uint64_t radix_hist_size(uint64_t n);
 int radix_sort_pairs(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, uint64_t n, uint32_t key_bits,
                      uint32_t* hist, uint32_t* offs, uint32_t* partials, hipStream_t s);
-void launch_fill_neighbors(pbf_context* c, uint64_t fb, uint64_t fe, bool want_skin);
+void launch_fill_neighbors(pbf_context* c, uint64_t fb, uint64_t fe);
 int radix_sort_u32(uint32_t* keys, uint32_t* vals, uint64_t n, uint32_t key_bits, hipStream_t s);
 void launch_bounds_counting(const uint32_t* sorted, uint64_t n, uint64_t b, uint64_t e, uint32_t* out,
                             int upper, hipStream_t s);
@@ -319,11 +332,11 @@ void launch_dp(pbf_context* c, uint64_t b, uint64_t e);                     // x
 void launch_update_position_stars(pbf_context* c, uint64_t b, uint64_t e);
 void launch_update_velocities(pbf_context* c, uint64_t b, uint64_t e);
 void launch_update_positions(pbf_context* c, uint64_t b, uint64_t e);
-void launch_viscosity(pbf_context* c, const float4* vin, float4* vout, int write_positions, uint64_t b,
-                      uint64_t e);
+void launch_viscosity(pbf_context* c, const float4* vin, float4* vout, uint64_t b, uint64_t e);
 void launch_vorticity(pbf_context* c, const float4* vin, uint64_t b, uint64_t e);
 void launch_apply_vorticity(pbf_context* c, float4* vio, uint64_t b, uint64_t e);
-void launch_surface_tension(pbf_context* c, uint64_t cb, uint64_t ce, uint64_t b, uint64_t e);
+// skin: the colour field may walk the skin lists
+void launch_surface_tension(pbf_context* c, uint64_t cb, uint64_t ce, uint64_t b, uint64_t e, bool skin);
 void launch_copy_f4(const float4* src, float4* dst, uint64_t n, hipStream_t s);
 void launch_copy_f1(const float* src, float* dst, uint64_t n, hipStream_t s);
 void launch_scale_f1(const float* src, float* dst, float scale, uint64_t n, hipStream_t s);

@@ -238,10 +238,13 @@ static int alloc_grid(pbf_context* c) {
   if (need <= c->grid_alloc) return PBF_OK;
   dfree(c->cell_start);
   dfree(c->cbox);
+  dfree(c->cstamp);
   c->cell_start = nullptr;
   c->cbox = nullptr;
+  c->cstamp = nullptr;
   int rc;
-  if ((rc = dalloc(&c->cell_start, need)) || (rc = dalloc(&c->cbox, 6 * need))) return rc;
+  if ((rc = dalloc(&c->cell_start, need)) || (rc = dalloc(&c->cbox, 6 * need)) || (rc = dalloc(&c->cstamp, need)))
+    return rc;
   c->grid_alloc = need;
   return PBF_OK;
 }
@@ -251,7 +254,7 @@ static void free_all(pbf_context* c) {
                   c->scra, c->rho,  c->lam,  c->rhoa, c->lama, c->oid,  c->oida,       c->key,
                   c->keya, c->slot, c->tmp,  c->tmpo, c->nbr,  c->nbr_count, c->counters, c->stage,
                   c->stage64, c->cell_start, c->scan_partials, c->sk[0], c->sk[1], c->sv[0], c->sv[1],
-                  c->rhist, c->roffs, c->rpart, c->heavy, c->cnb, c->cnb_count, c->moved, c->dirty,
+                  c->rhist, c->roffs, c->rpart, c->heavy, c->cnb, c->cnb_count, c->cstamp, c->dirty, c->ehist_row, c->esum_row,
                   c->ehist, c->lsum, c->lsuma, c->wlam, c->wgiven, c->xsave, c->esum, c->feat, c->mw1,
                   c->mw2, c->mp, c->scenes, c->sid, c->sida, c->cbox, c->chbox, c->wmask, c->mflag,
                   c->slog, c->slog_count, c->snb, c->snb_count, c->xs0, c->skin_hint};
@@ -398,6 +401,7 @@ int pbf_create(const pbf_params* params, pbf_context** out) {
     return rc;
   }
   const uint64_t N = c->capacity;
+  const uint64_t kErrWords = ((uint64_t)kMaxSolveSlots + 1) * kErrShards;
   // position buffers carry kRowPad rows of padding: the neighbour walk loads
   // candidates 8 at a time past the end of a cell's range
   const uint64_t NP = N + kRowPad;
@@ -419,10 +423,11 @@ int pbf_create(const pbf_params* params, pbf_context** out) {
       (rc = dalloc(&c->cnb, list_size(N, c->K.stride))) || (rc = dalloc(&c->cnb_count, N)) ||
       (rc = dalloc(&c->snb, list_size(N, c->K.stride))) || (rc = dalloc(&c->snb_count, N)) ||
       (rc = dalloc(&c->xs0, NP)) || (rc = dalloc(&c->skin_hint, 1)) ||
-      (rc = dalloc(&c->moved, N)) || (rc = dalloc(&c->dirty, N)) || (rc = dalloc(&c->mflag, N)) ||
-      (rc = dalloc(&c->ehist, (uint64_t)kMaxSolveSlots + 1)) || (rc = dalloc(&c->lsum, N)) ||
+      (rc = dalloc(&c->dirty, N)) || (rc = dalloc(&c->mflag, N)) ||
+      (rc = dalloc(&c->ehist, kErrWords)) || (rc = dalloc(&c->ehist_row, (uint64_t)kMaxSolveSlots + 1)) ||
+      (rc = dalloc(&c->esum_row, (uint64_t)kMaxSolveSlots + 1)) || (rc = dalloc(&c->lsum, N)) ||
       (rc = dalloc(&c->lsuma, N)) || (rc = dalloc(&c->wlam, N)) || (rc = dalloc(&c->wgiven, N)) ||
-      (rc = dalloc(&c->xsave, N)) || (rc = dalloc(&c->esum, (uint64_t)kMaxSolveSlots + 1)) ||
+      (rc = dalloc(&c->xsave, N)) || (rc = dalloc(&c->esum, kErrWords)) ||
       (rc = dalloc(&c->feat, N * PBF_WARM_FEATURES)) || (rc = dalloc(&c->mw1, (uint64_t)PBF_WARM_HIDDEN * 16)) ||
       (rc = dalloc(&c->mw2, (uint64_t)PBF_WARM_HIDDEN * PBF_WARM_HIDDEN)) ||
       (rc = dalloc(&c->mp, (uint64_t)PBF_WARM_PARAMS)) ||
@@ -445,8 +450,8 @@ int pbf_create(const pbf_params* params, pbf_context** out) {
   launch_fill_u32(c->dirty, 0u, N, c->stream);
   launch_fill_u32(c->mflag, 0u, N, c->stream);
   launch_fill_u32((uint32_t*)c->lsum, 0u, N, c->stream);
-  launch_fill_u32(c->ehist, 0u, (uint64_t)kMaxSolveSlots + 1, c->stream);
-  launch_fill_u64(c->esum, 0ull, (uint64_t)kMaxSolveSlots + 1, c->stream);
+  launch_fill_u32(c->ehist, 0u, kErrWords, c->stream);
+  launch_fill_u64(c->esum, 0ull, kErrWords, c->stream);
   launch_fill_u64(c->slog_count, 0ull, 1, c->stream);
   launch_fill_u64(c->skin_hint, 1ull, 1, c->stream);
   if ((rc = check_hip(hipStreamSynchronize(c->stream), "pbf_create"))) {
@@ -850,8 +855,7 @@ static void step_body(pbf_context* c) {
     else for (uint32_t it = 0; it < I; ++it) {
       ++c->dirty_stamp;
       launch_density_lambda_masked(c, (int)it, 0, S);       // xs -> xt, rho, lam, compact lists
-      launch_mark_dirty(c, (int)it, S);                     // only if the density fix fired
-      launch_lambda_repair(c, (int)it, S);
+      launch_lambda_repair(c, (int)it, S);                  // only if the density fix fired
       launch_dp_update_masked(c, (int)it, it + 1 == I, S);  // xt, lam -> xs (+ v)
     }
     if (I == 0) launch_update_velocities(c, 0, n);
@@ -943,8 +947,8 @@ static int solve_body(pbf_context* c, float tolerance, uint32_t max_iterations, 
   }
   launch_fill_u64(c->counters + C_ITERS, (unsigned long long)max_iterations, 1, c->stream);
   launch_fill_u64(c->counters + C_WARM_KEPT, (unsigned long long)warm, 1, c->stream);
-  launch_fill_u32(c->ehist, 0u, (uint64_t)max_iterations + 1, c->stream);
-  launch_fill_u64(c->esum, 0ull, (uint64_t)max_iterations + 1, c->stream);
+  launch_fill_u32(c->ehist, 0u, ((uint64_t)max_iterations + 1) * kErrShards, c->stream);
+  launch_fill_u64(c->esum, 0ull, ((uint64_t)max_iterations + 1) * kErrShards, c->stream);
   launch_forces_predict(c, F_FORCES | F_PREDICT, 0, n);
   find_neighbors_impl(c, n, 0, n, true);  // carries the previous sums to the new order
   // lsuma: the previous sums; lsum: this solve's
@@ -983,7 +987,6 @@ static int solve_body(pbf_context* c, float tolerance, uint32_t max_iterations, 
   else for (uint32_t it = 0; it < max_iterations; ++it) {
     ++c->dirty_stamp;
     launch_density_lambda_masked(c, (int)it, (int)it + 1, S);
-    launch_mark_dirty(c, (int)it, S);
     launch_lambda_repair(c, (int)it, S);
     launch_dp_update_masked(c, (int)it, 0, S);
     if (retry && it == 0) launch_warm_retry(c);  // (does nothing unless slot 0 rejected the warm start)
@@ -1161,10 +1164,11 @@ int pbf_get_solve_info(pbf_context* c, pbf_solve_info* out) {
   static_assert(kMaxSolveSlots + 1 <= 1024, "history size");
   uint32_t e[kMaxSolveSlots + 1];
   unsigned long long es[kMaxSolveSlots + 1];
+  launch_combine_errors(c);
   int rc = check_hip(hipMemcpyAsync(h, c->counters, sizeof(h), hipMemcpyDeviceToHost, c->stream), "solve info");
   if (rc) return rc;
-  if ((rc = check_hip(hipMemcpyAsync(e, c->ehist, sizeof(e), hipMemcpyDeviceToHost, c->stream), "solve info")) ||
-      (rc = check_hip(hipMemcpyAsync(es, c->esum, sizeof(es), hipMemcpyDeviceToHost, c->stream), "solve info")))
+  if ((rc = check_hip(hipMemcpyAsync(e, c->ehist_row, sizeof(e), hipMemcpyDeviceToHost, c->stream), "solve info")) ||
+      (rc = check_hip(hipMemcpyAsync(es, c->esum_row, sizeof(es), hipMemcpyDeviceToHost, c->stream), "solve info")))
     return rc;
   if ((rc = check_hip(hipStreamSynchronize(c->stream), "solve info"))) return rc;
   std::memset(out, 0, sizeof(*out));

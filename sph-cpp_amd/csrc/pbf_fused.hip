@@ -267,10 +267,10 @@ __device__ __forceinline__ unsigned long long fixed_error(float e) {
   return (unsigned long long)(fminf(e, 2147483648.0f) * 4294967296.0f);
 }
 
-// One block = one wavefront.  With S.ehist, the block's largest density
-// error goes into slot eslot (atomicMax on the bits of a non-negative float
-// orders like the float) and its fixed-point sum into S.esum[eslot].  With
-// S.tol >= 0 nothing runs once the solve is done.
+// With S.ehist, a wavefront's largest density error goes into a shard of row
+// eslot (atomicMax on the bits of a non-negative float orders like the float)
+// and its fixed-point sum into the same shard of S.esum.  With S.tol >= 0
+// nothing runs once the solve is done.
 // The learned warm start for one wavefront's 64 particles (every lane of the
 // wavefront calls it; fo holds the lane's features, zero past n): the
 // features go through LDS into the B operands of the network, which runs on
@@ -300,6 +300,44 @@ __device__ __forceinline__ void warm_network(const FeatCtl& F, uint32_t wave_fir
   }
 }
 
+// A particle is dirty when it or a particle in its list was moved by the
+// density fix: its fused lambda and its within-h mask may be stale.  A list
+// walk visits cells computed from floating-point coordinates (x + i*s,
+// neighbors.h:177-179), which lie within two cells of the particle's own cell
+// on every axis, so every particle that can list q sits within two cells of
+// q's cell: the wavefront that moved q stamps those 5x5x5 cells, and
+// lambda_repair takes every particle of a stamped cell.  Past kMaxMovedMarked
+// moved particles it scans the lists for moved ones instead (there the stamped
+// cells would hold nearly everything).  (Stamping cells, two stores a lane,
+// needs no launch of its own; stamping their particles took one, 4.5 us an
+// iteration also when nothing had moved.)
+constexpr uint32_t kMaxMovedMarked = 4096;
+__device__ __forceinline__ void stamp_cells(uint64_t movers, uint32_t p, uint32_t stamp, const KParams& K,
+                                            const uint32_t* __restrict__ key, uint32_t* __restrict__ cstamp) {
+  const uint32_t lane = threadIdx.x & 63;
+  while (movers != 0ull) {
+    const uint32_t i = (uint32_t)__builtin_ctzll(movers);
+    movers &= movers - 1ull;
+    const uint32_t q = (uint32_t)__builtin_amdgcn_readlane((int)p, (int)i);
+    const uint32_t kq = key[q];
+    if (kq >= K.ncells) {  // outside the grid: nobody lists it
+      if (lane == 0) cstamp[K.ncells] = stamp;
+      continue;
+    }
+    // cell coordinates in the moved particle's own grid (its scene's); a grid
+    // has fewer than 2^32 cells, so its layers do too
+    const GridView G = grid_of(K, q);
+    const uint32_t dxy = (uint32_t)G.dxy, lq = kq - G.off;
+    const int cz = (int)(lq / dxy), rest = (int)(lq % dxy);
+    const int cy = rest / (int)G.dimx, cx = rest % (int)G.dimx;
+    for (int j = (int)lane; j < 125; j += 64) {
+      const int z = cz - 2 + j / 25, y = cy - 2 + j / 5 % 5, x = cx - 2 + j % 5;
+      if (z >= 0 && z < (int)G.dimz && y >= 0 && y < (int)G.dimy && x >= 0 && x < (int)G.dimx)
+        cstamp[G.off + (uint32_t)z * dxy + (uint32_t)y * G.dimx + (uint32_t)x] = stamp;
+    }
+  }
+}
+
 // FM = 0: density and lambda only; 1: also the warm start's features (stored
 // when F.feat is set); 2: also the network on them (F.wlam).  FAST: the
 // PBF_OPT_FAST_MATH arithmetic.
@@ -317,7 +355,8 @@ __device__ __forceinline__ void density_pass(uint32_t vb, bool first, uint32_t n
                                              const int32_t* __restrict__ nbr,
                                              const int32_t* __restrict__ nbr_count,
                                              uint64_t* __restrict__ wmask,
-                                             uint32_t* __restrict__ moved, uint32_t stamp,
+                                             const uint32_t* __restrict__ key,
+                                             uint32_t* __restrict__ cstamp, uint32_t stamp,
                                              uint32_t* __restrict__ mflag,
                                              unsigned long long* __restrict__ counters,
                                              const int32_t* __restrict__ snb,
@@ -359,17 +398,16 @@ __device__ __forceinline__ void density_pass(uint32_t vb, bool first, uint32_t n
       atomicExch(&counters[C_HACK_FLAG + (it & 1)], 1ull);
     }
     base = __shfl(base, 0, 64);
-    if (hacks) {
-      moved[base + (unsigned long long)__popcll(hm & ((1ull << wl) - 1ull))] = p;
-      mflag[p] = stamp;
-    }
+    if (hacks) mflag[p] = stamp;
+    if (base < kMaxMovedMarked) stamp_cells(hm, p, stamp, K, key, cstamp);
   }
   if (S.ehist) {
     const unsigned long long es = wave_sum(fixed_error(e));
     e = wave_max(e);
+    const uint32_t row = (uint32_t)eslot * kErrShards + ((vb * blockDim.x + threadIdx.x) >> 6) % kErrShards;
     if ((threadIdx.x & 63) == 0) {
-      if (e > 0.0f) atomicMax(&S.ehist[eslot], __float_as_uint(e));
-      if (es) atomicAdd(&S.esum[eslot], es);
+      if (e > 0.0f) atomicMax(&S.ehist[row], __float_as_uint(e));
+      if (es) atomicAdd(&S.esum[row], es);
     }
   }
 }
@@ -384,91 +422,23 @@ k_density_lambda_c(uint32_t n, int it, int eslot, SolveCtl S, FeatCtl F,
                    const int32_t* __restrict__ nbr,
                    const int32_t* __restrict__ nbr_count,
                    uint64_t* __restrict__ wmask,
-                   uint32_t* __restrict__ moved, uint32_t stamp,
+                   const uint32_t* __restrict__ key,
+                   uint32_t* __restrict__ cstamp, uint32_t stamp,
                    uint32_t* __restrict__ mflag,
                    unsigned long long* __restrict__ counters,
                    const int32_t* __restrict__ snb,
                    const int32_t* __restrict__ snb_count) {
   density_pass<FM, FAST, SR, QUAD>(xcd_block(), blockIdx.x == 0 && threadIdx.x == 0, n, it, eslot, S, F, K, xs, v, xt, rho,
-                         lam, nbr, nbr_count, wmask, moved, stamp, mflag, counters, snb, snb_count);
-}
-
-// A particle is dirty when it or a particle in its list was moved by the
-// density fix: its fused lambda and its within-h mask may be stale.  A list
-// walk visits cells computed from floating-point coordinates (x + i*s,
-// neighbors.h:177-179), which lie within two cells of the particle's own cell
-// on every axis, so every particle that can list q sits within two cells of
-// q's cell: all particles of those 5x5x5 cells are marked, one wavefront per
-// moved particle (lanes 0..24 find the 25 rows of cells, then the wavefront
-// stamps each row's slot range).  Many moved particles, or a crowded
-// neighbourhood, leave the work to lambda_repair's exact scan instead.
-constexpr uint32_t kMaxMovedMarked = 4096;
-constexpr uint32_t kMaxMarkedPerMoved = 8192;
-constexpr uint32_t kMarkBlocks = 64;
-
-// (wave, nwaves: the calling wavefront among all wavefronts that share the pass)
-__device__ __forceinline__ void mark_pass(uint32_t wave, uint32_t nwaves, bool first, int it, uint32_t stamp,
-                                          const SolveCtl& S, const KParams& K, const uint32_t* __restrict__ key,
-                                          const uint32_t* __restrict__ start, const uint32_t* __restrict__ moved,
-                                          uint32_t* __restrict__ dirty, unsigned long long* __restrict__ counters) {
-  if (S.tol >= 0.0f && counters[C_DONE] != 0ull) return;
-  const uint32_t nmoved = (uint32_t)counters[C_MOVED_N + (it & 1)];
-  if (nmoved > kMaxMovedMarked) {
-    if (first) counters[C_MOVED_ALL + (it & 1)] = 1ull;
-    return;
-  }
-  const uint32_t lane = threadIdx.x & 63;
-  for (uint32_t i = wave; i < nmoved; i += nwaves) {
-    const uint32_t q = moved[i];
-    const uint32_t kq = key[q];
-    if (kq >= K.ncells) {  // outside the grid: no cell to start from
-      if (lane == 0) counters[C_MOVED_ALL + (it & 1)] = 1ull;
-      continue;
-    }
-    // cell coordinates in the moved particle's own grid (its scene's)
-    const GridView G = grid_of(K, q);
-    const uint32_t lq = kq - G.off;
-    const int cz = (int)(lq / G.dxy), cy = (int)((lq % G.dxy) / G.dimx), cx = (int)(lq % G.dimx);
-    uint32_t rb = 0, re = 0;
-    if (lane < 25) {
-      const int z = cz - 2 + (int)lane / 5, y = cy - 2 + (int)lane % 5;
-      if (z >= 0 && z < (int)G.dimz && y >= 0 && y < (int)G.dimy) {
-        const uint64_t row = G.off + (uint64_t)z * G.dxy + (uint64_t)y * G.dimx;
-        rb = start[row + max(cx - 2, 0)];
-        re = start[row + min(cx + 2, (int)G.dimx - 1) + 1];
-      }
-    }
-    uint32_t total = re - rb;
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) total += __shfl_xor(total, d, 64);
-    if (total > kMaxMarkedPerMoved) {  // crowded neighbourhood: leave it to the exact scan
-      if (lane == 0) counters[C_MOVED_ALL + (it & 1)] = 1ull;
-      continue;
-    }
-    for (int r = 0; r < 25; ++r) {
-      const uint32_t b = __shfl(rb, r, 64), e = __shfl(re, r, 64);
-      for (uint32_t t = b + lane; t < e; t += 64) dirty[t] = stamp;
-    }
-  }
-}
-
-__global__ void __launch_bounds__(kBlock) k_mark_dirty(int it, uint32_t stamp, SolveCtl S, KParams K,
-                                                       const uint32_t* __restrict__ key,
-                                                       const uint32_t* __restrict__ start,
-                                                       const uint32_t* __restrict__ moved,
-                                                       uint32_t* __restrict__ dirty,
-                                                       unsigned long long* __restrict__ counters) {
-  mark_pass((blockIdx.x * blockDim.x + threadIdx.x) >> 6, (gridDim.x * blockDim.x) >> 6,
-            blockIdx.x == 0 && threadIdx.x == 0, it, stamp, S, K, key, start, moved, dirty, counters);
+                         lam, nbr, nbr_count, wmask, key, cstamp, stamp, mflag, counters, snb, snb_count);
 }
 
 // compute_pressure_lambdas (particles.h:318-342) from xt for the dirty
 // particles of this iteration (plain walks).  The new lambda goes to lam and
 // to the particle's xt.w; positions are read as three words, so no lane reads
-// the w word that another lane writes.  When k_mark_dirty left the marking
-// (many moved particles or a crowded neighbourhood), a particle is dirty
-// exactly when it or an entry of its list carries this iteration's moved
-// stamp; this pass finds those and stamps them in dirty for the dp pass.
+// the w word that another lane writes.  Dirty are the particles of the stamped
+// cells, or with many moved particles exactly those that carry this
+// iteration's moved stamp or list one that does; they are stamped in dirty for
+// the dp pass.
 __device__ __forceinline__ f3 ld3_words(const float4* a, uint32_t i) {
   const float* f = reinterpret_cast<const float*>(a + i);
   return {f[0], f[1], f[2]};
@@ -481,11 +451,12 @@ __device__ __forceinline__ void repair_pass(uint32_t vb, uint32_t n, int it, uin
                                             const int32_t* __restrict__ nbr,
                                             const int32_t* __restrict__ nbr_count,
                                             const uint32_t* __restrict__ mflag,
-                                            uint32_t* __restrict__ dirty,
+                                            uint32_t* __restrict__ dirty, const uint32_t* __restrict__ key,
+                                            const uint32_t* __restrict__ cstamp,
                                             const unsigned long long* __restrict__ counters) {
   if (S.tol >= 0.0f && counters[C_DONE] != 0ull) return;
   if (counters[C_HACK_FLAG + (it & 1)] == 0ull) return;
-  const bool scan = counters[C_MOVED_ALL + (it & 1)] != 0ull;
+  const bool scan = counters[C_MOVED_N + (it & 1)] > kMaxMovedMarked;
   const uint32_t p = vb * blockDim.x + threadIdx.x;
   if (p >= n) return;
   const int cnt = nbr_count[p];
@@ -498,10 +469,10 @@ __device__ __forceinline__ void repair_pass(uint32_t vb, uint32_t n, int it, uin
       for (int u = 0; u < kBatch; ++u) hit |= (k0 + u < cnt) & (mflag[q[u]] == stamp);
     }
     if (!hit) return;
-    dirty[p] = stamp;
-  } else if (dirty[p] != stamp) {
+  } else if (cstamp[key[p]] != stamp) {
     return;
   }
+  dirty[p] = stamp;
   const f3 xp = ld3_words(xt, p);
   float sum_C = 0.0f;
   f3 sg = {0.f, 0.f, 0.f};
@@ -538,12 +509,24 @@ __global__ void __launch_bounds__(kBlock) k_lambda_repair(uint32_t n, int it, ui
                                                           const int32_t* __restrict__ nbr_count,
                                                           const uint32_t* __restrict__ mflag,
                                                           uint32_t* __restrict__ dirty,
+                                                          const uint32_t* __restrict__ key,
+                                                          const uint32_t* __restrict__ cstamp,
                                                           const unsigned long long* __restrict__ counters) {
-  repair_pass<FAST>(xcd_block(), n, it, stamp, S, K, xt, rho, lam, nbr, nbr_count, mflag, dirty, counters);
+  repair_pass<FAST>(xcd_block(), n, it, stamp, S, K, xt, rho, lam, nbr, nbr_count, mflag, dirty, key, cstamp,
+                    counters);
 }
 
 __device__ __forceinline__ float mean_error(unsigned long long sum, uint32_t n) {
   return (float)((double)sum / 4294967296.0 / (double)n);
+}
+
+// A row's error, its shards combined (every lane of the wavefront calls them)
+__device__ __forceinline__ float max_error_of(const SolveCtl& S, int row) {
+  static_assert(kErrShards == 64, "one shard per lane");
+  return wave_max(__uint_as_float(S.ehist[(uint32_t)row * kErrShards + (threadIdx.x & 63u)]));
+}
+__device__ __forceinline__ float mean_error_of(const SolveCtl& S, int row, uint32_t n) {
+  return mean_error(wave_sum(S.esum[(uint32_t)row * kErrShards + (threadIdx.x & 63u)]), n);
 }
 
 // The pressure update's sum over the entries of one particle's list within h
@@ -633,7 +616,6 @@ __device__ __forceinline__ void dp_pass(uint32_t vb, bool first, uint32_t n, int
   if (first) {
     counters[C_HACK_FLAG + ((it + 1) & 1)] = 0ull;
     counters[C_MOVED_N + ((it + 1) & 1)] = 0ull;
-    counters[C_MOVED_ALL + ((it + 1) & 1)] = 0ull;
   }
   const uint32_t p = QUAD ? (vb * blockDim.x + threadIdx.x) >> 2 : vb * blockDim.x + threadIdx.x;
   // (every lane of a quad computes the particle's new state; lane 0 writes it)
@@ -642,15 +624,14 @@ __device__ __forceinline__ void dp_pass(uint32_t vb, bool first, uint32_t n, int
   // rejected warm start's restore, 2 the end of the solve (x* = xt)
   int mode = 0;
   if (S.ehist) {
-    const float e = S.mean ? mean_error(S.esum[it + 1], n) : __uint_as_float(S.ehist[it + 1]);
-    const float e_pre = S.mean ? mean_error(S.esum[0], n) : __uint_as_float(S.ehist[0]);
+    const float e = S.mean ? mean_error_of(S, it + 1, n) : max_error_of(S, it + 1);
     bool grew = false;
     // slot 0 checks the warm start; with the retry, slot 1 checks the damped one
     if (S.warm && (it == 0 || (it == 1 && S.retry && counters[C_RETRY] != 0ull))) {
-      grew = e > e_pre;
+      grew = e > (S.mean ? mean_error_of(S, 0, n) : max_error_of(S, 0));
       if (S.strict) {  // the other error measure must not grow either
-        const float o = S.mean ? __uint_as_float(S.ehist[1]) : mean_error(S.esum[1], n);
-        const float o_pre = S.mean ? __uint_as_float(S.ehist[0]) : mean_error(S.esum[0], n);
+        const float o = S.mean ? max_error_of(S, 1) : mean_error_of(S, 1, n);
+        const float o_pre = S.mean ? max_error_of(S, 0) : mean_error_of(S, 0, n);
         grew = grew || o > o_pre;
       }
     }
@@ -1176,12 +1157,12 @@ static void launch_density_as(pbf_context* c, const char* name, int it, int eslo
   if constexpr (QUAD)
     PBF_LAUNCH_QUADS(c, name, (k_density_lambda_c<FM, FAST, SR, true>), it, eslot, S, F, c->K, (const float4*)c->xs,
                      (const float4*)c->v, c->xt, c->rho, c->lam, (const int32_t*)c->nbr,
-                     (const int32_t*)c->nbr_count, c->wmask, c->moved, c->dirty_stamp, c->mflag, c->counters,
+                     (const int32_t*)c->nbr_count, c->wmask, (const uint32_t*)c->key, c->cstamp, c->dirty_stamp, c->mflag, c->counters,
                      (const int32_t*)c->snb, (const int32_t*)c->snb_count);
   else
     PBF_LAUNCH(c, name, (k_density_lambda_c<FM, FAST, SR, false>), it, eslot, S, F, c->K, (const float4*)c->xs,
                (const float4*)c->v, c->xt, c->rho, c->lam, (const int32_t*)c->nbr, (const int32_t*)c->nbr_count,
-               c->wmask, c->moved, c->dirty_stamp, c->mflag, c->counters, (const int32_t*)c->snb,
+               c->wmask, (const uint32_t*)c->key, c->cstamp, c->dirty_stamp, c->mflag, c->counters, (const int32_t*)c->snb,
                (const int32_t*)c->snb_count);
 }
 
@@ -1206,20 +1187,11 @@ void launch_density_lambda_masked(pbf_context* c, int it, int eslot, const Solve
                       : launch_density_fm<0, false>(c, "density_lambda", it, eslot, S, F);
 }
 
-void launch_mark_dirty(pbf_context* c, int it, const SolveCtl& S) {
-  const uint32_t n = (uint32_t)c->n;
-  if (!n) return;
-  KernelTimer* t = timer_begin(c, "mark_dirty");
-  hipLaunchKernelGGL(k_mark_dirty, dim3(kMarkBlocks), dim3(kBlock), 0, c->stream, it, c->dirty_stamp, S, c->K,
-                     (const uint32_t*)c->key, (const uint32_t*)c->cell_start, (const uint32_t*)c->moved, c->dirty,
-                     c->counters);
-  timer_end(c, t);
-}
-
 void launch_lambda_repair(pbf_context* c, int it, const SolveCtl& S) {
   PBF_LAUNCH_ARITH(PBF_LAUNCH, c, "lambda_repair", k_lambda_repair, it, c->dirty_stamp, S, c->K, c->xt,
              (const float*)c->rho, c->lam, (const int32_t*)c->nbr, (const int32_t*)c->nbr_count,
-             (const uint32_t*)c->mflag, c->dirty, (const unsigned long long*)c->counters);
+             (const uint32_t*)c->mflag, c->dirty, (const uint32_t*)c->key, (const uint32_t*)c->cstamp,
+             (const unsigned long long*)c->counters);
 }
 
 #define PBF_DP_ARGS                                                                                              \
@@ -1256,8 +1228,8 @@ void launch_warm_dp(pbf_context* c) {
 
 // ---------------------------------------------------------------------------
 // The Jacobi iterations of a step or the slots of a solve in one cooperative
-// launch (PBF_OPT_PERSISTENT): each iteration runs the density, dirty-marking,
-// lambda-repair and pressure-update bodies above over the whole particle
+// launch (PBF_OPT_PERSISTENT): each iteration runs the density, lambda-repair
+// and pressure-update bodies above over the whole particle
 // range, separated by grid-wide barriers instead of kernel boundaries, and a
 // solve leaves the loop on the device once its slot met the tolerance (every
 // block reads the done flag after the same barrier).  Each block takes a
@@ -1276,8 +1248,8 @@ struct JacobiArgs {
   float *rho, *lam;
   const int32_t *nbr, *nbr_count, *snb, *snb_count;
   uint64_t* wmask;
-  uint32_t *moved, *mflag, *dirty;
-  const uint32_t *key, *start;
+  uint32_t *cstamp, *mflag, *dirty;
+  const uint32_t* key;
   unsigned long long* counters;
 };
 
@@ -1287,7 +1259,6 @@ __global__ void __launch_bounds__(kBlock) k_jacobi_persistent(JacobiArgs A) {
   const uint32_t nvb = (A.n + blockDim.x - 1) / blockDim.x;
   const uint32_t per = (nvb + gridDim.x - 1) / gridDim.x;
   const uint32_t vb0 = xcd_block() * per, vb1 = min(nvb, vb0 + per);
-  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, nwaves = (gridDim.x * blockDim.x) >> 6;
   const FeatCtl F0{nullptr, nullptr, nullptr, nullptr, nullptr, 0.0f, nullptr};
   for (uint32_t it = 0; it < A.iters; ++it) {
     if (A.S.tol >= 0.0f && __atomic_load_n(&A.counters[C_DONE], __ATOMIC_RELAXED) != 0ull) break;
@@ -1295,15 +1266,12 @@ __global__ void __launch_bounds__(kBlock) k_jacobi_persistent(JacobiArgs A) {
     const int eslot = A.solve ? (int)it + 1 : 0;
     for (uint32_t vb = vb0; vb < vb1; ++vb)
       density_pass<0, FAST, SR, false>(vb, vb == 0 && threadIdx.x == 0, A.n, (int)it, eslot, A.S, F0, A.K, A.xs, A.v, A.xt,
-                            A.rho, A.lam, A.nbr, A.nbr_count, A.wmask, A.moved, stamp, A.mflag, A.counters, A.snb,
+                            A.rho, A.lam, A.nbr, A.nbr_count, A.wmask, A.key, A.cstamp, stamp, A.mflag, A.counters, A.snb,
                             A.snb_count);
-    grid.sync();
-    mark_pass(wave, nwaves, wave == 0 && threadIdx.x == 0, (int)it, stamp, A.S, A.K, A.key, A.start, A.moved,
-              A.dirty, A.counters);
     grid.sync();
     for (uint32_t vb = vb0; vb < vb1; ++vb)
       repair_pass<FAST>(vb, A.n, (int)it, stamp, A.S, A.K, A.xt, A.rho, A.lam, A.nbr, A.nbr_count, A.mflag,
-                        A.dirty, A.counters);
+                        A.dirty, A.key, A.cstamp, A.counters);
     grid.sync();
     const int last = A.last_vel && it + 1 == A.iters;
     for (uint32_t vb = vb0; vb < vb1; ++vb)
@@ -1359,8 +1327,7 @@ int launch_jacobi_persistent(pbf_context* c, uint32_t iters, bool solve, bool la
   JacobiArgs A{n, iters, solve ? 1 : 0, last_vel ? 1 : 0, c->dirty_stamp + 1, S, c->K, c->xs, c->v, c->xt,
                (const float4*)c->x, (const float4*)c->xs0, c->rho, c->lam, (const int32_t*)c->nbr,
                (const int32_t*)c->nbr_count, (const int32_t*)c->snb, (const int32_t*)c->snb_count, c->wmask,
-               c->moved, c->mflag, c->dirty, (const uint32_t*)c->key, (const uint32_t*)c->cell_start,
-               c->counters};
+               c->cstamp, c->mflag, c->dirty, (const uint32_t*)c->key, c->counters};
   void* args[] = {&A};
   KernelTimer* t = timer_begin(c, "jacobi_persistent");
   const void* kern = persistent_kernel(c);
@@ -1373,12 +1340,12 @@ int launch_jacobi_persistent(pbf_context* c, uint32_t iters, bool solve, bool la
 
 // The record of the solve that just ran (pbf_get_solve_log): slots used,
 // whether the warm start was kept, the last used slot's errors and the errors
-// before the warm start.  One thread: the ring index advances on the device,
-// so graph replays record every solve.
-__global__ void k_log_solve(uint32_t n, const unsigned long long* __restrict__ counters,
-                            const uint32_t* __restrict__ ehist, const unsigned long long* __restrict__ esum,
-                            pbf_solve_record* __restrict__ log, unsigned long long* __restrict__ count) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
+// before the warm start.  One wavefront: the ring index advances on the
+// device, so graph replays record every solve.
+__global__ void __launch_bounds__(64) k_log_solve(uint32_t n, SolveCtl S,
+                                                  const unsigned long long* __restrict__ counters,
+                                                  pbf_solve_record* __restrict__ log,
+                                                  unsigned long long* __restrict__ count) {
   const unsigned long long idx = *count;
   const uint32_t k = (uint32_t)counters[C_ITERS];  // 1..kMaxSolveSlots
   const uint32_t nn = n ? n : 1u;
@@ -1386,18 +1353,36 @@ __global__ void k_log_solve(uint32_t n, const unsigned long long* __restrict__ c
   r.index = idx;
   r.iterations = k;
   r.warm_start_kept = (int32_t)counters[C_WARM_KEPT];
-  r.max_error = __uint_as_float(ehist[k]);
-  r.mean_error = mean_error(esum[k], nn);
-  r.max_error_before_warm_start = __uint_as_float(ehist[0]);
-  r.mean_error_before_warm_start = mean_error(esum[0], nn);
+  r.max_error = max_error_of(S, (int)k);
+  r.mean_error = mean_error_of(S, (int)k, nn);
+  r.max_error_before_warm_start = max_error_of(S, 0);
+  r.mean_error_before_warm_start = mean_error_of(S, 0, nn);
+  if (threadIdx.x != 0) return;
   log[idx % PBF_SOLVE_LOG_SIZE] = r;
   *count = idx + 1;
 }
 
 void launch_log_solve(pbf_context* c) {
-  hipLaunchKernelGGL(k_log_solve, dim3(1), dim3(64), 0, c->stream, (uint32_t)c->n,
-                     (const unsigned long long*)c->counters, (const uint32_t*)c->ehist,
-                     (const unsigned long long*)c->esum, c->slog, c->slog_count);
+  const SolveCtl S{-1.0f, 0, 0, c->ehist, c->esum, nullptr, nullptr, 0, 0};
+  hipLaunchKernelGGL(k_log_solve, dim3(1), dim3(64), 0, c->stream, (uint32_t)c->n, S,
+                     (const unsigned long long*)c->counters, c->slog, c->slog_count);
+}
+
+// every row's shards combined, for the host
+__global__ void __launch_bounds__(64) k_combine_errors(SolveCtl S, uint32_t* __restrict__ ehist_row,
+                                                       unsigned long long* __restrict__ esum_row) {
+  const float e = max_error_of(S, (int)blockIdx.x);
+  const unsigned long long s = wave_sum(S.esum[blockIdx.x * kErrShards + threadIdx.x]);
+  if (threadIdx.x == 0) {
+    ehist_row[blockIdx.x] = __float_as_uint(e);
+    esum_row[blockIdx.x] = s;
+  }
+}
+
+void launch_combine_errors(pbf_context* c) {
+  const SolveCtl S{-1.0f, 0, 0, c->ehist, c->esum, nullptr, nullptr, 0, 0};
+  hipLaunchKernelGGL(k_combine_errors, dim3(kMaxSolveSlots + 1), dim3(64), 0, c->stream, S, c->ehist_row,
+                     c->esum_row);
 }
 
 void launch_add_warm(pbf_context* c) {

@@ -186,10 +186,12 @@ void launch_bin(pbf_context* c, uint64_t bin_end, bool fused) {
 
 // find_bin_bounds (neighbors.h:137-148): begin[c] = lower_bound(keys, c);
 // end[c] = upper_bound(keys, c) = lower_bound(keys, c + 1) = begin[c + 1].
+// (the stamps of the cells next to moved particles start every step at zero)
 __global__ void k_cell_start(const uint32_t* __restrict__ sorted, uint32_t n, uint32_t ncells,
-                             uint32_t* __restrict__ start) {
+                             uint32_t* __restrict__ start, uint32_t* __restrict__ cstamp) {
   const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c > ncells + 1) return;
+  cstamp[c] = 0u;
   uint32_t lo = 0, hi = n;
   while (lo < hi) {
     const uint32_t mid = (lo + hi) >> 1;
@@ -209,7 +211,7 @@ void launch_sort(pbf_context* c) {
                                      c->rpart, c->stream);
   c->perm = c->sv[which];
   hipLaunchKernelGGL(k_cell_start, dim3(nblocks((uint64_t)c->K.ncells + 2)), dim3(kBlock), 0, c->stream,
-                     (const uint32_t*)c->sk[which], n, c->K.ncells, c->cell_start);
+                     (const uint32_t*)c->sk[which], n, c->K.ncells, c->cell_start, c->cstamp);
   timer_end(c, t);
 }
 

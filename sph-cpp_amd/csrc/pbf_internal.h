@@ -28,7 +28,10 @@
 //   far row          row `capacity` of the position stars (xs, xsa, xt) holds +inf: a padding
 //                                entry of a list reads it and lies outside every radius
 //   counters         u64[16]     overflow, outside, hacks, hack flags, solve state, ...
-//   ehist            uint32[kMaxSolveSlots+1]  max density error per solve slot (float bits)
+//   ehist, esum      uint32, u64[kMaxSolveSlots+1][kErrShards]  max (float bits) and sum of the
+//                                density errors per solve slot, in shards that their readers combine
+//   cstamp           uint32[C+1] == the iteration's stamp: a particle within two cells was moved
+//                                by the density fix (cleared with cell_start)
 //   lsum, lsuma      float[n]    multipliers summed over the updates of the last solve
 //                                (carried through the reorder while a warm start may use them)
 //   wlam, wgiven     float[n]    warm-start multipliers (slot order / original order)
@@ -98,7 +101,6 @@ enum Counter {
   C_HEAVY = 5,      // number of entries in the heavy list
   C_EMAX = 6,       // float bits of the max density error (atomicMax on non-negative floats)
   C_MOVED_N = 7,    // two counts (7, 8): particles moved by the density fix, per iteration parity
-  C_MOVED_ALL = 9,  // two flags (9, 10): too many moved particles or marked cells -> treat all as dirty
   C_DONE = 11,      // iterate-to-tolerance: 0, or the slot whose error fell below the tolerance plus one
   C_ITERS = 12,     // iterate-to-tolerance: slots used
   C_WARM_KEPT = 13, // the warm-start positions were kept (2: the damped retry's, PBF_OPT_WARM_RETRY)
@@ -112,6 +114,11 @@ enum Counter {
 };
 
 constexpr uint32_t kMaxSolveSlots = PBF_MAX_SOLVE_ITERATIONS;
+// The error of a slot is gathered by atomics of every wavefront: on one
+// address they queue up in the cache (16,384 of them at 1,048,576 particles),
+// so they are spread over this many, one per lane of the wavefront that reads
+// them back.
+constexpr uint32_t kErrShards = 64;
 constexpr uint64_t kRowPad = 8;  // padding rows of the float4 particle buffers
 constexpr float kWarmLambdaScale = PBF_WARM_LAMBDA_SCALE;
 
@@ -121,8 +128,8 @@ struct SolveCtl {
   float tol;                   // >= 0: stop once the slot's density error is <= tol
   int warm;                    // a warm-start update was applied before slot 0
   int mean;                    // compare the mean error (else the maximum)
-  uint32_t* ehist;             // max error as float bits: [0] before the warm start, [k+1] slot k
-  unsigned long long* esum;    // sum of the errors in 2^-32 units, same slots
+  uint32_t* ehist;             // max error as float bits: row 0 before the warm start, k+1 slot k
+  unsigned long long* esum;    // sum of the errors in 2^-32 units, same rows (kErrShards each)
   float* lsum;                 // sum of the applied multipliers (null: not kept)
   const float4* xsave;         // position stars to restore when the warm start is rejected
   int strict;                  // reject the warm start when the max or the mean error grows
@@ -198,7 +205,7 @@ struct pbf_context {
   uint32_t *rhist = nullptr, *roffs = nullptr, *rpart = nullptr;
   uint32_t* perm = nullptr;  // sorted slot -> previous slot (points into sv or tmpo)
   uint32_t* heavy = nullptr;
-  uint32_t* moved = nullptr;  // particles moved by the density fix in the current iteration
+  uint32_t* cstamp = nullptr;  // [cells + 1] == dirty_stamp: a particle within two cells was moved
   uint32_t* dirty = nullptr;  // == dirty_stamp: the particle or one of its neighbours moved
   uint32_t* mflag = nullptr;  // == dirty_stamp: the density fix moved the particle in that iteration
   uint32_t* cell_start = nullptr;
@@ -217,6 +224,8 @@ struct pbf_context {
   unsigned long long* counters = nullptr;
   uint32_t* ehist = nullptr;
   unsigned long long* esum = nullptr;
+  uint32_t* ehist_row = nullptr;            // their shards combined, for the host
+  unsigned long long* esum_row = nullptr;
   float* feat = nullptr;       // [n][8] features of the last warm-started solve
   bool feat_valid = false;
   short *mw1 = nullptr, *mw2 = nullptr;  // learned warm start: bf16 weights
@@ -311,7 +320,7 @@ void launch_density(pbf_context* c, uint64_t b, uint64_t e);  // xs -> xt, rho
 // ---- fused-step launchers (pbf_fused.hip): they build and use the compact lists ----
 void launch_density_lambda_masked(pbf_context* c, int it, int eslot, const SolveCtl& S,
                                   const FeatCtl& F = FeatCtl{nullptr, nullptr});  // xs -> xt, rho, lam
-void launch_mark_dirty(pbf_context* c, int it, const SolveCtl& S);     // particles next to a moved one
+void launch_combine_errors(pbf_context* c);                            // ehist, esum -> ehist_row, esum_row
 void launch_lambda_repair(pbf_context* c, int it, const SolveCtl& S);  // lam from xt for dirty particles
 void launch_dp_update_masked(pbf_context* c, int it, int last, const SolveCtl& S);
 void launch_warm_dp(pbf_context* c);      // xt, wlam -> xs (warm start), xsave = xt

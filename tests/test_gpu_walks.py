@@ -145,3 +145,30 @@ def test_few_particles(pbf, scenes, n):
     o.step(1)
     _same(g, o, f"{n} particles, pass by pass")
     g.close()
+
+
+@pytest.mark.parametrize("counts", [(11, 9, 10), (49, 46, 44)])
+@pytest.mark.parametrize("pairs", [2, 40])
+def test_density_fix_next_to_the_walls(pbf, scenes, counts, pairs):
+    """Coincident pairs (moved by the density fix) in the corner cells of the
+    grid, on its edges and inside, in scenes walked by quads and by single
+    lanes: the 5x5x5 cells stamped around a moved particle are cut off at the
+    grid's faces, and every particle that lists a moved one is repaired."""
+    params, pos, vel = _scene(scenes, counts, 1.0, 60)
+    box = np.array(params.boundary_max[:], dtype=np.float32)
+    rng = np.random.default_rng(pairs)
+    spots = np.stack([rng.choice([0.0, 0.5, 1.0], pairs) for _ in range(3)], axis=1).astype(np.float32)
+    lo, hi = pos.min(axis=0), pos.max(axis=0)
+    at = lo + spots * (hi - lo)
+    ids = rng.permutation(len(pos))[:2 * pairs]
+    pos[ids] = np.repeat(np.clip(at, 0.0, box), 2, axis=0)
+    vel[ids] = np.repeat(rng.uniform(-0.2, 0.2, (pairs, 3)), 2, axis=0).astype(np.float32)
+    g = pbf.Particles(params)
+    g.add(pos, pos, vel)
+    o = O.Oracle(O.params_from_pbf(params), mode=O.JACOBI, threads=THREADS)
+    o.set_state(pos, pos, vel)
+    g.step(1)
+    o.step(1)
+    assert g.stats()["density_hacks"] > 0
+    _same(g, o, f"{pairs} pairs, {len(pos)} particles")
+    g.close()

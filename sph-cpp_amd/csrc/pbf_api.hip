@@ -252,9 +252,9 @@ static int alloc_grid(pbf_context* c) {
 static void free_all(pbf_context* c) {
   void* ptrs[] = {c->x,    c->xs,   c->v,    c->xa,   c->xsa,  c->va,   c->xt,         c->scr,
                   c->scra, c->rho,  c->lam,  c->rhoa, c->lama, c->oid,  c->oida,       c->key,
-                  c->keya, c->slot, c->tmp,  c->tmpo, c->nbr,  c->nbr_count, c->counters, c->stage,
+                  c->slot, c->tmp,  c->tmpo, c->nbr,  c->nbr_count, c->counters, c->stage,
                   c->stage64, c->cell_start, c->scan_partials, c->sk[0], c->sk[1], c->sv[0], c->sv[1],
-                  c->rhist, c->roffs, c->rpart, c->heavy, c->cnb, c->cnb_count, c->cstamp, c->dirty, c->ehist_row, c->esum_row,
+                  c->rhist, c->rsum, c->heavy, c->cnb, c->cnb_count, c->cstamp, c->dirty, c->ehist_row, c->esum_row,
                   c->ehist, c->lsum, c->lsuma, c->wlam, c->wgiven, c->xsave, c->esum, c->feat, c->mw1,
                   c->mw2, c->mp, c->scenes, c->sid, c->sida, c->cbox, c->chbox, c->wmask, c->mflag,
                   c->slog, c->slog_count, c->snb, c->snb_count, c->xs0, c->skin_hint};
@@ -297,7 +297,8 @@ __global__ void k_compact_perm(uint32_t n, const uint32_t* __restrict__ oid, uin
 }
 
 // neighbour search body shared by pbf_find_neighbors and pbf_step
-static void find_neighbors_impl(pbf_context* c, uint64_t bin_end, uint64_t fb, uint64_t fe, bool fused);
+static void find_neighbors_impl(pbf_context* c, uint64_t bin_end, uint64_t fb, uint64_t fe);
+static void build_neighbors_fused(pbf_context* c, const StepInit& I);
 
 void drop_graph(pbf_context* c) {
   if (c->graph_exec) hipGraphExecDestroy(c->graph_exec);
@@ -317,7 +318,7 @@ static void drop_solve_graph(pbf_context* c) {
 // is valid only while they are where they were at capture.
 static std::vector<void*> buffer_sig(const pbf_context* c) {
   return {c->x, c->xs, c->v, c->xa, c->xsa, c->va, c->xt, c->scr, c->scra, c->rho, c->lam, c->rhoa, c->lama,
-          c->oid, c->oida, c->key, c->keya, c->lsum, c->lsuma, c->sid, c->sida, (void*)(uintptr_t)c->track_lsum};
+          c->oid, c->oida, c->key, c->lsum, c->lsuma, c->sid, c->sida, (void*)(uintptr_t)c->track_lsum};
 }
 
 // The grid of every scene of a batched context (boxes: 3 extents per scene)
@@ -411,14 +412,13 @@ int pbf_create(const pbf_params* params, pbf_context** out) {
       (rc = dalloc(&c->scr, NP)) || (rc = dalloc(&c->scra, NP)) || (rc = dalloc(&c->rho, NP)) ||
       (rc = dalloc(&c->lam, NP)) || (rc = dalloc(&c->rhoa, NP)) || (rc = dalloc(&c->lama, NP)) ||
       (rc = dalloc(&c->oid, N)) || (rc = dalloc(&c->oida, N)) || (rc = dalloc(&c->key, N)) ||
-      (rc = dalloc(&c->keya, N)) || (rc = dalloc(&c->slot, N)) || (rc = dalloc(&c->tmp, N + 1)) ||
+      (rc = dalloc(&c->slot, N)) || (rc = dalloc(&c->tmp, N + 1)) ||
       (rc = dalloc(&c->tmpo, N + 1)) || (rc = dalloc(&c->nbr, list_size(N, c->K.stride))) ||
       (rc = dalloc(&c->nbr_count, N)) || (rc = dalloc(&c->counters, (uint64_t)C_NUM)) ||
       (rc = dalloc(&c->stage, 4 * N)) || (rc = dalloc(&c->stage64, N + 1)) || (rc = alloc_grid(c)) ||
       (rc = dalloc(&c->sk[0], N + 1)) || (rc = dalloc(&c->sk[1], N + 1)) || (rc = dalloc(&c->sv[0], N + 1)) ||
       (rc = dalloc(&c->sv[1], N + 1)) || (rc = dalloc(&c->rhist, radix_hist_size(N))) ||
-      (rc = dalloc(&c->roffs, radix_hist_size(N) + 1)) ||
-      (rc = dalloc(&c->rpart, scan_partials_size(radix_hist_size(N) + 1))) || (rc = dalloc(&c->heavy, N)) ||
+      (rc = dalloc(&c->rsum, kRadixSumWords)) || (rc = dalloc(&c->heavy, N)) ||
       (rc = dalloc(&c->chbox, 2 * ((N + 63) / 64))) || (rc = dalloc(&c->wmask, 2 * N)) ||
       (rc = dalloc(&c->cnb, list_size(N, c->K.stride))) || (rc = dalloc(&c->cnb_count, N)) ||
       (rc = dalloc(&c->snb, list_size(N, c->K.stride))) || (rc = dalloc(&c->snb_count, N)) ||
@@ -632,9 +632,8 @@ int pbf_remove(pbf_context* c, uint64_t count) {
   launch_exclusive_scan(c->tmp, c->tmpo, n, c->scan_partials, c->stream);
   hipLaunchKernelGGL(k_compact_perm, dim3(nb), dim3(256), 0, c->stream, n, (const uint32_t*)c->oid, newn,
                      (const uint32_t*)c->tmpo, c->slot);
-  c->perm = c->slot;
   c->n = newn;
-  launch_reorder(c);
+  launch_reorder_by(c, c->slot);
   c->lists_valid = false;
   return check_hip(hipStreamSynchronize(c->stream), "pbf_remove");
 }
@@ -725,7 +724,7 @@ int pbf_find_neighbors(pbf_context* c, pbf_index_span bin_span, pbf_index_span f
   if (bin_span.begin != 0)
     return set_error(PBF_ERR_ARG, "bin span must start at 0: sort_bins sorts [0, count) (neighbors.h:130-132)");
   launch_fill_u64(c->counters, 0ull, 3, c->stream);  // overflow, outside, hacks
-  find_neighbors_impl(c, bin_span.end, fill_span.begin, fill_span.end, false);
+  find_neighbors_impl(c, bin_span.end, fill_span.begin, fill_span.end);
   c->pass_skin = c->K.skin_mode != 0;
   return check_hip(hipGetLastError(), "find_neighbors");
 }
@@ -839,15 +838,9 @@ static int check_persistent(pbf_context* c) {
 static void step_body(pbf_context* c) {
   const uint64_t n = c->n;
   {
-    // the multiplier sums move with the reorder inside find_neighbors
-    if (c->capturing) {  // stamps repeat on every replay
-      launch_fill_u32(c->dirty, 0u, n, c->stream);
-      launch_fill_u32(c->mflag, 0u, n, c->stream);
-    }
-    if (!n) launch_fill_u64(c->counters, 0ull, C_NUM, c->stream);
-    launch_forces_predict(c, F_FORCES | F_PREDICT | F_CLEAR, 0, n);  // (counters zeroed there)
-    find_neighbors_impl(c, n, 0, n, true);
-    if (c->track_lsum) launch_fill_u32((uint32_t*)c->lsum, 0u, n, c->stream);
+    // the multiplier sums move with the reorder
+    build_neighbors_fused(c, StepInit{0ull, 0ull, nullptr, nullptr, 0u});
+    if (c->track_lsum && c->P.solve_step_count == 0) launch_fill_u32((uint32_t*)c->lsum, 0u, n, c->stream);
     const SolveCtl S{-1.0f, 0, 0, nullptr, nullptr, c->track_lsum ? c->lsum : nullptr, nullptr};
     const uint32_t I = c->P.solve_step_count;
     c->coop_grid = 0;
@@ -940,23 +933,14 @@ static int solve_body(pbf_context* c, float tolerance, uint32_t max_iterations, 
   const int warm = warm_start != PBF_WARM_NONE;
   const bool had_lsum = c->track_lsum;
   c->track_lsum = true;
-  launch_fill_u64(c->counters, 0ull, C_NUM, c->stream);
-  if (c->capturing) {  // stamps repeat on every replay
-    launch_fill_u32(c->dirty, 0u, n, c->stream);
-    launch_fill_u32(c->mflag, 0u, n, c->stream);
-  }
-  launch_fill_u64(c->counters + C_ITERS, (unsigned long long)max_iterations, 1, c->stream);
-  launch_fill_u64(c->counters + C_WARM_KEPT, (unsigned long long)warm, 1, c->stream);
-  launch_fill_u32(c->ehist, 0u, ((uint64_t)max_iterations + 1) * kErrShards, c->stream);
-  launch_fill_u64(c->esum, 0ull, ((uint64_t)max_iterations + 1) * kErrShards, c->stream);
-  launch_forces_predict(c, F_FORCES | F_PREDICT, 0, n);
-  find_neighbors_impl(c, n, 0, n, true);  // carries the previous sums to the new order
-  // lsuma: the previous sums; lsum: this solve's
+  // carries the previous sums to the new order
+  build_neighbors_fused(c, StepInit{max_iterations, (unsigned long long)warm, c->ehist, c->esum,
+                                    (max_iterations + 1) * kErrShards});
+  // lsuma: the previous sums; lsum: this solve's (slot 0's update starts them)
   std::swap(c->lsum, c->lsuma);
   if (!had_lsum) launch_fill_u32((uint32_t*)c->lsuma, 0u, n, c->stream);
-  launch_fill_u32((uint32_t*)c->lsum, 0u, n, c->stream);
-  if (warm_start == PBF_WARM_PREVIOUS) launch_copy_f1(c->lsuma, c->wlam, n, c->stream);
-  else if (warm_start == PBF_WARM_GIVEN) launch_scatter_in_f1(c, c->wgiven, c->wlam);
+  if (warm_start == PBF_WARM_GIVEN) launch_scatter_in_f1(c, c->wgiven, c->wlam);
+  const float* wlam = warm_start == PBF_WARM_PREVIOUS ? c->lsuma : c->wlam;
   const int mean = (c->P.options & PBF_OPT_SOLVE_MEAN_ERROR) ? 1 : 0;
   const int strict = (c->P.options & PBF_OPT_WARM_STRICT) ? 1 : 0;
   const int retry = (warm && (c->P.options & PBF_OPT_WARM_RETRY)) ? 1 : 0;
@@ -979,7 +963,7 @@ static int solve_body(pbf_context* c, float tolerance, uint32_t max_iterations, 
     }
     launch_density_lambda_masked(c, 1, 0, S0, F);
     c->feat_valid = keep;
-    launch_warm_dp(c);
+    launch_warm_dp(c, wlam);
   }
   constexpr uint32_t kChunk = 8;
   c->coop_grid = 0;
@@ -989,7 +973,7 @@ static int solve_body(pbf_context* c, float tolerance, uint32_t max_iterations, 
     launch_density_lambda_masked(c, (int)it, (int)it + 1, S);
     launch_lambda_repair(c, (int)it, S);
     launch_dp_update_masked(c, (int)it, 0, S);
-    if (retry && it == 0) launch_warm_retry(c);  // (does nothing unless slot 0 rejected the warm start)
+    if (retry && it == 0) launch_warm_retry(c, wlam);  // (does nothing unless slot 0 rejected the warm start)
     if (host_chunks && (it + 1) % kChunk == 0 && it + 1 < max_iterations) {
       int rc = check_hip(hipMemcpyAsync(c->done_host, c->counters + C_DONE, sizeof(unsigned long long),
                                         hipMemcpyDeviceToHost, c->stream), "pbf_solve");
@@ -998,9 +982,7 @@ static int solve_body(pbf_context* c, float tolerance, uint32_t max_iterations, 
       if (*c->done_host) break;
     }
   }
-  if (warm) launch_add_warm(c);
-  launch_update_velocities(c, 0, n);
-  launch_log_solve(c);
+  launch_solve_end(c, warm ? wlam : nullptr);
   c->last_iterations = max_iterations;
   c->last_was_solve = true;
   step_tail(c);
@@ -1350,7 +1332,7 @@ int pbf_autotune_layout(pbf_context* c, uint32_t steps, pbf_layout* best) {
     if ((rc = pbf_set_params(c, &P)) || (rc = S.restore())) break;
     launch_fill_u64(c->counters, 0ull, C_NUM, c->stream);
     launch_forces_predict(c, F_FORCES | F_PREDICT, 0, c->n);
-    find_neighbors_impl(c, c->n, 0, c->n, false);
+    find_neighbors_impl(c, c->n, 0, c->n);
     unsigned long long over = 0;
     uint32_t longest = 0;
     if ((rc = check_hip(hipMemcpyAsync(&over, c->counters + C_OVERFLOW, sizeof(over), hipMemcpyDeviceToHost,
@@ -1590,15 +1572,26 @@ int pbf_region_end(pbf_context* c, double* ms) {
 
 namespace pbf {
 
-static void find_neighbors_impl(pbf_context* c, uint64_t bin_end, uint64_t fb, uint64_t fe, bool fused) {
-  launch_bin(c, bin_end, fused);  // (clears the list build's counters)
+// after the keys: sort, cell order, lists
+static void build_neighbors(pbf_context* c, uint64_t fb, uint64_t fe, bool fused) {
   launch_sort(c);
   // a fused step recomputes densities, multipliers and the scratch vector
   // before reading them (with at least one Jacobi iteration): they stay unsorted
-  launch_reorder(c, !(fused && c->P.solve_step_count > 0));
+  launch_reorder_cells(c, !(fused && c->P.solve_step_count > 0), fused);
   launch_fill_neighbors(c, fb, fe);
   c->lists_valid = true;
   c->pass_skin = false;
+}
+
+static void find_neighbors_impl(pbf_context* c, uint64_t bin_end, uint64_t fb, uint64_t fe) {
+  launch_bin(c, bin_end);  // (clears the list build's counters)
+  build_neighbors(c, fb, fe, false);
+}
+
+// the start of a fused step: forces, prediction, neighbour search
+static void build_neighbors_fused(pbf_context* c, const StepInit& I) {
+  launch_predict_bin(c, I);
+  build_neighbors(c, 0, c->n, true);
 }
 
 }  // namespace pbf

@@ -658,10 +658,12 @@ __device__ __forceinline__ void dp_pass(uint32_t vb, bool first, uint32_t n, int
   if (p < n && mode == 1) {
     const float4 sv = S.xsave[p];
     if (writes) xs[p] = sv;
+    if (S.lsum && it == 0 && writes) S.lsum[p] = 0.0f;
     if (track) mv = move2(xyz(sv), xs0[p]);
   } else if (p < n && mode == 2) {
     const float4 t = xt[p];
     if (writes) xs[p] = t;
+    if (S.lsum && it == 0 && writes) S.lsum[p] = 0.0f;
     if (track) mv = move2(xyz(t), xs0[p]);
   } else if (p < n) {
     // a dirty particle (moved by the density fix, or next to one) walks its
@@ -692,7 +694,7 @@ __device__ __forceinline__ void dp_pass(uint32_t vb, bool first, uint32_t n, int
     boundary(nw, K, p);
     if (writes) st3(xs, p, nw);
     if (track) mv = move2(nw, xs0[p]);
-    if (S.lsum && writes) S.lsum[p] += lp;
+    if (S.lsum && writes) S.lsum[p] = (it == 0 ? 0.0f : S.lsum[p]) + lp;  // (slot 0 starts the sum)
     if (last && writes) {  // the density rides in v.w for the XSPH passes' gathers
       f3 vel = div3(sub3(nw, ld3(x, p)), K.dt);
       if ((double)magsq3(vel) < K.vthr) vel = {0.f, 0.f, 0.f};
@@ -769,15 +771,6 @@ __global__ void __launch_bounds__(kBlock) k_warm_dp(uint32_t n, KParams K, const
   }
   // slot 0 reads parity 0
   if (track) record_move(mv, counters, C_DISP + 0, K);
-}
-
-// After the Jacobi loop: the kept warm-start multipliers join the sum.
-__global__ void k_add_warm(uint32_t n, const float* __restrict__ wlam, float* __restrict__ lsum,
-                           const unsigned long long* __restrict__ counters) {
-  const unsigned long long kept = counters[C_WARM_KEPT];
-  if (kept == 0ull) return;
-  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < n) lsum[p] += kept == 2ull ? kWarmRetryScale * wlam[p] : wlam[p];
 }
 
 // PBF_OPT_WARM_RETRY, after slot 0's pressure update: when that update put x*
@@ -1215,14 +1208,14 @@ void launch_dp_update_masked(pbf_context* c, int it, int last, const SolveCtl& S
     launch_dp_as<false, false>(c, it, last, S);
 }
 
-void launch_warm_retry(pbf_context* c) {
+void launch_warm_retry(pbf_context* c, const float* warm) {
   PBF_LAUNCH_ARITH(PBF_LAUNCH, c, "warm_retry", k_warm_retry, c->K, (const float4*)c->xsave,
-                   (const float*)c->wlam, (const int32_t*)c->nbr, (const int32_t*)c->nbr_count, c->xs, c->counters,
+                   warm, (const int32_t*)c->nbr, (const int32_t*)c->nbr_count, c->xs, c->counters,
                    (const float4*)c->xs0);
 }
 
-void launch_warm_dp(pbf_context* c) {
-  PBF_LAUNCH_ARITH(PBF_LAUNCH, c, "warm_dp", k_warm_dp, c->K, (const float4*)c->xt, (const float*)c->wlam, (const int32_t*)c->nbr,
+void launch_warm_dp(pbf_context* c, const float* warm) {
+  PBF_LAUNCH_ARITH(PBF_LAUNCH, c, "warm_dp", k_warm_dp, c->K, (const float4*)c->xt, warm, (const int32_t*)c->nbr,
              (const int32_t*)c->nbr_count, c->xs, c->xsave, c->counters, (const float4*)c->xs0);
 }
 
@@ -1342,10 +1335,10 @@ int launch_jacobi_persistent(pbf_context* c, uint32_t iters, bool solve, bool la
 // whether the warm start was kept, the last used slot's errors and the errors
 // before the warm start.  One wavefront: the ring index advances on the
 // device, so graph replays record every solve.
-__global__ void __launch_bounds__(64) k_log_solve(uint32_t n, SolveCtl S,
-                                                  const unsigned long long* __restrict__ counters,
-                                                  pbf_solve_record* __restrict__ log,
-                                                  unsigned long long* __restrict__ count) {
+__device__ __forceinline__ void log_solve(uint32_t n, const SolveCtl& S,
+                                          const unsigned long long* __restrict__ counters,
+                                          pbf_solve_record* __restrict__ log,
+                                          unsigned long long* __restrict__ count) {
   const unsigned long long idx = *count;
   const uint32_t k = (uint32_t)counters[C_ITERS];  // 1..kMaxSolveSlots
   const uint32_t nn = n ? n : 1u;
@@ -1357,15 +1350,40 @@ __global__ void __launch_bounds__(64) k_log_solve(uint32_t n, SolveCtl S,
   r.mean_error = mean_error_of(S, (int)k, nn);
   r.max_error_before_warm_start = max_error_of(S, 0);
   r.mean_error_before_warm_start = mean_error_of(S, 0, nn);
-  if (threadIdx.x != 0) return;
+  if ((threadIdx.x & 63u) != 0u) return;
   log[idx % PBF_SOLVE_LOG_SIZE] = r;
   *count = idx + 1;
 }
 
-void launch_log_solve(pbf_context* c) {
+// The end of a solve: update_velocities (particles.h:375-385; the density
+// rides in v.w for the passes that follow), the kept warm multipliers (null:
+// none) join the sum, and block 0's first wavefront writes the record.
+__global__ void __launch_bounds__(kBlock) k_solve_end(uint32_t n, KParams K, SolveCtl S,
+                                                      const float4* __restrict__ x, const float4* __restrict__ xs,
+                                                      const float* __restrict__ rho, float4* __restrict__ v,
+                                                      const float* __restrict__ warm, float* __restrict__ lsum,
+                                                      const unsigned long long* __restrict__ counters,
+                                                      pbf_solve_record* __restrict__ log,
+                                                      unsigned long long* __restrict__ count) {
+  if (blockIdx.x == 0 && threadIdx.x < 64u) log_solve(n, S, counters, log, count);
+  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n) return;
+  f3 vel = div3(sub3(ld3(xs, p), ld3(x, p)), K.dt);
+  if ((double)magsq3(vel) < K.vthr) vel = {0.f, 0.f, 0.f};
+  v[p] = make_float4(vel.x, vel.y, vel.z, rho[p]);
+  if (warm) {
+    const unsigned long long kept = counters[C_WARM_KEPT];
+    if (kept != 0ull) lsum[p] += kept == 2ull ? kWarmRetryScale * warm[p] : warm[p];
+  }
+}
+
+void launch_solve_end(pbf_context* c, const float* warm) {
   const SolveCtl S{-1.0f, 0, 0, c->ehist, c->esum, nullptr, nullptr, 0, 0};
-  hipLaunchKernelGGL(k_log_solve, dim3(1), dim3(64), 0, c->stream, (uint32_t)c->n, S,
+  KernelTimer* t = timer_begin(c, "solve_end");
+  hipLaunchKernelGGL(k_solve_end, dim3(std::max(1u, nblocks(c->n))), dim3(kBlock), 0, c->stream, (uint32_t)c->n,
+                     c->K, S, (const float4*)c->x, (const float4*)c->xs, (const float*)c->rho, c->v, warm, c->lsum,
                      (const unsigned long long*)c->counters, c->slog, c->slog_count);
+  timer_end(c, t);
 }
 
 // every row's shards combined, for the host
@@ -1383,10 +1401,6 @@ void launch_combine_errors(pbf_context* c) {
   const SolveCtl S{-1.0f, 0, 0, c->ehist, c->esum, nullptr, nullptr, 0, 0};
   hipLaunchKernelGGL(k_combine_errors, dim3(kMaxSolveSlots + 1), dim3(64), 0, c->stream, S, c->ehist_row,
                      c->esum_row);
-}
-
-void launch_add_warm(pbf_context* c) {
-  PBF_LAUNCH(c, "add_warm", k_add_warm, (const float*)c->wlam, c->lsum, (const unsigned long long*)c->counters);
 }
 
 #define PBF_VISC_ARGS                                                                                          \

@@ -10,9 +10,8 @@
 // particle index).  Particles here live in cell order from the previous
 // step, so a stable sort of the current slots would order by
 // (key, previous key, index).  Instead the (key, slot) pairs are listed in
-// original-index order (through the inverse permutation written by the
-// binning pass) and sorted by a stable LSD radix sort on the key bits (8-bit
-// digits, per-tile histograms, wavefront ballot ranking in LDS): the result is
+// original-index order (written there by the binning pass) and sorted by a stable LSD radix sort on the key bits (up to 8
+// a pass, per-tile histograms, wavefront ballot ranking): the result is
 // exactly the (key, original index) order the reference produces.
 //
 // Lists.  One lane per particle walks the 27 cells in the reference's order
@@ -139,124 +138,187 @@ void launch_exclusive_scan(const uint32_t* in, uint32_t* out, uint64_t n, uint32
 }
 
 // ---------------------------------------------------------------------------
-// calculate_bins (neighbors.h:120-125): cell key of every slot, and the
-// inverse permutation (original index -> slot) so that the keys can be
-// listed in original-index order for the stable sort.
-// Also lists the (key, slot) pairs by original index: a stable sort of that
-// sequence by key is the reference's stable sort of (key, index) pairs.
+// calculate_bins (neighbors.h:120-125): the cell key of every slot, listed
+// with the slot by original index: a stable sort of that sequence by key is
+// the reference's stable sort of (key, index) pairs.
+struct BinOut {
+  uint32_t *sk, *sv;       // (key, slot) pairs by original index
+  uint32_t* gsum;          // the sort's group sums, cleared for its counting passes
+  uint32_t gsum_words;
+  unsigned long long* counters;
+};
+__device__ __forceinline__ uint32_t bin_key(f3 ps, uint32_t p, const KParams& K) {
+  return cell_key(bin_coord(ps.x, K.s), bin_coord(ps.y, K.s), bin_coord(ps.z, K.s), grid_of(K, p), K);
+}
+
 __global__ void __launch_bounds__(kBlock) k_bin(const float4* __restrict__ xs, uint32_t n, uint32_t bin_end,
-                                                KParams K, const uint32_t* __restrict__ oid,
-                                                uint32_t* __restrict__ key, uint32_t* __restrict__ inv,
-                                                unsigned long long* __restrict__ counters,
-                                                uint32_t* __restrict__ sk, uint32_t* __restrict__ sv,
+                                                KParams K, const uint32_t* __restrict__ oid, BinOut B,
                                                 unsigned long long* __restrict__ hint) {
   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+  for (uint32_t i = p; i < B.gsum_words; i += gridDim.x * blockDim.x) B.gsum[i] = 0u;
   if (p == 0) {  // counted by the list build that follows
-    counters[C_HEAVY] = 0ull;
-    counters[C_TILE] = 0ull;
-    if (hint) {  // per-pass: skin lists if the moves since the last build kept them usable
-      *hint = counters[C_DISP_ALL] == 0ull ? 1ull : 0ull;
-      counters[C_DISP_ALL] = 0ull;
-      counters[C_SKIN] = 0ull;
-    }
+    B.counters[C_HEAVY] = 0ull;
+    B.counters[C_TILE] = 0ull;
+    // skin lists if the moves since the last build kept them usable
+    *hint = B.counters[C_DISP_ALL] == 0ull ? 1ull : 0ull;
+    B.counters[C_DISP_ALL] = 0ull;
+    B.counters[C_SKIN] = 0ull;
   }
   if (p >= n) return;
   const uint32_t o = oid[p];
   uint32_t k = K.ncells;  // particles past the bin span are placed in no cell
   if (o < bin_end) {
-    const f3 ps = ld3(xs, p);
-    k = cell_key(bin_coord(ps.x, K.s), bin_coord(ps.y, K.s), bin_coord(ps.z, K.s), grid_of(K, p), K);
-    if (k == K.ncells) atomicAdd(&counters[C_OUTSIDE], 1ull);
+    k = bin_key(ld3(xs, p), p, K);
+    if (k == K.ncells) atomicAdd(&B.counters[C_OUTSIDE], 1ull);
   }
-  key[p] = k;
-  inv[o] = p;
-  sk[o] = k;
-  sv[o] = p;
+  B.sk[o] = k;
+  B.sv[o] = p;
 }
 
-void launch_bin(pbf_context* c, uint64_t bin_end, bool fused) {
+// The start of a fused step in one pass over the particles: what it counts is
+// cleared (StepInit), external forces (particles.h:263-270), prediction
+// (:275-287) and the cell keys.  (As three launches the forces and the keys
+// each read the particles again: 14.2 + 11.7 us at 1,048,576 particles against
+// 18.0 so.)  Particles outside the grid are counted with the cell bounds.
+__global__ void __launch_bounds__(kBlock) k_predict_bin(uint32_t n, KParams K, const uint32_t* __restrict__ oid,
+                                                        const float4* __restrict__ x, float4* __restrict__ v,
+                                                        float4* __restrict__ xs, BinOut B, StepInit I) {
+  const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t all = gridDim.x * blockDim.x;
+  for (uint32_t i = p; i < B.gsum_words; i += all) B.gsum[i] = 0u;
+  for (uint32_t i = p; i < I.error_words; i += all) {
+    I.ehist[i] = 0u;
+    I.esum[i] = 0ull;
+  }
+  if (p < (uint32_t)C_NUM) B.counters[p] = p == C_ITERS ? I.iterations : (p == C_WARM_KEPT ? I.warm : 0ull);
+  if (p >= n) return;
+  const uint32_t o = oid[p];
+  f3 vp = ld3(v, p);
+  vp.y += K.g * K.dt;
+  st3(v, p, vp);
+  f3 ps = add3(ld3(x, p), mul3(vp, K.dt));
+  boundary(ps, K, p);
+  st3(xs, p, ps);
+  B.sk[o] = bin_key(ps, p, K);
+  B.sv[o] = p;
+}
+
+// the sort of a context's particles: keys go up to ncells (the outside bucket)
+static RadixPlan cell_sort_plan(const pbf_context* c) {
+  uint32_t bits = 1;
+  while (bits < 32 && (c->K.ncells >> bits) != 0) ++bits;
+  return radix_plan(c->n, bits);
+}
+static BinOut bin_out(pbf_context* c) {
+  return BinOut{c->sk[0], c->sv[0], c->rsum, cell_sort_plan(c).sum_words(), c->counters};
+}
+
+void launch_bin(pbf_context* c, uint64_t bin_end) {
   const uint32_t n = (uint32_t)c->n;
   if (!n) return;
   KernelTimer* t = timer_begin(c, "bin");
   hipLaunchKernelGGL(k_bin, dim3(nblocks(n)), dim3(kBlock), 0, c->stream, (const float4*)c->xs, n,
-                     (uint32_t)bin_end, c->K, (const uint32_t*)c->oid, c->key, c->slot, c->counters, c->sk[0],
-                     c->sv[0], fused ? nullptr : c->skin_hint);
+                     (uint32_t)bin_end, c->K, (const uint32_t*)c->oid, bin_out(c), c->skin_hint);
+  timer_end(c, t);
+}
+
+void launch_predict_bin(pbf_context* c, const StepInit& I) {
+  const uint32_t n = (uint32_t)c->n;
+  KernelTimer* t = timer_begin(c, "predict_bin");
+  hipLaunchKernelGGL(k_predict_bin, dim3(std::max(1u, nblocks(n))), dim3(kBlock), 0, c->stream, n, c->K,
+                     (const uint32_t*)c->oid, (const float4*)c->x, c->v, c->xs, bin_out(c), I);
+  timer_end(c, t);
+}
+
+void launch_sort(pbf_context* c) {
+  if (!c->n) return;
+  KernelTimer* t = timer_begin(c, "sort");
+  c->sorted = radix_sort_pairs(c->sk[0], c->sv[0], c->sk[1], c->sv[1], cell_sort_plan(c), c->rhist, c->rsum,
+                               c->stream);
   timer_end(c, t);
 }
 
 // find_bin_bounds (neighbors.h:137-148): begin[c] = lower_bound(keys, c);
 // end[c] = upper_bound(keys, c) = lower_bound(keys, c + 1) = begin[c + 1].
-// (the stamps of the cells next to moved particles start every step at zero)
-__global__ void k_cell_start(const uint32_t* __restrict__ sorted, uint32_t n, uint32_t ncells,
-                             uint32_t* __restrict__ start, uint32_t* __restrict__ cstamp) {
-  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c > ncells + 1) return;
-  cstamp[c] = 0u;
-  uint32_t lo = 0, hi = n;
+// The stamps of the cells next to moved particles start every step at zero;
+// in a fused step the particles of the outside bucket are counted here.
+struct CellOut {
+  const uint32_t* sorted;
+  uint32_t n, ncells, count_outside;
+  uint32_t *start, *cstamp;
+  unsigned long long* counters;
+};
+__device__ __forceinline__ void cell_bounds(uint32_t c, const CellOut& C) {
+  if (c > C.ncells + 1) return;
+  C.cstamp[c] = 0u;
+  uint32_t lo = 0, hi = C.n;
   while (lo < hi) {
     const uint32_t mid = (lo + hi) >> 1;
-    if (sorted[mid] < c) lo = mid + 1;
+    if (C.sorted[mid] < c) lo = mid + 1;
     else hi = mid;
   }
-  start[c] = lo;
+  C.start[c] = lo;
+  if (c == C.ncells && C.count_outside) C.counters[C_OUTSIDE] = C.n - lo;
 }
 
-void launch_sort(pbf_context* c) {
-  const uint32_t n = (uint32_t)c->n;
-  if (!n) return;
-  KernelTimer* t = timer_begin(c, "sort");
-  uint32_t bits = 1;
-  while (bits < 32 && (c->K.ncells >> bits) != 0) ++bits;  // keys go up to ncells (the outside bucket)
-  const int which = radix_sort_pairs(c->sk[0], c->sv[0], c->sk[1], c->sv[1], n, bits, c->rhist, c->roffs,
-                                     c->rpart, c->stream);
-  c->perm = c->sv[which];
-  hipLaunchKernelGGL(k_cell_start, dim3(nblocks((uint64_t)c->K.ncells + 2)), dim3(kBlock), 0, c->stream,
-                     (const uint32_t*)c->sk[which], n, c->K.ncells, c->cell_start, c->cstamp);
-  timer_end(c, t);
-}
-
-// gather the persistent state into cell order
-__global__ void __launch_bounds__(kBlock) k_reorder(uint32_t n, const uint32_t* __restrict__ perm,
+// Gathers the persistent state into cell order; the first cell_blocks blocks
+// find the cells' bounds meanwhile (chains of dependent loads, which the
+// gather's traffic covers: 8 us at 1,048,576 particles as a launch of its
+// own).
+struct ReorderOut {
+  float4 *x, *xs, *v, *scr;
+  float *rho, *lam, *lsum;
+  uint32_t *oid, *key, *sid;
+  uint32_t *dirty, *mflag;  // cleared when set (a captured step's stamps repeat)
+};
+__global__ void __launch_bounds__(kBlock) k_reorder(uint32_t n, uint32_t cell_blocks, CellOut C,
+                                                    const uint32_t* __restrict__ perm,
                                                     const float4* __restrict__ x, const float4* __restrict__ xs,
                                                     const float4* __restrict__ v, const float* __restrict__ rho,
                                                     const float* __restrict__ lam, const float4* __restrict__ scr,
                                                     const uint32_t* __restrict__ oid,
-                                                    const uint32_t* __restrict__ key,
                                                     const float* __restrict__ lsum,
-                                                    const uint32_t* __restrict__ sid, float4* __restrict__ xo,
-                                                    float4* __restrict__ xso, float4* __restrict__ vo,
-                                                    float* __restrict__ rhoo, float* __restrict__ lamo,
-                                                    float4* __restrict__ scro, uint32_t* __restrict__ oido,
-                                                    uint32_t* __restrict__ keyo, float* __restrict__ lsumo,
-                                                    uint32_t* __restrict__ sido) {
-  const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+                                                    const uint32_t* __restrict__ sid, ReorderOut O) {
+  if (blockIdx.x < cell_blocks) {
+    cell_bounds(blockIdx.x * blockDim.x + threadIdx.x, C);
+    return;
+  }
+  const uint32_t s = (blockIdx.x - cell_blocks) * blockDim.x + threadIdx.x;
   if (s >= n) return;
   const uint32_t p = perm[s];
-  if (lsum) lsumo[s] = lsum[p];
-  if (sid) sido[s] = sid[p];
-  xo[s] = x[p];
-  xso[s] = xs[p];
-  vo[s] = v[p];
+  if (lsum) O.lsum[s] = lsum[p];
+  if (sid) O.sid[s] = sid[p];
+  O.x[s] = x[p];
+  O.xs[s] = xs[p];
+  O.v[s] = v[p];
   if (rho) {
-    rhoo[s] = rho[p];
-    lamo[s] = lam[p];
-    scro[s] = scr[p];
+    O.rho[s] = rho[p];
+    O.lam[s] = lam[p];
+    O.scr[s] = scr[p];
   }
-  oido[s] = oid[p];
-  keyo[s] = key[p];
+  if (O.dirty) O.dirty[s] = O.mflag[s] = 0u;
+  O.oid[s] = oid[p];
+  if (O.key) O.key[s] = C.sorted[s];
 }
 
-void launch_reorder(pbf_context* c, bool all_fields) {
+// all_fields: densities, multipliers and the scratch vector move too; cells:
+// after a sort by cell (keys and cell bounds follow), otherwise only by perm
+static void reorder(pbf_context* c, const uint32_t* perm, bool all_fields, bool cells, bool fused) {
   const uint32_t n = (uint32_t)c->n;
   if (!n) return;
   KernelTimer* t = timer_begin(c, "reorder");
-  hipLaunchKernelGGL(k_reorder, dim3(nblocks(n)), dim3(kBlock), 0, c->stream, n, (const uint32_t*)c->perm,
+  const CellOut C{cells ? c->sk[c->sorted] : nullptr, n, c->K.ncells, fused ? 1u : 0u, c->cell_start, c->cstamp,
+                  c->counters};
+  const uint32_t cell_blocks = cells ? nblocks((uint64_t)c->K.ncells + 2) : 0u;
+  const bool clear = fused && c->capturing;
+  const ReorderOut O{c->xa,   c->xsa,  c->va,  c->scra, c->rhoa, c->lama, c->lsuma,
+                     c->oida, cells ? c->key : nullptr, c->sida, clear ? c->dirty : nullptr,
+                     clear ? c->mflag : nullptr};
+  hipLaunchKernelGGL(k_reorder, dim3(cell_blocks + nblocks(n)), dim3(kBlock), 0, c->stream, n, cell_blocks, C, perm,
                      (const float4*)c->x, (const float4*)c->xs, (const float4*)c->v,
-                     all_fields ? (const float*)c->rho : nullptr,
-                     (const float*)c->lam, (const float4*)c->scr, (const uint32_t*)c->oid,
-                     (const uint32_t*)c->key, c->track_lsum ? (const float*)c->lsum : nullptr,
-                     c->K.batched ? (const uint32_t*)c->sid : nullptr, c->xa, c->xsa, c->va, c->rhoa, c->lama,
-                     c->scra, c->oida, c->keya, c->lsuma, c->sida);
+                     all_fields ? (const float*)c->rho : nullptr, (const float*)c->lam, (const float4*)c->scr,
+                     (const uint32_t*)c->oid, c->track_lsum ? (const float*)c->lsum : nullptr,
+                     c->K.batched ? (const uint32_t*)c->sid : nullptr, O);
   timer_end(c, t);
   if (c->track_lsum) std::swap(c->lsum, c->lsuma);
   if (c->K.batched) {
@@ -272,8 +334,11 @@ void launch_reorder(pbf_context* c, bool all_fields) {
     std::swap(c->scr, c->scra);
   }
   std::swap(c->oid, c->oida);
-  std::swap(c->key, c->keya);
 }
+void launch_reorder_cells(pbf_context* c, bool all_fields, bool fused) {
+  reorder(c, c->sv[c->sorted], all_fields, true, fused);
+}
+void launch_reorder_by(pbf_context* c, const uint32_t* perm) { reorder(c, perm, true, false, false); }
 
 // ---------------------------------------------------------------------------
 // Bounding box of every cell's particles, 6 order-preserving integer
@@ -301,15 +366,20 @@ __device__ __forceinline__ float ord_dec(uint32_t u) {
   return __uint_as_float((u & 0x80000000u) ? (u & 0x7FFFFFFFu) : ~u);
 }
 
+// an empty box (word i of the boxes)
+__device__ __forceinline__ uint32_t box_empty(uint64_t i) { return (i % 6 < 3) ? 0xFFFFFFFFu : 0u; }
 __global__ void k_box_init(uint32_t* __restrict__ box, uint64_t count, const unsigned long long* __restrict__ counters) {
   if (counters[C_HEAVY] == 0ull) return;  // the boxes serve only the wavefront builder
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < count) box[i] = (i % 6 < 3) ? 0xFFFFFFFFu : 0u;
+  if (i < count) box[i] = box_empty(i);
 }
 
 // Slots are in cell order: each wavefront reduces its runs of equal keys and
-// the first lane of a run updates the cell's box.
-__global__ void __launch_bounds__(kBlock) k_cell_box(uint32_t n, uint32_t ncells, const uint32_t* __restrict__ key,
+// the first lane of a run updates the cell's box.  A block whose slots all lie
+// in one cell (a crowded cell holds thousands) updates it once: one update per
+// wavefront on the same six words queued up in the cache.
+constexpr int kBoxBlock = 1024;
+__global__ void __launch_bounds__(kBoxBlock) k_cell_box(uint32_t n, uint32_t ncells, const uint32_t* __restrict__ key,
                                                      const float4* __restrict__ xs, uint32_t* __restrict__ box,
                                                      float4* __restrict__ chbox,
                                                      const unsigned long long* __restrict__ counters) {
@@ -362,62 +432,32 @@ __global__ void __launch_bounds__(kBlock) k_cell_box(uint32_t n, uint32_t ncells
       }
     }
   }
-  // a wavefront inside one cell (all 64 keys equal) leaves the cell box to
-  // k_cell_box_chunks, which merges such chunks before touching the cell
-  const bool inside = __shfl(k, 0, 64) == __shfl(k, 63, 64) && __shfl(k, 63, 64) < ncells;
-  const uint32_t prev = __shfl_up(k, 1, 64);
-  if (!inside && valid && k < ncells && (lane == 0 || prev != k)) {
-    uint32_t* b = box + 6ull * k;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      atomicMin(&b[a], mn[a]);
-      atomicMax(&b[3 + a], mx[a]);
-    }
-  }
-}
-
-// The chunks that lie inside one cell (a crowded cell holds thousands): one
-// thread per chunk, runs of equal cells reduced per wavefront, one update of
-// the cell box per run -- instead of one per chunk on the same six words.
-__global__ void __launch_bounds__(kBlock) k_cell_box_chunks(uint32_t n, uint32_t ncells,
-                                                            const uint32_t* __restrict__ key,
-                                                            const float4* __restrict__ chbox,
-                                                            uint32_t* __restrict__ box,
-                                                            const unsigned long long* __restrict__ counters) {
-  if (counters[C_HEAVY] == 0ull) return;
-  const uint32_t ch = blockIdx.x * blockDim.x + threadIdx.x;
-  const int lane = threadIdx.x & 63;
-  const uint32_t nch = (n + 63) / 64;
-  uint32_t k = 0xFFFFFFFFu;
-  uint32_t mn[3] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu}, mx[3] = {0u, 0u, 0u};
-  if (ch < nch && 64ull * ch + 63 < n) {
-    const uint32_t k0 = key[64 * ch], k1 = key[64 * ch + 63];
-    if (k0 == k1 && k1 < ncells) {
-      k = k0;
-      const float4 lo = chbox[2 * ch], hi = chbox[2 * ch + 1];
-      mn[0] = ord_enc(lo.x), mn[1] = ord_enc(lo.y), mn[2] = ord_enc(lo.z);
-      mx[0] = ord_enc(hi.x), mx[1] = ord_enc(hi.y), mx[2] = ord_enc(hi.z);
-    }
-  }
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const uint32_t kk = __shfl_down(k, d, 64);
-    uint32_t omn[3], omx[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      omn[a] = __shfl_down(mn[a], d, 64);
-      omx[a] = __shfl_down(mx[a], d, 64);
-    }
-    if (lane + d < 64 && kk == k) {
+  const uint32_t first = blockIdx.x * blockDim.x, last = first + blockDim.x - 1;
+  const uint32_t kf = key[first];
+  if (last < n && key[last] == kf) {  // (the same for the whole block)
+    __shared__ uint32_t s_box[6][kBoxBlock / 64];
+    if (kf >= ncells) return;
+    const uint32_t w = threadIdx.x >> 6;
+    if (lane == 0)  // the wavefront is one run: its first lane holds the reduction
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
-        mn[a] = min(mn[a], omn[a]);
-        mx[a] = max(mx[a], omx[a]);
+        s_box[a][w] = mn[a];
+        s_box[3 + a][w] = mx[a];
       }
+    __syncthreads();
+    if (threadIdx.x < 6) {
+      uint32_t m = s_box[threadIdx.x][0];
+      for (int i = 1; i < kBoxBlock / 64; ++i)
+        m = threadIdx.x < 3 ? min(m, s_box[threadIdx.x][i]) : max(m, s_box[threadIdx.x][i]);
+      if (threadIdx.x < 3)
+        atomicMin(&box[6ull * kf + threadIdx.x], m);
+      else
+        atomicMax(&box[6ull * kf + threadIdx.x], m);
     }
+    return;
   }
   const uint32_t prev = __shfl_up(k, 1, 64);
-  if (k < ncells && (lane == 0 || prev != k)) {
+  if (valid && k < ncells && (lane == 0 || prev != k)) {
     uint32_t* b = box + 6ull * k;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
@@ -427,17 +467,20 @@ __global__ void __launch_bounds__(kBlock) k_cell_box_chunks(uint32_t n, uint32_t
   }
 }
 
-void launch_cell_box(pbf_context* c) {
+// Whether the list build clears the cell boxes on its way (a grid with few
+// cells beside its particles: 8 MB at 1,048,576 particles under a kernel of
+// 300 us); a sparse grid's are cleared only when they are needed.
+static bool boxes_in_fill(const pbf_context* c) { return (uint64_t)c->K.ncells <= 2 * c->n; }
+
+static void launch_cell_box(pbf_context* c) {
   const uint32_t n = (uint32_t)c->n;
-  if (!n) return;
   KernelTimer* t = timer_begin(c, "cell_box");
   const uint64_t count = 6ull * c->K.ncells;
   const unsigned long long* heavy = c->counters;
-  hipLaunchKernelGGL(k_box_init, dim3(nblocks(count)), dim3(kBlock), 0, c->stream, c->cbox, count, heavy);
-  hipLaunchKernelGGL(k_cell_box, dim3(nblocks(n)), dim3(kBlock), 0, c->stream, n, c->K.ncells,
+  if (!boxes_in_fill(c))
+    hipLaunchKernelGGL(k_box_init, dim3(nblocks(count)), dim3(kBlock), 0, c->stream, c->cbox, count, heavy);
+  hipLaunchKernelGGL(k_cell_box, dim3(nblocks(n, kBoxBlock)), dim3(kBoxBlock), 0, c->stream, n, c->K.ncells,
                      (const uint32_t*)c->key, (const float4*)c->xs, c->cbox, c->chbox, heavy);
-  hipLaunchKernelGGL(k_cell_box_chunks, dim3(nblocks((n + 63) / 64)), dim3(kBlock), 0, c->stream, n, c->K.ncells,
-                     (const uint32_t*)c->key, (const float4*)c->chbox, c->cbox, heavy);
   timer_end(c, t);
 }
 
@@ -528,6 +571,11 @@ struct ListWriter {
   }
 };
 
+// candidates a lane scans of a particle that may go to the wavefront builder
+__host__ __device__ __forceinline__ uint32_t lane_budget(const KParams& K) {
+  return K.heavy_budget < kMaxCellOffset - 8u ? K.heavy_budget : kMaxCellOffset - 8u;
+}
+
 // The lane walk of particle p: writes its list and count and returns true,
 // or returns false when the particle goes to the wavefront builder.  ovf
 // receives the candidates dropped by the cap.
@@ -557,7 +605,7 @@ __device__ __forceinline__ bool walk_list(uint32_t p, uint32_t n, uint32_t lane,
   for (int c = 0; c < 27; ++c) total += ce[c] - cb[c];
   // the lane's budget; below kMaxCellOffset - 8 so that a staged offset fits
   // in 10 bits (a batch of 8 may pass the budget before the test)
-  const uint32_t hb = min(K.heavy_budget, kMaxCellOffset - 8u);
+  const uint32_t hb = lane_budget(K);
   // every candidate must be seen to count the overflow: route by the total
   if (K.count_overflow && total > hb) return false;
   // otherwise the walk ends when the list is full; a lane whose 27 cells hold
@@ -861,8 +909,8 @@ __global__ void __launch_bounds__(kFillBlock) k_fill_neighbors(uint32_t n, uint3
                                                                const uint32_t* __restrict__ oid,
                                                                const uint32_t* __restrict__ key,
                                                                const uint32_t* __restrict__ start,
-                                                               const uint32_t* __restrict__ box, KParams K,
-                                                               int32_t* __restrict__ nbr,
+                                                               uint32_t* __restrict__ box, uint64_t box_words,
+                                                               KParams K, int32_t* __restrict__ nbr,
                                                                int32_t* __restrict__ nbr_count,
                                                                uint32_t* __restrict__ heavy,
                                                                unsigned long long* __restrict__ counters,
@@ -878,6 +926,8 @@ __global__ void __launch_bounds__(kFillBlock) k_fill_neighbors(uint32_t n, uint3
   const uint32_t lane = threadIdx.x;
   const uint32_t tb = xcd_block() * blockDim.x;
   const uint32_t p = tb + threadIdx.x;
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + lane; i < box_words; i += (uint64_t)gridDim.x * blockDim.x)
+    box[i] = box_empty(i);
   // skin lists only when the previous step kept them usable to its end
   const int skin = skin_mode && *hint != 0ull;
   if (skin && blockIdx.x == 0 && lane == 0) counters[C_SKIN] = 1ull;
@@ -1054,10 +1104,15 @@ void launch_fill_neighbors(pbf_context* c, uint64_t fb, uint64_t fe) {
   hipLaunchKernelGGL(k_fill_neighbors, dim3(nblocks(n, kFillBlock)), dim3(kFillBlock), stage, c->stream, n,
                      (uint32_t)fb,
                      (uint32_t)fe, (const float4*)c->xs, (const uint32_t*)c->oid, (const uint32_t*)c->key,
-                     (const uint32_t*)c->cell_start,
-                     (const uint32_t*)c->cbox, c->K, c->nbr, c->nbr_count, c->heavy, c->counters, skin,
+                     (const uint32_t*)c->cell_start, c->cbox, boxes_in_fill(c) ? 6ull * c->K.ncells : 0ull, c->K, c->nbr, c->nbr_count, c->heavy, c->counters, skin,
                      (const unsigned long long*)c->skin_hint, c->snb, c->snb_count, c->xs0);
   timer_end(c, t);
+  // no particle of a small scene has enough candidates for the wavefront
+  // builder: every particle is a candidate at most once (a grid of at least
+  // three cells an axis gives 27 different cells)
+  const bool wide = c->K.batched || (c->K.dimx >= 3 && c->K.dimy >= 3 && c->K.dimz >= 3);
+  const uint32_t hb = lane_budget(c->K);
+  if (wide && n <= (c->K.count_overflow ? hb : std::min(2u * hb, kMaxCellOffset))) return;
   // the cell and chunk boxes of the wavefront builder, built only when some particle went to it
   launch_cell_box(c);
   // enough waves to cover the chip; each loops over the heavy list (usually empty)
@@ -1071,92 +1126,194 @@ void launch_fill_neighbors(pbf_context* c, uint64_t fb, uint64_t fe) {
 }
 
 // ---------------------------------------------------------------------------
-// Stable LSD radix sort of (u32 key, u32 value) for the sort_by_key primitive.
-// Digit = 8 bits.  Per pass: tile histograms (digit-major), scan, stable
-// scatter.  Inside a tile, each element's rank among equal digits keeps
-// input order: waves rank with ballots, waves are combined through LDS.
-constexpr int kRadixItems = 4;                    // items per thread
-constexpr int kRadixTile = kBlock * kRadixItems;  // 1024 keys per tile
+// Stable LSD radix sort of (u32 key, u32 value), up to 8 bits a pass, two
+// launches a pass.
+//
+// Count: a tile's digit histogram, and its sum over groups of tiles (atomics
+// of one group's few tiles).  Place: a block adds up what lies before its tile
+// in its digits -- the groups before its own, then the tiles before it in the
+// group, one coalesced kilobyte of counts each -- scans the digits, ranks its
+// keys and stores them.  The counts of a million keys are 16 + 15 rows of that
+// at most; the tile-by-tile scan between counting and placing that they
+// replace took three launches of 4.5 us each.
+//
+// Ranks: a wavefront takes its keys of a tile 64 at a time, finds the lanes of
+// equal digit with one ballot per digit bit and keeps its running counts in
+// LDS, so that the block meets at a barrier twice a tile instead of four times
+// every 256 keys.
+//
+// Tiles of 1,024 keys while there are few (a tile is a block: 32,768 keys give
+// 32), of 4,096 above 262,144.  Past 2,048 tiles the rows before a tile are
+// too many to add up in every block; k_radix_prefix then turns the groups'
+// rows into prefixes first.
+RadixPlan radix_plan(uint64_t n, uint32_t key_bits) {
+  RadixPlan P{};
+  P.n = n;
+  P.items = n <= (1ull << 18) ? 4u : 16u;
+  const uint64_t tile = (uint64_t)kBlock * P.items;
+  P.ntiles = (uint32_t)((n + tile - 1) / tile);
+  P.passes = (key_bits + 7) / 8;
+  P.bits = (key_bits + P.passes - 1) / P.passes;
+  P.key_bits = key_bits;
+  P.prefixed = P.ntiles > 2048u;
+  if (P.prefixed) {
+    P.per_group = (P.ntiles + 63) / 64;
+  } else {
+    P.per_group = 1;
+    while (P.per_group * P.per_group < P.ntiles) P.per_group *= 2;
+  }
+  // (at most 64: 46 of a square root's size, or the prefixed sort's 64)
+  P.ngroups = P.ntiles ? (P.ntiles + P.per_group - 1) / P.per_group : 0u;
+  return P;
+}
 
-__global__ void __launch_bounds__(kBlock) k_radix_hist(const uint32_t* __restrict__ keys, uint64_t n, int shift,
-                                                       uint32_t ntiles, uint32_t* __restrict__ hist) {
+template <int ITEMS>
+__global__ void __launch_bounds__(kBlock) k_radix_count(const uint32_t* __restrict__ keys, uint64_t n, uint32_t shift,
+                                                        uint32_t mask, uint32_t per_group,
+                                                        uint32_t* __restrict__ hist, uint32_t* __restrict__ gsum) {
   __shared__ uint32_t h[256];
   h[threadIdx.x] = 0;
   __syncthreads();
-  const uint64_t base = (uint64_t)blockIdx.x * kRadixTile;
-  for (int i = 0; i < kRadixItems; ++i) {
+  const uint64_t base = (uint64_t)blockIdx.x * (kBlock * ITEMS);
+  uint32_t k[ITEMS];
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
     const uint64_t idx = base + (uint64_t)i * kBlock + threadIdx.x;
-    if (idx < n) atomicAdd(&h[(keys[idx] >> shift) & 255u], 1u);
+    k[i] = idx < n ? keys[idx] : 0u;
   }
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i)
+    if (base + (uint64_t)i * kBlock + threadIdx.x < n) atomicAdd(&h[(k[i] >> shift) & mask], 1u);
   __syncthreads();
-  hist[(uint64_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
+  const uint32_t c = h[threadIdx.x];
+  hist[(uint64_t)blockIdx.x * 256u + threadIdx.x] = c;
+  if (c) atomicAdd(&gsum[(uint64_t)(blockIdx.x / per_group) * 256u + threadIdx.x], c);
 }
 
-// Scatter one tile.  Elements are processed in rounds of 256 (one per
-// thread, in input order); within a round, rank = number of earlier lanes of
-// the round with the same digit, found with 8 ballots per wave.
-__global__ void __launch_bounds__(kBlock) k_radix_scatter(const uint32_t* __restrict__ keys,
-                                                          const uint32_t* __restrict__ vals, uint64_t n, int shift,
-                                                          uint32_t ntiles, const uint32_t* __restrict__ offs,
-                                                          uint32_t* __restrict__ okeys, uint32_t* __restrict__ ovals) {
-  __shared__ uint32_t base_d[256];       // running output offset per digit for this tile
-  __shared__ uint32_t wave_cnt[4][256];  // per wave, count of each digit in this round
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  base_d[threadIdx.x] = offs[(uint64_t)threadIdx.x * ntiles + blockIdx.x];
-  const uint64_t tbase = (uint64_t)blockIdx.x * kRadixTile;
-  for (int r = 0; r < kRadixItems; ++r) {
-    for (int i = 0; i < 4; ++i) wave_cnt[i][threadIdx.x] = 0;
-    __syncthreads();
-    const uint64_t idx = tbase + (uint64_t)r * kBlock + threadIdx.x;
-    const bool valid = idx < n;
-    const uint32_t k = valid ? keys[idx] : 0u;
-    const uint32_t d = (k >> shift) & 255u;
-    // lanes of this wave with the same digit
-    uint64_t peers = __ballot(valid);
+// a group's rows become the counts before each tile within the group
+__global__ void __launch_bounds__(kBlock) k_radix_prefix(uint32_t ntiles, uint32_t per_group,
+                                                         uint32_t* __restrict__ hist) {
+  const uint32_t t0 = blockIdx.x * per_group, t1 = min(ntiles, t0 + per_group);
+  uint32_t run = 0;
+  for (uint32_t t = t0; t < t1; t += 16) {
+    uint32_t c[16];
 #pragma unroll
-    for (int b = 0; b < 8; ++b) {
+    for (uint32_t i = 0; i < 16; ++i) c[i] = t + i < t1 ? hist[(uint64_t)(t + i) * 256u + threadIdx.x] : 0u;
+#pragma unroll
+    for (uint32_t i = 0; i < 16; ++i) {
+      if (t + i < t1) hist[(uint64_t)(t + i) * 256u + threadIdx.x] = run;
+      run += c[i];
+    }
+  }
+}
+
+template <int ITEMS>
+__global__ void __launch_bounds__(kBlock) k_radix_place(const uint32_t* __restrict__ keys,
+                                                        const uint32_t* __restrict__ vals, RadixPlan P,
+                                                        uint32_t shift, uint32_t bits,
+                                                        const uint32_t* __restrict__ hist,
+                                                        const uint32_t* __restrict__ gsum,
+                                                        uint32_t* __restrict__ okeys, uint32_t* __restrict__ ovals) {
+  constexpr int kWaves = kBlock / 64;
+  // per wavefront: its running count of each digit, then its first output slot
+  // (every access of a wavefront's row between the barriers is that
+  // wavefront's own, in program order)
+  __shared__ volatile uint32_t s_cnt[kWaves][256];
+  const uint32_t d0 = threadIdx.x, lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+  const uint64_t base = (uint64_t)blockIdx.x * (kBlock * ITEMS) + w * (64u * ITEMS) + lane;
+  uint32_t k[ITEMS], v[ITEMS];
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    const uint64_t idx = base + (uint64_t)i * 64u;
+    k[i] = idx < P.n ? keys[idx] : 0u;
+    v[i] = idx < P.n ? vals[idx] : 0u;
+  }
+#pragma unroll
+  for (int i = 0; i < kWaves; ++i) s_cnt[i][threadIdx.x] = 0u;
+  // digit d0: all of it, and what lies before this tile
+  const uint32_t group = blockIdx.x / P.per_group;
+  uint32_t total = 0, before = 0;
+  for (uint32_t g0 = 0; g0 < P.ngroups; g0 += 8) {
+    uint32_t c[8];
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i) c[i] = g0 + i < P.ngroups ? gsum[(uint64_t)(g0 + i) * 256u + d0] : 0u;
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i) {
+      total += c[i];
+      before += g0 + i < group ? c[i] : 0u;
+    }
+  }
+  if (P.prefixed) {
+    before += hist[(uint64_t)blockIdx.x * 256u + d0];
+  } else {
+    for (uint32_t t0 = group * P.per_group; t0 < blockIdx.x; t0 += 8) {
+      uint32_t c[8];
+#pragma unroll
+      for (uint32_t i = 0; i < 8; ++i) c[i] = t0 + i < blockIdx.x ? hist[(uint64_t)(t0 + i) * 256u + d0] : 0u;
+#pragma unroll
+      for (uint32_t i = 0; i < 8; ++i) before += c[i];
+    }
+  }
+  uint32_t all;
+  before += block_excl_scan(total, &all);  // (its barriers also cover the cleared counts)
+  const uint32_t mask = (1u << bits) - 1u;
+  const uint64_t lower = (1ull << lane) - 1ull;
+  uint32_t rank[ITEMS];
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    const bool valid = base + (uint64_t)i * 64u < P.n;
+    const uint32_t d = (k[i] >> shift) & mask;
+    uint64_t peers = __ballot(valid);
+    for (uint32_t b = 0; b < bits; ++b) {
       const uint64_t bal = __ballot(((d >> b) & 1u) != 0u);
       peers &= ((d >> b) & 1u) ? bal : ~bal;
     }
-    const uint64_t lower = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    const uint32_t rank_in_wave = (uint32_t)__popcll(peers & lower);
-    const uint32_t wave_total = (uint32_t)__popcll(peers);
-    if (valid && rank_in_wave == 0) wave_cnt[w][d] = wave_total;
-    __syncthreads();
-    if (valid) {
-      uint32_t before = 0;
-      for (int i = 0; i < w; ++i) before += wave_cnt[i][d];
-      const uint32_t pos = base_d[d] + before + rank_in_wave;
-      okeys[pos] = k;
-      ovals[pos] = vals[idx];
-    }
-    __syncthreads();
-    // advance the digit offsets by this round's counts
-    {
-      const uint32_t dd = threadIdx.x;
-      base_d[dd] += wave_cnt[0][dd] + wave_cnt[1][dd] + wave_cnt[2][dd] + wave_cnt[3][dd];
-    }
-    __syncthreads();
+    const uint32_t done = s_cnt[w][d], mine = (uint32_t)__popcll(peers & lower);
+    rank[i] = done + mine;
+    if (valid && mine == 0u) s_cnt[w][d] = done + (uint32_t)__popcll(peers);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kWaves; ++i) {
+    const uint32_t c = s_cnt[i][d0];
+    s_cnt[i][d0] = before;
+    before += c;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    if (base + (uint64_t)i * 64u >= P.n) continue;
+    const uint32_t pos = s_cnt[w][(k[i] >> shift) & mask] + rank[i];
+    okeys[pos] = k[i];
+    ovals[pos] = v[i];
   }
 }
 
-uint64_t radix_hist_size(uint64_t n) { return 256ull * ((n + kRadixTile - 1) / kRadixTile); }
+uint64_t radix_hist_size(uint64_t n) { return 256ull * ((n + 1023) / 1024); }
+template <int ITEMS>
+static void radix_pass(const uint32_t* ki, const uint32_t* vi, uint32_t* ko, uint32_t* vo, const RadixPlan& P,
+                       uint32_t shift, uint32_t bits, uint32_t* hist, uint32_t* gsum, hipStream_t s) {
+  hipLaunchKernelGGL(k_radix_count<ITEMS>, dim3(P.ntiles), dim3(kBlock), 0, s, ki, P.n, shift, (1u << bits) - 1u,
+                     P.per_group, hist, gsum);
+  if (P.prefixed) hipLaunchKernelGGL(k_radix_prefix, dim3(P.ngroups), dim3(kBlock), 0, s, P.ntiles, P.per_group, hist);
+  hipLaunchKernelGGL(k_radix_place<ITEMS>, dim3(P.ntiles), dim3(kBlock), 0, s, ki, vi, P, shift, bits,
+                     (const uint32_t*)hist, (const uint32_t*)gsum, ko, vo);
+}
 
-// Stable LSD sort of (keys, vals) over key_bits bits, ping-ponging between
-// (k0, v0) and (k1, v1).  Returns 0 or 1: the buffer pair holding the result.
-int radix_sort_pairs(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, uint64_t n, uint32_t key_bits,
-                     uint32_t* hist, uint32_t* offs, uint32_t* partials, hipStream_t s) {
-  if (n <= 1) return 0;
-  const uint32_t ntiles = (uint32_t)((n + kRadixTile - 1) / kRadixTile);
-  const uint64_t hn = 256ull * ntiles;
+// Stable LSD sort of (keys, vals) by P.key_bits bits, ping-ponging between
+// (k0, v0) and (k1, v1); gsum starts at zero.  Returns 0 or 1: the buffer pair
+// holding the result.
+int radix_sort_pairs(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, const RadixPlan& P, uint32_t* hist,
+                     uint32_t* gsum, hipStream_t s) {
+  if (P.n <= 1) return 0;
   uint32_t *ki = k0, *vi = v0, *ko = k1, *vo = v1;
   int which = 0;
-  for (uint32_t shift = 0; shift < key_bits; shift += 8) {
-    hipLaunchKernelGGL(k_radix_hist, dim3(ntiles), dim3(kBlock), 0, s, (const uint32_t*)ki, n, (int)shift, ntiles,
-                       hist);
-    launch_exclusive_scan(hist, offs, hn, partials, s);
-    hipLaunchKernelGGL(k_radix_scatter, dim3(ntiles), dim3(kBlock), 0, s, (const uint32_t*)ki,
-                       (const uint32_t*)vi, n, (int)shift, ntiles, (const uint32_t*)offs, ko, vo);
+  for (uint32_t shift = 0; shift < P.key_bits; shift += P.bits, gsum += 256ull * P.ngroups) {
+    const uint32_t bits = std::min(P.bits, P.key_bits - shift);
+    if (P.items == 4)
+      radix_pass<4>(ki, vi, ko, vo, P, shift, bits, hist, gsum, s);
+    else
+      radix_pass<16>(ki, vi, ko, vo, P, shift, bits, hist, gsum, s);
     std::swap(ki, ko);
     std::swap(vi, vo);
     which ^= 1;
@@ -1164,28 +1321,30 @@ int radix_sort_pairs(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, uin
   return which;
 }
 
+// the sort_by_key primitive, the result back in keys and vals
+int radix_sort_in_place(uint32_t* keys, uint32_t* vals, uint64_t n, uint32_t key_bits, uint32_t* k2, uint32_t* v2,
+                        uint32_t* hist, uint32_t* gsum, hipStream_t s) {
+  const RadixPlan P = radix_plan(n, key_bits);
+  launch_fill_u32(gsum, 0u, P.sum_words(), s);
+  int rc = PBF_OK;
+  if (radix_sort_pairs(keys, vals, k2, v2, P, hist, gsum, s)) {
+    rc = check_hip(hipMemcpyAsync(keys, k2, n * 4, hipMemcpyDeviceToDevice, s), "sort_by_key copy");
+    if (!rc) rc = check_hip(hipMemcpyAsync(vals, v2, n * 4, hipMemcpyDeviceToDevice, s), "sort_by_key copy");
+  }
+  if (!rc) rc = check_hip(hipGetLastError(), "radix sort launch");
+  return rc;
+}
+
 int radix_sort_u32(uint32_t* keys, uint32_t* vals, uint64_t n, uint32_t key_bits, hipStream_t s) {
   if (n <= 1) return PBF_OK;
   if (n > 0xFFFFFFFFull) return set_error(PBF_ERR_UNSUPPORTED, "sort_by_key: n must be < 2^32");
   if (key_bits == 0 || key_bits > 32) key_bits = 32;
-  const uint64_t hn = radix_hist_size(n);
-  uint32_t *k2 = nullptr, *v2 = nullptr, *hist = nullptr, *offs = nullptr, *part = nullptr;
-  int rc = PBF_OK;
-  if ((rc = check_hip(hipMallocAsync((void**)&k2, n * 4, s), "hipMallocAsync")) ||
-      (rc = check_hip(hipMallocAsync((void**)&v2, n * 4, s), "hipMallocAsync")) ||
-      (rc = check_hip(hipMallocAsync((void**)&hist, hn * 4, s), "hipMallocAsync")) ||
-      (rc = check_hip(hipMallocAsync((void**)&offs, (hn + 1) * 4, s), "hipMallocAsync")) ||
-      (rc = check_hip(hipMallocAsync((void**)&part, scan_partials_size(hn) * 4, s), "hipMallocAsync"))) {
-    // the buffers allocated before the failure are freed below
-  } else {
-    if (radix_sort_pairs(keys, vals, k2, v2, n, key_bits, hist, offs, part, s)) {
-      rc = check_hip(hipMemcpyAsync(keys, k2, n * 4, hipMemcpyDeviceToDevice, s), "sort_by_key copy");
-      if (!rc) rc = check_hip(hipMemcpyAsync(vals, v2, n * 4, hipMemcpyDeviceToDevice, s), "sort_by_key copy");
-    }
-    if (!rc) rc = check_hip(hipGetLastError(), "radix sort launch");
-  }
-  for (uint32_t* b : {k2, v2, hist, offs, part})
-    if (b) (void)hipFreeAsync(b, s);
+  uint32_t* ws = nullptr;
+  const uint64_t hist = radix_hist_size(n);
+  int rc = check_hip(hipMallocAsync((void**)&ws, (2 * n + hist + kRadixSumWords) * 4, s), "hipMallocAsync");
+  if (rc) return rc;
+  rc = radix_sort_in_place(keys, vals, n, key_bits, ws, ws + n, ws + 2 * n, ws + 2 * n + hist, s);
+  (void)hipFreeAsync(ws, s);
   return rc;
 }
 

@@ -9,10 +9,10 @@
 //   scr              float4[n]   scratch vector: dp, vorticity or colour field
 //   rho, lam         float[n]
 //   oid, oida        uint32[n]   original index of each sorted slot
-//   key, keya        uint32[n]   cell key of each slot
-//   slot             uint32[n]   inverse permutation (original index -> slot)
+//   key              uint32[n]   cell key of each slot
+//   slot             uint32[n]   the kept slots of pbf_remove
 //   sk[2], sv[2]     uint32[n]   radix-sort ping-pong buffers (cell key, slot)
-//   rhist, roffs     uint32[256 * tiles]  radix digit histograms and their scan
+//   rhist, rsum      uint32      radix digit histograms of the tiles, and their sums over groups
 //   cell_start       uint32[C+2] first sorted slot of every cell (C = the outside bucket)
 //   heavy            uint32[n]   particles whose 27 cells hold too many candidates
 //                                for one lane (built by a whole wavefront instead)
@@ -199,11 +199,11 @@ struct pbf_context {
   float4 *xt = nullptr, *scr = nullptr;
   float *rho = nullptr, *lam = nullptr, *rhoa = nullptr, *lama = nullptr;
   float4* scra = nullptr;
-  uint32_t *oid = nullptr, *oida = nullptr, *key = nullptr, *keya = nullptr;
+  uint32_t *oid = nullptr, *oida = nullptr, *key = nullptr;
   uint32_t *slot = nullptr, *tmp = nullptr, *tmpo = nullptr;
   uint32_t *sk[2] = {nullptr, nullptr}, *sv[2] = {nullptr, nullptr};
-  uint32_t *rhist = nullptr, *roffs = nullptr, *rpart = nullptr;
-  uint32_t* perm = nullptr;  // sorted slot -> previous slot (points into sv or tmpo)
+  uint32_t *rhist = nullptr, *rsum = nullptr;
+  int sorted = 0;  // which of sk, sv the last sort left its result in
   uint32_t* heavy = nullptr;
   uint32_t* cstamp = nullptr;  // [cells + 1] == dirty_stamp: a particle within two cells was moved
   uint32_t* dirty = nullptr;  // == dirty_stamp: the particle or one of its neighbours moved
@@ -297,16 +297,37 @@ void launch_fill_u64(unsigned long long* p, unsigned long long value, uint64_t n
 // exclusive scan of in[0..n) into out[0..n]; out[n] = total.  partials needs scan_partials_size(n).
 uint64_t scan_partials_size(uint64_t n);
 void launch_exclusive_scan(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* partials, hipStream_t s);
-// fused: part of a fused step (its counters are clear and its hint set)
-void launch_bin(pbf_context* c, uint64_t bin_end, bool fused);  // key, inverse permutation, keys by original index
-void launch_sort(pbf_context* c);            // radix sort -> perm, cell_start
-void launch_cell_box(pbf_context* c);        // bounding box of each cell's particles
-// gather state by perm (without all_fields: densities, multipliers and the
-// scratch vector stay where they are)
-void launch_reorder(pbf_context* c, bool all_fields = true);
-uint64_t radix_hist_size(uint64_t n);
-int radix_sort_pairs(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, uint64_t n, uint32_t key_bits,
-                     uint32_t* hist, uint32_t* offs, uint32_t* partials, hipStream_t s);
+void launch_bin(pbf_context* c, uint64_t bin_end);  // (key, slot) pairs by original index
+// What a fused step starts from: iterations and warm for the solve's counters,
+// and the first error_words words of its error history cleared.
+struct StepInit {
+  unsigned long long iterations, warm;
+  uint32_t* ehist;
+  unsigned long long* esum;
+  uint32_t error_words;
+};
+void launch_predict_bin(pbf_context* c, const StepInit& I);  // forces, prediction and bins of a fused step
+void launch_sort(pbf_context* c);                            // radix sort -> c->sorted
+// gather the state into cell order, keys and cell bounds with it (without
+// all_fields: densities, multipliers and the scratch vector stay where they
+// are), or by a permutation of slots
+void launch_reorder_cells(pbf_context* c, bool all_fields, bool fused);
+void launch_reorder_by(pbf_context* c, const uint32_t* perm);
+// How a sort of n keys is cut into tiles, groups of tiles and passes.
+struct RadixPlan {
+  uint64_t n;
+  uint32_t items, ntiles, per_group, ngroups, passes, bits, key_bits;
+  bool prefixed;
+  uint32_t sum_words() const { return passes * ngroups * 256u; }
+};
+RadixPlan radix_plan(uint64_t n, uint32_t key_bits);
+uint64_t radix_hist_size(uint64_t n);  // words, for any sort of up to n keys
+// words of the group sums of any sort: four passes, at most 64 groups
+constexpr uint64_t kRadixSumWords = 4ull * 64ull * 256ull;
+int radix_sort_pairs(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, const RadixPlan& P, uint32_t* hist,
+                     uint32_t* gsum, hipStream_t s);
+int radix_sort_in_place(uint32_t* keys, uint32_t* vals, uint64_t n, uint32_t key_bits, uint32_t* k2, uint32_t* v2,
+                        uint32_t* hist, uint32_t* gsum, hipStream_t s);
 void launch_fill_neighbors(pbf_context* c, uint64_t fb, uint64_t fe);
 int radix_sort_u32(uint32_t* keys, uint32_t* vals, uint64_t n, uint32_t key_bits, hipStream_t s);
 void launch_bounds_counting(const uint32_t* sorted, uint64_t n, uint64_t b, uint64_t e, uint32_t* out,
@@ -314,7 +335,7 @@ void launch_bounds_counting(const uint32_t* sorted, uint64_t n, uint64_t b, uint
 
 // ---- launchers (pbf_passes.hip) ----
 // flags for the particle-local kernel
-enum { F_FORCES = 1, F_PREDICT = 2, F_CLEAR = 4 };  // F_CLEAR: zero the counters first
+enum { F_FORCES = 1, F_PREDICT = 2 };
 void launch_forces_predict(pbf_context* c, int flags, uint64_t b, uint64_t e);
 void launch_density(pbf_context* c, uint64_t b, uint64_t e);  // xs -> xt, rho
 // ---- fused-step launchers (pbf_fused.hip): they build and use the compact lists ----
@@ -323,10 +344,11 @@ void launch_density_lambda_masked(pbf_context* c, int it, int eslot, const Solve
 void launch_combine_errors(pbf_context* c);                            // ehist, esum -> ehist_row, esum_row
 void launch_lambda_repair(pbf_context* c, int it, const SolveCtl& S);  // lam from xt for dirty particles
 void launch_dp_update_masked(pbf_context* c, int it, int last, const SolveCtl& S);
-void launch_warm_dp(pbf_context* c);      // xt, wlam -> xs (warm start), xsave = xt
-void launch_add_warm(pbf_context* c);     // lsum += wlam when the warm start was kept
-void launch_log_solve(pbf_context* c);    // one pbf_solve_record of the solve just queued
-void launch_warm_retry(pbf_context* c);   // the damped warm start after a rejected one (a no-op otherwise)
+void launch_warm_dp(pbf_context* c, const float* warm);      // xt, multipliers -> xs (warm start), xsave = xt
+// the end of a solve: velocities, the kept warm multipliers (null: none) into
+// the sums, and its record
+void launch_solve_end(pbf_context* c, const float* warm);
+void launch_warm_retry(pbf_context* c, const float* warm);   // the damped warm start after a rejected one (a no-op otherwise)
 // the Jacobi loop in one cooperative launch (PBF_OPT_PERSISTENT); advances dirty_stamp by iters
 bool persistent_available(pbf_context* c);
 uint32_t persistent_capacity(pbf_context* c);  // blocks of it the device holds at once (occupancy query)
@@ -346,9 +368,6 @@ void launch_vorticity(pbf_context* c, const float4* vin, uint64_t b, uint64_t e)
 void launch_apply_vorticity(pbf_context* c, float4* vio, uint64_t b, uint64_t e);
 // skin: the colour field may walk the skin lists
 void launch_surface_tension(pbf_context* c, uint64_t cb, uint64_t ce, uint64_t b, uint64_t e, bool skin);
-void launch_copy_f4(const float4* src, float4* dst, uint64_t n, hipStream_t s);
-void launch_copy_f1(const float* src, float* dst, uint64_t n, hipStream_t s);
-void launch_scale_f1(const float* src, float* dst, float scale, uint64_t n, hipStream_t s);
 // ---- learned warm start (pbf_mlp.hip) ----
 // original-order transfer helpers
 void launch_gather_out_f4(pbf_context* c, const float4* src, float* dst3, int comps);

@@ -73,10 +73,8 @@ constexpr uint64_t kPassQuads = 131072;
 __global__ void __launch_bounds__(kBlock) k_forces_predict(uint32_t n, uint32_t b, uint32_t e, int flags, KParams K,
                                                            const uint32_t* __restrict__ oid,
                                                            const float4* __restrict__ x, float4* __restrict__ v,
-                                                           float4* __restrict__ xs,
-                                                           unsigned long long* __restrict__ counters) {
+                                                           float4* __restrict__ xs) {
   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-  if ((flags & F_CLEAR) && p < (uint32_t)C_NUM) counters[p] = 0ull;  // a fused step's counters start at zero
   if (p >= n || !in_span(oid[p], b, e)) return;
   f3 vp = ld3(v, p);
   if (flags & F_FORCES) {
@@ -95,7 +93,7 @@ void launch_forces_predict(pbf_context* c, int flags, uint64_t b, uint64_t e) {
   if (!n) return;
   KernelTimer* t = timer_begin(c, "forces_predict");
   hipLaunchKernelGGL(k_forces_predict, dim3(nblocks(n)), dim3(kBlock), 0, c->stream, n, (uint32_t)b, (uint32_t)e,
-                     flags, c->K, (const uint32_t*)c->oid, (const float4*)c->x, c->v, c->xs, c->counters);
+                     flags, c->K, (const uint32_t*)c->oid, (const float4*)c->x, c->v, c->xs);
   timer_end(c, t);
 }
 
@@ -492,29 +490,6 @@ void launch_surface_tension(pbf_context* c, uint64_t cb, uint64_t ce, uint64_t b
   launch_color(c, cb, ce, skin);
   launch_tension(c, b, e);
   timer_end(c, t);
-}
-
-__global__ void k_copy_f4(const float4* __restrict__ src, float4* __restrict__ dst, uint64_t n) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = src[i];
-}
-void launch_copy_f4(const float4* src, float4* dst, uint64_t n, hipStream_t s) {
-  if (n) hipLaunchKernelGGL(k_copy_f4, dim3(nblocks(n)), dim3(kBlock), 0, s, src, dst, n);
-}
-
-__global__ void k_copy_f1(const float* __restrict__ src, float* __restrict__ dst, uint64_t n) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = src[i];
-}
-void launch_copy_f1(const float* src, float* dst, uint64_t n, hipStream_t s) {
-  if (n) hipLaunchKernelGGL(k_copy_f1, dim3(nblocks(n)), dim3(kBlock), 0, s, src, dst, n);
-}
-__global__ void k_scale_f1(const float* __restrict__ src, float* __restrict__ dst, float scale, uint64_t n) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = src[i] * scale;
-}
-void launch_scale_f1(const float* src, float* dst, float scale, uint64_t n, hipStream_t s) {
-  if (n) hipLaunchKernelGGL(k_scale_f1, dim3(nblocks(n)), dim3(kBlock), 0, s, src, dst, scale, n);
 }
 
 // ---- original-order transfers through the staging buffer ----

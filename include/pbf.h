@@ -105,10 +105,9 @@ typedef struct pbf_params {
  * bit for bit.  This option turns the skin lists off (for comparison). */
 #define PBF_OPT_FULL_LISTS 32u
 /* The list builder walks every particle's 27 cells with one lane of its own.  By default
- * the particles of ordinary cells are listed by a walk shared by all particles of a cell
- * (each candidate tested by one lane against the cell's particles in turn); the lists are
- * the same, bit for bit.  This option keeps the per-lane walk for every particle (for
- * comparison). */
+ * the particles of a cell are listed by a walk that they share (each candidate tested by
+ * one lane against the cell's particles in turn); the lists are the same, bit for bit.
+ * This option keeps the per-lane walk for every particle (for comparison). */
 #define PBF_OPT_LANE_LISTS 64u
 /* pbf_step and pbf_solve run their Jacobi iterations (the density, dirty-marking,
  * lambda-repair and pressure-update passes of every iteration or solve slot) in one
@@ -139,7 +138,7 @@ typedef struct pbf_stats {
   uint64_t density_hacks;      /* triggers of the near-coincidence fix (particles.h:303-305) */
   uint64_t iterations;         /* Jacobi iterations run in the last step */
   double max_density_error;    /* max_p max(rho_p/rho0 - 1, 0) of the last density pass */
-  uint64_t tile_listed;        /* particles the last list build listed with the cell-tile walk
+  uint64_t tile_listed;        /* particles the last list build listed with the shared cell walk
                                   (PBF_OPT_LANE_LISTS); counted only with PBF_OPT_COUNT_OVERFLOW */
   uint64_t persistent_grid;    /* blocks of the last cooperative Jacobi launch (PBF_OPT_PERSISTENT; 0: none) */
   uint64_t persistent_capacity; /* blocks of that kernel the device runs at once (0 without the option) */
@@ -364,11 +363,12 @@ int pbf_step_graph(pbf_context* ctx, uint32_t nsteps);
 
 /* ---- launch tuning (no counterpart in the reference) ----
  * Launch parameters that do not change any result: the block size of the fused
- * per-particle kernels (64, 128 or 256), the candidate budget after which the neighbour
- * walk of one particle is handed from one lane to a whole wavefront (64..65536, used up to
- * 2040; it applies to particles whose 27 cells hold more than twice that many candidates,
- * or more than 2048), and the number
- * of blocks of that wavefront builder (1..65536).  The bin spacing and the list cap
+ * per-particle kernels (64, 128 or 256), the candidate budget that decides when a particle
+ * gets a whole wavefront for its neighbour walk (64..65536: with more than four times that
+ * many candidates in its 27 cells, when twice that many are tested and its list is not full;
+ * with PBF_OPT_COUNT_OVERFLOW with more than twice that many; with PBF_OPT_LANE_LISTS when
+ * one lane has scanned that many, at most 2040, of more than twice as many or more than
+ * 2048), and the number of blocks of that wavefront builder (1..65536).  The bin spacing and the list cap
  * are not tuned: both are part of the reference's neighbour semantics (neighbors.h:39,198).
  * pbf_autotune times `steps` fused steps from the current state for each candidate,
  * restores the state (the following steps are bit-identical to an untuned run), keeps

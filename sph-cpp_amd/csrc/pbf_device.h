@@ -31,6 +31,8 @@ __device__ __forceinline__ float4 gather4(const float4* __restrict__ a, uint32_t
   return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(a) + (i << 4));
 }
 
+__device__ __forceinline__ f3 xyz3(float4 t) { return {t.x, t.y, t.z}; }
+
 // vec.h operator-, operator+, vec*scalar, scalar*vec, vec/scalar, +=, -=
 __device__ __forceinline__ f3 sub3(f3 a, f3 b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
 __device__ __forceinline__ f3 add3(f3 a, f3 b) { return {a.x + b.x, a.y + b.y, a.z + b.z}; }
@@ -226,7 +228,7 @@ __device__ __forceinline__ float bin_coord(float p, float s) { return floorf((p 
 __device__ __forceinline__ uint32_t cell_key(float fx, float fy, float fz, const GridView& G, const KParams& K) {
   if (!(fx >= 0.f) || !(fy >= 0.f) || !(fz >= 0.f)) return K.ncells;
   if (fx > 4.0e9f || fy > 4.0e9f || fz > 4.0e9f) return K.ncells;
-  const uint64_t bx = (uint64_t)fx, by = (uint64_t)fy, bz = (uint64_t)fz;
+  const uint64_t bx = (uint32_t)fx, by = (uint32_t)fy, bz = (uint32_t)fz;  // (below 2^32)
   const uint64_t k = G.dxy * bz + (by * (uint64_t)G.dimx + bx);
   return k < (uint64_t)G.ncells ? G.off + (uint32_t)k : K.ncells;
 }

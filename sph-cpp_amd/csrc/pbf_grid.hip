@@ -14,13 +14,12 @@
 // a pass, per-tile histograms, wavefront ballot ranking): the result is
 // exactly the (key, original index) order the reference produces.
 //
-// Lists.  One lane per particle walks the 27 cells in the reference's order
-// and stages its entries in LDS, then writes them tiled by groups of 64
-// particles, four entries at a time (list_at).  A
-// particle with many candidates whose walk passes a budget is handed to a
-// list of heavy particles that one wavefront each finishes with
-// ballot-compacted appends, so that collapsed cells do not serialise a
-// wavefront on one lane.
+// Lists.  Particles of one cell walk the same 27 cells: a wavefront takes
+// them together, one candidate per lane, and appends every particle's accepted
+// candidates in walk order through ballots (the cell walk, below).  Particles
+// with very many candidates go to a list that one wavefront each works off,
+// skipping cells and runs of slots that are too far (k_fill_heavy).  With
+// PBF_OPT_LANE_LISTS one lane per particle walks its cells by itself.
 #include "pbf_device.h"
 
 namespace pbf {
@@ -502,12 +501,11 @@ __device__ __forceinline__ bool cell_far(const uint32_t* __restrict__ box, uint3
 // coordinates x + i*s, neighbors.h:171-185), skips itself and accepts
 // d^2 < s^2 while the list has room.  Lists hold sorted slots (list_at).
 //
-// Two tiers with identical results: one lane per particle, unless its 27
-// cells hold more than twice K.heavy_budget candidates and its walk scans
-// K.heavy_budget of them without filling the list (with the overflow count
-// on: more than K.heavy_budget candidates); such a particle goes to a list
-// that k_fill_heavy walks with a whole wavefront (64 candidates per step,
-// accepted ones appended in order through a ballot).
+// Tiers with identical results: the cell walk, and k_fill_heavy (a wavefront
+// per particle) for those that it hands on; with PBF_OPT_LANE_LISTS one lane per particle
+// unless its cells hold more than twice K.heavy_budget candidates and its walk
+// scans K.heavy_budget of them without filling the list (with the overflow
+// count on: more than K.heavy_budget candidates).
 
 struct WalkCells {
   float cx[3], cy[3], cz[3];
@@ -529,23 +527,20 @@ __device__ __forceinline__ WalkCells walk_cells(f3 ps, float s) {
   return w;
 }
 
-// One wavefront per block; each lane stages its entries in its own LDS
-// column (entry k of the 64 lanes is contiguous) and writes them out at the
-// end, four entries of a particle in one 16-byte store and those of the
-// wavefront's 64 particles one contiguous kilobyte (ListWriter), instead of
-// 64 scattered 4-byte writes per entry.  A staged entry is
-// 16 bits: the slot's offset in its cell (10 bits), the cell's place in the
-// 27-cell walk (c, 5 bits) and whether the candidate lies within the skin
-// radius (bit 15), which halves the staging and doubles the wavefronts the
-// LDS holds.  The offset stays below kMaxCellOffset because a lane walks a
-// cell in full only when its 27 cells hold at most that many candidates, and
-// otherwise stops after a budget below it.
-//
 // Skin lists (with `skin`): the entries within 1.1 h (K.skin2) of the
 // positions the lists are built from, in list order; x*_0 = x*.
 // The Jacobi passes walk them instead of the full lists while no particle has
 // moved far enough for an entry outside them to come within h
 // (pbf_fused.hip).
+//
+// The lane walk: one wavefront per block; each lane stages its entries in its
+// own LDS column (entry k of the 64 lanes is contiguous) and writes them out
+// at the end.  A staged entry is 16 bits: the slot's offset in its cell (10
+// bits), the cell's place in the 27-cell walk (c, 5 bits) and whether the
+// candidate lies within the skin radius (bit 15).  The offset stays below
+// kMaxCellOffset because a lane walks a cell in full only when its 27 cells
+// hold at most that many candidates, and otherwise stops after a budget below
+// it.
 constexpr int kFillBlock = 64;
 constexpr uint32_t kMaxCellOffset = 1024u;
 
@@ -677,300 +672,408 @@ done:
 }
 
 // ---------------------------------------------------------------------------
-// The cell-tile walk: the default for particles of ordinary cells.  A
-// wavefront's 64 consecutive slots fall into runs of one cell each
-// (segments).  All particles of a segment walk the same candidate stream:
-// the 27 cells around their cell in walk order, each cell's slots in order,
-// i.e. the sequence the lane walk visits.  The stream (at most kTileMaxCand
-// candidates) is held in registers, 64 candidates per round, one per lane;
-// for each particle of the segment the wavefront tests every round's 64
-// candidates at once, and the ballot of the accepted ones is that particle's
-// next 64 acceptance bits, kept in the particle's own lane of two registers
-// (the particle's position comes from its lane by readlane).
-// Afterwards every lane stages its accepted stream positions in order up to
-// the cap, then turns them into slots through the segment's table of cell
-// starts.  The lists, counts, overflow counts and skin lists are the lane
-// walk's, bit for bit: the same candidates in the same order under the same
-// test.  Each candidate is tested by one lane for the whole segment instead
-// of by every particle's lane for itself, with no divergence between lanes
-// whose cells differ in size.
+// The cell walk.  A wavefront takes `width` consecutive slots.  Particles with
+// the same walk cells (those of a cell, but for rounding in x + i*s) have the
+// same candidates in the same order, the cells' slots one after the other: a
+// stream.  Eight of them at a time have their positions broadcast into
+// registers and go through the stream together, 64 candidates a round, one per
+// lane: the ballot of a particle's accepted candidates gives each its place in
+// the particle's row in LDS (the accepted before it: mbcnt).  A row takes the
+// particle itself too, and the sign bit of an entry says whether it lies
+// within the skin radius; one pass over the finished row, a lane per entry,
+// takes the particle out and splits the skin list off, which costs less than
+// either test in every round.  The eight particles' lists are then written out
+// together, 16 bytes a lane.
 //
-// A particle is not covered when its cell coordinates, computed in floating
-// point like the walk's (x + i*s), are not exactly its cell's neighbours,
-// when its cell is the outside bucket or one of its neighbour cells wraps
-// onto its own, when its 27 cells hold more than kTileMaxCand candidates, or
-// when its wavefront has more than kTileSegs segments; a wavefront with a
-// particle that is not covered takes the lane walk for all its particles.
-constexpr uint32_t kTileRounds = 8;
-constexpr uint32_t kTileMaxCand = 64u * kTileRounds;
-// (12 segment tables keep the wavefront's LDS under 10 KB, so that 16
-// wavefronts share a CU, as many as the registers allow; 16 tables cover a few
-// more particles at rest but fit only 14)
-constexpr uint32_t kTileSegs = 12;
-constexpr uint32_t kTileTab = 28;  // per segment: 27 cell starts; 28 stream offsets (the last is the total)
+// The slot of a stream position: each cell marks the position where its slots
+// begin, and a running maximum over the lanes (DPP) carries the cell's number
+// on to the positions that follow, so that a cell of any size takes the same
+// time.
+//
+// Bound: vector instructions, 14 a particle and round out of 170 a particle
+// (at rest 373 candidates in six rounds, 56 accepted; issue 98% busy), and in
+// small scenes the chain cells -> bounds -> slots -> positions -> tests, which
+// is why `width` falls with the scene.  Six wavefronts a SIMD: with the eight
+// rounds of a stream in registers there are four, 358 us instead of 306.
+// Measured, us a launch at rest, by width (in brackets one wavefront's 64
+// particles with bits of acceptance in registers and a lane writing each
+// list, which this replaces):
+//   particles      4     8    16    32
+//         960     14    16    23    38   (66)
+//      32,768     28    25    32    47   (76)
+//     131,072     68    56    58    65   (93)
+//     524,288    229   180   172   173  (203)
+//   1,048,576    445   341   314   306  (341)
+constexpr uint32_t kRounds = 4;
+constexpr uint32_t kChunk = 64u * kRounds;
+constexpr uint32_t kMembers = 8;  // particles tested and written out together
+constexpr uint32_t kUnit = 2;     // of these, without a branch between them
 
-// v_writelane_b32: lane `lane` of v takes the uniform value `val`
-__device__ __forceinline__ uint32_t write_lane(uint32_t v, uint32_t val, uint32_t lane) {
-  asm("v_writelane_b32 %0, %1, m0" : "+v"(v) : "s"(val), "{m0}"(lane));
+// The cell walk hands particles with more than crowded() candidates to
+// k_fill_heavy, which skips whole cells and runs of slots that are too far: at
+// once when the overflow is counted (every candidate must be seen), otherwise
+// when it has tested walk_budget() of them and some list of the group is not
+// full.  Measured on a collapsed scene of 1,048,576 particles (lists at their
+// cap), us a step in both kernels: budget 768 556, 1,536 545, 2,304 567,
+// 3,072 584; all candidates up to 3,072, none above 770.
+__host__ __device__ __forceinline__ uint32_t crowded(const KParams& K) {
+  return (K.count_overflow ? 2u : 4u) * K.heavy_budget;
+}
+__device__ __forceinline__ uint32_t walk_budget(const KParams& K, uint32_t total) {
+  return total > crowded(K) ? (K.count_overflow ? 0u : 2u * K.heavy_budget) : 0xFFFFFFFFu;
+}
+
+// v with the lanes' values moved by a DPP control; lanes without a source, and
+// rows outside the mask, get 0
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp0(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, false);
+}
+// inclusive sum over lanes 0..31
+__device__ __forceinline__ uint32_t sum_scan32(uint32_t v) {
+  v += dpp0<0x111, 0xF>(v);  // row_shr 1, 2, 4, 8
+  v += dpp0<0x112, 0xF>(v);
+  v += dpp0<0x114, 0xF>(v);
+  v += dpp0<0x118, 0xF>(v);
+  v += dpp0<0x142, 0xA>(v);  // row_bcast 15
+  return v;
+}
+// inclusive maximum over the wavefront
+__device__ __forceinline__ uint32_t max_scan64(uint32_t v) {
+  v = max(v, dpp0<0x111, 0xF>(v));
+  v = max(v, dpp0<0x112, 0xF>(v));
+  v = max(v, dpp0<0x114, 0xF>(v));
+  v = max(v, dpp0<0x118, 0xF>(v));
+  v = max(v, dpp0<0x142, 0xA>(v));
+  v = max(v, dpp0<0x143, 0xC>(v));  // row_bcast 31
   return v;
 }
 __device__ __forceinline__ float read_lane(float v, uint32_t lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), (int)lane));
 }
+// a lane's place among the lanes of mask m
+__device__ __forceinline__ uint32_t rank_in(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+// a uniform value in a vector register: an operation on vector registers alone
+// issues in half the time of one with a scalar operand
+__device__ __forceinline__ float in_vgpr(float v) {
+  float r;
+  asm("v_mov_b32 %0, %1" : "=v"(r) : "s"(v));
+  return r;
+}
 
-template <bool SKIN>
-__device__ __forceinline__ bool tile_walk(uint32_t tb, uint32_t lane, uint32_t n, bool query, f3 ps,
-                                          const uint32_t* __restrict__ key, const float4* __restrict__ xs,
-                                          const uint32_t* __restrict__ start, const KParams& K,
-                                          int32_t* __restrict__ nbr, int32_t* __restrict__ nbr_count,
-                                          int32_t* __restrict__ snb, int32_t* __restrict__ snb_count,
-                                          uint16_t* __restrict__ s_list, uint32_t* __restrict__ s_tab,
-                                          uint16_t* __restrict__ s_off, uint64_t* __restrict__ s_qm,
-                                          uint32_t& ovf) {
-  const uint32_t p = tb + lane;
-  const bool valid = p < n;
-  const uint32_t kk = valid ? key[p] : 0xFFFFFFFFu;
-  const WalkCells w = walk_cells(ps, K.s);
-  const uint32_t prev = __shfl_up(kk, 1, 64);
-  uint64_t heads = __builtin_amdgcn_ballot_w64(valid && (lane == 0 || kk != prev));
-  const uint32_t last = min(64u, n - tb);
-  // the current segment's stream (the slot of every stream position) lives in
-  // the staging area, which the lists use only after the segments
-  uint32_t* __restrict__ s_stream = reinterpret_cast<uint32_t*>(s_list);
-  uint32_t wa[2 * kTileRounds], ws[2 * kTileRounds];
+// CAP: the largest cap
+template <uint32_t CAP>
+struct CellWalkLds {
+  // words of a row: the list's entries, the particle itself once for each of
+  // its walk cells, and a round's past them; in the end the list and, from
+  // kNear on, the skin list
+  static constexpr uint32_t kPitch = CAP + 92u > 2u * CAP ? CAP + 92u : 2u * CAP, kNear = kPitch - CAP;
+  uint32_t row[kMembers * kPitch];
+  uint32_t mark[64];  // position j of a chunk: byte j / 64 of word j % 64
+  uint32_t base[28];  // first slot of the cell minus its stream offset
+};
+
+// the candidates of stream positions [c0, c0 + kChunk): slots and positions
+// (past the stream's end: the far row)
+template <class Lds>
+__device__ __forceinline__ void load_chunk(uint32_t c0, uint32_t total, uint32_t off, uint32_t cm, uint32_t lane, Lds& S, const float4* __restrict__ xs, uint32_t pad,
+                                           uint32_t (&slot)[kRounds], f3 (&t)[kRounds]) {
+  S.mark[lane] = 0u;
+  __syncthreads();
+  if (cm != 0u && off >= c0 && off < c0 + kChunk)
+    reinterpret_cast<uint8_t*>(S.mark)[((off - c0) & 63u) * 4u + ((off - c0) >> 6)] = (uint8_t)(lane + 1u);
+  // the cell that the chunk begins in: the last one that begins at or before c0
+  const uint64_t begun = __builtin_amdgcn_ballot_w64(cm != 0u && off <= c0);
+  uint32_t carry = 64u - (uint32_t)__builtin_clzll(begun | 1ull);
+  __syncthreads();
+  const uint32_t word = S.mark[lane];
 #pragma unroll
-  for (uint32_t i = 0; i < 2 * kTileRounds; ++i) wa[i] = ws[i] = 0u;
-  // pass 1: every segment's table of cells, and which particles it covers
-  bool mine = false;
-  uint32_t my_seg = 0, seg = 0;
-  while (heads != 0ull) {
-    const uint32_t s0 = (uint32_t)__builtin_ctzll(heads);
-    heads &= heads - 1ull;
-    const uint32_t s1 = heads ? (uint32_t)__builtin_ctzll(heads) : last;
-    const uint32_t ck = (uint32_t)__builtin_amdgcn_readlane((int)kk, (int)s0);
-    if (ck >= K.ncells) continue;  // the outside bucket (its particles are not covered)
-    if (seg >= kTileSegs) continue;
-    // the segment cell's coordinates in its grid (its scene's)
-    const GridView G = grid_of(K, tb + s0);
-    if (G.dxy > 0xFFFFFFFFull) continue;  // (a layer of 2^32 cells: coordinates need 64-bit division)
-    const uint32_t local = ck - G.off;
-    const uint32_t dxy = (uint32_t)G.dxy;
-    const uint32_t bz = local / dxy, rem = local - bz * dxy;
-    const uint32_t by = rem / G.dimx, bx = rem - by * G.dimx;
-    const float fx = (float)bx, fy = (float)by, fz = (float)bz;
-    // lanes 0..26: cell `lane` of the walk order (x outer, z inner)
-    uint32_t cb = 0, cm = 0, cellk = K.ncells;
-    if (lane < 27) {
-      const float ox = (float)((int)(lane / 9u) - 1), oy = (float)((int)((lane / 3u) % 3u) - 1),
-                  oz = (float)((int)(lane % 3u) - 1);
-      cellk = cell_key(fx + ox, fy + oy, fz + oz, G, K);
-      if (cellk < K.ncells) {
-        cb = start[cellk];
-        cm = start[cellk + 1] - cb;
+  for (uint32_t r = 0; r < kRounds; ++r) {
+    slot[r] = pad;
+    if (c0 + r * 64u < total) {
+      const uint32_t cell = max(max_scan64((word >> (8u * r)) & 255u), carry);
+      carry = (uint32_t)__builtin_amdgcn_readlane((int)cell, 63);
+      const uint32_t j = c0 + r * 64u + lane;
+      if (j < total) slot[r] = S.base[cell - 1u] + j;
+    }
+  }
+#pragma unroll
+  for (uint32_t r = 0; r < kRounds; ++r) t[r] = ld3(xs, slot[r]);
+}
+
+template <class Lds>
+__device__ __forceinline__ void cell_walk(uint32_t tb, uint32_t lane, uint64_t todo, f3 ps, uint32_t key,
+                                          const float4* __restrict__ xs, const uint32_t* __restrict__ start,
+                                          const KParams& K, int32_t* __restrict__ nbr,
+                                          int32_t* __restrict__ nbr_count, int32_t* __restrict__ snb,
+                                          int32_t* __restrict__ snb_count, bool skin, Lds& S, uint64_t& heavy,
+                                          uint32_t& ovf) {
+  constexpr uint32_t kPitch = Lds::kPitch, kNear = Lds::kNear;
+  f3 mid;
+  uint64_t even;
+  {
+    const WalkCells w = walk_cells(ps, K.s);
+    mid = {w.cx[1], w.cy[1], w.cz[1]};
+    even = __builtin_amdgcn_ballot_w64(w.cx[0] == mid.x - 1.0f && w.cx[2] == mid.x + 1.0f && w.cy[0] == mid.y - 1.0f &&
+                                       w.cy[2] == mid.y + 1.0f && w.cz[0] == mid.z - 1.0f && w.cz[2] == mid.z + 1.0f);
+  }
+  const uint32_t cap = (uint32_t)K.cap;
+  const float ss = in_vgpr(K.ss), ks = in_vgpr(K.skin2);
+  while (todo != 0ull) {
+    // the particles that walk the same cells as the first one left
+    const uint32_t i0 = (uint32_t)__builtin_ctzll(todo);
+    const uint32_t key0 = (uint32_t)__builtin_amdgcn_readlane((int)key, (int)i0);
+    const f3 mid0 = {read_lane(mid.x, i0), read_lane(mid.y, i0), read_lane(mid.z, i0)};
+    uint64_t members = 1ull << i0;
+    WalkCells w;
+    if (even & members) {
+      members = __builtin_amdgcn_ballot_w64(key == key0) & __builtin_amdgcn_ballot_w64(mid.x == mid0.x) &
+                __builtin_amdgcn_ballot_w64(mid.y == mid0.y) & __builtin_amdgcn_ballot_w64(mid.z == mid0.z) & even & todo;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const float d = (float)(a - 1);
+        w.cx[a] = mid0.x + d, w.cy[a] = mid0.y + d, w.cz[a] = mid0.z + d;
+      }
+    } else {
+      // (x + i*s rounds into another cell, or a coordinate is not finite)
+      w = walk_cells({read_lane(ps.x, i0), read_lane(ps.y, i0), read_lane(ps.z, i0)}, K.s);
+    }
+    todo &= ~members;
+    // lanes 0..26: cell `lane` of the walk (x outer, z inner)
+    const GridView G = grid_of(K, tb + i0);
+    uint32_t cb = 0, cm = 0, cell = K.ncells;
+    if (lane < 27u) {
+      cell = cell_key(pick3(w.cx, (int)(lane / 9u)), pick3(w.cy, (int)((lane / 3u) % 3u)),
+                      pick3(w.cz, (int)(lane % 3u)), G, K);
+      if (cell < K.ncells) {
+        cb = start[cell];
+        cm = start[cell + 1] - cb;
       }
     }
-    // exclusive scan of the cell sizes: lane c gets the stream offset of cell c, lane 27 the total
-    uint32_t incl = cm;
-#pragma unroll
-    for (int d = 1; d < 32; d <<= 1) {
-      const uint32_t t = __shfl_up(incl, d, 64);
-      if ((int)lane >= d) incl += t;
-    }
-    const uint32_t off = incl - cm;
+    const uint32_t incl = sum_scan32(cm), off = incl - cm;
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 26);
-    // the segment's particles whose own walk cells are the segment's
-    const bool canon = lane >= s0 && lane < s1 && query && w.cx[0] == fx - 1.0f && w.cx[1] == fx &&
-                       w.cx[2] == fx + 1.0f && w.cy[0] == fy - 1.0f && w.cy[1] == fy && w.cy[2] == fy + 1.0f &&
-                       w.cz[0] == fz - 1.0f && w.cz[1] == fz && w.cz[2] == fz + 1.0f;
-    const uint64_t qm = __builtin_amdgcn_ballot_w64(canon);
-    // a grid so narrow that a neighbour cell wraps onto the centre cell lists
-    // a particle's own slot twice
-    const bool dup = __builtin_amdgcn_ballot_w64(lane < 27 && lane != 13 && cellk == ck) != 0ull;
-    if (total > kTileMaxCand || dup || qm == 0ull) continue;
-    if (lane < 27) s_tab[seg * kTileTab + lane] = cb;
-    if (lane < kTileTab) s_off[seg * kTileTab + lane] = (uint16_t)off;
-    if (lane == 0) s_qm[seg] = qm;
-    if (canon) {
-      mine = true;
-      my_seg = seg;
+    const uint32_t budget = walk_budget(K, total);
+    if (budget == 0u) {
+      heavy |= members;
+      continue;
     }
-    ++seg;
-  }
-  // a wavefront takes the lane walk throughout unless every particle that
-  // needs a list is covered: the lane walk costs nearly as much for a few
-  // lanes as for all of them (measured: leaving the uncovered lanes alone to
-  // it was no faster at rest and 1-6% slower over the collapse)
-  if (__builtin_amdgcn_ballot_w64(query && !mine) != 0ull) return false;
-  __syncthreads();  // one wavefront per block
-  // pass 2: the segments' streams
-  for (uint32_t sg = 0; sg < seg; ++sg) {
-    // (the same in every lane: read into scalar registers)
-    const uint64_t qv = s_qm[sg];
-    const uint64_t qm = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)qv) |
-                        ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(qv >> 32)) << 32);
-    const uint32_t total = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_off[sg * kTileTab + 27]);
-    uint32_t cb = 0, off = 0, cm = 0;
-    if (lane < 27) {
-      cb = s_tab[sg * kTileTab + lane];
-      off = s_off[sg * kTileTab + lane];
-      cm = (uint32_t)s_off[sg * kTileTab + lane + 1] - off;
-    }
-    // the candidates' slots through a table in the staging area (which the
-    // lists use only afterwards), then their positions into registers: every
-    // round's candidates stay there while the segment's particles go by
-    for (uint32_t u = 0; u < cm; ++u) s_stream[off + u] = cb + u;
-    __syncthreads();
-    f3 t[kTileRounds];
+    // how often a particle meets itself
+    const uint32_t own = (uint32_t)__builtin_popcountll(
+        __builtin_amdgcn_ballot_w64(lane < 27u && cell == key0 && cell < K.ncells));
+    // bytes of a full row: the list's entries and the particle itself; what a
+    // round adds past them is overwritten by the next
+    const uint32_t room = 4u * (cap + own);
+    __syncthreads();  // (the previous stream's reads are done)
+    if (lane < 27u) S.base[lane] = cb - off;
+    uint32_t idx[kMembers], at[kMembers], ne = 0;  // lanes; LDS bytes of the rows so far
+    f3 pi[kMembers];
+    uint32_t found = 0;
+    auto next_group = [&]() {
+      ne = 0;
 #pragma unroll
-    for (uint32_t r = 0; r < kTileRounds; ++r) {
-      const uint32_t j = r * 64u + lane;
-      t[r] = f3{__builtin_inff(), __builtin_inff(), __builtin_inff()};
-      if (j < total) t[r] = ld3(xs, s_stream[j]);
-    }
-    // a particle's own stream position: its slot in the centre cell (place 13)
-    const uint32_t jself0 = (uint32_t)__builtin_amdgcn_readlane((int)off, 13) + tb -
-                            (uint32_t)__builtin_amdgcn_readlane((int)cb, 13);
-    uint64_t qq = qm;
-    while (qq != 0ull) {
-      const uint32_t i = (uint32_t)__builtin_ctzll(qq);
-      qq &= qq - 1ull;
-      const f3 pi = {read_lane(ps.x, i), read_lane(ps.y, i), read_lane(ps.z, i)};
-      const uint32_t js = jself0 + i;  // the particle itself is no candidate
+      for (uint32_t e = 0; e < kMembers; ++e) {
+        const bool on = members != 0ull;
+        idx[e] = on ? (uint32_t)__builtin_ctzll(members) : 0u;
+        // (places left over never accept)
+        pi[e] = {in_vgpr(on ? read_lane(ps.x, idx[e]) : __builtin_inff()), in_vgpr(read_lane(ps.y, idx[e])),
+                 in_vgpr(read_lane(ps.z, idx[e]))};
+        at[e] = on ? 0u : room;
+        members &= members - (on ? 1ull : 0ull);
+        ne += on ? 1u : 0u;
+      }
+    };
+    auto test = [&](uint32_t c, const uint32_t (&slot)[kRounds], const f3 (&t)[kRounds]) {
 #pragma unroll
-      for (uint32_t r = 0; r < kTileRounds; ++r) {
-        if (r * 64u >= total) break;
-        const float d2 = magsq3(sub3(pi, t[r]));
-        const uint64_t self = (js >> 6) == r ? 1ull << (js & 63u) : 0ull;
-        const uint64_t am = __builtin_amdgcn_ballot_w64(d2 < K.ss) & ~self;
-        wa[2 * r] = write_lane(wa[2 * r], (uint32_t)am, i);
-        wa[2 * r + 1] = write_lane(wa[2 * r + 1], (uint32_t)(am >> 32), i);
-        if (SKIN) {
-          const uint64_t sm = __builtin_amdgcn_ballot_w64(d2 < K.skin2) & am;
-          ws[2 * r] = write_lane(ws[2 * r], (uint32_t)sm, i);
-          ws[2 * r + 1] = write_lane(ws[2 * r + 1], (uint32_t)(sm >> 32), i);
+      for (uint32_t r = 0; r < kRounds; ++r) {
+        if (c + r * 64u >= total) break;
+#pragma unroll
+        for (uint32_t e0 = 0; e0 < kMembers; e0 += kUnit) {
+          if (e0 >= ne) break;
+#pragma unroll
+          for (uint32_t e = e0; e < e0 + kUnit; ++e) {
+            const float d2 = magsq3(sub3(pi[e], t[r]));
+            const uint64_t m = __builtin_amdgcn_ballot_w64(d2 < ss);
+            // bit 31: within the skin radius (the sign of the difference)
+            const uint32_t v = (__float_as_uint(d2 - ks) & 0x80000000u) | slot[r];
+            if (__builtin_amdgcn_inverse_ballot_w64(m))
+              *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(S.row + e * kPitch) + (at[e] + (rank_in(m) << 2))) = v;
+            const uint32_t f = (uint32_t)__builtin_popcountll(m);
+            found += f;
+            at[e] = min(at[e] + 4u * f, room);
+          }
         }
       }
-    }
-    __syncthreads();  // the next segment rewrites the stream
-  }
-  if (!mine) return false;
-  // stage the accepted stream positions (with the skin bit) in order, up to the cap
-  const uint32_t base = my_seg * kTileTab;
-  const uint32_t total = s_off[base + 27];
-  const uint32_t cap = (uint32_t)K.cap;
-  uint32_t k = 0, acc = 0;
+    };
+    // the lists of the group: the rows in order without the particle itself,
+    // and their entries within the skin radius
+    auto finish = [&]() {
+      __syncthreads();
+      const uint32_t mine = lane & (kMembers - 1u), q0 = lane / kMembers;
+      uint32_t x[kMembers], p = 0, kept = 0, near = 0;
 #pragma unroll
-  for (uint32_t wi = 0; wi < 2 * kTileRounds; ++wi) {
-    if (32u * wi < total) {
-      uint32_t bits = wa[wi];
-      const uint32_t rest = total - 32u * wi;
-      if (rest < 32u) bits &= (1u << rest) - 1u;
-      acc += (uint32_t)__builtin_popcount(bits);
-      const uint32_t sb = SKIN ? ws[wi] : 0u;
-      while (bits != 0u && k < cap) {
-        const uint32_t b = (uint32_t)__builtin_ctz(bits);
-        bits &= bits - 1u;
-        s_list[k * kFillBlock + lane] = (uint16_t)((32u * wi + b) | (((sb >> b) & 1u) << 15));
-        ++k;
+      for (uint32_t e = 0; e < kMembers; ++e) x[e] = S.row[e * kPitch + lane];
+#pragma unroll
+      for (uint32_t e = 0; e < kMembers; ++e) {
+        if (e >= ne) break;
+        const uint32_t pe = tb + idx[e], have = at[e] >> 2;
+        uint32_t* __restrict__ row = S.row + e * kPitch;
+        uint32_t k = 0, s = 0;
+        auto compact = [&](uint32_t k0, uint32_t x) {
+          const uint32_t q = x & 0x7FFFFFFFu;
+          const uint64_t m = __builtin_amdgcn_ballot_w64(q != pe) & __builtin_amdgcn_ballot_w64(k0 + lane < have);
+          const uint32_t to = k + rank_in(m);
+          const uint64_t in = m & __builtin_amdgcn_ballot_w64(to < cap);
+          if (__builtin_amdgcn_inverse_ballot_w64(in)) row[to] = q;
+          k += (uint32_t)__builtin_popcountll(in);
+          if (skin) {
+            const uint64_t ms = in & __builtin_amdgcn_ballot_w64((int32_t)x < 0);
+            if (__builtin_amdgcn_inverse_ballot_w64(ms)) (row + kNear + s)[rank_in(ms)] = q;
+            s += (uint32_t)__builtin_popcountll(ms);
+          }
+        };
+        if (have <= 64u) {
+          compact(0u, x[e]);
+        } else {  // (everything is read before the lists go over it)
+          const uint32_t x1 = row[64u + lane], x2 = kPitch >= 192u ? row[128u + lane] : 0u;
+          compact(0u, x[e]);
+          compact(64u, x1);
+          if (kPitch >= 192u) compact(128u, x2);
+        }
+        if (mine == e) p = pe, kept = k, near = s;
+        found -= k;
+      }
+      __syncthreads();
+      // out, padded to whole batches of eight
+      if (mine < ne) {
+        const uint64_t to = list_at(0, p, (uint32_t)K.stride);
+        const int pad = (int)K.pad;
+        auto write = [&](const uint32_t* from, int32_t* __restrict__ list, uint32_t n) {
+          int4* out = reinterpret_cast<int4*>(list + to);
+          for (uint32_t q = q0; 4u * q < ((n + 7u) & ~7u); q += 64u / kMembers) {
+            const uint32_t k = 4u * q;
+            const int4 x = *reinterpret_cast<const int4*>(from + k);
+            out[q * 64u] = make_int4(k < n ? x.x : pad, k + 1u < n ? x.y : pad, k + 2u < n ? x.z : pad,
+                                     k + 3u < n ? x.w : pad);
+          }
+        };
+        write(S.row + mine * kPitch, nbr, kept);
+        if (skin) write(S.row + mine * kPitch + kNear, snb, near);
+        if (q0 == 0u) {
+          nbr_count[p] = (int32_t)kept;
+          if (skin) snb_count[p] = (int32_t)near;
+        }
+      }
+      found -= ne * own;
+      if (lane == 0u) ovf += found;
+      found = 0u;
+      __syncthreads();
+    };
+    uint32_t slot[kRounds];
+    f3 t[kRounds];
+    while (members != 0ull) {
+      const uint64_t group = members;
+      next_group();
+      bool full = false;
+      uint32_t c = 0;
+      for (; c < total && c < budget && !full; c += kChunk) {
+        load_chunk(c, total, off, cm, lane, S, xs, K.pad, slot, t);
+        test(c, slot, t);
+        uint32_t least = at[0];
+#pragma unroll
+        for (uint32_t e = 1; e < kMembers; ++e) least = min(least, at[e]);
+        full = least >= room && !K.count_overflow;
+      }
+      if (c >= total || full) {
+        finish();
+      } else {
+        heavy |= group & ~members;
+        found = 0u;
       }
     }
   }
-  if (acc > k) ovf = acc - k;
-  nbr_count[p] = (int32_t)k;
-  // flush: stream positions to slots, cell by cell
-  uint32_t c = 0, co = 0, nxt = s_off[base + 1], cs = s_tab[base];
-  ListWriter full(nbr, p, K), near(snb, p, K);
-  for (uint32_t e = 0; e < k; ++e) {
-    const uint32_t e16 = s_list[e * kFillBlock + lane];
-    const uint32_t j = e16 & 1023u;
-    while (j >= nxt) {
-      ++c;
-      co = nxt;
-      cs = s_tab[base + c];
-      nxt = s_off[base + c + 1];
-    }
-    const uint32_t slot = cs + (j - co);
-    full.add(slot);
-    if (SKIN && (e16 >> 15)) near.add(slot);
-  }
-  full.close();
-  if (SKIN) {
-    near.close();
-    snb_count[p] = (int32_t)near.count;
-  }
-  return true;
 }
 
 // Hand-offs and overflow counts go to the shared counters once per
 // wavefront (a same-address atomic per lane serialises in L2 when many
 // particles of a collapsed region hand off together).
-__global__ void __launch_bounds__(kFillBlock) k_fill_neighbors(uint32_t n, uint32_t fb, uint32_t fe,
-                                                               const float4* __restrict__ xs,
-                                                               const uint32_t* __restrict__ oid,
-                                                               const uint32_t* __restrict__ key,
-                                                               const uint32_t* __restrict__ start,
-                                                               uint32_t* __restrict__ box, uint64_t box_words,
-                                                               KParams K, int32_t* __restrict__ nbr,
-                                                               int32_t* __restrict__ nbr_count,
-                                                               uint32_t* __restrict__ heavy,
-                                                               unsigned long long* __restrict__ counters,
-                                                               int skin_mode,
-                                                               const unsigned long long* __restrict__ hint,
-                                                               int32_t* __restrict__ snb,
-                                                               int32_t* __restrict__ snb_count,
-                                                               float4* __restrict__ xs0) {
-  extern __shared__ uint16_t s_list[];  // [cap + 1][kFillBlock], or the cell-tile walk's stream
-  __shared__ uint32_t s_tab[kTileSegs * kTileTab];
-  __shared__ uint16_t s_off[kTileSegs * kTileTab];
-  __shared__ uint64_t s_qm[kTileSegs];
-  const uint32_t lane = threadIdx.x;
-  const uint32_t tb = xcd_block() * blockDim.x;
-  const uint32_t p = tb + threadIdx.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + lane; i < box_words; i += (uint64_t)gridDim.x * blockDim.x)
-    box[i] = box_empty(i);
-  // skin lists only when the previous step kept them usable to its end
-  const int skin = skin_mode && *hint != 0ull;
-  if (skin && blockIdx.x == 0 && lane == 0) counters[C_SKIN] = 1ull;
-  bool to_heavy = false;
-  uint32_t ovf = 0;
-  const uint32_t o = p < n ? oid[p] : 0u;
-  const bool query = p < n && o >= fb && o < fe;
-  bool built = false;
-  if (K.tile_lists) {  // every lane of the wavefront takes part
-    const f3 ps = p < n ? ld3(xs, p) : f3{0.f, 0.f, 0.f};
-    built = skin ? tile_walk<true>(tb, lane, n, query, ps, key, xs, start, K, nbr, nbr_count, snb, snb_count,
-                                   s_list, s_tab, s_off, s_qm, ovf)
-                 : tile_walk<false>(tb, lane, n, query, ps, key, xs, start, K, nbr, nbr_count, snb, snb_count,
-                                    s_list, s_tab, s_off, s_qm, ovf);
-  }
-  if (p < n) {
-    if (skin_mode) xs0[p] = xs[p];
-    if (built) {
-      // listed by the cell-tile walk
-    } else if (!query) {
-      nbr_count[p] = 0;
-      if (skin) snb_count[p] = 0;
-    } else {
-      to_heavy = skin ? !walk_list<true>(p, n, lane, s_list, xs, start, K, nbr, nbr_count, ovf, snb, snb_count)
-                      : !walk_list<false>(p, n, lane, s_list, xs, start, K, nbr, nbr_count, ovf, snb, snb_count);
-    }
-  }
-  // every lane of the wavefront (one per block) is here
-  const uint64_t hm = __ballot(to_heavy);
-  if (hm) {
+__device__ __forceinline__ void count_fill(uint64_t hm, uint32_t p, uint32_t ovf, bool listed, uint32_t lane,
+                                           const KParams& K, uint32_t* __restrict__ heavy,
+                                           unsigned long long* __restrict__ counters) {
+  if (hm != 0ull) {
     unsigned long long base = 0;
     if (lane == 0) base = atomicAdd(&counters[C_HEAVY], (unsigned long long)__popcll(hm));
     base = __shfl(base, 0, 64);
-    if (to_heavy) heavy[base + (unsigned long long)__popcll(hm & ((1ull << lane) - 1ull))] = p;
+    if ((hm >> lane) & 1ull) heavy[base + (unsigned long long)__popcll(hm & ((1ull << lane) - 1ull))] = p;
+    if (listed && K.count_overflow && lane == 0) atomicAdd(&counters[C_TILE], 0ull - (unsigned long long)__popcll(hm));
   }
   if (K.count_overflow) {
     unsigned long long ov = ovf;
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) ov += __shfl_xor(ov, d, 64);
-    const unsigned long long tiles = (unsigned long long)__popcll(__ballot(built && p < n));
     if (lane == 0 && ov) atomicAdd(&counters[C_OVERFLOW], ov);
-    if (lane == 0 && tiles) atomicAdd(&counters[C_TILE], tiles);
   }
+}
+
+struct FillArgs {
+  uint32_t n, fb, fe, width;
+  const float4* xs;
+  const uint32_t *oid, *key, *start;
+  uint32_t* box;
+  uint64_t box_words;
+  int32_t *nbr, *nbr_count, *snb, *snb_count;
+  uint32_t* heavy;
+  unsigned long long* counters;
+  int skin_mode;
+  const unsigned long long* hint;
+  float4* xs0;
+};
+
+// LANES: one lane per particle (PBF_OPT_LANE_LISTS); CAP: the longest list
+template <bool LANES, uint32_t CAP>
+__global__ void __launch_bounds__(kFillBlock, LANES ? 1 : (CAP <= 64 ? 6 : 5)) k_fill_neighbors(FillArgs A, KParams K) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char s_mem[];
+  const uint32_t lane = threadIdx.x;
+  const uint32_t tb = xcd_block() * A.width;
+  const bool valid = lane < A.width && tb + lane < A.n;
+  const uint32_t p = valid ? tb + lane : tb;
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + lane; i < A.box_words; i += (uint64_t)gridDim.x * blockDim.x)
+    A.box[i] = box_empty(i);
+  // skin lists only when the previous step kept them usable to its end
+  const int skin = A.skin_mode && *A.hint != 0ull;
+  if (skin && blockIdx.x == 0 && lane == 0) A.counters[C_SKIN] = 1ull;
+  const uint32_t o = A.oid[p];
+  const bool query = valid && o >= A.fb && o < A.fe;
+  const float4 ps4 = A.xs[p];
+  if (valid) {
+    if (A.skin_mode) A.xs0[p] = ps4;
+    if (!query) {
+      A.nbr_count[p] = 0;
+      if (skin) A.snb_count[p] = 0;
+    }
+  }
+  uint32_t ovf = 0;
+  uint64_t hm = 0ull;
+  if constexpr (LANES) {
+    uint16_t* s_list = reinterpret_cast<uint16_t*>(s_mem);  // [cap + 1][kFillBlock]
+    bool to_heavy = false;
+    if (query)
+      to_heavy = skin ? !walk_list<true>(p, A.n, lane, s_list, A.xs, A.start, K, A.nbr, A.nbr_count, ovf, A.snb, A.snb_count)
+                      : !walk_list<false>(p, A.n, lane, s_list, A.xs, A.start, K, A.nbr, A.nbr_count, ovf, A.snb, A.snb_count);
+    hm = __ballot(to_heavy);
+  } else {
+    __shared__ __attribute__((aligned(16))) CellWalkLds<CAP> S;
+    const uint64_t todo = __builtin_amdgcn_ballot_w64(query);
+    uint32_t key = A.key[p];
+    if (K.batched && key == K.ncells) key += K.sid[p];  // (outside every cell, but in its own scene's grid)
+    cell_walk(tb, lane, todo, xyz3(ps4), key, A.xs, A.start, K, A.nbr, A.nbr_count, A.snb, A.snb_count, skin != 0, S, hm,
+              ovf);
+    // all listed here (but for those handed on): an atomic a wavefront took 0.5 ms at 8 million particles
+    if (K.count_overflow && blockIdx.x == 0 && lane == 0)
+      atomicAdd(&A.counters[C_TILE], (unsigned long long)(min(A.fe, A.n) - min(A.fb, A.n)));
+  }
+  count_fill(hm, p, ovf, !LANES, lane, K, A.heavy, A.counters);
 }
 
 // A group of 64 candidates of the wavefront builder, one per lane (valid:
@@ -1091,6 +1194,9 @@ __global__ void __launch_bounds__(kBlock) k_fill_heavy(uint32_t n, const float4*
   }
 }
 
+// slots a wavefront of the cell walk takes (see there)
+static uint32_t fill_width(uint64_t n) { return n <= 16384 ? 4u : (n <= 131072 ? 8u : (n <= 524288 ? 16u : 32u)); }
+
 void launch_fill_neighbors(pbf_context* c, uint64_t fb, uint64_t fe) {
   const uint32_t n = (uint32_t)c->n;
   if (!n) return;
@@ -1098,21 +1204,28 @@ void launch_fill_neighbors(pbf_context* c, uint64_t fb, uint64_t fe) {
   // previous step's moves stayed below their limit (c->skin_hint)
   const int skin = c->K.skin_mode;
   KernelTimer* t = timer_begin(c, "fill_neighbors");
-  // the staging area holds a wavefront's lists, or the cell-tile walk's stream of slots
-  const uint32_t stage = std::max<uint32_t>(kFillBlock * (c->K.cap + 1) * sizeof(uint16_t),
-                                            kTileMaxCand * sizeof(uint32_t));
-  hipLaunchKernelGGL(k_fill_neighbors, dim3(nblocks(n, kFillBlock)), dim3(kFillBlock), stage, c->stream, n,
-                     (uint32_t)fb,
-                     (uint32_t)fe, (const float4*)c->xs, (const uint32_t*)c->oid, (const uint32_t*)c->key,
-                     (const uint32_t*)c->cell_start, c->cbox, boxes_in_fill(c) ? 6ull * c->K.ncells : 0ull, c->K, c->nbr, c->nbr_count, c->heavy, c->counters, skin,
-                     (const unsigned long long*)c->skin_hint, c->snb, c->snb_count, c->xs0);
+  const bool lanes = !c->K.tile_lists;
+  const uint32_t width = lanes ? (uint32_t)kFillBlock : fill_width(n);
+  const FillArgs A{n, (uint32_t)fb, (uint32_t)fe, width, c->xs, c->oid, c->key, c->cell_start, c->cbox,
+                   boxes_in_fill(c) ? 6ull * c->K.ncells : 0ull, c->nbr, c->nbr_count, c->snb, c->snb_count, c->heavy,
+                   c->counters, skin, c->skin_hint, c->xs0};
+  const dim3 grid(nblocks(n, (int)width)), block(kFillBlock);
+  if (lanes)
+    hipLaunchKernelGGL((k_fill_neighbors<true, 0>), grid, block, kFillBlock * (c->K.cap + 1) * sizeof(uint16_t), c->stream,
+                       A, c->K);
+  else
+    // (rows for lists of up to 64 or 128 entries: the longer ones leave LDS for five wavefronts a SIMD instead of six)
+    hipLaunchKernelGGL((c->K.cap <= 64 ? k_fill_neighbors<false, 64> : k_fill_neighbors<false, 128>), grid, block, 0,
+                       c->stream, A, c->K);
   timer_end(c, t);
   // no particle of a small scene has enough candidates for the wavefront
   // builder: every particle is a candidate at most once (a grid of at least
   // three cells an axis gives 27 different cells)
   const bool wide = c->K.batched || (c->K.dimx >= 3 && c->K.dimy >= 3 && c->K.dimz >= 3);
   const uint32_t hb = lane_budget(c->K);
-  if (wide && n <= (c->K.count_overflow ? hb : std::min(2u * hb, kMaxCellOffset))) return;
+  const uint32_t most = !lanes ? crowded(c->K)
+                               : (c->K.count_overflow ? hb : std::min(2u * hb, kMaxCellOffset));
+  if (wide && n <= most) return;
   // the cell and chunk boxes of the wavefront builder, built only when some particle went to it
   launch_cell_box(c);
   // enough waves to cover the chip; each loops over the heavy list (usually empty)

@@ -356,6 +356,43 @@ static int build_scene_geo(const pbf_params& params, const float* boxes, uint32_
 
 using namespace pbf;
 
+// a caller's array to c->stage or the like; a device pointer is copied as one
+static int upload(pbf_context* c, void* dev, const void* host, uint64_t bytes) {
+  if (!on_device(host)) return c->host.upload(dev, host, bytes, c->stream);
+  return check_hip(hipMemcpyAsync(dev, host, bytes, hipMemcpyDefault, c->stream), "upload");
+}
+// and back; waits for the stream
+static int download(pbf_context* c, void* host, const void* dev, uint64_t bytes) {
+  if (!on_device(host)) return c->host.download(host, dev, bytes, c->stream);
+  int rc = check_hip(hipMemcpyAsync(host, dev, bytes, hipMemcpyDefault, c->stream), "download");
+  return rc ? rc : check_hip(hipStreamSynchronize(c->stream), "download");
+}
+
+// Short arrays skip the device staging: the kernel that puts them in order
+// reads or writes the pinned memory, which saves the copy's launch.
+template <class Order>
+static int get_array(pbf_context* c, float* out, uint64_t bytes, Order order) {
+  if (bytes > HostStage::kDirect || on_device(out)) {
+    order(c->stage);
+    return download(c, out, c->stage, bytes);
+  }
+  order((float*)c->host.pin);
+  if (int rc = check_hip(hipStreamSynchronize(c->stream), "download")) return rc;
+  std::memcpy(out, c->host.pin, bytes);
+  return PBF_OK;
+}
+template <class Order>
+static int set_array(pbf_context* c, const float* in, uint64_t bytes, Order order) {
+  if (bytes > HostStage::kDirect || on_device(in)) {
+    if (int rc = upload(c, c->stage, in, bytes)) return rc;
+    order(c->stage);
+  } else {
+    std::memcpy(c->host.pin, in, bytes);
+    order((const float*)c->host.pin);
+  }
+  return check_hip(hipStreamSynchronize(c->stream), "upload");
+}
+
 // ---------------------------------------------------------------------------
 extern "C" {
 
@@ -434,9 +471,11 @@ int pbf_create(const pbf_params* params, pbf_context** out) {
       (rc = dalloc(&c->scan_partials, scan_partials_size(N + 1))) ||
       (rc = dalloc(&c->slog, (uint64_t)PBF_SOLVE_LOG_SIZE)) || (rc = dalloc(&c->slog_count, 1)) ||
       (rc = check_hip(hipHostMalloc((void**)&c->done_host, sizeof(unsigned long long)), "hipHostMalloc")) ||
+      (rc = c->host.create(N * 3 * sizeof(float))) ||
       (rc = check_hip(hipEventCreate(&c->region_a), "hipEventCreate")) ||
       (rc = check_hip(hipEventCreate(&c->region_b), "hipEventCreate"))) {
     free_all(c);
+    c->host.destroy();
     if (c->done_host) (void)hipHostFree(c->done_host);
     if (c->region_a) (void)hipEventDestroy(c->region_a);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -470,6 +509,7 @@ int pbf_destroy(pbf_context* c) {
   drop_solve_graph(c);
   timers_release(c);
   free_all(c);
+  c->host.destroy();
   if (c->done_host) hipHostFree(c->done_host);
   if (c->region_a) hipEventDestroy(c->region_a);
   if (c->region_b) hipEventDestroy(c->region_b);
@@ -551,9 +591,9 @@ int pbf_add(pbf_context* c, const float* pos, const float* pos_star, const float
   const float* src[3] = {pos, pos_star, vel};
   float4* dst[3] = {c->x, c->xs, c->v};
   for (int a = 0; a < 3; ++a) {
-    int rc = check_hip(hipMemcpyAsync(c->stage, src[a], count * 3 * sizeof(float), hipMemcpyHostToDevice,
-                                      c->stream), "add");
-    if (rc) return rc;
+    if (a)  // (the arrays share the staging memory)
+      if (int rc = check_hip(hipStreamSynchronize(c->stream), "add")) return rc;
+    if (int rc = upload(c, c->stage, src[a], count * 3 * sizeof(float))) return rc;
     hipLaunchKernelGGL(k_widen3, dim3(nb), dim3(256), 0, c->stream, (const float*)c->stage, dst[a], first, count);
   }
   hipLaunchKernelGGL(k_iota, dim3(nb), dim3(256), 0, c->stream, c->oid, first, count);
@@ -643,40 +683,25 @@ static int get_vec(pbf_context* c, const float4* src, float* out) {
   PBF_TRACE("pbf_get_state");
   if (!c || !out) return set_error(PBF_ERR_ARG, "null argument");
   if (!c->n) return PBF_OK;
-  launch_gather_out_f4(c, src, c->stage, 3);
-  int rc = check_hip(hipMemcpyAsync(out, c->stage, c->n * 3 * sizeof(float), hipMemcpyDeviceToHost, c->stream),
-                     "download");
-  if (rc) return rc;
-  return check_hip(hipStreamSynchronize(c->stream), "download");
+  return get_array(c, out, c->n * 3 * sizeof(float), [&](float* to) { launch_gather_out_f4(c, src, to, 3); });
 }
 static int get_scalar(pbf_context* c, const float* src, float* out) {
   PBF_TRACE("pbf_get_state");
   if (!c || !out) return set_error(PBF_ERR_ARG, "null argument");
   if (!c->n) return PBF_OK;
-  launch_gather_out_f1(c, src, c->stage);
-  int rc = check_hip(hipMemcpyAsync(out, c->stage, c->n * sizeof(float), hipMemcpyDeviceToHost, c->stream),
-                     "download");
-  if (rc) return rc;
-  return check_hip(hipStreamSynchronize(c->stream), "download");
+  return get_array(c, out, c->n * sizeof(float), [&](float* to) { launch_gather_out_f1(c, src, to); });
 }
 static int set_vec(pbf_context* c, float4* dst, const float* in) {
   PBF_TRACE("pbf_set_state");
   if (!c || !in) return set_error(PBF_ERR_ARG, "null argument");
   if (!c->n) return PBF_OK;
-  int rc = check_hip(hipMemcpyAsync(c->stage, in, c->n * 3 * sizeof(float), hipMemcpyHostToDevice, c->stream),
-                     "upload");
-  if (rc) return rc;
-  launch_scatter_in_f4(c, c->stage, dst);
-  return check_hip(hipStreamSynchronize(c->stream), "upload");
+  return set_array(c, in, c->n * 3 * sizeof(float), [&](const float* from) { launch_scatter_in_f4(c, from, dst); });
 }
 static int set_scalar(pbf_context* c, float* dst, const float* in) {
   PBF_TRACE("pbf_set_state");
   if (!c || !in) return set_error(PBF_ERR_ARG, "null argument");
   if (!c->n) return PBF_OK;
-  int rc = check_hip(hipMemcpyAsync(c->stage, in, c->n * sizeof(float), hipMemcpyHostToDevice, c->stream), "upload");
-  if (rc) return rc;
-  launch_scatter_in_f1(c, c->stage, dst);
-  return check_hip(hipStreamSynchronize(c->stream), "upload");
+  return set_array(c, in, c->n * sizeof(float), [&](const float* from) { launch_scatter_in_f1(c, from, dst); });
 }
 
 int pbf_get_positions(pbf_context* c, float* out) { return get_vec(c, c ? c->x : nullptr, out); }
@@ -1092,8 +1117,7 @@ int pbf_get_warm_features(pbf_context* c, float* out) {
   int rc = check_hip(hipMallocAsync((void**)&tmp, c->n * PBF_WARM_FEATURES * sizeof(float), c->stream), "alloc");
   if (rc) return rc;
   launch_gather_out_rows(c, c->feat, tmp, PBF_WARM_FEATURES);
-  rc = check_hip(hipMemcpyAsync(out, tmp, c->n * PBF_WARM_FEATURES * sizeof(float), hipMemcpyDeviceToHost,
-                                c->stream), "download");
+  rc = download(c, out, tmp, c->n * PBF_WARM_FEATURES * sizeof(float));
   hipFreeAsync(tmp, c->stream);
   if (rc) return rc;
   return check_hip(hipStreamSynchronize(c->stream), "download");
@@ -1103,8 +1127,7 @@ int pbf_set_warm_lambdas(pbf_context* c, const float* lambdas) {
   PBF_TRACE("pbf_set_warm_lambdas");
   if (!c || !lambdas) return set_error(PBF_ERR_ARG, "null argument");
   if (c->n) {
-    int rc = check_hip(hipMemcpyAsync(c->wgiven, lambdas, c->n * sizeof(float), hipMemcpyHostToDevice, c->stream),
-                       "upload");
+    int rc = upload(c, c->wgiven, lambdas, c->n * sizeof(float));
     if (rc) return rc;
     if ((rc = check_hip(hipStreamSynchronize(c->stream), "upload"))) return rc;
   }
@@ -1116,11 +1139,8 @@ int pbf_set_lambda_sums(pbf_context* c, const float* in) {
   PBF_TRACE("pbf_set_lambda_sums");
   if (!c || !in) return set_error(PBF_ERR_ARG, "null argument");
   if (c->n) {
-    int rc = check_hip(hipMemcpyAsync(c->stage, in, c->n * sizeof(float), hipMemcpyHostToDevice, c->stream),
-                       "upload");
+    const int rc = set_array(c, in, c->n * sizeof(float), [&](const float* from) { launch_scatter_in_f1(c, from, c->lsum); });
     if (rc) return rc;
-    launch_scatter_in_f1(c, c->stage, c->lsum);
-    if ((rc = check_hip(hipStreamSynchronize(c->stream), "upload"))) return rc;
   }
   c->track_lsum = true;
   return PBF_OK;
@@ -1131,11 +1151,7 @@ int pbf_get_lambda_sums(pbf_context* c, float* out) {
   if (!c || !out) return set_error(PBF_ERR_ARG, "null argument");
   if (!c->track_lsum) return set_error(PBF_ERR_STATE, "no pbf_solve has run");
   if (!c->n) return PBF_OK;
-  launch_gather_out_f1(c, c->lsum, c->stage);
-  int rc = check_hip(hipMemcpyAsync(out, c->stage, c->n * sizeof(float), hipMemcpyDeviceToHost, c->stream),
-                     "download");
-  if (rc) return rc;
-  return check_hip(hipStreamSynchronize(c->stream), "download");
+  return get_array(c, out, c->n * sizeof(float), [&](float* to) { launch_gather_out_f1(c, c->lsum, to); });
 }
 
 int pbf_get_solve_info(pbf_context* c, pbf_solve_info* out) {
@@ -1384,9 +1400,7 @@ int pbf_get_stats(pbf_context* c, pbf_stats* out) {
   int rc = check_hip(hipMemcpyAsync(h, c->counters, sizeof(h), hipMemcpyDeviceToHost, c->stream), "stats");
   if (rc) return rc;
   std::vector<float> rho(c->n);
-  if (c->n && (rc = check_hip(hipMemcpyAsync(rho.data(), c->rho, c->n * 4, hipMemcpyDeviceToHost, c->stream),
-                              "stats")))
-    return rc;
+  if (c->n && (rc = download(c, rho.data(), c->rho, c->n * 4))) return rc;
   if ((rc = check_hip(hipStreamSynchronize(c->stream), "stats"))) return rc;
   out->neighbor_overflow = h[C_OVERFLOW];
   out->outside_grid = h[C_OUTSIDE];
@@ -1416,9 +1430,7 @@ uint64_t pbf_num_cells(const pbf_context* c) { return c ? c->ncells : 0; }
 static int download_u32(pbf_context* c, const uint32_t* src, uint64_t count, std::vector<uint32_t>& out) {
   out.resize(count);
   if (!count) return PBF_OK;
-  int rc = check_hip(hipMemcpyAsync(out.data(), src, count * 4, hipMemcpyDeviceToHost, c->stream), "download");
-  if (rc) return rc;
-  return check_hip(hipStreamSynchronize(c->stream), "download");
+  return download(c, out.data(), src, count * 4);
 }
 
 int pbf_get_bin_ids(pbf_context* c, uint64_t* out) {

@@ -167,6 +167,38 @@ __host__ __device__ __forceinline__ uint64_t list_at(uint32_t k, uint32_t p, uin
 // rows that a walk may load ahead
 inline uint64_t list_size(uint64_t capacity, uint64_t stride) { return ((capacity + 63) / 64 * stride + 8) * 64; }
 
+// Pinned memory of one object (a context, a warm-start model) that its copies
+// from and to ordinary memory go through (pbf_transfer.hip).  One transfer at
+// a time: the caller synchronizes the stream before the next one.
+struct HostStage {
+  static constexpr uint32_t kSlots = 8;
+  static constexpr uint64_t kSlot = 2u << 20;    // bytes of a slot: 16 MB in all at most
+  static constexpr uint64_t kTwo = 8u << 20, kFour = 32u << 20;  // from here on two and four threads copy
+  static constexpr uint64_t kDirect = 1u << 16;  // up to here kernels read the pinned memory themselves
+  unsigned char* pin = nullptr;
+  uint64_t slot_bytes = 0;
+  uint32_t nslots = 0;
+  hipEvent_t done[kSlots] = {};
+  int create(uint64_t most);  // most: bytes of the largest transfer
+  void destroy();
+  // queues the copy on s; host may be reused when it returns
+  int upload(void* dev, const void* host, uint64_t bytes, hipStream_t s);
+  // waits for s and the copy
+  int download(void* host, const void* dev, uint64_t bytes, hipStream_t s);
+
+ private:
+  int device = 0;
+  hipError_t upload_part(unsigned char* dev, const unsigned char* host, uint64_t bytes, uint64_t chunk, uint32_t first,
+                         uint32_t count, hipStream_t s);
+  hipError_t download_part(unsigned char* host, const unsigned char* dev, uint64_t bytes, uint64_t chunk,
+                           uint32_t first, uint32_t count, hipStream_t s);
+  template <class Part>
+  hipError_t in_parts(uint64_t bytes, Part part);
+};
+
+// whether p is device memory (callers may pass it where an array is expected)
+bool on_device(const void* p);
+
 struct KernelTimer {
   std::string name;
   uint64_t launches = 0;
@@ -264,6 +296,7 @@ struct pbf_context {
   float4* xsave = nullptr;
   bool has_given = false;
   float* stage = nullptr;  // device staging for original-order transfers (4 floats / particle)
+  pbf::HostStage host;     // and host staging
   uint64_t* stage64 = nullptr;
 
   hipEvent_t region_a = nullptr, region_b = nullptr;

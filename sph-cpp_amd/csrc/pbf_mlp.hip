@@ -330,12 +330,28 @@ struct pbf_warm_model {
   float *part = nullptr, *lpart = nullptr, *loss = nullptr, *loss_acc = nullptr;
   float *feat = nullptr, *tgt = nullptr;
   uint32_t *perm = nullptr, *iota = nullptr;
+  float *pfeat = nullptr, *pout = nullptr;  // predict's rows, up to kPredictRows
+  pbf::HostStage host;
   uint64_t count = 0, max_samples = 0;
   uint64_t adam_t = 0;
   bool has_params = false;
 };
 
 namespace pbf {
+
+// Rows of one launch of predict: the workspace of a model, so that a call
+// allocates nothing (two allocations and their release took about 150 us)
+constexpr uint64_t kPredictRows = 32768;
+
+static int upload(pbf_warm_model* M, void* dev, const void* host, uint64_t bytes) {
+  if (!on_device(host)) return M->host.upload(dev, host, bytes, M->stream);
+  return check_hip(hipMemcpyAsync(dev, host, bytes, hipMemcpyDefault, M->stream), "upload");
+}
+static int download(pbf_warm_model* M, void* host, const void* dev, uint64_t bytes) {
+  if (!on_device(host)) return M->host.download(host, dev, bytes, M->stream);
+  int rc = check_hip(hipMemcpyAsync(host, dev, bytes, hipMemcpyDefault, M->stream), "download");
+  return rc ? rc : check_hip(hipStreamSynchronize(M->stream), "download");
+}
 
 static MlpW model_weights(const pbf_warm_model* M) { return MlpW{M->w1, M->w2, M->w2t, M->p}; }
 
@@ -391,7 +407,8 @@ int pbf_warm_model_create(uint64_t max_samples, pbf_warm_model** out) {
       (rc = A((void**)&M->lpart, kMaxTrainWaves * 4)) || (rc = A((void**)&M->loss, 4)) ||
       (rc = A((void**)&M->loss_acc, 4)) || (rc = A((void**)&M->feat, max_samples * kFeat * 4)) ||
       (rc = A((void**)&M->tgt, max_samples * 4)) || (rc = A((void**)&M->perm, max_samples * 4)) ||
-      (rc = A((void**)&M->iota, max_samples * 4))) {
+      (rc = A((void**)&M->iota, max_samples * 4)) || (rc = A((void**)&M->pfeat, kPredictRows * kFeat * 4)) ||
+      (rc = A((void**)&M->pout, kPredictRows * 4)) || (rc = M->host.create(kPredictRows * kFeat * 4))) {
     pbf_warm_model_destroy(M);
     return rc;
   }
@@ -409,9 +426,10 @@ int pbf_warm_model_destroy(pbf_warm_model* M) {
   if (!M) return PBF_OK;
   if (M->stream) hipStreamSynchronize(M->stream);
   void* ptrs[] = {M->p, M->w1, M->w2, M->w2t, M->m, M->v, M->grad, M->part, M->lpart, M->loss, M->loss_acc,
-                  M->feat, M->tgt, M->perm, M->iota};
+                  M->feat, M->tgt, M->perm, M->iota, M->pfeat, M->pout};
   for (void* q : ptrs)
     if (q) hipFree(q);
+  M->host.destroy();
   if (M->stream) hipStreamDestroy(M->stream);
   delete M;
   return PBF_OK;
@@ -419,7 +437,7 @@ int pbf_warm_model_destroy(pbf_warm_model* M) {
 
 int pbf_warm_model_set_params(pbf_warm_model* M, const float* params) {
   if (!M || !params) return set_error(PBF_ERR_ARG, "null argument");
-  int rc = check_hip(hipMemcpyAsync(M->p, params, kNPar * 4, hipMemcpyHostToDevice, M->stream), "upload");
+  int rc = upload(M, M->p, params, kNPar * 4);
   if (rc) return rc;
   refresh(M);
   launch_fill_u32((uint32_t*)M->m, 0u, kNPar, M->stream);
@@ -432,9 +450,7 @@ int pbf_warm_model_set_params(pbf_warm_model* M, const float* params) {
 int pbf_warm_model_get_params(pbf_warm_model* M, float* params) {
   if (!M || !params) return set_error(PBF_ERR_ARG, "null argument");
   if (!M->has_params) return set_error(PBF_ERR_STATE, "model has no parameters");
-  int rc = check_hip(hipMemcpyAsync(params, M->p, kNPar * 4, hipMemcpyDeviceToHost, M->stream), "download");
-  if (rc) return rc;
-  return check_hip(hipStreamSynchronize(M->stream), "download");
+  return download(M, params, M->p, kNPar * 4);
 }
 
 // Uniform(-1/sqrt(fan_in), 1/sqrt(fan_in)) weights, zero biases.
@@ -461,12 +477,9 @@ int pbf_warm_model_clear_samples(pbf_warm_model* M) {
 int pbf_warm_model_add_samples(pbf_warm_model* M, const float* features, const float* targets, uint64_t count) {
   if (!M || (count && (!features || !targets))) return set_error(PBF_ERR_ARG, "null argument");
   if (M->count + count > M->max_samples) return set_error(PBF_ERR_CAPACITY, "sample store is full");
-  int rc = check_hip(hipMemcpyAsync(M->feat + M->count * kFeat, features, count * kFeat * 4, hipMemcpyHostToDevice,
-                                    M->stream), "upload");
-  if (rc) return rc;
-  if ((rc = check_hip(hipMemcpyAsync(M->tgt + M->count, targets, count * 4, hipMemcpyHostToDevice, M->stream),
-                      "upload")))
-    return rc;
+  int rc = upload(M, M->feat + M->count * kFeat, features, count * kFeat * 4);
+  if (rc || (rc = check_hip(hipStreamSynchronize(M->stream), "upload"))) return rc;  // (one staging memory)
+  if ((rc = upload(M, M->tgt + M->count, targets, count * 4))) return rc;
   if ((rc = check_hip(hipStreamSynchronize(M->stream), "upload"))) return rc;
   M->count += count;
   return PBF_OK;
@@ -506,18 +519,16 @@ int pbf_warm_model_gradient(pbf_warm_model* M, uint64_t first, uint32_t count, f
   if (!M->has_params) return set_error(PBF_ERR_STATE, "model has no parameters");
   if (count == 0 || first + count > M->count) return set_error(PBF_ERR_ARG, "sample range out of bounds");
   run_batch(M, M->iota + first, count, nullptr, nullptr);
-  int rc = check_hip(hipMemcpyAsync(grad, M->grad, kNPar * 4, hipMemcpyDeviceToHost, M->stream), "download");
-  if (rc) return rc;
-  if (loss && (rc = check_hip(hipMemcpyAsync(loss, M->loss, 4, hipMemcpyDeviceToHost, M->stream), "download")))
-    return rc;
-  return check_hip(hipStreamSynchronize(M->stream), "gradient");
+  int rc = download(M, grad, M->grad, kNPar * 4);
+  if (!rc && loss) rc = download(M, loss, M->loss, 4);
+  return rc;
 }
 
 int pbf_warm_model_adam_step(pbf_warm_model* M, const float* grad, float learning_rate) {
   PBF_TRACE("pbf_warm_model_adam_step");
   if (!M || !grad) return set_error(PBF_ERR_ARG, "null argument");
   if (!M->has_params) return set_error(PBF_ERR_STATE, "model has no parameters");
-  int rc = check_hip(hipMemcpyAsync(M->grad, grad, kNPar * 4, hipMemcpyHostToDevice, M->stream), "upload");
+  int rc = upload(M, M->grad, grad, kNPar * 4);
   if (rc) return rc;
   hipLaunchKernelGGL(k_mlp_adam, dim3((kNPar + 255) / 256), dim3(256), 0, M->stream, (const float*)M->grad,
                      next_adam(M, learning_rate), M->w1, M->w2, M->w2t);
@@ -541,9 +552,7 @@ int pbf_warm_model_train(pbf_warm_model* M, uint32_t epochs, uint32_t batch, flo
     // the permutation buffer is rewritten only after the previous epoch's batches ran
     int rc = check_hip(hipStreamSynchronize(M->stream), "train");
     if (rc) return rc;
-    if ((rc = check_hip(hipMemcpyAsync(M->perm, perm.data(), M->count * 4, hipMemcpyHostToDevice, M->stream),
-                        "upload")))
-      return rc;
+    if ((rc = upload(M, M->perm, perm.data(), M->count * 4))) return rc;
     for (uint64_t s = 0; s < M->count; s += batch) {
       const uint32_t cnt = (uint32_t)std::min<uint64_t>(batch, M->count - s);
       const AdamStep adam = next_adam(M, learning_rate);
@@ -552,9 +561,7 @@ int pbf_warm_model_train(pbf_warm_model* M, uint32_t epochs, uint32_t batch, flo
     }
   }
   float acc = 0.f;
-  int rc = check_hip(hipMemcpyAsync(&acc, M->loss_acc, 4, hipMemcpyDeviceToHost, M->stream), "download");
-  if (rc) return rc;
-  if ((rc = check_hip(hipStreamSynchronize(M->stream), "train"))) return rc;
+  if (int rc = download(M, &acc, M->loss_acc, 4)) return rc;
   if (mean_loss) *mean_loss = batches ? acc / (float)batches : 0.f;
   return PBF_OK;
 }
@@ -565,24 +572,15 @@ int pbf_warm_model_predict(pbf_warm_model* M, const float* features, uint64_t co
   if (!M->has_params) return set_error(PBF_ERR_STATE, "model has no parameters");
   if (!count) return PBF_OK;
   if (count >= (1ull << 32)) return set_error(PBF_ERR_ARG, "count out of range");
-  float *f = nullptr, *o = nullptr;
-  int rc = check_hip(hipMalloc((void**)&f, count * kFeat * 4), "hipMalloc");
-  if (rc) return rc;
-  if ((rc = check_hip(hipMalloc((void**)&o, count * 4), "hipMalloc"))) {
-    hipFree(f);
-    return rc;
+  for (uint64_t first = 0; first < count; first += kPredictRows) {
+    const uint64_t rows = std::min<uint64_t>(kPredictRows, count - first);
+    if (int rc = upload(M, M->pfeat, features + first * kFeat, rows * kFeat * 4)) return rc;
+    const uint32_t groups = (uint32_t)((rows + 15) / 16);
+    hipLaunchKernelGGL(k_mlp_forward, dim3(std::min<uint32_t>(groups, 4096u)), dim3(64), 0, M->stream, (uint32_t)rows,
+                       (const float*)M->pfeat, model_weights(M), 1.0f, nullptr, M->pout);
+    if (int rc = download(M, out + first, M->pout, rows * 4)) return rc;
   }
-  rc = check_hip(hipMemcpyAsync(f, features, count * kFeat * 4, hipMemcpyHostToDevice, M->stream), "upload");
-  if (!rc) {
-    const uint32_t groups = (uint32_t)((count + 15) / 16);
-    hipLaunchKernelGGL(k_mlp_forward, dim3(std::min<uint32_t>(groups, 4096u)), dim3(64), 0, M->stream,
-                       (uint32_t)count, (const float*)f, model_weights(M), 1.0f, nullptr, o);
-    rc = check_hip(hipMemcpyAsync(out, o, count * 4, hipMemcpyDeviceToHost, M->stream), "download");
-  }
-  if (!rc) rc = check_hip(hipStreamSynchronize(M->stream), "predict");
-  hipFree(f);
-  hipFree(o);
-  return rc;
+  return PBF_OK;
 }
 
 int pbf_set_warm_gain(pbf_context* c, float gain) {

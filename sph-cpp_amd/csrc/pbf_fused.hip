@@ -17,8 +17,8 @@
 //    appends the entries within h of the final positions to a compact row
 //    (cnb); vorticity, vorticity-apply and the second XSPH pass walk only that
 //    row, in the same order.
-//  * A particle is walked by one lane, or in small scenes by four (quad walks,
-//    below).
+//  * A particle is walked by one lane, or in small scenes by four or sixteen
+//    (pbf_walk.h).
 //  * The density pass writes lambda into the w word of its x* output, so the
 //    dp pass gathers a neighbour's x* and lambda in one 16-byte load.
 //  * The near-coincidence fix of compute_densities (particles.h:303-305) moves
@@ -202,10 +202,10 @@ __device__ __forceinline__ float density_lambda_one(uint32_t p, uint32_t n, cons
   return constraint > 0.0f ? constraint : 0.0f;
 }
 
-// The same by a quad (no features); lane 0 writes, counts the fixes and
+// The same by L lanes (no features); lane 0 writes, counts the fixes and
 // returns the error, the other lanes return 0.
-template <bool FAST, bool SR>
-__device__ __forceinline__ float density_lambda_quad(uint32_t p, const KParams& K, const float4* __restrict__ xs,
+template <bool FAST, bool SR, int L>
+__device__ __forceinline__ float density_lambda_group(uint32_t p, const KParams& K, const float4* __restrict__ xs,
                                                      const float4* __restrict__ v, float4* __restrict__ xt,
                                                      float* __restrict__ rho, float* __restrict__ lam,
                                                      const int32_t* __restrict__ nbr,
@@ -216,15 +216,18 @@ __device__ __forceinline__ float density_lambda_quad(uint32_t p, const KParams& 
   const int cnt = skin ? snb_count[p] : nbr_count[p];
   DensitySums s = density_start(K);
   bool hack = false;
-  const uint32_t* __restrict__ row = quad_row(skin ? snb : nbr, p, K.stride);
-  uint32_t q[2] = {row[0], row[256]};
-  for (int k0 = 0; k0 < cnt && !hack; k0 += kBatch) {
-    const float4 t[2] = {gather4(xs, q[0]), gather4(xs, q[1])};
-    row += kBatch * 64;
-    q[0] = row[0], q[1] = row[256];  // the next batch
+  GroupRow<L> row(skin ? snb : nbr, p, K.stride);
+  constexpr int kMine = GroupRow<L>::kMine;
+  for (int k0 = 0; k0 < cnt && !hack; k0 += GroupRow<L>::kEntries) {
+    uint32_t q[kMine];
+    float4 t[kMine];
+    row.template entries<true>(cnt - k0, K.pad, q);
+#pragma unroll
+    for (int j = 0; j < kMine; ++j) t[j] = gather4(xs, q[j]);
+    row.advance();
     bool near = false;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < kMine; ++j) {
       const f3 d = sub3(xp, xyz(t[j]));
       const float d2 = magsq3(d);
       near |= d2 < K.T_hack;
@@ -236,15 +239,15 @@ __device__ __forceinline__ float density_lambda_quad(uint32_t p, const KParams& 
         grad = smul3(K.neg_inv_rho0, nb_spiky<FAST, SR>(d, r, K));
         c2 = magsq3(grad);
       }
-      quad_add(s.density, dens);
-      quad_sub(s.sg.x, grad.x);
-      quad_sub(s.sg.y, grad.y);
-      quad_sub(s.sg.z, grad.z);
-      quad_add(s.sum_C, c2);
+      group_sum<L, false>(s.density, dens);
+      group_sum<L, true>(s.sg.x, grad.x);
+      group_sum<L, true>(s.sg.y, grad.y);
+      group_sum<L, true>(s.sg.z, grad.z);
+      group_sum<L, false>(s.sum_C, c2);
     }
-    hack = quad_any(near);
+    hack = group_bits<L>(near) != 0u;
   }
-  if ((threadIdx.x & 3u) != 0u) return 0.0f;
+  if (lane_in_group<L>() != 0u) return 0.0f;
   if (hack) s = density_plain<false, FAST>(p, xp, f3{0.f, 0.f, 0.f}, K, xs, v, nbr, nbr_count, hacks);
   float sum_C, lp;
   const float constraint = density_finish(p, s, xp, K, xt, rho, lam, sum_C, lp);
@@ -345,8 +348,8 @@ __device__ __forceinline__ void stamp_cells(uint64_t movers, uint32_t p, uint32_
 // calling thread is the one that clears the pass's flags (first): the same
 // bodies run as their own kernels (vb from xcd_block()) and inside the
 // persistent Jacobi kernel (vb from the calling block's share).
-// QUAD: by quads, a block of vb holding a quarter as many particles.
-template <int FM, bool FAST, bool SR, bool QUAD>
+// L: lanes per particle; a block of vb holds blockDim.x / L particles.
+template <int FM, bool FAST, bool SR, int L>
 __device__ __forceinline__ void density_pass(uint32_t vb, bool first, uint32_t n, int it, int eslot,
                                              const SolveCtl& S, const FeatCtl& F,
                                              const KParams& K, const float4* __restrict__ xs,
@@ -362,7 +365,7 @@ __device__ __forceinline__ void density_pass(uint32_t vb, bool first, uint32_t n
                                              const int32_t* __restrict__ snb,
                                              const int32_t* __restrict__ snb_count) {
   if (S.tol >= 0.0f && counters[C_DONE] != 0ull) return;
-  const uint32_t p = QUAD ? (vb * blockDim.x + threadIdx.x) >> 2 : vb * blockDim.x + threadIdx.x;
+  const uint32_t p = (vb * blockDim.x + threadIdx.x) / (uint32_t)L;
   // this iteration's pressure update records its moves in the other slot
   const bool skin = FM == 0 && skin_usable(counters, C_DISP + (it & 1));
   if (first) counters[C_DISP + ((it + 1) & 1)] = 0ull;
@@ -370,8 +373,8 @@ __device__ __forceinline__ void density_pass(uint32_t vb, bool first, uint32_t n
   uint32_t hacks = 0;
   float fo[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (p < n) {
-    if constexpr (QUAD)
-      e = density_lambda_quad<FAST, SR>(p, K, xs, v, xt, rho, lam, nbr, nbr_count, hacks, snb, snb_count, skin);
+    if constexpr (L != 1)
+      e = density_lambda_group<FAST, SR, L>(p, K, xs, v, xt, rho, lam, nbr, nbr_count, hacks, snb, snb_count, skin);
     else
       e = density_lambda_one<FM != 0, FAST, SR>(p, n, K, xs, v, xt, rho, lam, nbr, nbr_count, wmask, F, hacks, fo,
                                                 snb, snb_count, skin);
@@ -413,7 +416,7 @@ __device__ __forceinline__ void density_pass(uint32_t vb, bool first, uint32_t n
 }
 
 // (the exact and fast instances of the plain pass fit 64 registers: 8 wavefronts per SIMD)
-template <int FM, bool FAST, bool SR, bool QUAD>
+template <int FM, bool FAST, bool SR, int L>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu((FM == 0 && (SR || FAST)) ? 8 : 1)))
 k_density_lambda_c(uint32_t n, int it, int eslot, SolveCtl S, FeatCtl F,
                    KParams K, const float4* __restrict__ xs,
@@ -428,7 +431,7 @@ k_density_lambda_c(uint32_t n, int it, int eslot, SolveCtl S, FeatCtl F,
                    unsigned long long* __restrict__ counters,
                    const int32_t* __restrict__ snb,
                    const int32_t* __restrict__ snb_count) {
-  density_pass<FM, FAST, SR, QUAD>(xcd_block(), blockIdx.x == 0 && threadIdx.x == 0, n, it, eslot, S, F, K, xs, v, xt, rho,
+  density_pass<FM, FAST, SR, L>(xcd_block(), blockIdx.x == 0 && threadIdx.x == 0, n, it, eslot, S, F, K, xs, v, xt, rho,
                          lam, nbr, nbr_count, wmask, key, cstamp, stamp, mflag, counters, snb, snb_count);
 }
 
@@ -558,19 +561,22 @@ __device__ __forceinline__ f3 dp_walk(const int32_t* __restrict__ walk, int cnt,
   return dp;
 }
 
-// The same by a quad.
-template <bool FAST, bool SR>
-__device__ __forceinline__ f3 dp_walk_quad(const int32_t* __restrict__ walk, int cnt, uint32_t p, f3 xp, float lp,
+// The same by L lanes.
+template <bool FAST, bool SR, int L>
+__device__ __forceinline__ f3 dp_walk_group(const int32_t* __restrict__ walk, int cnt, uint32_t p, f3 xp, float lp,
                                            const KParams& K, const float4* __restrict__ xt) {
   f3 dp = {0.f, 0.f, 0.f};
-  const uint32_t* __restrict__ row = quad_row(walk, p, K.stride);
-  uint32_t q[2] = {row[0], row[256]};
-  for (int k0 = 0; k0 < cnt; k0 += kBatch) {
-    const float4 t[2] = {gather4(xt, q[0]), gather4(xt, q[1])};
-    row += kBatch * 64;
-    q[0] = row[0], q[1] = row[256];
+  GroupRow<L> row(walk, p, K.stride);
+  constexpr int kMine = GroupRow<L>::kMine;
+  for (int k0 = 0; k0 < cnt; k0 += GroupRow<L>::kEntries) {
+    uint32_t q[kMine];
+    float4 t[kMine];
+    row.template entries<true>(cnt - k0, K.pad, q);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < kMine; ++j) t[j] = gather4(xt, q[j]);
+    row.advance();
+#pragma unroll
+    for (int j = 0; j < kMine; ++j) {
       const f3 d = sub3(xp, xyz(t[j]));
       const float d2 = magsq3(d);
       f3 term = {0.f, 0.f, 0.f};
@@ -578,7 +584,7 @@ __device__ __forceinline__ f3 dp_walk_quad(const int32_t* __restrict__ walk, int
         const float r = nb_sqrt<FAST, SR>(d2);
         term = smul3(lp + t[j].w, nb_spiky<FAST, SR>(d, r, K));
       }
-      quad_add3(dp, term);
+      group_add3<L>(dp, term);
     }
   }
   return dp;
@@ -591,7 +597,7 @@ __device__ __forceinline__ f3 dp_walk_quad(const int32_t* __restrict__ walk, int
 // before the warm start; with the retry, also slot 1's after the damped
 // start) restores xsave; an error <= tol ends the solve with x* = xt.
 // Neither applies an update.
-template <bool FAST, bool SR, bool QUAD>
+template <bool FAST, bool SR, int L>
 __device__ __forceinline__ void dp_pass(uint32_t vb, bool first, uint32_t n, int it, int last, uint32_t stamp,
                                         const SolveCtl& S,
                                         const KParams& K, const float4* __restrict__ xt,
@@ -617,9 +623,9 @@ __device__ __forceinline__ void dp_pass(uint32_t vb, bool first, uint32_t n, int
     counters[C_HACK_FLAG + ((it + 1) & 1)] = 0ull;
     counters[C_MOVED_N + ((it + 1) & 1)] = 0ull;
   }
-  const uint32_t p = QUAD ? (vb * blockDim.x + threadIdx.x) >> 2 : vb * blockDim.x + threadIdx.x;
-  // (every lane of a quad computes the particle's new state; lane 0 writes it)
-  const bool writes = !QUAD || (threadIdx.x & 3u) == 0u;
+  const uint32_t p = (vb * blockDim.x + threadIdx.x) / (uint32_t)L;
+  // (every lane of a group computes the particle's new state; lane 0 writes it)
+  const bool writes = lane_in_group<L>() == 0u;
   // what this slot does, the same for every thread: 0 the update, 1 the
   // rejected warm start's restore, 2 the end of the solve (x* = xt)
   int mode = 0;
@@ -678,12 +684,12 @@ __device__ __forceinline__ void dp_pass(uint32_t vb, bool first, uint32_t n, int
     const float lp = xp4.w;
     const int cnt = skin ? snb_count[p] : nbr_count[p];
     // with no dirty lane in the wavefront every pair within h is one the
-    // density pass accepted at the same positions (static ranges); the quads
-    // find them by the same test, the single lanes by the mask it left
+    // density pass accepted at the same positions (static ranges); the lanes
+    // of a group find them by the same test, single lanes by the mask it left
     f3 dp;
-    if constexpr (QUAD)
-      dp = (SR && __ballot(plain) == 0ull) ? dp_walk_quad<FAST, SR>(walk, cnt, p, xp, lp, K, xt)
-                                           : dp_walk_quad<FAST, false>(walk, cnt, p, xp, lp, K, xt);
+    if constexpr (L != 1)
+      dp = (SR && __ballot(plain) == 0ull) ? dp_walk_group<FAST, SR, L>(walk, cnt, p, xp, lp, K, xt)
+                                           : dp_walk_group<FAST, false, L>(walk, cnt, p, xp, lp, K, xt);
     else {
       const uint64_t m0 = plain ? ~0ull : wmask[p];
       const uint64_t m1 = (plain || K.cap <= 64) ? ~0ull : wmask[n + p];
@@ -704,7 +710,7 @@ __device__ __forceinline__ void dp_pass(uint32_t vb, bool first, uint32_t n, int
   if (track) record_move(mv, counters, C_DISP + ((it + 1) & 1), K);
 }
 
-template <bool FAST, bool SR, bool QUAD>
+template <bool FAST, bool SR, int L>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) k_dp_update_c(uint32_t n, int it, int last, uint32_t stamp, SolveCtl S,
                                                         KParams K, const float4* __restrict__ xt,
                                                         const float4* __restrict__ x, float4* __restrict__ xs,
@@ -717,7 +723,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))
                                                         const int32_t* __restrict__ snb_count,
                                                         const float4* __restrict__ xs0,
                                                         const float* __restrict__ rho) {
-  dp_pass<FAST, SR, QUAD>(xcd_block(), blockIdx.x == 0 && threadIdx.x == 0, n, it, last, stamp, S, K, xt, x, xs, v, nbr,
+  dp_pass<FAST, SR, L>(xcd_block(), blockIdx.x == 0 && threadIdx.x == 0, n, it, last, stamp, S, K, xt, x, xs, v, nbr,
                 nbr_count, wmask, dirty, counters, snb, snb_count, xs0, rho);
 }
 
@@ -824,7 +830,7 @@ __global__ void __launch_bounds__(kBlock) k_warm_retry(uint32_t n, KParams K, co
 }
 
 // ---------------------------------------------------------------------------
-// The passes after the pressure solve, by quads.  A compact row (cnb) holds
+// The passes after the pressure solve, by groups of lanes.  A compact row (cnb) holds
 // the entries within h of the final positions as byte offsets into the
 // particle arrays.
 __device__ __forceinline__ float4 gather_at(const float4* __restrict__ a, uint32_t offset) {
@@ -841,7 +847,8 @@ __device__ __forceinline__ f3 xsph_term(f3 xp, f3 vp, float4 t, float4 vq, const
 // apply_viscosity (particles.h:436-447), first call: walks the skin or full
 // list and leaves the compact rows of the final positions for the passes that
 // follow.  An accepted entry's place in the row is the number accepted before
-// it: the quad's four verdicts come from one ballot.
+// it: the group's verdicts come from one ballot.
+template <int L>
 __global__ void __launch_bounds__(kBlock) k_viscosity_first(uint32_t n, KParams K, const float4* __restrict__ xs,
                                                             const float4* __restrict__ vin,
                                                             float4* __restrict__ vout,
@@ -853,8 +860,8 @@ __global__ void __launch_bounds__(kBlock) k_viscosity_first(uint32_t n, KParams 
                                                             const int32_t* __restrict__ snb,
                                                             const int32_t* __restrict__ snb_count,
                                                             unsigned long long* __restrict__ skin_hint) {
-  const uint32_t p = (xcd_block() * blockDim.x + threadIdx.x) >> 2;
-  const uint32_t u = threadIdx.x & 3u;
+  const uint32_t p = particle_of<L>();
+  const uint32_t u = lane_in_group<L>();
   // the next step builds skin lists only if this one's moves kept them usable to the end
   if (K.skin_mode && blockIdx.x == 0 && threadIdx.x == 0) *skin_hint = counters[C_DISP_ALL] == 0ull ? 1ull : 0ull;
   if (p >= n) return;
@@ -865,22 +872,26 @@ __global__ void __launch_bounds__(kBlock) k_viscosity_first(uint32_t n, KParams 
   // 0.045 h over the step (skin lists, above)
   const bool skin = skin_usable(counters, C_DISP_ALL);
   const int cnt = skin ? snb_count[p] : nbr_count[p];
-  const uint32_t* __restrict__ row = quad_row(skin ? snb : nbr, p, K.stride);
+  GroupRow<L> row(skin ? snb : nbr, p, K.stride);
+  constexpr int kMine = GroupRow<L>::kMine;
   int32_t* __restrict__ out = cnb + list_at(0, p, K.stride);
-  const uint32_t shift = threadIdx.x & 60u, before = (1u << u) - 1u;
+  const uint32_t before = (1u << u) - 1u;
   f3 dv = {0.f, 0.f, 0.f};
   uint32_t nc = 0;
-  uint32_t q[2] = {row[0], row[256]};
-  for (int k0 = 0; k0 < cnt; k0 += kBatch) {
-    const uint32_t at[2] = {q[0] << 4, q[1] << 4};
-    const float4 t[2] = {gather_at(xs, at[0]), gather_at(xs, at[1])};
-    const float4 vq[2] = {gather_at(vin, at[0]), gather_at(vin, at[1])};
-    row += kBatch * 64;
-    q[0] = row[0], q[1] = row[256];
+  for (int k0 = 0; k0 < cnt; k0 += GroupRow<L>::kEntries) {
+    uint32_t at[kMine];
+    float4 t[kMine], vq[kMine];
+    row.template entries<true>(cnt - k0, K.pad, at);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < kMine; ++j) {
+      at[j] <<= 4;
+      t[j] = gather_at(xs, at[j]), vq[j] = gather_at(vin, at[j]);
+    }
+    row.advance();
+#pragma unroll
+    for (int j = 0; j < kMine; ++j) {
       const bool in = within_h(magsq3(sub3(xp, xyz(t[j]))), K);
-      const uint32_t bits = (uint32_t)(__ballot(in) >> shift) & 15u;
+      const uint32_t bits = group_bits<L>(in);
       f3 term = {0.f, 0.f, 0.f};
       if (in) {
         const uint32_t k = nc + (uint32_t)__popc(bits & before);
@@ -888,7 +899,7 @@ __global__ void __launch_bounds__(kBlock) k_viscosity_first(uint32_t n, KParams 
         term = xsph_term(xp, vp, t[j], vq[j], K);
       }
       nc += (uint32_t)__popc(bits);
-      quad_add3(dv, term);
+      group_add3<L>(dv, term);
     }
   }
   if (u != 0u) return;
@@ -898,28 +909,28 @@ __global__ void __launch_bounds__(kBlock) k_viscosity_first(uint32_t n, KParams 
   vout[p] = make_float4(nv.x, nv.y, nv.z, v4.w);  // the density stays in w
 }
 
-// A quad's walk over a compact row: TERM(offset) gives the three terms of an
-// entry, which enter `sum` in list order.  Lanes past the row's end gather
-// the particle itself and add +0.
-template <class Load, class Term>
-__device__ __forceinline__ void quad_walk_compact(const int32_t* __restrict__ cnb, int cnt, uint32_t p,
-                                                  const KParams& K, f3& sum, Load load, Term term) {
-  const uint32_t* __restrict__ row = quad_row(cnb, p, K.stride);
-  const int u = (int)(threadIdx.x & 3u);
-  uint32_t q[2] = {row[0], row[256]};
-  for (int k0 = 0; k0 < cnt; k0 += kBatch) {
-    const bool on[2] = {k0 + u < cnt, k0 + 4 + u < cnt};
-    const uint32_t at[2] = {on[0] ? q[0] : p << 4, on[1] ? q[1] : p << 4};
-    const auto a = load(at[0]);
-    const auto b = load(at[1]);
-    row += kBatch * 64;
-    q[0] = row[0], q[1] = row[256];
-    f3 t = {0.f, 0.f, 0.f};
-    if (on[0]) t = term(a);
-    quad_add3(sum, t);
-    t = f3{0.f, 0.f, 0.f};
-    if (on[1]) t = term(b);
-    quad_add3(sum, t);
+// A group's walk over a compact row: TERM(load(offset)) gives the three terms
+// of an entry, which enter `sum` in list order.  Lanes past the row's end
+// gather the particle itself and add +0.
+template <int L, class Load, class Term>
+__device__ __forceinline__ void group_walk_compact(const int32_t* __restrict__ cnb, int cnt, uint32_t p,
+                                                   const KParams& K, f3& sum, Load load, Term term) {
+  GroupRow<L> row(cnb, p, K.stride);
+  constexpr int kMine = GroupRow<L>::kMine;
+  const int u = (int)lane_in_group<L>();
+  for (int k0 = 0; k0 < cnt; k0 += GroupRow<L>::kEntries) {
+    uint32_t at[kMine];
+    decltype(load(0u)) a[kMine];
+    row.template entries<false>(cnt - k0, p << 4, at);
+#pragma unroll
+    for (int j = 0; j < kMine; ++j) a[j] = load(at[j]);
+    row.advance();
+#pragma unroll
+    for (int j = 0; j < kMine; ++j) {
+      f3 t = {0.f, 0.f, 0.f};
+      if (u + j * L < cnt - k0) t = term(a[j]);
+      group_add3<L>(sum, t);
+    }
   }
 }
 struct Pair2 {  // a neighbour's position and its velocity or vorticity
@@ -950,29 +961,29 @@ __device__ __forceinline__ void lane_walk_compact(const int32_t* __restrict__ cn
   }
 }
 
-template <bool QUAD, class Load, class Term>
+template <int L, class Load, class Term>
 __device__ __forceinline__ void walk_compact(const int32_t* __restrict__ cnb, int cnt, uint32_t p, const KParams& K,
                                              f3& sum, Load load, Term term) {
-  if constexpr (QUAD)
-    quad_walk_compact(cnb, cnt, p, K, sum, load, term);
+  if constexpr (L != 1)
+    group_walk_compact<L>(cnb, cnt, p, K, sum, load, term);
   else
     lane_walk_compact(cnb, cnt, p, K, sum, load, term);
 }
 // apply_viscosity, second call, fused with update_positions (particles.h:390-394)
-template <bool QUAD>
+template <int L>
 __global__ void __launch_bounds__(kBlock) k_viscosity_last(uint32_t n, KParams K, const float4* __restrict__ xs,
                                                            const float4* __restrict__ vin, float4* __restrict__ vout,
                                                            float4* __restrict__ x, const int32_t* __restrict__ cnb,
                                                            const int32_t* __restrict__ cnb_count) {
-  const uint32_t p = particle_of<QUAD>();
+  const uint32_t p = particle_of<L>();
   if (p >= n) return;
   const f3 xp = ld3(xs, p);
   const f3 vp = ld3(vin, p);
   f3 dv = {0.f, 0.f, 0.f};
-  walk_compact<QUAD>(
+  walk_compact<L>(
       cnb, cnb_count[p], p, K, dv, [&](uint32_t at) { return Pair2{gather_at(xs, at), gather_at(vin, at)}; },
       [&](const Pair2& q) { return xsph_term(xp, vp, q.t, q.w, K); });
-  if (QUAD && (threadIdx.x & 3u) != 0u) return;
+  if (lane_in_group<L>() != 0u) return;
   f3 nv = vp;
   acc3(nv, smul3(K.visc, dv));
   st3(vout, p, nv);
@@ -980,46 +991,46 @@ __global__ void __launch_bounds__(kBlock) k_viscosity_last(uint32_t n, KParams K
 }
 
 // compute_vorticity (particles.h:452-466) -> scr (omega, and |omega| in w)
-template <bool SR, bool QUAD>
+template <bool SR, int L>
 __global__ void __launch_bounds__(kBlock) k_vorticity_c(uint32_t n, KParams K, const float4* __restrict__ xs,
                                                         const float4* __restrict__ vin, float4* __restrict__ scr,
                                                         const int32_t* __restrict__ cnb,
                                                         const int32_t* __restrict__ cnb_count) {
-  const uint32_t p = particle_of<QUAD>();
+  const uint32_t p = particle_of<L>();
   if (p >= n) return;
   const f3 xp = ld3(xs, p);
   const f3 vp = ld3(vin, p);
   f3 w = {0.f, 0.f, 0.f};
-  walk_compact<QUAD>(
+  walk_compact<L>(
       cnb, cnb_count[p], p, K, w, [&](uint32_t at) { return Pair2{gather_at(xs, at), gather_at(vin, at)}; },
       [&](const Pair2& q) {
         const f3 d = sub3(xp, xyz(q.t));
         const float r = sqrt_cr(magsq3(d));
         return cross3(sub3(xyz(q.w), vp), nb_spiky<false, SR>(d, r, K));
       });
-  if (QUAD && (threadIdx.x & 3u) != 0u) return;
+  if (lane_in_group<L>() != 0u) return;
   scr[p] = make_float4(w.x, w.y, w.z, sqrtf(magsq3(w)));  // |omega| for apply_vorticity's gathers
 }
 
 // apply_vorticity (particles.h:471-487), v in place (own particle only)
-template <bool SR, bool QUAD>
+template <bool SR, int L>
 __global__ void __launch_bounds__(kBlock) k_apply_vorticity_c(uint32_t n, KParams K, const float4* __restrict__ xs,
                                                               const float4* __restrict__ scr,
                                                               float4* __restrict__ v,
                                                               const int32_t* __restrict__ cnb,
                                                               const int32_t* __restrict__ cnb_count) {
-  const uint32_t p = particle_of<QUAD>();
+  const uint32_t p = particle_of<L>();
   if (p >= n) return;
   const f3 xp = ld3(xs, p);
   f3 eta = {0.f, 0.f, 0.f};
-  walk_compact<QUAD>(
+  walk_compact<L>(
       cnb, cnb_count[p], p, K, eta, [&](uint32_t at) { return Pair2{gather_at(xs, at), gather_at(scr, at)}; },
       [&](const Pair2& q) {
         const f3 d = sub3(xp, xyz(q.t));
         const float r = sqrt_cr(magsq3(d));
         return smul3(q.w.w, nb_spiky<false, SR>(d, r, K));  // |omega_q|, computed by the vorticity pass
       });
-  if (QUAD && (threadIdx.x & 3u) != 0u) return;
+  if (lane_in_group<L>() != 0u) return;
   const f3 N = div3(eta, sqrtf(magsq3(eta)) + K.r_eps);
   const float4 v4 = v[p];
   f3 vp = xyz(v4);
@@ -1094,11 +1105,20 @@ __global__ void __launch_bounds__(kStageBlock) k_viscosity_first_lane(
     timer_end((c), t_);                                                                                   \
   } while (0)
 
-// Whether a pass goes by quads or by single lanes (same results).  Quads take
-// a quarter of the steps with four times the wavefronts and pay for their
-// ordered sums with twelve to twenty DPP additions per four pairs, so they win
-// while single lanes leave the chip short of wavefronts (524,288 lanes fill
-// it).  Measured, quads against lanes, us per launch on a dam break at rest:
+// How many lanes of a pass share a particle (same results): sixteen, four or
+// one.  More lanes take fewer steps with more wavefronts and pay for their
+// ordered sums, a DPP addition for every entry and term in all lanes, so they
+// win while fewer leave the chip short of wavefronts (524,288 single lanes
+// fill it).  Measured, us per launch on a dam break at rest, timed with events
+// (some 3 us above the kernels' own time); 16 lanes against 4:
+//   particles            960          8,192        16,384       32,768
+//   density              10.3 / 11.6  11.1 / 12.2  12.3 / 12.3  16.6 / 13.7
+//   pressure update       8.1 /  9.8   8.9 /  9.8  10.3 / 10.1  13.6 / 11.0
+//   first XSPH            8.5 / 10.6   8.7 / 11.1  10.2 / 11.2  12.9 / 12.3
+//   vorticity             6.4 /  8.6   6.8 /  8.8   8.1 /  8.8   9.6 /  9.4
+//   confinement           6.4 /  8.5   6.7 /  8.5   7.6 /  8.5   9.9 /  9.1
+//   second XSPH           7.1 /  9.1   7.3 /  9.2   7.7 /  9.1   9.3 /  9.7
+// and 4 against 1:
 //   particles            32,768       131,072      262,144      1,048,576
 //   density              10.7 / 14.3  19.8 / 18.0  30.8 / 25.8  95 / 80
 //   pressure update       9.6 / 15.0  17.1 / 18.1  27.7 / 25.5  91 / 77
@@ -1106,21 +1126,22 @@ __global__ void __launch_bounds__(kStageBlock) k_viscosity_first_lane(
 //   vorticity             8.8 / 13.1  15.9 / 17.8  25.8 / 27.1  111 / 96
 //   confinement           8.6 / 13.1  15.3 / 16.3  26.8 / 27.6  87 / 84
 //   second XSPH           9.1 / 15.0  15.3 / 17.1  26.0 / 27.4  86 / 83
-// (lanes overtake between 65,536 and 131,072 particles in the pressure solve,
-// and near 524,288 in the passes after it)
-constexpr uint64_t kQuadsPressure = 98304;
-constexpr uint64_t kQuadsTail = 524288;
-static bool pressure_quads(const pbf_context* c) { return c->n <= kQuadsPressure; }
-static bool tail_quads(const pbf_context* c) { return c->n <= kQuadsTail; }
+// (single lanes overtake between 65,536 and 131,072 particles in the pressure
+// solve, and near 524,288 in the passes after it)
+constexpr uint64_t kRowsPressure = 12288, kQuadsPressure = 98304;
+constexpr uint64_t kRowsTail = 24576, kQuadsTail = 524288;
+static int pressure_lanes(const pbf_context* c) { return c->n <= kRowsPressure ? 16 : (c->n <= kQuadsPressure ? 4 : 1); }
+static int tail_lanes(const pbf_context* c) { return c->n <= kRowsTail ? 16 : (c->n <= kQuadsTail ? 4 : 1); }
 
-// four lanes per particle
-#define PBF_LAUNCH_QUADS(c, name, kern, ...)                                                              \
+// `lanes` lanes per particle
+#define PBF_LAUNCH_LANES(c, name, lanes, kern, ...)                                                       \
   do {                                                                                                    \
-    const uint32_t n_ = (uint32_t)(c)->n;                                                                 \
+    const uint64_t n_ = (c)->n;                                                                           \
     if (!n_) return;                                                                                      \
     KernelTimer* t_ = timer_begin((c), name);                                                             \
     const uint32_t b_ = (c)->tune.block_size;                                                             \
-    hipLaunchKernelGGL(kern, dim3((n_ + b_ / 4 - 1) / (b_ / 4)), dim3(b_), 0, (c)->stream, n_, __VA_ARGS__); \
+    hipLaunchKernelGGL(kern, dim3((uint32_t)((n_ * (lanes) + b_ - 1) / b_)), dim3(b_), 0, (c)->stream,    \
+                       (uint32_t)n_, __VA_ARGS__);                                                        \
     timer_end((c), t_);                                                                                   \
   } while (0)
 
@@ -1144,40 +1165,37 @@ static bool tail_quads(const pbf_context* c) { return c->n <= kQuadsTail; }
       launch(c, name, (KT<false>), __VA_ARGS__);          \
   } while (0)
 
-template <int FM, bool FAST, bool SR, bool QUAD>
+template <int FM, bool FAST, bool SR, int L>
 static void launch_density_as(pbf_context* c, const char* name, int it, int eslot, const SolveCtl& S,
                               const FeatCtl& F) {
-  if constexpr (QUAD)
-    PBF_LAUNCH_QUADS(c, name, (k_density_lambda_c<FM, FAST, SR, true>), it, eslot, S, F, c->K, (const float4*)c->xs,
-                     (const float4*)c->v, c->xt, c->rho, c->lam, (const int32_t*)c->nbr,
-                     (const int32_t*)c->nbr_count, c->wmask, (const uint32_t*)c->key, c->cstamp, c->dirty_stamp, c->mflag, c->counters,
-                     (const int32_t*)c->snb, (const int32_t*)c->snb_count);
-  else
-    PBF_LAUNCH(c, name, (k_density_lambda_c<FM, FAST, SR, false>), it, eslot, S, F, c->K, (const float4*)c->xs,
-               (const float4*)c->v, c->xt, c->rho, c->lam, (const int32_t*)c->nbr, (const int32_t*)c->nbr_count,
-               c->wmask, (const uint32_t*)c->key, c->cstamp, c->dirty_stamp, c->mflag, c->counters, (const int32_t*)c->snb,
-               (const int32_t*)c->snb_count);
+  PBF_LAUNCH_LANES(c, name, L, (k_density_lambda_c<FM, FAST, SR, L>), it, eslot, S, F, c->K, (const float4*)c->xs,
+                   (const float4*)c->v, c->xt, c->rho, c->lam, (const int32_t*)c->nbr, (const int32_t*)c->nbr_count,
+                   c->wmask, (const uint32_t*)c->key, c->cstamp, c->dirty_stamp, c->mflag, c->counters,
+                   (const int32_t*)c->snb, (const int32_t*)c->snb_count);
 }
 
-template <int FM, bool QUAD>
+template <int FM, int L>
 static void launch_density_fm(pbf_context* c, const char* name, int it, int eslot, const SolveCtl& S,
                               const FeatCtl& F) {
   if (c->K.fast)
-    launch_density_as<FM, true, false, QUAD>(c, name, it, eslot, S, F);
+    launch_density_as<FM, true, false, L>(c, name, it, eslot, S, F);
   else if (c->K.static_ranges)
-    launch_density_as<FM, false, true, QUAD>(c, name, it, eslot, S, F);
+    launch_density_as<FM, false, true, L>(c, name, it, eslot, S, F);
   else
-    launch_density_as<FM, false, false, QUAD>(c, name, it, eslot, S, F);
+    launch_density_as<FM, false, false, L>(c, name, it, eslot, S, F);
 }
 
 void launch_density_lambda_masked(pbf_context* c, int it, int eslot, const SolveCtl& S, const FeatCtl& F) {
   if (F.wlam)
-    launch_density_fm<2, false>(c, "density_warm_network", it, eslot, S, F);
+    launch_density_fm<2, 1>(c, "density_warm_network", it, eslot, S, F);
   else if (F.feat)
-    launch_density_fm<1, false>(c, "density_features", it, eslot, S, F);
+    launch_density_fm<1, 1>(c, "density_features", it, eslot, S, F);
   else
-    pressure_quads(c) ? launch_density_fm<0, true>(c, "density_lambda", it, eslot, S, F)
-                      : launch_density_fm<0, false>(c, "density_lambda", it, eslot, S, F);
+    switch (pressure_lanes(c)) {
+      case 16: return launch_density_fm<0, 16>(c, "density_lambda", it, eslot, S, F);
+      case 4: return launch_density_fm<0, 4>(c, "density_lambda", it, eslot, S, F);
+      default: return launch_density_fm<0, 1>(c, "density_lambda", it, eslot, S, F);
+    }
 }
 
 void launch_lambda_repair(pbf_context* c, int it, const SolveCtl& S) {
@@ -1193,10 +1211,11 @@ void launch_lambda_repair(pbf_context* c, int it, const SolveCtl& S) {
       (const int32_t*)c->snb, (const int32_t*)c->snb_count, (const float4*)c->xs0, (const float*)c->rho
 template <bool FAST, bool SR>
 static void launch_dp_as(pbf_context* c, int it, int last, const SolveCtl& S) {
-  if (pressure_quads(c))
-    PBF_LAUNCH_QUADS(c, "dp_update", (k_dp_update_c<FAST, SR, true>), PBF_DP_ARGS);
-  else
-    PBF_LAUNCH(c, "dp_update", (k_dp_update_c<FAST, SR, false>), PBF_DP_ARGS);
+  switch (pressure_lanes(c)) {
+    case 16: PBF_LAUNCH_LANES(c, "dp_update", 16, (k_dp_update_c<FAST, SR, 16>), PBF_DP_ARGS); break;
+    case 4: PBF_LAUNCH_LANES(c, "dp_update", 4, (k_dp_update_c<FAST, SR, 4>), PBF_DP_ARGS); break;
+    default: PBF_LAUNCH_LANES(c, "dp_update", 1, (k_dp_update_c<FAST, SR, 1>), PBF_DP_ARGS);
+  }
 }
 
 void launch_dp_update_masked(pbf_context* c, int it, int last, const SolveCtl& S) {
@@ -1258,7 +1277,7 @@ __global__ void __launch_bounds__(kBlock) k_jacobi_persistent(JacobiArgs A) {
     const uint32_t stamp = A.stamp0 + it;
     const int eslot = A.solve ? (int)it + 1 : 0;
     for (uint32_t vb = vb0; vb < vb1; ++vb)
-      density_pass<0, FAST, SR, false>(vb, vb == 0 && threadIdx.x == 0, A.n, (int)it, eslot, A.S, F0, A.K, A.xs, A.v, A.xt,
+      density_pass<0, FAST, SR, 1>(vb, vb == 0 && threadIdx.x == 0, A.n, (int)it, eslot, A.S, F0, A.K, A.xs, A.v, A.xt,
                             A.rho, A.lam, A.nbr, A.nbr_count, A.wmask, A.key, A.cstamp, stamp, A.mflag, A.counters, A.snb,
                             A.snb_count);
     grid.sync();
@@ -1268,7 +1287,7 @@ __global__ void __launch_bounds__(kBlock) k_jacobi_persistent(JacobiArgs A) {
     grid.sync();
     const int last = A.last_vel && it + 1 == A.iters;
     for (uint32_t vb = vb0; vb < vb1; ++vb)
-      dp_pass<FAST, SR, false>(vb, vb == 0 && threadIdx.x == 0, A.n, (int)it, last, stamp, A.S, A.K, A.xt, A.x, A.xs, A.v,
+      dp_pass<FAST, SR, 1>(vb, vb == 0 && threadIdx.x == 0, A.n, (int)it, last, stamp, A.S, A.K, A.xt, A.x, A.xs, A.v,
                     A.nbr, A.nbr_count, A.wmask, A.dirty, A.counters, A.snb, A.snb_count, A.xs0, A.rho);
     grid.sync();
   }
@@ -1408,46 +1427,47 @@ void launch_combine_errors(pbf_context* c) {
       c->cnb, c->cnb_count, (const unsigned long long*)c->counters, (const int32_t*)c->snb,                     \
       (const int32_t*)c->snb_count, c->skin_hint
 void launch_viscosity_first(pbf_context* c) {
-  if (tail_quads(c))
-    PBF_LAUNCH_QUADS(c, "viscosity", k_viscosity_first, PBF_VISC_ARGS);
-  else
-    PBF_LAUNCH_STAGED(c, "viscosity", k_viscosity_first_lane, PBF_VISC_ARGS);
+  switch (tail_lanes(c)) {
+    case 16: PBF_LAUNCH_LANES(c, "viscosity", 16, k_viscosity_first<16>, PBF_VISC_ARGS); break;
+    case 4: PBF_LAUNCH_LANES(c, "viscosity", 4, k_viscosity_first<4>, PBF_VISC_ARGS); break;
+    default: PBF_LAUNCH_STAGED(c, "viscosity", k_viscosity_first_lane, PBF_VISC_ARGS);
+  }
 }
 
 // the vorticity passes stay exact in both arithmetic modes; the static-range
 // instance of the divide where KParams::static_ranges holds
-#define PBF_LAUNCH_SR(c, name, KT, Q, ...)                                  \
-  do {                                                                      \
-    if ((c)->K.static_ranges) {                                             \
-      if (Q)                                                                \
-        PBF_LAUNCH_QUADS(c, name, (KT<true, true>), __VA_ARGS__);           \
-      else                                                                  \
-        PBF_LAUNCH(c, name, (KT<true, false>), __VA_ARGS__);                \
-    } else {                                                                \
-      if (Q)                                                                \
-        PBF_LAUNCH_QUADS(c, name, (KT<false, true>), __VA_ARGS__);          \
-      else                                                                  \
-        PBF_LAUNCH(c, name, (KT<false, false>), __VA_ARGS__);               \
-    }                                                                       \
+#define PBF_LAUNCH_SR_AS(c, name, KT, L, ...)                         \
+  do {                                                                \
+    if ((c)->K.static_ranges)                                         \
+      PBF_LAUNCH_LANES(c, name, L, (KT<true, L>), __VA_ARGS__);       \
+    else                                                              \
+      PBF_LAUNCH_LANES(c, name, L, (KT<false, L>), __VA_ARGS__);      \
   } while (0)
+#define PBF_LAUNCH_SR(c, name, KT, ...)                               \
+  switch (tail_lanes(c)) {                                            \
+    case 16: PBF_LAUNCH_SR_AS(c, name, KT, 16, __VA_ARGS__); break;   \
+    case 4: PBF_LAUNCH_SR_AS(c, name, KT, 4, __VA_ARGS__); break;     \
+    default: PBF_LAUNCH_SR_AS(c, name, KT, 1, __VA_ARGS__);           \
+  }
 
 void launch_vorticity_masked(pbf_context* c) {
-  PBF_LAUNCH_SR(c, "vorticity", k_vorticity_c, tail_quads(c), c->K, (const float4*)c->xs, (const float4*)c->va, c->scr,
+  PBF_LAUNCH_SR(c, "vorticity", k_vorticity_c, c->K, (const float4*)c->xs, (const float4*)c->va, c->scr,
                 (const int32_t*)c->cnb, (const int32_t*)c->cnb_count);
 }
 
 void launch_apply_vorticity_masked(pbf_context* c) {
-  PBF_LAUNCH_SR(c, "apply_vorticity", k_apply_vorticity_c, tail_quads(c), c->K, (const float4*)c->xs,
+  PBF_LAUNCH_SR(c, "apply_vorticity", k_apply_vorticity_c, c->K, (const float4*)c->xs,
                 (const float4*)c->scr, c->va, (const int32_t*)c->cnb, (const int32_t*)c->cnb_count);
 }
 
 #define PBF_LAST_ARGS \
   c->K, (const float4*)c->xs, (const float4*)c->va, c->v, c->x, (const int32_t*)c->cnb, (const int32_t*)c->cnb_count
 void launch_viscosity_last(pbf_context* c) {
-  if (tail_quads(c))
-    PBF_LAUNCH_QUADS(c, "viscosity_positions", k_viscosity_last<true>, PBF_LAST_ARGS);
-  else
-    PBF_LAUNCH(c, "viscosity_positions", k_viscosity_last<false>, PBF_LAST_ARGS);
+  switch (tail_lanes(c)) {
+    case 16: PBF_LAUNCH_LANES(c, "viscosity_positions", 16, k_viscosity_last<16>, PBF_LAST_ARGS); break;
+    case 4: PBF_LAUNCH_LANES(c, "viscosity_positions", 4, k_viscosity_last<4>, PBF_LAST_ARGS); break;
+    default: PBF_LAUNCH_LANES(c, "viscosity_positions", 1, k_viscosity_last<1>, PBF_LAST_ARGS);
+  }
 }
 
 }  // namespace pbf

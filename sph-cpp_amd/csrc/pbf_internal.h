@@ -163,9 +163,9 @@ struct FeatCtl {
 __host__ __device__ __forceinline__ uint64_t list_at(uint32_t k, uint32_t p, uint32_t stride) {
   return ((uint64_t)(p >> 6) * stride + (k & ~3u)) * 64u + (p & 63u) * 4u + (k & 3u);
 }
-// entries of the lists of `capacity` particles, with one more batch of eight
-// rows that a walk may load ahead
-inline uint64_t list_size(uint64_t capacity, uint64_t stride) { return ((capacity + 63) / 64 * stride + 8) * 64; }
+// entries of the lists of `capacity` particles, with the rows past the last
+// list that a walk may load ahead (up to 31 past an entry)
+inline uint64_t list_size(uint64_t capacity, uint64_t stride) { return ((capacity + 63) / 64 * stride + 32) * 64; }
 
 // Pinned memory of one object (a context, a warm-start model) that its copies
 // from and to ordinary memory go through (pbf_transfer.hip).  One transfer at

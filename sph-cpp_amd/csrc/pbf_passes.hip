@@ -48,9 +48,9 @@ __device__ __forceinline__ Walk walk_of(const PassLists& L, uint32_t p) {
   const bool skin = L.skin && skin_usable(L.counters, C_DISP_ALL);
   return Walk{skin ? L.snb : L.nbr, skin ? L.snb_count[p] : L.nbr_count[p]};
 }
-template <bool QUAD>
+template <int LANES>
 __device__ __forceinline__ bool pass_writes() {
-  return !QUAD || (threadIdx.x & 3u) == 0u;
+  return lane_in_group<LANES>() == 0u;
 }
 
 // Quads below this many particles, single lanes above, for the reason given at
@@ -63,9 +63,9 @@ constexpr uint64_t kPassQuads = 131072;
     if (!n_) return;                                                                                             \
     KernelTimer* t_ = timer_begin((c), name);                                                                    \
     if (n_ <= kPassQuads)                                                                                        \
-      hipLaunchKernelGGL(kern<true>, dim3(nblocks(4ull * n_)), dim3(kBlock), 0, (c)->stream, n_, __VA_ARGS__);   \
+      hipLaunchKernelGGL(kern<4>, dim3(nblocks(4ull * n_)), dim3(kBlock), 0, (c)->stream, n_, __VA_ARGS__);   \
     else                                                                                                         \
-      hipLaunchKernelGGL(kern<false>, dim3(nblocks(n_)), dim3(kBlock), 0, (c)->stream, n_, __VA_ARGS__);         \
+      hipLaunchKernelGGL(kern<1>, dim3(nblocks(n_)), dim3(kBlock), 0, (c)->stream, n_, __VA_ARGS__);         \
     timer_end((c), t_);                                                                                          \
   } while (0)
 
@@ -100,27 +100,27 @@ void launch_forces_predict(pbf_context* c, int flags, uint64_t b, uint64_t e) {
 // compute_densities (particles.h:292-313).  Reads xs, writes xt (the position
 // star with the near-coincidence fix applied, particles.h:303-305) and rho;
 // the API swaps xs and xt afterwards.
-template <bool QUAD>
+template <int LANES>
 __global__ void __launch_bounds__(kBlock) k_density(uint32_t n, uint32_t b, uint32_t e, KParams K,
                                                     const uint32_t* __restrict__ oid, const float4* __restrict__ xs,
                                                     const float4* __restrict__ v, float4* __restrict__ xt,
                                                     float* __restrict__ rho, PassLists L,
                                                     const float4* __restrict__ xs0,
                                                     unsigned long long* __restrict__ counters) {
-  const uint32_t p = particle_of<QUAD>();
+  const uint32_t p = particle_of<LANES>();
   if (p >= n) return;
   f3 xp = ld3(xs, p);
   if (!in_span(oid[p], b, e)) {
-    if (pass_writes<QUAD>()) st3(xt, p, xp);
+    if (pass_writes<LANES>()) st3(xt, p, xp);
     return;
   }
   Terms<1> sum{{K.mass_W0}};
   bool near = false;
   const Walk w = walk_of(L, p);
-  walk_within<QUAD>(
+  walk_within<LANES>(
       w.list, w.cnt, p, xp, K, xs, sum, near, [](uint32_t) { return NoData{}; },
       [&](f3, float d2, NoData, Terms<1>& t) { t.a[0] = K.mass * poly6_in(sqrt_cr(d2), K); });
-  if (!pass_writes<QUAD>()) return;
+  if (!pass_writes<LANES>()) return;
   uint32_t hacks = 0;
   if (near) {
     // magnitude(x*_p - x*_q) < 1e-8 (particles.h:304): the particle again, entry by entry
@@ -159,24 +159,24 @@ void launch_density(pbf_context* c, uint64_t b, uint64_t e) {
 }
 
 // compute_pressure_lambdas (particles.h:318-342) from positions `pos`
-template <bool QUAD>
+template <int LANES>
 __global__ void __launch_bounds__(kBlock) k_lambda(uint32_t n, uint32_t b, uint32_t e, KParams K,
                                                    const uint32_t* __restrict__ oid, const float4* __restrict__ pos,
                                                    const float* __restrict__ rho, float* __restrict__ lam,
                                                    PassLists L) {
-  const uint32_t p = particle_of<QUAD>();
+  const uint32_t p = particle_of<LANES>();
   if (p >= n || !in_span(oid[p], b, e)) return;
   // minus the sum of the gradients, and the sum of their squares
   Terms<4> sum{};
   bool near = false;
   const Walk w = walk_of(L, p);
-  walk_within<QUAD>(
+  walk_within<LANES>(
       w.list, w.cnt, p, ld3(pos, p), K, pos, sum, near, [](uint32_t) { return NoData{}; },
       [&](f3 d, float d2, NoData, Terms<4>& t) {
         const f3 grad = smul3(K.neg_inv_rho0, spiky_in(d, sqrt_cr(d2), K));
         t = Terms<4>{{-grad.x, -grad.y, -grad.z, magsq3(grad)}};
       });
-  if (!pass_writes<QUAD>()) return;
+  if (!pass_writes<LANES>()) return;
   const float sum_C = sum.a[3] + magsq3(f3{sum.a[0], sum.a[1], sum.a[2]});
   const float constraint = rho[p] / K.rho0 - 1.0f;
   const float C_p = ((double)constraint < 0.0) ? 0.0f : constraint;
@@ -189,23 +189,23 @@ void launch_lambda(pbf_context* c, const float4* pos, uint64_t b, uint64_t e) {
 }
 
 // compute_pressure_dps (particles.h:348-358): dp sum in list order
-template <bool QUAD>
+template <int LANES>
 __global__ void __launch_bounds__(kBlock) k_dp(uint32_t n, uint32_t b, uint32_t e, KParams K,
                                                const uint32_t* __restrict__ oid, const float4* __restrict__ pos,
                                                const float* __restrict__ lam, float4* __restrict__ scr, PassLists L) {
-  const uint32_t p = particle_of<QUAD>();
+  const uint32_t p = particle_of<LANES>();
   if (p >= n || !in_span(oid[p], b, e)) return;
   const float lp = lam[p];
   Terms<3> sum{};
   bool near = false;
   const Walk w = walk_of(L, p);
-  walk_within<QUAD>(
+  walk_within<LANES>(
       w.list, w.cnt, p, ld3(pos, p), K, pos, sum, near, [&](uint32_t q) { return lam[q]; },
       [&](f3 d, float d2, float lq, Terms<3>& t) {
         const f3 s = smul3(lp + lq, spiky_in(d, sqrt_cr(d2), K));
         t = Terms<3>{{s.x, s.y, s.z}};
       });
-  if (pass_writes<QUAD>()) st3(scr, p, smul3(K.inv_rho0, f3{sum.a[0], sum.a[1], sum.a[2]}));
+  if (pass_writes<LANES>()) st3(scr, p, smul3(K.inv_rho0, f3{sum.a[0], sum.a[1], sum.a[2]}));
 }
 
 void launch_dp(pbf_context* c, uint64_t b, uint64_t e) {
@@ -288,30 +288,30 @@ struct VelocityDensity {
   float4 v;
   float rho;
 };
-template <bool QUAD>
+template <int LANES>
 __global__ void __launch_bounds__(kBlock) k_viscosity(uint32_t n, uint32_t b, uint32_t e, KParams K,
                                                       const uint32_t* __restrict__ oid,
                                                       const float4* __restrict__ xs, const float* __restrict__ rho,
                                                       const float4* __restrict__ vin, float4* __restrict__ vout,
                                                       PassLists L) {
-  const uint32_t p = particle_of<QUAD>();
+  const uint32_t p = particle_of<LANES>();
   if (p >= n) return;
   const f3 vp = ld3(vin, p);
   if (!in_span(oid[p], b, e)) {
-    if (pass_writes<QUAD>()) st3(vout, p, vp);
+    if (pass_writes<LANES>()) st3(vout, p, vp);
     return;
   }
   Terms<3> sum{};
   bool near = false;
   const Walk w = walk_of(L, p);
-  walk_within<QUAD>(
+  walk_within<LANES>(
       w.list, w.cnt, p, ld3(xs, p), K, xs, sum, near,
       [&](uint32_t q) { return VelocityDensity{gather4(vin, q), rho[q]}; },
       [&](f3, float d2, const VelocityDensity& q, Terms<3>& t) {
         const f3 s = div3_shared(mul3(sub3(xyz(q.v), vp), poly6_in(sqrt_cr(d2), K)), q.rho);
         t = Terms<3>{{s.x, s.y, s.z}};
       });
-  if (!pass_writes<QUAD>()) return;
+  if (!pass_writes<LANES>()) return;
   f3 nv = vp;
   acc3(nv, smul3(K.visc, f3{sum.a[0], sum.a[1], sum.a[2]}));
   st3(vout, p, nv);
@@ -323,25 +323,25 @@ void launch_viscosity(pbf_context* c, const float4* vin, float4* vout, uint64_t 
 }
 
 // compute_vorticity (particles.h:452-466): omega -> scr
-template <bool QUAD>
+template <int LANES>
 __global__ void __launch_bounds__(kBlock) k_vorticity(uint32_t n, uint32_t b, uint32_t e, KParams K,
                                                       const uint32_t* __restrict__ oid,
                                                       const float4* __restrict__ xs,
                                                       const float4* __restrict__ vin, float4* __restrict__ scr,
                                                       PassLists L) {
-  const uint32_t p = particle_of<QUAD>();
+  const uint32_t p = particle_of<LANES>();
   if (p >= n || !in_span(oid[p], b, e)) return;
   const f3 vp = ld3(vin, p);
   Terms<3> sum{};
   bool near = false;
   const Walk w = walk_of(L, p);
-  walk_within<QUAD>(
+  walk_within<LANES>(
       w.list, w.cnt, p, ld3(xs, p), K, xs, sum, near, [&](uint32_t q) { return gather4(vin, q); },
       [&](f3 d, float d2, float4 vq, Terms<3>& t) {
         const f3 s = cross3(sub3(xyz(vq), vp), spiky_in(d, sqrt_cr(d2), K));
         t = Terms<3>{{s.x, s.y, s.z}};
       });
-  if (pass_writes<QUAD>()) st3(scr, p, f3{sum.a[0], sum.a[1], sum.a[2]});
+  if (pass_writes<LANES>()) st3(scr, p, f3{sum.a[0], sum.a[1], sum.a[2]});
 }
 
 void launch_vorticity(pbf_context* c, const float4* vin, uint64_t b, uint64_t e) {
@@ -350,24 +350,24 @@ void launch_vorticity(pbf_context* c, const float4* vin, uint64_t b, uint64_t e)
 }
 
 // apply_vorticity (particles.h:471-487): reads |omega_q| of neighbours, own v
-template <bool QUAD>
+template <int LANES>
 __global__ void __launch_bounds__(kBlock) k_apply_vorticity(uint32_t n, uint32_t b, uint32_t e, KParams K,
                                                             const uint32_t* __restrict__ oid,
                                                             const float4* __restrict__ xs,
                                                             const float4* __restrict__ scr, float4* __restrict__ v,
                                                             PassLists L) {
-  const uint32_t p = particle_of<QUAD>();
+  const uint32_t p = particle_of<LANES>();
   if (p >= n || !in_span(oid[p], b, e)) return;
   Terms<3> sum{};
   bool near = false;
   const Walk w = walk_of(L, p);
-  walk_within<QUAD>(
+  walk_within<LANES>(
       w.list, w.cnt, p, ld3(xs, p), K, xs, sum, near, [&](uint32_t q) { return gather4(scr, q); },
       [&](f3 d, float d2, float4 wq, Terms<3>& t) {
         const f3 s = smul3(sqrt_cr(magsq3(xyz(wq))), spiky_in(d, sqrt_cr(d2), K));
         t = Terms<3>{{s.x, s.y, s.z}};
       });
-  if (!pass_writes<QUAD>()) return;
+  if (!pass_writes<LANES>()) return;
   const f3 eta = {sum.a[0], sum.a[1], sum.a[2]};
   const f3 N = div3(eta, sqrtf(magsq3(eta)) + K.r_eps);
   f3 vp = ld3(v, p);
@@ -381,23 +381,23 @@ void launch_apply_vorticity(pbf_context* c, float4* vio, uint64_t b, uint64_t e)
 }
 
 // apply_surface_tension (particles.h:400-431).  Pass 1: colour field -> scr.
-template <bool QUAD>
+template <int LANES>
 __global__ void __launch_bounds__(kBlock) k_color(uint32_t n, uint32_t b, uint32_t e, KParams K,
                                                   const uint32_t* __restrict__ oid, const float4* __restrict__ xs,
                                                   const float* __restrict__ rho, float4* __restrict__ scr,
                                                   PassLists L) {
-  const uint32_t p = particle_of<QUAD>();
+  const uint32_t p = particle_of<LANES>();
   if (p >= n || !in_span(oid[p], b, e)) return;
   Terms<3> sum{};
   bool near = false;
   const Walk w = walk_of(L, p);
-  walk_within<QUAD>(
+  walk_within<LANES>(
       w.list, w.cnt, p, ld3(xs, p), K, xs, sum, near, [&](uint32_t q) { return rho[q]; },
       [&](f3 d, float d2, float rq, Terms<3>& t) {
         const f3 s = div3_shared(spiky_in(d, sqrt_cr(d2), K), rq);
         t = Terms<3>{{s.x, s.y, s.z}};
       });
-  if (pass_writes<QUAD>()) st3(scr, p, smul3(K.h, f3{sum.a[0], sum.a[1], sum.a[2]}));
+  if (pass_writes<LANES>()) st3(scr, p, smul3(K.h, f3{sum.a[0], sum.a[1], sum.a[2]}));
 }
 
 // One pair's cohesion and curvature force (particles.h:415-426).  The
@@ -419,20 +419,20 @@ __device__ __forceinline__ f3 tension_term(f3 r, f3 sp, float4 sq, float rp, flo
 // Pass 2: cohesion + curvature force into own v.  The r > h shortcut does
 // not apply here: curvature (scratch_p - scratch_q) has no kernel factor, so
 // the walk takes every entry of the full list.
-template <bool QUAD>
+template <int LANES>
 __global__ void __launch_bounds__(kBlock) k_tension(uint32_t n, uint32_t b, uint32_t e, KParams K,
                                                     const uint32_t* __restrict__ oid, const float4* __restrict__ xs,
                                                     const float* __restrict__ rho, const float4* __restrict__ scr,
                                                     float4* __restrict__ v, const int32_t* __restrict__ nbr,
                                                     const int32_t* __restrict__ nbr_count) {
-  const uint32_t p = particle_of<QUAD>();
+  const uint32_t p = particle_of<LANES>();
   if (p >= n || !in_span(oid[p], b, e)) return;
   const f3 xp = ld3(xs, p);
   const f3 sp = ld3(scr, p);
   const float rp = rho[p];
   f3 f = {0.f, 0.f, 0.f};
   const int cnt = nbr_count[p];
-  if constexpr (QUAD) {
+  if constexpr (LANES != 1) {
     const uint32_t* __restrict__ row = quad_row(nbr, p, K.stride);
     const int u = (int)(threadIdx.x & 3u);
     for (int k0 = 0; k0 < cnt; k0 += kBatch) {

@@ -75,7 +75,7 @@ __device__ __forceinline__ void record_move(float m, unsigned long long* __restr
 // are mostly consecutive slots of one cell (about 15 distinct lines of 128
 // bytes a gather at rest, against 31 for 64 particles' k-th neighbours).  The
 // price is the ordered sums (a DPP addition takes twice a plain one's time),
-// so large scenes stay with single lanes (pressure_quads, tail_quads).
+// so large scenes stay with single lanes (pressure_lanes, tail_lanes).
 template <int CTRL>
 __device__ __forceinline__ float quad_lane(float t) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), CTRL, 0xF, 0xF, true));
@@ -109,11 +109,74 @@ __device__ __forceinline__ const uint32_t* quad_row(const int32_t* __restrict__ 
   return reinterpret_cast<const uint32_t*>(list) + list_at(0, p, stride) + (threadIdx.x & 3u);
 }
 
-template <bool QUAD>
+// L lanes share a particle: 1, 4 (a quad) or 16 (a row of the wavefront, whose
+// walks take one entry a lane at a time, summed with row broadcasts)
+template <int L>
 __device__ __forceinline__ uint32_t particle_of() {
-  const uint32_t t = xcd_block() * blockDim.x + threadIdx.x;
-  return QUAD ? t >> 2 : t;
+  return (xcd_block() * blockDim.x + threadIdx.x) / (uint32_t)L;
 }
+template <int L>
+__device__ __forceinline__ uint32_t lane_in_group() {
+  return threadIdx.x & (uint32_t)(L - 1);
+}
+template <int I>
+__device__ __forceinline__ float row_lane(float t) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), 0x150 + I, 0xF, 0xF, true));
+}
+template <int L, bool SUB>
+__device__ __forceinline__ void group_sum(float& a, float t) {
+  if constexpr (L == 4) {
+    SUB ? quad_sub(a, t) : quad_add(a, t);
+  } else {
+    static_assert(L == 16, "a row");
+#define PBF_ROW_STEP(I) a = SUB ? a - row_lane<I>(t) : a + row_lane<I>(t);
+    PBF_ROW_STEP(0) PBF_ROW_STEP(1) PBF_ROW_STEP(2) PBF_ROW_STEP(3) PBF_ROW_STEP(4) PBF_ROW_STEP(5)
+    PBF_ROW_STEP(6) PBF_ROW_STEP(7) PBF_ROW_STEP(8) PBF_ROW_STEP(9) PBF_ROW_STEP(10) PBF_ROW_STEP(11)
+    PBF_ROW_STEP(12) PBF_ROW_STEP(13) PBF_ROW_STEP(14) PBF_ROW_STEP(15)
+#undef PBF_ROW_STEP
+  }
+}
+template <int L>
+__device__ __forceinline__ void group_add3(f3& a, f3 t) {
+  group_sum<L, false>(a.x, t.x);
+  group_sum<L, false>(a.y, t.y);
+  group_sum<L, false>(a.z, t.z);
+}
+// the group's lanes of a ballot
+template <int L>
+__device__ __forceinline__ uint32_t group_bits(bool b) {
+  return (uint32_t)(__ballot(b) >> (threadIdx.x & 63u & ~(uint32_t)(L - 1))) & ((1u << L) - 1u);
+}
+// A group's way along a list, kEntries entries a step, kMine of them the
+// lane's own.  entries() gives the step's, those at or past `left` replaced by
+// `past` (PADDED: the list's last eight are whole, and `past` is the far row);
+// advance(), after the gathers, loads the next step's under them.
+template <int L>
+struct GroupRow {
+  static constexpr int kEntries = L == 4 ? 8 : 16, kMine = kEntries / L;
+  const uint32_t* __restrict__ row;
+  uint32_t q[kMine];
+  __device__ __forceinline__ GroupRow(const int32_t* __restrict__ list, uint32_t p, uint32_t stride)
+      : row(reinterpret_cast<const uint32_t*>(list) + list_at(lane_in_group<L>(), p, stride)) {
+    load();
+  }
+  template <bool PADDED>
+  __device__ __forceinline__ void entries(int left, uint32_t past, uint32_t (&out)[kMine]) const {
+#pragma unroll
+    for (int j = 0; j < kMine; ++j)
+      out[j] = (PADDED && L == 4) || (int)lane_in_group<L>() + j * L < left ? q[j] : past;
+  }
+  __device__ __forceinline__ void advance() {
+    row += kEntries * 64;
+    load();
+  }
+
+ private:
+  __device__ __forceinline__ void load() {
+#pragma unroll
+    for (int j = 0; j < kMine; ++j) q[j] = row[j * L * 64];
+  }
+};
 
 // Sums of N terms over the entries of a padded list within h of xp, in list
 // order.  data(q) loads what the terms need of neighbour q beyond its
@@ -124,11 +187,11 @@ template <int N>
 struct Terms {
   float a[N];
 };
-template <bool QUAD, int N, class Data, class Term>
+template <int L, int N, class Data, class Term>
 __device__ __forceinline__ void walk_within(const int32_t* __restrict__ list, int cnt, uint32_t p, f3 xp,
                                             const KParams& K, const float4* __restrict__ pos, Terms<N>& sum,
                                             bool& near, Data data, Term term) {
-  if constexpr (QUAD) {
+  if constexpr (L != 1) {
     const uint32_t* __restrict__ row = quad_row(list, p, K.stride);
     uint32_t q[2] = {row[0], row[256]};
     for (int k0 = 0; k0 < cnt; k0 += kBatch) {

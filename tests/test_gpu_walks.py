@@ -172,3 +172,22 @@ def test_density_fix_next_to_the_walls(pbf, scenes, counts, pairs):
     assert g.stats()["density_hacks"] > 0
     _same(g, o, f"{pairs} pairs, {len(pos)} particles")
     g.close()
+
+
+# at and past the sizes where sixteen lanes give way to four (12,288 particles
+# in the pressure solve, 24,576 after it), with lists that end inside a step of
+# sixteen, within its first eight and past the 64th entry
+@pytest.mark.parametrize("counts,squeeze,cap", [((1, 1, 1), 1.0, 60), ((5, 4, 3), 0.84, 128), ((9, 9, 9), 1.0, 17),
+                                                ((24, 16, 32), 0.84, 128), ((1, 12289, 1), 0.9, 60),
+                                                ((32, 24, 32), 0.9, 71), ((24, 32, 33), 1.0, 41)])
+def test_sixteen_lanes_equal_oracle(pbf, scenes, counts, squeeze, cap):
+    params, pos, vel = _scene(scenes, counts, squeeze, cap)
+    g = pbf.Particles(params)
+    g.add(pos, pos, vel)
+    o = O.Oracle(O.params_from_pbf(params), mode=O.JACOBI, threads=THREADS)
+    o.set_state(pos, pos, vel)
+    for k in range(3):  # (the later steps over skin lists, where no particle moves far)
+        g.step(1)
+        o.step(1)
+        _same(g, o, f"{counts}, squeeze {squeeze}, cap {cap}, step {k + 1}")
+    g.close()

@@ -20,7 +20,7 @@
 
 namespace pbf {
 
-constexpr int kMaxTrainWaves = 1024;
+constexpr int kMaxTrainBlocks = 1024;
 
 __device__ __forceinline__ v4s feature_operand(const float* __restrict__ f, bool valid, int g) {
   v4s xb = {0, 0, 0, 0};
@@ -51,126 +51,141 @@ __global__ void __launch_bounds__(64) k_mlp_forward(uint32_t n, const float* __r
 }
 
 // Gradient of the mean squared error over `count` samples idx[0..count) for
-// one batch.  Block b (one wavefront) handles sample groups b, b + grid, ...
-// and writes its partial gradient to part[b][kNPar] and its partial sum of
-// squared errors to lpart[b].
-__global__ void __launch_bounds__(64) k_mlp_train(uint32_t count, const uint32_t* __restrict__ idx,
-                                                  const float* __restrict__ feat, const float* __restrict__ tgt,
-                                                  MlpW W, float inv_batch, float* __restrict__ part,
-                                                  float* __restrict__ lpart) {
-  __shared__ __attribute__((aligned(16))) short sA[kHid * 16];  // [unit][particle]: dZ2, then dZ1
-  __shared__ __attribute__((aligned(16))) short sH[kHid * 16];  // [unit][particle]: H1
-  __shared__ __attribute__((aligned(16))) short sX[16 * 16];    // [particle][feature]
-  const int l = threadIdx.x, c = l & 15, g = l >> 4;
-  v4s a1[4], a2[4][4], a2t[4][4];
-  load_forward_operands(W, c, g, a1, a2);
+// one batch.  Block b handles sample groups b, b + grid, ... of 16 and writes
+// its partial gradient to part[b][kNPar] and its partial sum of squared errors
+// to lpart[b].
+//
+// Bound by the chain of one group: operands, two layers and their derivatives
+// with an exponential and a divide for every unit, then 19 KB of partials.  A
+// block is four wavefronts, each with one of the four tiles of 16 units of
+// either layer: a quarter of the operands, exponentials, MFMA and stores each.
+// They exchange the activations and derivatives as B operands, and the
+// outputs' products, which every wavefront adds up in the order of the units.
+// Measured at 4,096 samples (256 blocks), us: 15.4 with one wavefront a block,
+// 9.6 so.
+__global__ void __launch_bounds__(256) k_mlp_train(uint32_t count, const uint32_t* __restrict__ idx,
+                                                   const float* __restrict__ feat, const float* __restrict__ tgt,
+                                                   MlpW W, float inv_batch, float* __restrict__ part,
+                                                   float* __restrict__ lpart) {
+  __shared__ __attribute__((aligned(16))) short sA[kHid * 16];   // [unit][particle]: dZ2
+  __shared__ __attribute__((aligned(16))) short sA1[kHid * 16];  // [unit][particle]: dZ1
+  __shared__ __attribute__((aligned(16))) short sH[kHid * 16];   // [unit][particle]: H1
+  __shared__ __attribute__((aligned(16))) short sX[16 * 16];     // [particle][feature]
+  __shared__ v4s sB[4][64], sD[4][64];                           // B operands: H1, dZ2
+  __shared__ v4f sP[4][64];                                      // w3 * H2
+  const int l = threadIdx.x & 63, t = threadIdx.x >> 6, c = l & 15, g = l >> 4;
+  const int r0 = 16 * t + 4 * g;  // the lane's units: r0 .. r0 + 3
+  // (the first of two dependent loads of a group goes out before the operands')
+  auto sample_of = [&](uint32_t gi) { return gi * 16 + c < count ? idx[gi * 16 + c] : 0u; };
+  uint32_t next = sample_of(blockIdx.x);
+  const v4s a1 = *(const v4s*)(W.w1 + (16 * t + c) * 16 + 4 * g);
+  v4s a2[4], a2t[4];
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int k = 0; k < 4; ++k) a2t[t][k] = *(const v4s*)(W.w2t + (16 * t + c) * kHid + 16 * k + 4 * g);
-  v4f gW2[4][4], gW1[4];
-  float db1[4][4], db2[4][4], dw3[4][4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    gW1[t] = v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      gW2[t][k] = v4f{0.f, 0.f, 0.f, 0.f};
-      db1[t][k] = db2[t][k] = dw3[t][k] = 0.f;
-    }
+  for (int k = 0; k < 4; ++k) {
+    a2[k] = *(const v4s*)(W.w2 + (16 * t + c) * kHid + 16 * k + 4 * g);
+    a2t[k] = *(const v4s*)(W.w2t + (16 * t + c) * kHid + 16 * k + 4 * g);
   }
+  const v4f b1 = *(const v4f*)(W.p + OFF_B1 + r0), b2 = *(const v4f*)(W.p + OFF_B2 + r0),
+            w3 = *(const v4f*)(W.p + OFF_W3 + r0);
+  const float b3 = W.p[OFF_B3];
+  const v4f zero = {0.f, 0.f, 0.f, 0.f};
+  v4f gW2[4] = {zero, zero, zero, zero}, gW1 = zero, db1 = zero, db2 = zero, dw3 = zero;
   float db3 = 0.f, loss = 0.f;
   const uint32_t groups = (count + 15) / 16;
   for (uint32_t gi = blockIdx.x; gi < groups; gi += gridDim.x) {
-    const uint32_t s = gi * 16 + c;
-    const bool valid = s < count;
-    const uint32_t sample = valid ? idx[s] : 0u;
+    const bool valid = gi * 16 + c < count;
+    const uint32_t sample = next;
     const v4s xb = feature_operand(feat + (uint64_t)sample * kFeat, valid, g);
+    next = gi + gridDim.x < groups ? sample_of(gi + gridDim.x) : 0u;
+    const float target = valid ? tgt[sample] : 0.f;
+    if (t == 0) *(v4s*)(sX + c * 16 + 4 * g) = xb;
+    const v4f acc1 = mfma16(a1, xb, zero);
+    v4f z1, z2, h2;
+    v4s hb;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) sX[c * 16 + 4 * g + j] = xb[j];
-    v4f z1[4], h1[4], z2[4], h2[4];
-    const float out = mlp_forward(W, a1, a2, xb, g, z1, h1, z2, h2);
-    const float diff = valid ? out - tgt[sample] : 0.f;
+    for (int j = 0; j < 4; ++j) {
+      z1[j] = acc1[j] + b1[j];
+      hb[j] = f2bf(silu(z1[j]));
+      sH[(r0 + j) * 16 + c] = hb[j];
+    }
+    sB[t][l] = hb;
+    __syncthreads();
+    v4f acc2 = zero, prod;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc2 = mfma16(a2[k], sB[k][l], acc2);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      z2[j] = acc2[j] + b2[j];
+      h2[j] = silu(z2[j]);
+      prod[j] = w3[j] * h2[j];
+    }
+    sP[t][l] = prod;
+    __syncthreads();
+    float y = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const v4f q = sP[k][l];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y += q[j];
+    }
+    y += __shfl_xor(y, 16, 64);
+    y += __shfl_xor(y, 32, 64);
+    const float diff = valid ? (y + b3) - target : 0.f;
     const float dout = 2.0f * diff * inv_batch;
     if (g == 0) {
       loss += diff * diff;
       db3 += dout;
     }
-    v4f dz2[4];
+    v4s db;
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int r = 16 * t + 4 * g + j;
-        dw3[t][j] += dout * h2[t][j];
-        const float d = dout * W.p[OFF_W3 + r] * dsilu(z2[t][j]);
-        dz2[t][j] = d;
-        db2[t][j] += d;
-        sA[r * 16 + c] = f2bf(d);
-        sH[r * 16 + c] = f2bf(h1[t][j]);
-      }
+    for (int j = 0; j < 4; ++j) {
+      dw3[j] += dout * h2[j];
+      const float d = dout * w3[j] * dsilu(z2[j]);
+      db2[j] += d;
+      db[j] = f2bf(d);
+      sA[(r0 + j) * 16 + c] = db[j];
+    }
+    sD[t][l] = db;
     __syncthreads();
     // dW2 += dZ2 . H1^T (contraction over the 16 particles)
+    const v4s A2 = *(const v4s*)(sA + (16 * t + c) * 16 + 4 * g);
 #pragma unroll
-    for (int to = 0; to < 4; ++to) {
-      const v4s A = *(const v4s*)(sA + (16 * to + c) * 16 + 4 * g);
-#pragma unroll
-      for (int ti = 0; ti < 4; ++ti) {
-        const v4s B = *(const v4s*)(sH + (16 * ti + c) * 16 + 4 * g);
-        gW2[to][ti] = mfma16(A, B, gW2[to][ti]);
-      }
-    }
+    for (int ti = 0; ti < 4; ++ti)
+      gW2[ti] = mfma16(A2, *(const v4s*)(sH + (16 * ti + c) * 16 + 4 * g), gW2[ti]);
     // dH1 = W2^T . dZ2, dZ1 = dH1 * silu'(Z1)
-    v4f dz1[4];
+    v4f acc = zero;
 #pragma unroll
-    for (int ti = 0; ti < 4; ++ti) {
-      v4f acc = {0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < 4; ++k) acc = mfma16(a2t[k], sD[k][l], acc);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const v4s bz = {f2bf(dz2[k][0]), f2bf(dz2[k][1]), f2bf(dz2[k][2]), f2bf(dz2[k][3])};
-        acc = mfma16(a2t[ti][k], bz, acc);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        dz1[ti][j] = acc[j] * dsilu(z1[ti][j]);
-        db1[ti][j] += dz1[ti][j];
-      }
+    for (int j = 0; j < 4; ++j) {
+      const float d = acc[j] * dsilu(z1[j]);
+      db1[j] += d;
+      sA1[(r0 + j) * 16 + c] = f2bf(d);
     }
-    __syncthreads();
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) sA[(16 * t + 4 * g + j) * 16 + c] = f2bf(dz1[t][j]);
     __syncthreads();
     // dW1 += dZ1 . X^T
     const v4s B1 = {sX[(4 * g + 0) * 16 + c], sX[(4 * g + 1) * 16 + c], sX[(4 * g + 2) * 16 + c],
                     sX[(4 * g + 3) * 16 + c]};
-#pragma unroll
-    for (int to = 0; to < 4; ++to) {
-      const v4s A = *(const v4s*)(sA + (16 * to + c) * 16 + 4 * g);
-      gW1[to] = mfma16(A, B1, gW1[to]);
-    }
+    gW1 = mfma16(*(const v4s*)(sA1 + (16 * t + c) * 16 + 4 * g), B1, gW1);
     __syncthreads();
   }
   float* P = part + (uint64_t)blockIdx.x * kNPar;
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int j = 0; j < 4; ++j) {
+    const int r = r0 + j;
+    if (c < kFeat) P[OFF_W1 + r * kFeat + c] = gW1[j];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int r = 16 * t + 4 * g + j;
-      if (c < kFeat) P[OFF_W1 + r * kFeat + c] = gW1[t][j];
-#pragma unroll
-      for (int ti = 0; ti < 4; ++ti) P[OFF_W2 + r * kHid + 16 * ti + c] = gW2[t][ti][j];
-      const float b1s = red16(db1[t][j]), b2s = red16(db2[t][j]), w3s = red16(dw3[t][j]);
-      if (c == 0) {
-        P[OFF_B1 + r] = b1s;
-        P[OFF_B2 + r] = b2s;
-        P[OFF_W3 + r] = w3s;
-      }
+    for (int ti = 0; ti < 4; ++ti) P[OFF_W2 + r * kHid + 16 * ti + c] = gW2[ti][j];
+    const float b1s = red16(db1[j]), b2s = red16(db2[j]), w3s = red16(dw3[j]);
+    if (c == 0) {
+      P[OFF_B1 + r] = b1s;
+      P[OFF_B2 + r] = b2s;
+      P[OFF_W3 + r] = w3s;
     }
+  }
   db3 = red16(db3);
   loss = red16(loss);
-  if (l == 0) {
+  if (threadIdx.x == 0) {
     P[OFF_B3] = db3;
     lpart[blockIdx.x] = loss;
   }
@@ -218,7 +233,8 @@ __device__ __forceinline__ void refresh_operand(uint32_t i, float p, short* __re
 // Measured for a training epoch of 131,072 samples in batches of 4,096 (256
 // rows) with the gradient over all of them: 3.58 ms with one lane per
 // parameter reading row after row (72 us a batch, and 4.7 us each for Adam and
-// the operands in kernels of their own), 1.23 ms so.
+// the operands in kernels of their own), 1.23 ms so (1.01 with k_mlp_train's
+// four wavefronts a block).
 constexpr int kSumBlock = 512;
 constexpr uint32_t kRows = 128;
 template <bool TRAIN>
@@ -230,7 +246,7 @@ __global__ void __launch_bounds__(kSumBlock) k_mlp_finish(uint32_t nblk, const f
                                                           short* __restrict__ w2t) {
   constexpr int kWaves = kSumBlock / 64, kPer = kRows / kWaves;
   __shared__ float s_row[kRows][64];
-  __shared__ float s_loss[kMaxTrainWaves];
+  __shared__ float s_loss[kMaxTrainBlocks];
   const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const uint32_t i = blockIdx.x * 64 + lane;
   const uint32_t ic = min(i, (uint32_t)kNPar - 1u);
@@ -372,9 +388,9 @@ static AdamStep next_adam(pbf_warm_model* M, float learning_rate) {
 // its loss and the Adam update
 static void run_batch(pbf_warm_model* M, const uint32_t* idx, uint32_t count, float* loss_acc, const AdamStep* adam) {
   const uint32_t groups = (count + 15) / 16;
-  const uint32_t blocks = std::min<uint32_t>(groups, (uint32_t)kMaxTrainWaves);
+  const uint32_t blocks = std::min<uint32_t>(groups, (uint32_t)kMaxTrainBlocks);
   const float inv = 1.0f / (float)count;
-  hipLaunchKernelGGL(k_mlp_train, dim3(blocks), dim3(64), 0, M->stream, count, idx, (const float*)M->feat,
+  hipLaunchKernelGGL(k_mlp_train, dim3(blocks), dim3(256), 0, M->stream, count, idx, (const float*)M->feat,
                      (const float*)M->tgt, model_weights(M), inv, M->part, M->lpart);
   const dim3 grid((kNPar + 63) / 64);
   if (adam)
@@ -403,8 +419,8 @@ int pbf_warm_model_create(uint64_t max_samples, pbf_warm_model** out) {
       (rc = A((void**)&M->p, kNPar * 4)) || (rc = A((void**)&M->w1, kHid * 16 * 2)) ||
       (rc = A((void**)&M->w2, kHid * kHid * 2)) || (rc = A((void**)&M->w2t, kHid * kHid * 2)) ||
       (rc = A((void**)&M->m, kNPar * 4)) || (rc = A((void**)&M->v, kNPar * 4)) ||
-      (rc = A((void**)&M->grad, kNPar * 4)) || (rc = A((void**)&M->part, (uint64_t)kMaxTrainWaves * kNPar * 4)) ||
-      (rc = A((void**)&M->lpart, kMaxTrainWaves * 4)) || (rc = A((void**)&M->loss, 4)) ||
+      (rc = A((void**)&M->grad, kNPar * 4)) || (rc = A((void**)&M->part, (uint64_t)kMaxTrainBlocks * kNPar * 4)) ||
+      (rc = A((void**)&M->lpart, kMaxTrainBlocks * 4)) || (rc = A((void**)&M->loss, 4)) ||
       (rc = A((void**)&M->loss_acc, 4)) || (rc = A((void**)&M->feat, max_samples * kFeat * 4)) ||
       (rc = A((void**)&M->tgt, max_samples * 4)) || (rc = A((void**)&M->perm, max_samples * 4)) ||
       (rc = A((void**)&M->iota, max_samples * 4)) || (rc = A((void**)&M->pfeat, kPredictRows * kFeat * 4)) ||

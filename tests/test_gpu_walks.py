@@ -191,3 +191,30 @@ def test_sixteen_lanes_equal_oracle(pbf, scenes, counts, squeeze, cap):
         o.step(1)
         _same(g, o, f"{counts}, squeeze {squeeze}, cap {cap}, step {k + 1}")
     g.close()
+
+
+@pytest.mark.parametrize("counts", [(10, 9, 8), (50, 53, 50)])
+def test_tension_after_a_partial_color_pass(pbf, scenes, counts):
+    """Surface tension takes a neighbour's density from the color pass when
+    that ran over every particle in the same call, and from the densities
+    otherwise: the color field in two halves, the second with the forces, must
+    give what one call gives (four lanes and one lane a particle)."""
+    params, pos, vel = _scene(scenes, counts, 0.9, 60, gamma=0.5)
+    n = pos.shape[0]
+    out = []
+    for halves in (False, True):
+        g = pbf.Particles(params)
+        g.add(pos, pos, vel)
+        g.find_neighbors()
+        g.compute_densities()
+        g.set_scratch(np.full_like(pos, 7.0))  # (no color left from before)
+        if halves:
+            g.apply_surface_tension(pbf.span(0, n // 2), pbf.span(0, 0))
+            g.apply_surface_tension(pbf.span(n // 2, n), pbf.span(0, n))
+        else:
+            g.apply_surface_tension()
+        out.append((g.scratch(), g.velocities()))
+        g.close()
+    assert not np.array_equal(out[0][1], vel)
+    assert np.array_equal(out[0][0], out[1][0])
+    assert np.array_equal(out[0][1], out[1][1])

@@ -51,3 +51,17 @@ def test_crowded_scene_around_the_lane_limit(pbf, scenes, n, count_overflow):
     if count_overflow:
         assert g.stats()["neighbor_overflow"] == o.counters()["overflow"]
     g.close()
+
+
+@pytest.mark.parametrize("bits", [1, 7, 8, 9, 17, 24, 32])
+@pytest.mark.parametrize("n", [2, 63, 64, 65, 1023, 1024, 1025, 2049, 4095, 4096, 4097])
+def test_sort_around_one_block(pbf, n, bits):
+    """Up to 1,024 and 4,096 keys are sorted by one block, in LDS: stable, and
+    equal to the sort of numpy, with one to four passes."""
+    rng = np.random.default_rng(100 * n + bits)
+    keys = rng.integers(0, 1 << (min(bits, 6) if n % 2 else bits), size=n, dtype=np.uint64).astype(np.uint32)
+    vals = rng.permutation(n).astype(np.uint32)
+    k, v = pbf.sort_by_key_u32(keys, vals, bits)
+    order = np.argsort(keys, kind="stable")
+    assert np.array_equal(k, keys[order])
+    assert np.array_equal(v, vals[order])

@@ -60,11 +60,9 @@ ALG_BYTES = {
     "viscosity_positions": 12 + 12 + 4 + 12 + 12,
     "vorticity": 12 + 12 + 12,             # R x*, v; W omega
     "apply_vorticity": 12 + 12 + 12 + 12,  # R x*, omega, v; W v
-    "forces_predict": 12 + 12 + 12 + 12,   # R x, v; W v, x*
-    "bin": 12 + 4 + 4,
+    "predict_bin": 12 + 12 + 12 + 12 + 4 + 4,  # R x, v; W v, x*, key, slot
     "sort": 4 * 4,
     "reorder": 2 * (3 * 12 + 4 + 4 + 12 + 4 + 4),
-    "scan": 8,
     "lambda_repair": 0,
 }
 
@@ -182,19 +180,19 @@ def _profile_valu(kernel: str):
         return None
 
 
-KERNELS = ["forces_predict", "bin", "scan", "sort", "reorder", "cell_box", "fill_neighbors", "fill_heavy",
-           "density_lambda",
-           "mark_dirty", "lambda_repair", "dp_update", "viscosity", "vorticity", "apply_vorticity",
-           "viscosity_positions"]
+KERNELS = ["predict_bin", "sort", "reorder", "fill_neighbors", "cell_box", "fill_heavy", "density_lambda",
+           "lambda_repair", "dp_update", "viscosity", "vorticity", "apply_vorticity", "viscosity_positions"]
 
-# HIP kernel behind each timer (the names rocprofv3 reports)
+# HIP kernel behind each timer (the names rocprofv3 reports at the benchmark's
+# size, where one lane walks a particle's list)
 HIP_KERNEL = {
-    "forces_predict": "pbf::k_forces_predict", "bin": "pbf::k_bin", "reorder": "pbf::k_reorder",
-    "cell_box": "pbf::k_cell_box", "fill_neighbors": "pbf::k_fill_neighbors", "fill_heavy": "pbf::k_fill_heavy",
-    "density_lambda": "pbf::k_density_lambda_c<0, false, true>", "mark_dirty": "pbf::k_mark_dirty",
-    "lambda_repair": "pbf::k_lambda_repair<false>", "dp_update": "pbf::k_dp_update_c<false, true>",
-    "viscosity": "pbf::k_viscosity_first", "vorticity": "pbf::k_vorticity_c<true>",
-    "apply_vorticity": "pbf::k_apply_vorticity_c<true>", "viscosity_positions": "pbf::k_viscosity_last",
+    "predict_bin": "pbf::k_predict_bin", "reorder": "pbf::k_reorder",
+    "cell_box": "pbf::k_cell_box", "fill_neighbors": "pbf::k_fill_neighbors<false, 64u>",
+    "fill_heavy": "pbf::k_fill_heavy",
+    "density_lambda": "pbf::k_density_lambda_c<0, false, true, 1>",
+    "lambda_repair": "pbf::k_lambda_repair<false>", "dp_update": "pbf::k_dp_update_c<false, true, 1>",
+    "viscosity": "pbf::k_viscosity_first_lane", "vorticity": "pbf::k_vorticity_c<true, 1>",
+    "apply_vorticity": "pbf::k_apply_vorticity_c<true, 1>", "viscosity_positions": "pbf::k_viscosity_last<1>",
 }
 
 

@@ -109,7 +109,7 @@ typedef struct pbf_params {
  * one lane against the cell's particles in turn); the lists are the same, bit for bit.
  * This option keeps the per-lane walk for every particle (for comparison). */
 #define PBF_OPT_LANE_LISTS 64u
-/* pbf_step and pbf_solve run their Jacobi iterations (the density, dirty-marking,
+/* pbf_step and pbf_solve run their Jacobi iterations (the density,
  * lambda-repair and pressure-update passes of every iteration or solve slot) in one
  * cooperative launch with grid-wide barriers between the passes, instead of one launch per
  * pass; a solve stops on the device.  Same results, bit for bit.  Used for up to 256

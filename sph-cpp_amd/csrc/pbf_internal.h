@@ -6,7 +6,8 @@
 //                                density of the last density pass (gathered by the XSPH passes)
 //   xa, xsa, va      float4[n]   reorder targets, swapped with the above
 //   xt               float4[n]   position stars after the density pass (hack applied)
-//   scr              float4[n]   scratch vector: dp, vorticity or colour field
+//   scr              float4[n]   scratch vector: dp, vorticity or colour field (w: |omega|, or the
+//                                density beside the colour)
 //   rho, lam         float[n]
 //   oid, oida        uint32[n]   original index of each sorted slot
 //   key              uint32[n]   cell key of each slot
@@ -14,8 +15,7 @@
 //   sk[2], sv[2]     uint32[n]   radix-sort ping-pong buffers (cell key, slot)
 //   rhist, rsum      uint32      radix digit histograms of the tiles, and their sums over groups
 //   cell_start       uint32[C+2] first sorted slot of every cell (C = the outside bucket)
-//   heavy            uint32[n]   particles whose 27 cells hold too many candidates
-//                                for one lane (built by a whole wavefront instead)
+//   heavy            uint32[n]   particles that a whole wavefront lists (k_fill_heavy)
 //   nbr              int32[n/64][K/4][64][4] neighbour lists tiled by groups of 64 particles:
 //                                nbr[list_at(k, p, K)] (entries 4j .. 4j+3 of a particle are one
 //                                16-byte load, a wavefront's one contiguous kilobyte, its whole
@@ -27,7 +27,7 @@
 //                                from (xs0), in list order (same tiling and padding)
 //   far row          row `capacity` of the position stars (xs, xsa, xt) holds +inf: a padding
 //                                entry of a list reads it and lies outside every radius
-//   counters         u64[16]     overflow, outside, hacks, hack flags, solve state, ...
+//   counters         u64[C_NUM]  overflow, outside, hacks, hack flags, solve state, ...
 //   ehist, esum      uint32, u64[kMaxSolveSlots+1][kErrShards]  max (float bits) and sum of the
 //                                density errors per solve slot, in shards that their readers combine
 //   cstamp           uint32[C+1] == the iteration's stamp: a particle within two cells was moved
@@ -82,11 +82,11 @@ struct KParams {
   float skin2;                   // (1.1 h)^2: the radius of the skin lists
   float disp_lim2;               // (0.045 h)^2: squared moves below it keep the skin lists usable
   int skin_mode;                 // skin lists allowed (no PBF_OPT_FULL_LISTS)
-  int tile_lists;                // the cell-tile list walk (no PBF_OPT_LANE_LISTS)
+  int tile_lists;                // the cell walk builds the lists (no PBF_OPT_LANE_LISTS)
   int fast;                      // PBF_OPT_FAST_MATH: hardware sqrt and reciprocal in the fused step
   int static_ranges;             // the exact sums' range tests hold for every accepted pair (nb_sqrt, nb_spiky)
   uint32_t pad;                  // the far row (the capacity): what the lists are padded with
-  uint32_t heavy_budget;         // candidates one lane scans before a wavefront takes over (see walk_list)
+  uint32_t heavy_budget;         // candidates before a particle gets a wavefront of its own (crowded, walk_budget, walk_list)
   // batched scenes: ncells is the total over the scenes, sid the scene of each slot
   int batched;
   const SceneGeo* scenes;
@@ -108,7 +108,7 @@ enum Counter {
                     // end of the previous Jacobi iteration (parity of the iteration that reads it)
   C_SKIN = 16,      // 1: this step's skin lists are built
   C_DISP_ALL = 17,  // the same over the whole step so far
-  C_TILE = 18,      // particles listed by the cell-tile walk (counted with PBF_OPT_COUNT_OVERFLOW)
+  C_TILE = 18,      // particles listed by the cell walk (counted with PBF_OPT_COUNT_OVERFLOW)
   C_RETRY = 19,     // the warm start grew the error at slot 0 and its damped retry was applied
   C_NUM = 24
 };

@@ -1126,11 +1126,14 @@ __global__ void __launch_bounds__(kStageBlock) k_viscosity_first_lane(
 //   vorticity             8.8 / 13.1  15.9 / 17.8  25.8 / 27.1  111 / 96
 //   confinement           8.6 / 13.1  15.3 / 16.3  26.8 / 27.6  87 / 84
 //   second XSPH           9.1 / 15.0  15.3 / 17.1  26.0 / 27.4  86 / 83
-// (single lanes overtake between 65,536 and 131,072 particles in the pressure
-// solve, and near 524,288 in the passes after it)
-constexpr uint64_t kRowsPressure = 12288, kQuadsPressure = 98304;
+// (single lanes overtake between 65,536 and 131,072 particles in the density
+// pass, between 131,072, where the update takes 17.3 us by quads and 18.8 by
+// lanes, and 196,608, 23.2 and 22.4, in the pressure update, and near 524,288
+// in the passes after it)
+constexpr uint64_t kRowsPressure = 12288, kQuadsDensity = 98304, kQuadsUpdate = 147456;
 constexpr uint64_t kRowsTail = 24576, kQuadsTail = 524288;
-static int pressure_lanes(const pbf_context* c) { return c->n <= kRowsPressure ? 16 : (c->n <= kQuadsPressure ? 4 : 1); }
+static int density_lanes(const pbf_context* c) { return c->n <= kRowsPressure ? 16 : (c->n <= kQuadsDensity ? 4 : 1); }
+static int update_lanes(const pbf_context* c) { return c->n <= kRowsPressure ? 16 : (c->n <= kQuadsUpdate ? 4 : 1); }
 static int tail_lanes(const pbf_context* c) { return c->n <= kRowsTail ? 16 : (c->n <= kQuadsTail ? 4 : 1); }
 
 // `lanes` lanes per particle
@@ -1191,7 +1194,7 @@ void launch_density_lambda_masked(pbf_context* c, int it, int eslot, const Solve
   else if (F.feat)
     launch_density_fm<1, 1>(c, "density_features", it, eslot, S, F);
   else
-    switch (pressure_lanes(c)) {
+    switch (density_lanes(c)) {
       case 16: return launch_density_fm<0, 16>(c, "density_lambda", it, eslot, S, F);
       case 4: return launch_density_fm<0, 4>(c, "density_lambda", it, eslot, S, F);
       default: return launch_density_fm<0, 1>(c, "density_lambda", it, eslot, S, F);
@@ -1211,7 +1214,7 @@ void launch_lambda_repair(pbf_context* c, int it, const SolveCtl& S) {
       (const int32_t*)c->snb, (const int32_t*)c->snb_count, (const float4*)c->xs0, (const float*)c->rho
 template <bool FAST, bool SR>
 static void launch_dp_as(pbf_context* c, int it, int last, const SolveCtl& S) {
-  switch (pressure_lanes(c)) {
+  switch (update_lanes(c)) {
     case 16: PBF_LAUNCH_LANES(c, "dp_update", 16, (k_dp_update_c<FAST, SR, 16>), PBF_DP_ARGS); break;
     case 4: PBF_LAUNCH_LANES(c, "dp_update", 4, (k_dp_update_c<FAST, SR, 4>), PBF_DP_ARGS); break;
     default: PBF_LAUNCH_LANES(c, "dp_update", 1, (k_dp_update_c<FAST, SR, 1>), PBF_DP_ARGS);

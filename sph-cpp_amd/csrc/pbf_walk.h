@@ -75,7 +75,7 @@ __device__ __forceinline__ void record_move(float m, unsigned long long* __restr
 // are mostly consecutive slots of one cell (about 15 distinct lines of 128
 // bytes a gather at rest, against 31 for 64 particles' k-th neighbours).  The
 // price is the ordered sums (a DPP addition takes twice a plain one's time),
-// so large scenes stay with single lanes (pressure_lanes, tail_lanes).
+// so large scenes stay with single lanes (density_lanes, update_lanes, tail_lanes).
 template <int CTRL>
 __device__ __forceinline__ float quad_lane(float t) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), CTRL, 0xF, 0xF, true));

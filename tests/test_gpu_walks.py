@@ -218,3 +218,18 @@ def test_tension_after_a_partial_color_pass(pbf, scenes, counts):
     assert not np.array_equal(out[0][1], vel)
     assert np.array_equal(out[0][0], out[1][0])
     assert np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("counts,squeeze,cap", [((64, 48, 48), 0.84, 128), ((73, 45, 45), 0.9, 71)])
+def test_density_by_lanes_and_update_by_quads(pbf, scenes, counts, squeeze, cap):
+    """At 147,456 particles (and one row more) the density pass goes by single
+    lanes and the pressure update by quads (by single lanes)."""
+    params, pos, vel = _scene(scenes, counts, squeeze, cap)
+    g = pbf.Particles(params)
+    g.add(pos, pos, vel)
+    o = O.Oracle(O.params_from_pbf(params), mode=O.JACOBI, threads=THREADS)
+    o.set_state(pos, pos, vel)
+    g.step(1)
+    o.step(1)
+    _same(g, o, f"{counts}, squeeze {squeeze}, cap {cap}")
+    g.close()

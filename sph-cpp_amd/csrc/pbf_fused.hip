@@ -1121,7 +1121,7 @@ __global__ void __launch_bounds__(kStageBlock) k_viscosity_first_lane(
 // and 4 against 1:
 //   particles            32,768       131,072      262,144      1,048,576
 //   density              10.7 / 14.3  19.8 / 18.0  30.8 / 25.8  95 / 80
-//   pressure update       9.6 / 15.0  17.1 / 18.1  27.7 / 25.5  91 / 77
+//   pressure update       9.6 / 15.0  17.1 / 18.1  27.7 / 24.6  92 / 72
 //   first XSPH           11.5 / 18.0  22.5 / 26.8  36.6 / 44.5  188 / 164
 //   vorticity             8.8 / 13.1  15.9 / 17.8  25.8 / 27.1  111 / 96
 //   confinement           8.6 / 13.1  15.3 / 16.3  26.8 / 27.6  87 / 84

@@ -13,8 +13,9 @@
 //    12.6 MB    400 /  490  (410 /  790)
 //      50 MB   1340 / 1800 (1790 / 3000)
 // Bound: PCIe (12.6 MB alone take 228 us from pinned memory), the host's copy
-// next to it, and some 15 us a queued copy, which is why chunks are large.  (A kernel that copies instead of the copy engine was no faster: 35
-// / 34 and 430 / 520 us at 393 KB and 12.6 MB.)
+// next to it, and some 15 us a queued copy, which is why chunks are large.  (A
+// kernel that copies instead of the copy engine was no faster: 35 / 34 and
+// 430 / 520 us at 393 KB and 12.6 MB.)
 #include <algorithm>
 #include <cstring>
 #include <thread>

@@ -309,9 +309,9 @@ __device__ __forceinline__ void warm_network(const FeatCtl& F, uint32_t wave_fir
 // neighbors.h:177-179), which lie within two cells of the particle's own cell
 // on every axis, so every particle that can list q sits within two cells of
 // q's cell: the wavefront that moved q stamps those 5x5x5 cells, and
-// lambda_repair takes every particle of a stamped cell.  Past kMaxMovedMarked
-// moved particles it scans the lists for moved ones instead (there the stamped
-// cells would hold nearly everything).  (Stamping cells, two stores a lane,
+// lambda_repair looks through the lists of the particles in stamped cells for
+// moved ones.  Past kMaxMovedMarked moved particles it looks through all of
+// them (there the stamped cells would hold nearly everything).  (Stamping cells, two stores a lane,
 // needs no launch of its own; stamping their particles took one, 4.5 us an
 // iteration also when nothing had moved.)
 constexpr uint32_t kMaxMovedMarked = 4096;
@@ -438,8 +438,7 @@ k_density_lambda_c(uint32_t n, int it, int eslot, SolveCtl S, FeatCtl F,
 // compute_pressure_lambdas (particles.h:318-342) from xt for the dirty
 // particles of this iteration (plain walks).  The new lambda goes to lam and
 // to the particle's xt.w; positions are read as three words, so no lane reads
-// the w word that another lane writes.  Dirty are the particles of the stamped
-// cells, or with many moved particles exactly those that carry this
+// the w word that another lane writes.  Dirty are the particles that carry this
 // iteration's moved stamp or list one that does; they are stamped in dirty for
 // the dp pass.
 __device__ __forceinline__ f3 ld3_words(const float4* a, uint32_t i) {
@@ -447,38 +446,10 @@ __device__ __forceinline__ f3 ld3_words(const float4* a, uint32_t i) {
   return {f[0], f[1], f[2]};
 }
 
+// the sums of one particle, by one lane
 template <bool FAST>
-__device__ __forceinline__ void repair_pass(uint32_t vb, uint32_t n, int it, uint32_t stamp, const SolveCtl& S,
-                                            const KParams& K, float4* __restrict__ xt,
-                                            const float* __restrict__ rho, float* __restrict__ lam,
-                                            const int32_t* __restrict__ nbr,
-                                            const int32_t* __restrict__ nbr_count,
-                                            const uint32_t* __restrict__ mflag,
-                                            uint32_t* __restrict__ dirty, const uint32_t* __restrict__ key,
-                                            const uint32_t* __restrict__ cstamp,
-                                            const unsigned long long* __restrict__ counters) {
-  if (S.tol >= 0.0f && counters[C_DONE] != 0ull) return;
-  if (counters[C_HACK_FLAG + (it & 1)] == 0ull) return;
-  const bool scan = counters[C_MOVED_N + (it & 1)] > kMaxMovedMarked;
-  const uint32_t p = vb * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  const int cnt = nbr_count[p];
-  if (scan) {
-    bool hit = mflag[p] == stamp;
-    for (int k0 = 0; k0 < cnt && !hit; k0 += kBatch) {
-      uint32_t q[kBatch];
-      load_batch(nbr, K.stride, k0, cnt, p, q);
-#pragma unroll
-      for (int u = 0; u < kBatch; ++u) hit |= (k0 + u < cnt) & (mflag[q[u]] == stamp);
-    }
-    if (!hit) return;
-  } else if (cstamp[key[p]] != stamp) {
-    return;
-  }
-  dirty[p] = stamp;
-  const f3 xp = ld3_words(xt, p);
-  float sum_C = 0.0f;
-  f3 sg = {0.f, 0.f, 0.f};
+__device__ __forceinline__ void repair_walk(uint32_t p, f3 xp, const KParams& K, const float4* __restrict__ xt,
+                                            const int32_t* __restrict__ nbr, int cnt, f3& sg, float& sum_C) {
   for (int k0 = 0; k0 < cnt; k0 += kBatch) {
     uint32_t q[kBatch];
     load_batch(nbr, K.stride, k0, cnt, p, q);
@@ -496,12 +467,149 @@ __device__ __forceinline__ void repair_pass(uint32_t vb, uint32_t n, int it, uin
       sum_C += magsq3(grad);
     }
   }
-  sum_C += magsq3(sg);
-  const float constraint = rho[p] / K.rho0 - 1.0f;
-  const float C_p = ((double)constraint < 0.0) ? 0.0f : constraint;
-  const float lp = -C_p / (sum_C + K.eps);
-  lam[p] = lp;
-  reinterpret_cast<float*>(xt + p)[3] = lp;
+}
+
+// the same by L
+template <bool FAST, int L>
+__device__ __forceinline__ void repair_walk_group(uint32_t p, f3 xp, const KParams& K, const float4* __restrict__ xt,
+                                                  const int32_t* __restrict__ nbr, int cnt, f3& sg, float& sum_C) {
+  GroupRow<L> row(nbr, p, K.stride);
+  constexpr int kMine = GroupRow<L>::kMine;
+  for (int k0 = 0; k0 < cnt; k0 += GroupRow<L>::kEntries) {
+    uint32_t q[kMine];
+    f3 t[kMine];
+    row.template entries<false>(cnt - k0, p, q);
+#pragma unroll
+    for (int j = 0; j < kMine; ++j) t[j] = ld3_words(xt, q[j]);
+    row.advance();
+#pragma unroll
+    for (int j = 0; j < kMine; ++j) {
+      const f3 d = sub3(xp, t[j]);
+      const float d2 = magsq3(d);
+      float c2 = 0.0f;
+      f3 grad = {0.f, 0.f, 0.f};
+      if (k0 + (int)lane_in_group<L>() + L * j < cnt && within_h(d2, K)) {
+        const float r = nb_sqrt<FAST>(d2);
+        grad = smul3(K.neg_inv_rho0, nb_spiky<FAST>(d, r, K));
+        c2 = magsq3(grad);
+      }
+      group_sum<L, true>(sg.x, grad.x);
+      group_sum<L, true>(sg.y, grad.y);
+      group_sum<L, true>(sg.z, grad.z);
+      group_sum<L, false>(sum_C, c2);
+    }
+  }
+}
+
+// Whether an entry of p's list was moved (its stamp in mflag), 16 entries a step.
+__device__ __forceinline__ bool lists_moved(uint32_t p, uint32_t stamp, const KParams& K,
+                                            const int32_t* __restrict__ nbr, int cnt,
+                                            const uint32_t* __restrict__ mflag) {
+  bool hit = mflag[p] == stamp;
+  for (int k0 = 0; k0 < cnt && !hit; k0 += 2 * kBatch) {
+    uint32_t q[2][kBatch];
+    load_batch(nbr, K.stride, k0, cnt, p, q[0]);
+    if (k0 + kBatch < cnt) load_batch(nbr, K.stride, k0 + kBatch, cnt, p, q[1]);
+    else
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) q[1][u] = p;
+    uint32_t f[2][kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) f[0][u] = mflag[q[0][u]], f[1][u] = mflag[q[1][u]];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) hit |= (f[0][u] == stamp) | (f[1][u] == stamp);
+  }
+  return hit;
+}
+
+// The particles p of the block's threads with `take`, gathered in LDS; their
+// count.  Every thread of the block calls it.
+__device__ __forceinline__ uint32_t block_gather(bool take, uint32_t p, uint32_t* s_p, uint32_t* s_count) {
+  const uint32_t wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  const uint64_t m = __ballot(take);
+  if ((threadIdx.x & 63u) == 0u) s_count[wave] = (uint32_t)__popcll(m);
+  __syncthreads();
+  uint32_t before = 0, total = 0;
+  for (uint32_t w = 0; w < waves; ++w) {
+    const uint32_t k = s_count[w];
+    before += w < wave ? k : 0u;
+    total += k;
+  }
+  if (take)
+    s_p[before + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = p;
+  __syncthreads();
+  return total;
+}
+
+template <bool FAST, int L>
+__device__ __forceinline__ void repair_gathered(const uint32_t* s_p, uint32_t total, uint32_t stamp,
+                                                const KParams& K, float4* __restrict__ xt,
+                                                const float* __restrict__ rho, float* __restrict__ lam,
+                                                const int32_t* __restrict__ nbr,
+                                                const int32_t* __restrict__ nbr_count,
+                                                uint32_t* __restrict__ dirty) {
+  for (uint32_t i = threadIdx.x / (uint32_t)L; i < total; i += blockDim.x / (uint32_t)L) {
+    const uint32_t p = s_p[i];
+    const f3 xp = ld3_words(xt, p);
+    const int cnt = nbr_count[p];
+    float sum_C = 0.0f;
+    f3 sg = {0.f, 0.f, 0.f};
+    if constexpr (L == 1)
+      repair_walk<FAST>(p, xp, K, xt, nbr, cnt, sg, sum_C);
+    else
+      repair_walk_group<FAST, L>(p, xp, K, xt, nbr, cnt, sg, sum_C);
+    if (L != 1 && lane_in_group<L>() != 0u) continue;
+    sum_C += magsq3(sg);
+    const float constraint = rho[p] / K.rho0 - 1.0f;
+    const float C_p = ((double)constraint < 0.0) ? 0.0f : constraint;
+    const float lp = -C_p / (sum_C + K.eps);
+    dirty[p] = stamp;
+    lam[p] = lp;
+    reinterpret_cast<float*>(xt + p)[3] = lp;
+  }
+}
+
+// Every thread of the block calls it.  A block gathers its candidates in LDS,
+// tests their lists and gathers the dirty ones, so that the walks fill their
+// wavefronts.  With few moved particles the launch takes as long as one walk,
+// so up to kQuadRepairs dirty particles in a block go four lanes a particle
+// (sixteen lanes for the fewest were no faster).  Measured on the million
+// particles of a dam break, us a launch timed with events (some 7 above the
+// kernel's own time): 26.5 with 16 moved particles, 76 with 1,000 and 110 with
+// 130,000 when every particle of a stamped cell was redone where it stood by
+// one lane; 20, 57 and 105 so.  (Limits of 64 and 256 instead of 128, before
+// the candidates were tested: 26.4 and 21.4 with 16 moved particles, 21.2 with
+// 128, and 77.7 and 115 with 1,000, 77.6 with 128.)
+constexpr uint32_t kQuadRepairs = 128;
+template <bool FAST>
+__device__ __forceinline__ void repair_pass(uint32_t vb, uint32_t n, int it, uint32_t stamp, const SolveCtl& S,
+                                            const KParams& K, float4* __restrict__ xt,
+                                            const float* __restrict__ rho, float* __restrict__ lam,
+                                            const int32_t* __restrict__ nbr,
+                                            const int32_t* __restrict__ nbr_count,
+                                            const uint32_t* __restrict__ mflag,
+                                            uint32_t* __restrict__ dirty, const uint32_t* __restrict__ key,
+                                            const uint32_t* __restrict__ cstamp,
+                                            const unsigned long long* __restrict__ counters) {
+  if (S.tol >= 0.0f && counters[C_DONE] != 0ull) return;
+  if (counters[C_HACK_FLAG + (it & 1)] == 0ull) return;
+  const bool scan = counters[C_MOVED_N + (it & 1)] > kMaxMovedMarked;
+  const uint32_t p0 = vb * blockDim.x + threadIdx.x;
+  __shared__ uint32_t s_dirty[kBlock], s_count[kBlock / 64];
+  uint32_t p = p0;
+  uint32_t total = block_gather(p0 < n && (scan || cstamp[key[p0]] == stamp), p0, s_dirty, s_count);
+  bool hit = threadIdx.x < total;
+  if (hit) {
+    p = s_dirty[threadIdx.x];
+    hit = lists_moved(p, stamp, K, nbr, nbr_count[p], mflag);
+  }
+  __syncthreads();
+  total = block_gather(hit, p, s_dirty, s_count);
+  if (total <= kQuadRepairs)
+    repair_gathered<FAST, 4>(s_dirty, total, stamp, K, xt, rho, lam, nbr, nbr_count, dirty);
+  else
+    repair_gathered<FAST, 1>(s_dirty, total, stamp, K, xt, rho, lam, nbr, nbr_count, dirty);
+  __syncthreads();  // a block of the persistent kernel uses the rows again
 }
 
 template <bool FAST>

@@ -301,8 +301,8 @@ def summarize(d: str, workload: str, out_dir: str = "") -> None:
     os.makedirs(prof, exist_ok=True)
     lines, per = _kernel_table(
         os.path.join(d, "trace", "c2_kernel_trace.csv"), workload, PROFILE_COMMANDS["trace"],
-        "then `python3 bench.py --summarize /tmp/pbf_prof`.  The command is the benchmark's timed run as the\n"
-        "driver runs it (`--steps 20 --warmup 5`) without the CPU baseline, the variants and the warm-start\n"
+        "then `python3 bench.py --summarize /tmp/pbf_prof`.  The command is the benchmark's timed run\n"
+        "(`--steps 20 --warmup 5`) without the CPU baseline, the variants and the warm-start\n"
         "comparison: a warm-up context advanced 10 substeps, the autotuner on it, a profiled replay, then the\n"
         "timed run of substeps 1-20 of the 1,048,576-particle dam break from the initial scene (neighbour cap\n"
         "60).  The table covers the timed run only (the launches after its particle upload); the benchmark's\n"

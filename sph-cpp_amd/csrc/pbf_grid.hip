@@ -572,10 +572,12 @@ __host__ __device__ __forceinline__ uint32_t lane_budget(const KParams& K) {
 }
 
 // The lane walk of particle p: writes its list and count and returns true,
-// or returns false when the particle goes to the wavefront builder.  ovf
-// receives the candidates dropped by the cap.
+// or returns false when the particle goes to the wavefront builder (only with
+// hand_on; without it there are at most kMaxCellOffset particles, so every
+// offset fits).  ovf receives the candidates dropped by the cap.
 template <bool SKIN>
-__device__ __forceinline__ bool walk_list(uint32_t p, uint32_t n, uint32_t lane, uint16_t* __restrict__ s_list,
+__device__ __forceinline__ bool walk_list(uint32_t p, uint32_t n, bool hand_on, uint32_t lane,
+                                          uint16_t* __restrict__ s_list,
                                           const float4* __restrict__ xs, const uint32_t* __restrict__ start,
                                           const KParams& K, int32_t* __restrict__ nbr,
                                           int32_t* __restrict__ nbr_count, uint32_t& ovf,
@@ -602,13 +604,13 @@ __device__ __forceinline__ bool walk_list(uint32_t p, uint32_t n, uint32_t lane,
   // in 10 bits (a batch of 8 may pass the budget before the test)
   const uint32_t hb = lane_budget(K);
   // every candidate must be seen to count the overflow: route by the total
-  if (K.count_overflow && total > hb) return false;
+  if (hand_on && K.count_overflow && total > hb) return false;
   // otherwise the walk ends when the list is full; a lane whose 27 cells hold
   // more than twice K.heavy_budget candidates and that has scanned
   // K.heavy_budget of them without filling its list hands the particle over
   // (the wavefront builder starts again and writes the same entries); lanes
   // with fewer candidates walk them all
-  const uint32_t budget = total > min(2u * hb, kMaxCellOffset) ? hb : 0xFFFFFFFFu;
+  const uint32_t budget = hand_on && total > min(2u * hb, kMaxCellOffset) ? hb : 0xFFFFFFFFu;
   uint32_t scanned = 0;
   int count = 0;
   const int cap = K.cap;
@@ -808,8 +810,8 @@ __device__ __forceinline__ void cell_walk(uint32_t tb, uint32_t lane, uint64_t t
                                           const float4* __restrict__ xs, const uint32_t* __restrict__ start,
                                           const KParams& K, int32_t* __restrict__ nbr,
                                           int32_t* __restrict__ nbr_count, int32_t* __restrict__ snb,
-                                          int32_t* __restrict__ snb_count, bool skin, Lds& S, uint64_t& heavy,
-                                          uint32_t& ovf) {
+                                          int32_t* __restrict__ snb_count, bool skin, bool hand_on, Lds& S,
+                                          uint64_t& heavy, uint32_t& ovf) {
   constexpr uint32_t kPitch = Lds::kPitch, kNear = Lds::kNear;
   f3 mid;
   uint64_t even;
@@ -854,7 +856,7 @@ __device__ __forceinline__ void cell_walk(uint32_t tb, uint32_t lane, uint64_t t
     }
     const uint32_t incl = sum_scan32(cm), off = incl - cm;
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 26);
-    const uint32_t budget = walk_budget(K, total);
+    const uint32_t budget = hand_on ? walk_budget(K, total) : 0xFFFFFFFFu;
     if (budget == 0u) {
       heavy |= members;
       continue;
@@ -1018,6 +1020,7 @@ __device__ __forceinline__ void count_fill(uint64_t hm, uint32_t p, uint32_t ovf
 
 struct FillArgs {
   uint32_t n, fb, fe, width;
+  int hand_on;  // k_fill_heavy follows and takes what the walks hand on
   const float4* xs;
   const uint32_t *oid, *key, *start;
   uint32_t* box;
@@ -1059,16 +1062,16 @@ __global__ void __launch_bounds__(kFillBlock, LANES ? 1 : (CAP <= 64 ? 6 : 5)) k
     uint16_t* s_list = reinterpret_cast<uint16_t*>(s_mem);  // [cap + 1][kFillBlock]
     bool to_heavy = false;
     if (query)
-      to_heavy = skin ? !walk_list<true>(p, A.n, lane, s_list, A.xs, A.start, K, A.nbr, A.nbr_count, ovf, A.snb, A.snb_count)
-                      : !walk_list<false>(p, A.n, lane, s_list, A.xs, A.start, K, A.nbr, A.nbr_count, ovf, A.snb, A.snb_count);
+      to_heavy = skin ? !walk_list<true>(p, A.n, A.hand_on != 0, lane, s_list, A.xs, A.start, K, A.nbr, A.nbr_count, ovf, A.snb, A.snb_count)
+                      : !walk_list<false>(p, A.n, A.hand_on != 0, lane, s_list, A.xs, A.start, K, A.nbr, A.nbr_count, ovf, A.snb, A.snb_count);
     hm = __ballot(to_heavy);
   } else {
     __shared__ __attribute__((aligned(16))) CellWalkLds<CAP> S;
     const uint64_t todo = __builtin_amdgcn_ballot_w64(query);
     uint32_t key = A.key[p];
     if (K.batched && key == K.ncells) key += K.sid[p];  // (outside every cell, but in its own scene's grid)
-    cell_walk(tb, lane, todo, xyz3(ps4), key, A.xs, A.start, K, A.nbr, A.nbr_count, A.snb, A.snb_count, skin != 0, S, hm,
-              ovf);
+    cell_walk(tb, lane, todo, xyz3(ps4), key, A.xs, A.start, K, A.nbr, A.nbr_count, A.snb, A.snb_count, skin != 0,
+              A.hand_on != 0, S, hm, ovf);
     // all listed here (but for those handed on): an atomic a wavefront took 0.5 ms at 8 million particles
     if (K.count_overflow && blockIdx.x == 0 && lane == 0)
       atomicAdd(&A.counters[C_TILE], (unsigned long long)(min(A.fe, A.n) - min(A.fb, A.n)));
@@ -1206,7 +1209,17 @@ void launch_fill_neighbors(pbf_context* c, uint64_t fb, uint64_t fe) {
   KernelTimer* t = timer_begin(c, "fill_neighbors");
   const bool lanes = !c->K.tile_lists;
   const uint32_t width = lanes ? (uint32_t)kFillBlock : fill_width(n);
-  const FillArgs A{n, (uint32_t)fb, (uint32_t)fe, width, c->xs, c->oid, c->key, c->cell_start, c->cbox,
+  // A small scene does without the wavefront builder (two launches, about 9 us
+  // of a step of 960 particles): its walks hand no particle on, whatever its
+  // candidates come to.  They come to more than n where walk cells repeat: x +
+  // i*s can round into the cell of x + (i-1)*s (at x = 2.4 with s = 0.12 the
+  // walk's x cells are 20, 20 and 21), up to twice an axis.
+  const bool wide = c->K.batched || (c->K.dimx >= 3 && c->K.dimy >= 3 && c->K.dimz >= 3);
+  const uint32_t hb = lane_budget(c->K);
+  const uint32_t most = !lanes ? crowded(c->K)
+                               : (c->K.count_overflow ? hb : std::min(2u * hb, kMaxCellOffset));
+  const bool hand_on = !wide || n > most;
+  const FillArgs A{n, (uint32_t)fb, (uint32_t)fe, width, hand_on ? 1 : 0, c->xs, c->oid, c->key, c->cell_start, c->cbox,
                    boxes_in_fill(c) ? 6ull * c->K.ncells : 0ull, c->nbr, c->nbr_count, c->snb, c->snb_count, c->heavy,
                    c->counters, skin, c->skin_hint, c->xs0};
   const dim3 grid(nblocks(n, (int)width)), block(kFillBlock);
@@ -1218,14 +1231,7 @@ void launch_fill_neighbors(pbf_context* c, uint64_t fb, uint64_t fe) {
     hipLaunchKernelGGL((c->K.cap <= 64 ? k_fill_neighbors<false, 64> : k_fill_neighbors<false, 128>), grid, block, 0,
                        c->stream, A, c->K);
   timer_end(c, t);
-  // no particle of a small scene has enough candidates for the wavefront
-  // builder: every particle is a candidate at most once (a grid of at least
-  // three cells an axis gives 27 different cells)
-  const bool wide = c->K.batched || (c->K.dimx >= 3 && c->K.dimy >= 3 && c->K.dimz >= 3);
-  const uint32_t hb = lane_budget(c->K);
-  const uint32_t most = !lanes ? crowded(c->K)
-                               : (c->K.count_overflow ? hb : std::min(2u * hb, kMaxCellOffset));
-  if (wide && n <= most) return;
+  if (!hand_on) return;
   // the cell and chunk boxes of the wavefront builder, built only when some particle went to it
   launch_cell_box(c);
   // enough waves to cover the chip; each loops over the heavy list (usually empty)

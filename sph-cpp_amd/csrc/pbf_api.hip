@@ -356,23 +356,31 @@ static int build_scene_geo(const pbf_params& params, const float* boxes, uint32_
 
 using namespace pbf;
 
-// a caller's array to c->stage or the like; a device pointer is copied as one
+// a caller's array to c->stage or the like; what the copy engine reaches is
+// copied as it is
 static int upload(pbf_context* c, void* dev, const void* host, uint64_t bytes) {
-  if (!on_device(host)) return c->host.upload(dev, host, bytes, c->stream);
+  if (memory_of(host) == Memory::kPageable) return c->host.upload(dev, host, bytes, c->stream);
   return check_hip(hipMemcpyAsync(dev, host, bytes, hipMemcpyDefault, c->stream), "upload");
 }
 // and back; waits for the stream
 static int download(pbf_context* c, void* host, const void* dev, uint64_t bytes) {
-  if (!on_device(host)) return c->host.download(host, dev, bytes, c->stream);
+  if (memory_of(host) == Memory::kPageable) return c->host.download(host, dev, bytes, c->stream);
   int rc = check_hip(hipMemcpyAsync(host, dev, bytes, hipMemcpyDefault, c->stream), "download");
   return rc ? rc : check_hip(hipStreamSynchronize(c->stream), "download");
 }
 
 // Short arrays skip the device staging: the kernel that puts them in order
-// reads or writes the pinned memory, which saves the copy's launch.
+// reads or writes the pinned memory, which saves the copy's launch.  (From
+// memory that is pinned already the copy is quicker, and is overtaken sooner:
+// 65 KB of scalars read / set so take 28 / 25 us, copied 22 / 21.)
+static bool in_place(const void* p, uint64_t bytes) {
+  if (bytes > HostStage::kDirect) return false;
+  const Memory m = memory_of(p);
+  return m == Memory::kPageable || (m == Memory::kPinned && bytes <= HostStage::kDirect / 2);
+}
 template <class Order>
 static int get_array(pbf_context* c, float* out, uint64_t bytes, Order order) {
-  if (bytes > HostStage::kDirect || on_device(out)) {
+  if (!in_place(out, bytes)) {
     order(c->stage);
     return download(c, out, c->stage, bytes);
   }
@@ -383,7 +391,7 @@ static int get_array(pbf_context* c, float* out, uint64_t bytes, Order order) {
 }
 template <class Order>
 static int set_array(pbf_context* c, const float* in, uint64_t bytes, Order order) {
-  if (bytes > HostStage::kDirect || on_device(in)) {
+  if (!in_place(in, bytes)) {
     if (int rc = upload(c, c->stage, in, bytes)) return rc;
     order(c->stage);
   } else {

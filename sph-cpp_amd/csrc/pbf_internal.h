@@ -196,8 +196,12 @@ struct HostStage {
   hipError_t in_parts(uint64_t bytes, Part part);
 };
 
-// whether p is device memory (callers may pass it where an array is expected)
-bool on_device(const void* p);
+// What a caller's array lies in: ordinary memory, which copies go through the
+// staging memory for, host memory that the runtime has pinned, or memory of
+// the device (which callers may pass where an array is expected; managed
+// memory counts as such).
+enum class Memory { kPageable, kPinned, kDevice };
+Memory memory_of(const void* p);
 
 struct KernelTimer {
   std::string name;

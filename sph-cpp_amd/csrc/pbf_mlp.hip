@@ -360,11 +360,11 @@ namespace pbf {
 constexpr uint64_t kPredictRows = 32768;
 
 static int upload(pbf_warm_model* M, void* dev, const void* host, uint64_t bytes) {
-  if (!on_device(host)) return M->host.upload(dev, host, bytes, M->stream);
+  if (memory_of(host) == Memory::kPageable) return M->host.upload(dev, host, bytes, M->stream);
   return check_hip(hipMemcpyAsync(dev, host, bytes, hipMemcpyDefault, M->stream), "upload");
 }
 static int download(pbf_warm_model* M, void* host, const void* dev, uint64_t bytes) {
-  if (!on_device(host)) return M->host.download(host, dev, bytes, M->stream);
+  if (memory_of(host) == Memory::kPageable) return M->host.download(host, dev, bytes, M->stream);
   int rc = check_hip(hipMemcpyAsync(host, dev, bytes, hipMemcpyDefault, M->stream), "download");
   return rc ? rc : check_hip(hipStreamSynchronize(M->stream), "download");
 }

@@ -16,6 +16,10 @@
 // next to it, and some 15 us a queued copy, which is why chunks are large.  (A
 // kernel that copies instead of the copy engine was no faster: 35 / 34 and
 // 430 / 520 us at 393 KB and 12.6 MB.)
+//
+// Memory that the caller has pinned takes no part in this: the copy engine
+// reads and writes it as it is, 257 / 266 us for 12.6 MB against 346 / 515
+// through the staging memory.
 #include <algorithm>
 #include <cstring>
 #include <thread>
@@ -24,13 +28,17 @@
 
 namespace pbf {
 
-bool on_device(const void* p) {
+Memory memory_of(const void* p) {
   hipPointerAttribute_t a{};
   if (hipPointerGetAttributes(&a, p) != hipSuccess) {
     (void)hipGetLastError();
-    return false;
+    return Memory::kPageable;
   }
-  return a.type == hipMemoryTypeDevice;
+  switch (a.type) {
+    case hipMemoryTypeUnregistered: return Memory::kPageable;
+    case hipMemoryTypeHost: return Memory::kPinned;
+    default: return Memory::kDevice;
+  }
 }
 
 int HostStage::create(uint64_t most) {

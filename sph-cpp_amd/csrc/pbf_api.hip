@@ -1436,9 +1436,12 @@ int pbf_grid_dims(const pbf_context* c, uint64_t dims[3]) {
 uint64_t pbf_num_cells(const pbf_context* c) { return c ? c->ncells : 0; }
 
 static int download_u32(pbf_context* c, const uint32_t* src, uint64_t count, std::vector<uint32_t>& out) {
+  // (straight into the vector, which the callers convert: through the staging
+  // memory 16,000 to 65,000 words took 3 us more)
   out.resize(count);
   if (!count) return PBF_OK;
-  return download(c, out.data(), src, count * 4);
+  int rc = check_hip(hipMemcpyAsync(out.data(), src, count * 4, hipMemcpyDeviceToHost, c->stream), "download");
+  return rc ? rc : check_hip(hipStreamSynchronize(c->stream), "download");
 }
 
 int pbf_get_bin_ids(pbf_context* c, uint64_t* out) {

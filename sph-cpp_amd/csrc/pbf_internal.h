@@ -179,9 +179,14 @@ struct HostStage {
   uint64_t slot_bytes = 0;
   uint32_t nslots = 0;
   hipEvent_t done[kSlots] = {};
-  int create(uint64_t most);  // most: bytes of the largest transfer
+  // most: bytes of the transfers that it is made for (much larger ones go
+  // through it where it has all its slots, and are the runtime's otherwise)
+  int create(uint64_t most, uint64_t slot = kSlot);
   void destroy();
-  // queues the copy on s; host may be reused when it returns
+  bool fits(uint64_t bytes) const {
+    return nslots == kSlots || bytes <= (nslots > 1 ? 2 : 1) * nslots * slot_bytes;
+  }
+  // queues the copy on s; a caller reuses host when it has waited for s
   int upload(void* dev, const void* host, uint64_t bytes, hipStream_t s);
   // waits for s and the copy
   int download(void* host, const void* dev, uint64_t bytes, hipStream_t s);

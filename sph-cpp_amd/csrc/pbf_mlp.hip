@@ -355,9 +355,14 @@ struct pbf_warm_model {
 
 namespace pbf {
 
-// Rows of one launch of predict: the workspace of a model, so that a call
-// allocates nothing (two allocations and their release took about 150 us)
+// Rows that predict has a workspace for, so that a call of as many allocates
+// nothing (two allocations and their release are 10 of 32 us for 100 rows).
+// Calls of more rows allocate theirs and take all rows in one upload, launch
+// and download: in blocks of this many with a wait between each, 131,072 and
+// 1,000,000 rows took 320 and 2,800 us against 240 and 1,450 so.
 constexpr uint64_t kPredictRows = 32768;
+// Two slots of staging memory: above 2 MB the runtime's copies are as fast.
+constexpr uint64_t kStageSlot = 512u << 10, kStageBytes = 2 * kStageSlot;
 
 static int upload(pbf_warm_model* M, void* dev, const void* host, uint64_t bytes) {
   if (memory_of(host) == Memory::kPageable) return M->host.upload(dev, host, bytes, M->stream);
@@ -424,7 +429,7 @@ int pbf_warm_model_create(uint64_t max_samples, pbf_warm_model** out) {
       (rc = A((void**)&M->loss_acc, 4)) || (rc = A((void**)&M->feat, max_samples * kFeat * 4)) ||
       (rc = A((void**)&M->tgt, max_samples * 4)) || (rc = A((void**)&M->perm, max_samples * 4)) ||
       (rc = A((void**)&M->iota, max_samples * 4)) || (rc = A((void**)&M->pfeat, kPredictRows * kFeat * 4)) ||
-      (rc = A((void**)&M->pout, kPredictRows * 4)) || (rc = M->host.create(kPredictRows * kFeat * 4))) {
+      (rc = A((void**)&M->pout, kPredictRows * 4)) || (rc = M->host.create(kStageBytes, kStageSlot))) {
     pbf_warm_model_destroy(M);
     return rc;
   }
@@ -559,10 +564,13 @@ int pbf_warm_model_train(pbf_warm_model* M, uint32_t epochs, uint32_t batch, flo
   if (M->count == 0) return set_error(PBF_ERR_STATE, "no samples");
   if (batch == 0) return set_error(PBF_ERR_ARG, "batch must be positive");
   std::mt19937_64 rng(seed);
-  std::vector<uint32_t> perm(M->count);
+  std::vector<uint32_t> perms[2];
   uint64_t batches = 0;
   launch_fill_u32((uint32_t*)M->loss_acc, 0u, 1, M->stream);
   for (uint32_t e = 0; e < epochs; ++e) {
+    // (drawn while the last epoch's may still be read, unless it was staged)
+    std::vector<uint32_t>& perm = perms[M->host.fits(M->count * 4) ? 0u : e & 1u];
+    perm.resize(M->count);
     for (uint64_t i = 0; i < M->count; ++i) perm[i] = (uint32_t)i;
     std::shuffle(perm.begin(), perm.end(), rng);
     // the permutation buffer is rewritten only after the previous epoch's batches ran
@@ -577,7 +585,7 @@ int pbf_warm_model_train(pbf_warm_model* M, uint32_t epochs, uint32_t batch, flo
     }
   }
   float acc = 0.f;
-  if (int rc = download(M, &acc, M->loss_acc, 4)) return rc;
+  if (int rc = download(M, &acc, M->loss_acc, 4)) return rc;  // (waits for everything)
   if (mean_loss) *mean_loss = batches ? acc / (float)batches : 0.f;
   return PBF_OK;
 }
@@ -588,15 +596,27 @@ int pbf_warm_model_predict(pbf_warm_model* M, const float* features, uint64_t co
   if (!M->has_params) return set_error(PBF_ERR_STATE, "model has no parameters");
   if (!count) return PBF_OK;
   if (count >= (1ull << 32)) return set_error(PBF_ERR_ARG, "count out of range");
-  for (uint64_t first = 0; first < count; first += kPredictRows) {
-    const uint64_t rows = std::min<uint64_t>(kPredictRows, count - first);
-    if (int rc = upload(M, M->pfeat, features + first * kFeat, rows * kFeat * 4)) return rc;
+  float *f = M->pfeat, *o = M->pout, *own = nullptr;
+  uint64_t most = kPredictRows;
+  if (count > kPredictRows) {
+    if (hipMallocAsync((void**)&own, count * (kFeat + 1) * 4, M->stream) == hipSuccess) {
+      f = own, o = own + count * kFeat, most = count;
+    } else {  // (no room: block by block)
+      (void)hipGetLastError();
+      own = nullptr;
+    }
+  }
+  int rc = PBF_OK;
+  for (uint64_t first = 0; !rc && first < count; first += most) {
+    const uint64_t rows = std::min<uint64_t>(most, count - first);
+    if ((rc = upload(M, f, features + first * kFeat, rows * kFeat * 4))) break;
     const uint32_t groups = (uint32_t)((rows + 15) / 16);
     hipLaunchKernelGGL(k_mlp_forward, dim3(std::min<uint32_t>(groups, 4096u)), dim3(64), 0, M->stream, (uint32_t)rows,
-                       (const float*)M->pfeat, model_weights(M), 1.0f, nullptr, M->pout);
-    if (int rc = download(M, out + first, M->pout, rows * 4)) return rc;
+                       (const float*)f, model_weights(M), 1.0f, nullptr, o);
+    rc = download(M, out + first, o, rows * 4);
   }
-  return PBF_OK;
+  if (own) (void)hipFreeAsync(own, M->stream);
+  return rc;
 }
 
 int pbf_set_warm_gain(pbf_context* c, float gain) {

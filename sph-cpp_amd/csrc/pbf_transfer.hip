@@ -41,8 +41,8 @@ Memory memory_of(const void* p) {
   }
 }
 
-int HostStage::create(uint64_t most) {
-  slot_bytes = std::min<uint64_t>(kSlot, (most + 255) / 256 * 256);
+int HostStage::create(uint64_t most, uint64_t slot) {
+  slot_bytes = std::min<uint64_t>(slot, (most + 255) / 256 * 256);
   const uint64_t slots = std::min<uint64_t>(kSlots, (most + slot_bytes - 1) / slot_bytes);
   int rc = check_hip(hipGetDevice(&device), "hipGetDevice");
   if (!rc) rc = check_hip(hipHostMalloc((void**)&pin, slots * slot_bytes), "hipHostMalloc");
@@ -139,7 +139,13 @@ hipError_t HostStage::in_parts(uint64_t bytes, Part part) {
   return hipSuccess;
 }
 
+// What a small object's few slots do not hold (many samples of a warm-start
+// model) would go through them chunk by chunk with a wait for each: 4 MB of
+// samples took 360 us through one slot of 1 MB, 160 by the runtime.  (One more
+// round of two slots is no slower than the runtime's copies of 1 to 2 MB,
+// which sometimes take 450 us.)
 int HostStage::upload(void* dev, const void* host, uint64_t bytes, hipStream_t s) {
+  if (!fits(bytes)) return check_hip(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s), "upload");
   return check_hip(in_parts(bytes, [&](uint64_t at, uint64_t len, uint64_t chunk, uint32_t first, uint32_t count) {
                      return upload_part((unsigned char*)dev + at, (const unsigned char*)host + at, len, chunk, first,
                                         count, s);
@@ -147,6 +153,10 @@ int HostStage::upload(void* dev, const void* host, uint64_t bytes, hipStream_t s
 }
 
 int HostStage::download(void* host, const void* dev, uint64_t bytes, hipStream_t s) {
+  if (!fits(bytes)) {
+    const int rc = check_hip(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s), "download");
+    return rc ? rc : check_hip(hipStreamSynchronize(s), "download");
+  }
   return check_hip(in_parts(bytes, [&](uint64_t at, uint64_t len, uint64_t chunk, uint32_t first, uint32_t count) {
                      return download_part((unsigned char*)host + at, (const unsigned char*)dev + at, len, chunk, first,
                                           count, s);

@@ -1491,7 +1491,18 @@ int pbf_get_neighbor_lists(pbf_context* c, uint64_t* out, int32_t* counts) {
     const uint64_t op = o[p];
     const int32_t cp = (int32_t)cnt[p];
     counts[op] = cp;
-    for (int32_t k = 0; k < cp; ++k) out[op * K + k] = o[lists[list_at((uint32_t)k, (uint32_t)p, c->K.stride)]];
+    // four entries together, the next four a kilobyte on: a line of each serves
+    // four particles, and is asked for sixteen particles ahead
+    const uint32_t* q = lists.data() + list_at(0, (uint32_t)p, c->K.stride);
+    if (p % 4 == 0)
+      for (int32_t j = 0; j < cp; j += 4) __builtin_prefetch(q + 64 * j + 64);
+    uint64_t* to = out + op * K;
+    int32_t k = 0;
+    for (; k + 4 <= cp; k += 4, q += 256, to += 4) {
+      const uint64_t e[4] = {o[q[0]], o[q[1]], o[q[2]], o[q[3]]};
+      to[0] = e[0], to[1] = e[1], to[2] = e[2], to[3] = e[3];
+    }
+    for (int32_t j = 0; k + j < cp; ++j) to[j] = o[q[j]];
   }
   return PBF_OK;
 }

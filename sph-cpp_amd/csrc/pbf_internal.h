@@ -169,7 +169,8 @@ inline uint64_t list_size(uint64_t capacity, uint64_t stride) { return ((capacit
 
 // Pinned memory of one object (a context, a warm-start model) that its copies
 // from and to ordinary memory go through (pbf_transfer.hip).  One transfer at
-// a time: the caller synchronizes the stream before the next one.
+// a time: the caller synchronizes the stream before the next one (but see
+// upload).
 struct HostStage {
   static constexpr uint32_t kSlots = 8;
   static constexpr uint64_t kSlot = 2u << 20;    // bytes of a slot: 16 MB in all at most
@@ -186,8 +187,12 @@ struct HostStage {
   bool fits(uint64_t bytes) const {
     return nslots == kSlots || bytes <= (nslots > 1 ? 2 : 1) * nslots * slot_bytes;
   }
-  // queues the copy on s; a caller reuses host when it has waited for s
-  int upload(void* dev, const void* host, uint64_t bytes, hipStream_t s);
+  // whether the host's threads share a transfer
+  bool threaded(uint64_t bytes) const { return nslots == kSlots && bytes >= kTwo; }
+  // queues the copy on s; a caller reuses host when it has waited for s.  The
+  // first chunk goes through slot `slot`: of two transfers with no wait
+  // between them the second begins past the first one's.
+  int upload(void* dev, const void* host, uint64_t bytes, hipStream_t s, uint32_t slot = 0);
   // waits for s and the copy
   int download(void* host, const void* dev, uint64_t bytes, hipStream_t s);
 

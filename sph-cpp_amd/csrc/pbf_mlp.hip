@@ -346,7 +346,6 @@ struct pbf_warm_model {
   float *part = nullptr, *lpart = nullptr, *loss = nullptr, *loss_acc = nullptr;
   float *feat = nullptr, *tgt = nullptr;
   uint32_t *perm = nullptr, *iota = nullptr;
-  float *pfeat = nullptr, *pout = nullptr;  // predict's rows, up to kPredictRows
   pbf::HostStage host;
   uint64_t count = 0, max_samples = 0;
   uint64_t adam_t = 0;
@@ -355,17 +354,19 @@ struct pbf_warm_model {
 
 namespace pbf {
 
-// Rows that predict has a workspace for, so that a call of as many allocates
-// nothing (two allocations and their release are 10 of 32 us for 100 rows).
+// Rows that predict has a workspace for (the training batches' partials, which
+// nothing holds between calls), so that a call of as many allocates nothing
+// (two allocations and their release are 10 of 32 us for 100 rows).
 // Calls of more rows allocate theirs and take all rows in one upload, launch
-// and download: in blocks of this many with a wait between each, 131,072 and
-// 1,000,000 rows took 320 and 2,800 us against 240 and 1,450 so.
-constexpr uint64_t kPredictRows = 32768;
-// Two slots of staging memory: above 2 MB the runtime's copies are as fast.
+// and download: in blocks of 32,768 with a wait between each, 131,072 and
+// 1,000,000 rows took 320 and 2,800 us against 215 and 1,380 so.
+constexpr uint64_t kPredictRows = 524288;
+static_assert(kPredictRows * (kFeat + 1) <= (uint64_t)kMaxTrainBlocks * kNPar, "predict's rows in the partials");
+// two slots of staging memory
 constexpr uint64_t kStageSlot = 512u << 10, kStageBytes = 2 * kStageSlot;
 
-static int upload(pbf_warm_model* M, void* dev, const void* host, uint64_t bytes) {
-  if (memory_of(host) == Memory::kPageable) return M->host.upload(dev, host, bytes, M->stream);
+static int upload(pbf_warm_model* M, void* dev, const void* host, uint64_t bytes, uint32_t slot = 0) {
+  if (memory_of(host) == Memory::kPageable) return M->host.upload(dev, host, bytes, M->stream, slot);
   return check_hip(hipMemcpyAsync(dev, host, bytes, hipMemcpyDefault, M->stream), "upload");
 }
 static int download(pbf_warm_model* M, void* host, const void* dev, uint64_t bytes) {
@@ -428,8 +429,7 @@ int pbf_warm_model_create(uint64_t max_samples, pbf_warm_model** out) {
       (rc = A((void**)&M->lpart, kMaxTrainBlocks * 4)) || (rc = A((void**)&M->loss, 4)) ||
       (rc = A((void**)&M->loss_acc, 4)) || (rc = A((void**)&M->feat, max_samples * kFeat * 4)) ||
       (rc = A((void**)&M->tgt, max_samples * 4)) || (rc = A((void**)&M->perm, max_samples * 4)) ||
-      (rc = A((void**)&M->iota, max_samples * 4)) || (rc = A((void**)&M->pfeat, kPredictRows * kFeat * 4)) ||
-      (rc = A((void**)&M->pout, kPredictRows * 4)) || (rc = M->host.create(kStageBytes, kStageSlot))) {
+      (rc = A((void**)&M->iota, max_samples * 4)) || (rc = M->host.create(kStageBytes, kStageSlot))) {
     pbf_warm_model_destroy(M);
     return rc;
   }
@@ -447,7 +447,7 @@ int pbf_warm_model_destroy(pbf_warm_model* M) {
   if (!M) return PBF_OK;
   if (M->stream) hipStreamSynchronize(M->stream);
   void* ptrs[] = {M->p, M->w1, M->w2, M->w2t, M->m, M->v, M->grad, M->part, M->lpart, M->loss, M->loss_acc,
-                  M->feat, M->tgt, M->perm, M->iota, M->pfeat, M->pout};
+                  M->feat, M->tgt, M->perm, M->iota};
   for (void* q : ptrs)
     if (q) hipFree(q);
   M->host.destroy();
@@ -498,9 +498,21 @@ int pbf_warm_model_clear_samples(pbf_warm_model* M) {
 int pbf_warm_model_add_samples(pbf_warm_model* M, const float* features, const float* targets, uint64_t count) {
   if (!M || (count && (!features || !targets))) return set_error(PBF_ERR_ARG, "null argument");
   if (M->count + count > M->max_samples) return set_error(PBF_ERR_CAPACITY, "sample store is full");
-  int rc = upload(M, M->feat + M->count * kFeat, features, count * kFeat * 4);
-  if (rc || (rc = check_hip(hipStreamSynchronize(M->stream), "upload"))) return rc;  // (one staging memory)
-  if ((rc = upload(M, M->tgt + M->count, targets, count * 4))) return rc;
+  float *f = M->feat + M->count * kFeat, *t = M->tgt + M->count;
+  const uint64_t bytes = count * kFeat * 4;
+  int rc;
+  if (bytes > kStageBytes) {  // (the runtime's copies need no wait in between)
+    if ((rc = check_hip(hipMemcpyAsync(f, features, bytes, hipMemcpyDefault, M->stream), "upload")) ||
+        (rc = check_hip(hipMemcpyAsync(t, targets, count * 4, hipMemcpyDefault, M->stream), "upload")))
+      return rc;
+  } else {
+    // the targets go through the second slot where the features take no more
+    // than the first: 1 to 100 samples 21 us, 30 with a wait in between
+    const bool apart = bytes <= kStageSlot;
+    if ((rc = upload(M, f, features, bytes))) return rc;
+    if (!apart && (rc = check_hip(hipStreamSynchronize(M->stream), "upload"))) return rc;
+    if ((rc = upload(M, t, targets, count * 4, apart ? 1 : 0))) return rc;
+  }
   if ((rc = check_hip(hipStreamSynchronize(M->stream), "upload"))) return rc;
   M->count += count;
   return PBF_OK;
@@ -596,7 +608,7 @@ int pbf_warm_model_predict(pbf_warm_model* M, const float* features, uint64_t co
   if (!M->has_params) return set_error(PBF_ERR_STATE, "model has no parameters");
   if (!count) return PBF_OK;
   if (count >= (1ull << 32)) return set_error(PBF_ERR_ARG, "count out of range");
-  float *f = M->pfeat, *o = M->pout, *own = nullptr;
+  float *f = M->part, *o = M->part + kPredictRows * kFeat, *own = nullptr;
   uint64_t most = kPredictRows;
   if (count > kPredictRows) {
     if (hipMallocAsync((void**)&own, count * (kFeat + 1) * 4, M->stream) == hipSuccess) {

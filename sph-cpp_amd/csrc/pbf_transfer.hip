@@ -112,7 +112,7 @@ hipError_t HostStage::download_part(unsigned char* host, const unsigned char* de
 // it, about as long as the device takes), through their own slots.
 template <class Part>
 hipError_t HostStage::in_parts(uint64_t bytes, Part part) {
-  const uint32_t parts = nslots < kSlots || bytes < kTwo ? 1u : (bytes < kFour ? 2u : 4u);
+  const uint32_t parts = !threaded(bytes) ? 1u : (bytes < kFour ? 2u : 4u);
   const uint64_t share = (bytes / parts + 255) / 256 * 256;
   const uint32_t count = nslots / parts;
   const uint64_t chunk = slot_bytes;
@@ -141,10 +141,13 @@ hipError_t HostStage::in_parts(uint64_t bytes, Part part) {
 
 // What a small object's few slots do not hold (many samples of a warm-start
 // model) would go through them chunk by chunk with a wait for each: 4 MB of
-// samples took 360 us through one slot of 1 MB, 160 by the runtime.  (One more
-// round of two slots is no slower than the runtime's copies of 1 to 2 MB,
-// which sometimes take 450 us.)
-int HostStage::upload(void* dev, const void* host, uint64_t bytes, hipStream_t s) {
+// samples took 360 us through one slot of 1 MB, 160 by the runtime.  (A second
+// round of two slots is about as fast as the runtime's copies of 1 to 2 MB,
+// which take 400 us where the caller makes and gives back an array a call.)
+int HostStage::upload(void* dev, const void* host, uint64_t bytes, hipStream_t s, uint32_t slot) {
+  if (slot)
+    return check_hip(upload_part((unsigned char*)dev, (const unsigned char*)host, bytes, slot_bytes, slot, nslots - slot, s),
+                     "upload");
   if (!fits(bytes)) return check_hip(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s), "upload");
   return check_hip(in_parts(bytes, [&](uint64_t at, uint64_t len, uint64_t chunk, uint32_t first, uint32_t count) {
                      return upload_part((unsigned char*)dev + at, (const unsigned char*)host + at, len, chunk, first,

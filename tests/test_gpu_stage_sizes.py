@@ -46,7 +46,7 @@ def test_samples_arrive(pbf, count):
     one.close()
 
 
-@pytest.mark.parametrize("count", [32768, 32769, 65537, 262144, 500001])
+@pytest.mark.parametrize("count", [32768, 65537, 524288, 524289, 600001])
 def test_predict_past_the_workspace(pbf, count):
     """Every row equals its prediction in calls of 1,000 rows."""
     m = pbf.WarmModel(8)

@@ -42,7 +42,10 @@ Memory memory_of(const void* p) {
 }
 
 int HostStage::create(uint64_t most, uint64_t slot) {
-  slot_bytes = std::min<uint64_t>(slot, (most + 255) / 256 * 256);
+  // (two slots from 1 MB on, so that the host's copy of one chunk goes next to
+  // the device's of the other: 1.6 MB up take 84 us in one piece)
+  const bool halves = most > kSlot / 2 && most <= slot;
+  slot_bytes = std::min<uint64_t>(slot, ((halves ? (most + 1) / 2 : most) + 255) / 256 * 256);
   const uint64_t slots = std::min<uint64_t>(kSlots, (most + slot_bytes - 1) / slot_bytes);
   int rc = check_hip(hipGetDevice(&device), "hipGetDevice");
   if (!rc) rc = check_hip(hipHostMalloc((void**)&pin, slots * slot_bytes), "hipHostMalloc");

@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstring>
 #include <limits>
+#include <numeric>
 #include <string>
 #include <vector>
 
@@ -768,7 +769,7 @@ int pbf_find_neighbors(pbf_context* c, pbf_index_span bin_span, pbf_index_span f
   PBF_CHECK_CTX_SPAN(c, fill_span);
   if (bin_span.begin != 0)
     return set_error(PBF_ERR_ARG, "bin span must start at 0: sort_bins sorts [0, count) (neighbors.h:130-132)");
-  launch_fill_u64(c->counters, 0ull, 3, c->stream);  // overflow, outside, hacks
+  launch_fill_u64(c->counters, 0ull, C_CLEARED, c->stream);  // overflow, outside, hacks
   find_neighbors_impl(c, bin_span.end, fill_span.begin, fill_span.end);
   c->pass_skin = c->K.skin_mode != 0;
   return check_hip(hipGetLastError(), "find_neighbors");
@@ -1369,13 +1370,14 @@ int pbf_autotune_layout(pbf_context* c, uint32_t steps, pbf_layout* best) {
     launch_fill_u64(c->counters, 0ull, C_NUM, c->stream);
     launch_forces_predict(c, F_FORCES | F_PREDICT, 0, c->n);
     find_neighbors_impl(c, c->n, 0, c->n);
-    unsigned long long over = 0;
+    unsigned long long over[kOverflowShards];
     uint32_t longest = 0;
-    if ((rc = check_hip(hipMemcpyAsync(&over, c->counters + C_OVERFLOW, sizeof(over), hipMemcpyDeviceToHost,
+    if ((rc = check_hip(hipMemcpyAsync(over, c->counters + C_OVERFLOW, sizeof(over), hipMemcpyDeviceToHost,
                                        c->stream), "autotune")) ||
         (rc = max_list_length(c, &longest)))
       break;
-    if (over != 0) continue;  // this spacing needs a longer list than the context holds
+    if (std::any_of(over, over + kOverflowShards, [](unsigned long long k) { return k != 0; }))
+      continue;  // this spacing needs a longer list than the context holds
     // room for 25% longer lists than the state's longest, in rows of 8
     uint32_t cap = (uint32_t)std::ceil(1.25 * (double)longest);
     cap = std::min<uint32_t>((cap + 7u) / 8u * 8u, (uint32_t)c->cap_alloc);
@@ -1422,10 +1424,10 @@ int pbf_get_stats(pbf_context* c, pbf_stats* out) {
   std::vector<float> rho(c->n);
   if (c->n && (rc = download(c, rho.data(), c->rho, c->n * 4))) return rc;
   if ((rc = check_hip(hipStreamSynchronize(c->stream), "stats"))) return rc;
-  out->neighbor_overflow = h[C_OVERFLOW];
+  out->neighbor_overflow = std::accumulate(h + C_OVERFLOW, h + C_OVERFLOW + kOverflowShards, 0ull);
   out->outside_grid = h[C_OUTSIDE];
   out->density_hacks = h[C_HACKS];
-  out->tile_listed = h[C_TILE];
+  out->tile_listed = h[C_TILE] ? h[C_TILE] - h[C_HEAVY] : 0;
   out->persistent_grid = c->coop_grid;
   out->persistent_capacity = (c->P.options & PBF_OPT_PERSISTENT) ? persistent_capacity(c) : 0;
   out->iterations = c->last_was_solve ? h[C_ITERS] : c->last_iterations;

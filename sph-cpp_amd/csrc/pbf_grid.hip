@@ -189,6 +189,7 @@ __global__ void __launch_bounds__(kBlock) k_predict_bin(uint32_t n, KParams K, c
     I.ehist[i] = 0u;
     I.esum[i] = 0ull;
   }
+  static_assert(C_NUM <= kBlock, "cleared by the first block");
   if (p < (uint32_t)C_NUM) B.counters[p] = p == C_ITERS ? I.iterations : (p == C_WARM_KEPT ? I.warm : 0ull);
   if (p >= n) return;
   const uint32_t o = oid[p];
@@ -1000,7 +1001,7 @@ __device__ __forceinline__ void cell_walk(uint32_t tb, uint32_t lane, uint64_t t
 // Hand-offs and overflow counts go to the shared counters once per
 // wavefront (a same-address atomic per lane serialises in L2 when many
 // particles of a collapsed region hand off together).
-__device__ __forceinline__ void count_fill(uint64_t hm, uint32_t p, uint32_t ovf, bool listed, uint32_t lane,
+__device__ __forceinline__ void count_fill(uint64_t hm, uint32_t p, uint32_t ovf, uint32_t lane,
                                            const KParams& K, uint32_t* __restrict__ heavy,
                                            unsigned long long* __restrict__ counters) {
   if (hm != 0ull) {
@@ -1008,13 +1009,12 @@ __device__ __forceinline__ void count_fill(uint64_t hm, uint32_t p, uint32_t ovf
     if (lane == 0) base = atomicAdd(&counters[C_HEAVY], (unsigned long long)__popcll(hm));
     base = __shfl(base, 0, 64);
     if ((hm >> lane) & 1ull) heavy[base + (unsigned long long)__popcll(hm & ((1ull << lane) - 1ull))] = p;
-    if (listed && K.count_overflow && lane == 0) atomicAdd(&counters[C_TILE], 0ull - (unsigned long long)__popcll(hm));
   }
   if (K.count_overflow) {
     unsigned long long ov = ovf;
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) ov += __shfl_xor(ov, d, 64);
-    if (lane == 0 && ov) atomicAdd(&counters[C_OVERFLOW], ov);
+    if (lane == 0 && ov) atomicAdd(&counters[C_OVERFLOW + blockIdx.x % kOverflowShards], ov);
   }
 }
 
@@ -1072,11 +1072,11 @@ __global__ void __launch_bounds__(kFillBlock, LANES ? 1 : (CAP <= 64 ? 6 : 5)) k
     if (K.batched && key == K.ncells) key += K.sid[p];  // (outside every cell, but in its own scene's grid)
     cell_walk(tb, lane, todo, xyz3(ps4), key, A.xs, A.start, K, A.nbr, A.nbr_count, A.snb, A.snb_count, skin != 0,
               A.hand_on != 0, S, hm, ovf);
-    // all listed here (but for those handed on): an atomic a wavefront took 0.5 ms at 8 million particles
+    // (once for all: an atomic a wavefront took 0.5 ms at 8 million particles)
     if (K.count_overflow && blockIdx.x == 0 && lane == 0)
       atomicAdd(&A.counters[C_TILE], (unsigned long long)(min(A.fe, A.n) - min(A.fb, A.n)));
   }
-  count_fill(hm, p, ovf, !LANES, lane, K, A.heavy, A.counters);
+  count_fill(hm, p, ovf, lane, K, A.heavy, A.counters);
 }
 
 // A group of 64 candidates of the wavefront builder, one per lane (valid:
@@ -1192,7 +1192,8 @@ __global__ void __launch_bounds__(kBlock) k_fill_heavy(uint32_t n, const float4*
     if (lane == 0) {
       nbr_count[p] = (int32_t)kept;
       if (skin) snb_count[p] = (int32_t)scount;
-      if (count > cap && K.count_overflow) atomicAdd(&counters[C_OVERFLOW], (unsigned long long)(count - cap));
+      if (count > cap && K.count_overflow)
+        atomicAdd(&counters[C_OVERFLOW + h % kOverflowShards], (unsigned long long)(count - cap));
     }
   }
 }

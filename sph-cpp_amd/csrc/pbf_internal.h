@@ -93,24 +93,32 @@ struct KParams {
   const uint32_t* sid;
 };
 
+// The candidates that the cap drops are counted by atomics of every wavefront
+// that drops some: on one address they queue up in the cache (500,000
+// particles in clumps of 200: 410 us for the list build, 31,250 of them, and
+// 150 without the count), so they are spread over this many, which the host
+// adds up.
+constexpr uint32_t kOverflowShards = 64;
 enum Counter {
-  C_OVERFLOW = 0,
-  C_OUTSIDE = 1,
-  C_HACKS = 2,
-  C_HACK_FLAG = 3,  // two flags (3, 4) used on alternate Jacobi iterations
-  C_HEAVY = 5,      // number of entries in the heavy list
-  C_EMAX = 6,       // float bits of the max density error (atomicMax on non-negative floats)
-  C_MOVED_N = 7,    // two counts (7, 8): particles moved by the density fix, per iteration parity
-  C_DONE = 11,      // iterate-to-tolerance: 0, or the slot whose error fell below the tolerance plus one
-  C_ITERS = 12,     // iterate-to-tolerance: slots used
-  C_WARM_KEPT = 13, // the warm-start positions were kept (2: the damped retry's, PBF_OPT_WARM_RETRY)
-  C_DISP = 14,      // two flags (14, 15): some particle has moved too far for the skin lists by the
-                    // end of the previous Jacobi iteration (parity of the iteration that reads it)
-  C_SKIN = 16,      // 1: this step's skin lists are built
-  C_DISP_ALL = 17,  // the same over the whole step so far
-  C_TILE = 18,      // particles listed by the cell walk (counted with PBF_OPT_COUNT_OVERFLOW)
-  C_RETRY = 19,     // the warm start grew the error at slot 0 and its damped retry was applied
-  C_NUM = 24
+  C_OVERFLOW = 0,   // kOverflowShards counts
+  C_FIRST = kOverflowShards,
+  C_OUTSIDE = C_FIRST,
+  C_HACKS,
+  C_CLEARED,        // pbf_find_neighbors clears the counters before this one
+  C_HACK_FLAG = C_CLEARED,     // two flags used on alternate Jacobi iterations
+  C_HEAVY = C_HACK_FLAG + 2,   // number of entries in the heavy list
+  C_MOVED_N,                   // two counts: particles moved by the density fix, per iteration parity
+  C_DONE = C_MOVED_N + 2,      // iterate-to-tolerance: 0, or the slot whose error fell below the tolerance plus one
+  C_ITERS,                     // iterate-to-tolerance: slots used
+  C_WARM_KEPT,                 // the warm-start positions were kept (2: the damped retry's, PBF_OPT_WARM_RETRY)
+  C_DISP,                      // two flags: some particle has moved too far for the skin lists by the
+                               // end of the previous Jacobi iteration (parity of the iteration that reads it)
+  C_SKIN = C_DISP + 2,         // 1: this step's skin lists are built
+  C_DISP_ALL,                  // the same over the whole step so far
+  C_TILE,                      // particles that the cell walk set out to list (with PBF_OPT_COUNT_OVERFLOW;
+                               // what it handed on is in C_HEAVY)
+  C_RETRY,                     // the warm start grew the error at slot 0 and its damped retry was applied
+  C_NUM
 };
 
 constexpr uint32_t kMaxSolveSlots = PBF_MAX_SOLVE_ITERATIONS;

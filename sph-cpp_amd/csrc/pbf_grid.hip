@@ -806,8 +806,87 @@ __device__ __forceinline__ void load_chunk(uint32_t c0, uint32_t total, uint32_t
   for (uint32_t r = 0; r < kRounds; ++r) t[r] = ld3(xs, slot[r]);
 }
 
+// Where particles share their walk cells with few others, or with none (no
+// cell at all for one that has left the grid), the cell walk sets up a stream
+// for every one or two of them.  There each lane lists a particle: its cells go
+// by three at a time, x and y the same, and their candidates four at a time as
+// one stream, so that a lane waits for memory nine times twice and rarely
+// oftener.  Returns false, with nothing listed, after kSparseMost candidates.
+//
+// A wavefront takes it when it would set up more streams than its particles
+// times 8 / sparse_eighths(): one for three particles, for two, for each; with
+// fewer slots a wavefront the streams stay the quicker ones for longer.
+// Measured on random points, us a launch by particles a cell, all by streams /
+// so (in brackets the tile walk that the cell walk replaced, which wrote no
+// skin lists here):
+//   particles           3                2               1               0.3             none in the grid
+//      32,768      32 (54)         33 (49)         34 (46)         37 / 33 (45)
+//     131,072      67 (67)         71 (61)         82 (60)         92 / 81 (58)      90 / 29 (11)
+//     300,000     121 / 118 (112) 136 / 122 (104) 159 / 110 (99)  190 / 82 (97)
+//   1,000,000     331 / 280 (258) 371 / 237 (245) 457 / 186 (237) 560 / 135 (232)   587 / 50 (35)
+// (At 8,192 particles, four slots a wavefront, streams are the quicker ones
+// always: 17 to 19, lanes 23 at 0.3 a cell and 42 at three.)
+constexpr uint32_t kSparseMost = 256;
+__device__ __forceinline__ uint32_t sparse_eighths(uint32_t width) {
+  return width >= 32u ? 24u : (width >= 16u ? 16u : (width >= 8u ? 9u : 0u));
+}
+__device__ __forceinline__ bool sparse_walk(uint32_t p, f3 ps, const float4* __restrict__ xs,
+                                            const uint32_t* __restrict__ start, const KParams& K,
+                                            int32_t* __restrict__ nbr, int32_t* __restrict__ nbr_count,
+                                            int32_t* __restrict__ snb, int32_t* __restrict__ snb_count, bool skin,
+                                            uint32_t& ovf) {
+  const WalkCells w = walk_cells(ps, K.s);
+  const GridView G = grid_of(K, p);
+  ListWriter full(nbr, p, K), near(snb, p, K);
+  uint32_t dropped = 0, seen = 0;
+#pragma unroll 1
+  for (int xy = 0; xy < 9; ++xy) {
+    uint32_t b[3], m[3];
+#pragma unroll
+    for (int z = 0; z < 3; ++z) {
+      const uint32_t cell = cell_key(pick3(w.cx, xy / 3), pick3(w.cy, xy % 3), w.cz[z], G, K);
+      const uint32_t c = cell < K.ncells ? cell : 0u;
+      b[z] = start[c];
+      m[z] = cell < K.ncells ? start[c + 1] - b[z] : 0u;
+    }
+    const uint32_t m1 = m[0], m2 = m1 + m[1], total = m2 + m[2];
+    seen += total;
+    if (seen > kSparseMost) return false;
+#pragma unroll 1
+    for (uint32_t j0 = 0; j0 < total; j0 += 4) {
+      uint32_t q[4];
+      f3 t[4];
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u) {
+        const uint32_t j = j0 + u;
+        q[u] = j < m1 ? b[0] + j : (j < m2 ? b[1] + (j - m1) : (j < total ? b[2] + (j - m2) : K.pad));
+        t[u] = ld3(xs, q[u]);
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u) {
+        const float d2 = magsq3(sub3(ps, t[u]));
+        if (!(d2 < K.ss) || q[u] == p) continue;
+        if (full.count < (uint32_t)K.cap) {
+          full.add(q[u]);
+          if (skin && d2 < K.skin2) near.add(q[u]);
+        } else {
+          ++dropped;
+        }
+      }
+    }
+  }
+  full.close();
+  nbr_count[p] = (int32_t)full.count;
+  if (skin) {
+    near.close();
+    snb_count[p] = (int32_t)near.count;
+  }
+  ovf += dropped;
+  return true;
+}
+
 template <class Lds>
-__device__ __forceinline__ void cell_walk(uint32_t tb, uint32_t lane, uint64_t todo, f3 ps, uint32_t key,
+__device__ __forceinline__ void cell_walk(uint32_t tb, uint32_t width, uint32_t lane, uint64_t todo, f3 ps, uint32_t key,
                                           const float4* __restrict__ xs, const uint32_t* __restrict__ start,
                                           const KParams& K, int32_t* __restrict__ nbr,
                                           int32_t* __restrict__ nbr_count, int32_t* __restrict__ snb,
@@ -821,6 +900,17 @@ __device__ __forceinline__ void cell_walk(uint32_t tb, uint32_t lane, uint64_t t
     mid = {w.cx[1], w.cy[1], w.cz[1]};
     even = __builtin_amdgcn_ballot_w64(w.cx[0] == mid.x - 1.0f && w.cx[2] == mid.x + 1.0f && w.cy[0] == mid.y - 1.0f &&
                                        w.cy[2] == mid.y + 1.0f && w.cz[0] == mid.z - 1.0f && w.cz[2] == mid.z + 1.0f);
+  }
+  {
+    // about as many streams as the cell walk would set up
+    const uint32_t before = (uint32_t)__shfl_up((int)key, 1, 64);
+    const uint64_t own = __builtin_amdgcn_ballot_w64(lane == 0u || key != before || key >= K.ncells) | ~even;
+    if (sparse_eighths(width) * (uint32_t)__builtin_popcountll(own & todo) > 8u * (uint32_t)__builtin_popcountll(todo)) {
+      bool listed = false;
+      if ((todo >> lane) & 1ull)
+        listed = sparse_walk(tb + lane, ps, xs, start, K, nbr, nbr_count, snb, snb_count, skin, ovf);
+      todo &= ~__builtin_amdgcn_ballot_w64(listed);
+    }
   }
   const uint32_t cap = (uint32_t)K.cap;
   const float ss = in_vgpr(K.ss), ks = in_vgpr(K.skin2);
@@ -1070,7 +1160,7 @@ __global__ void __launch_bounds__(kFillBlock, LANES ? 1 : (CAP <= 64 ? 6 : 5)) k
     const uint64_t todo = __builtin_amdgcn_ballot_w64(query);
     uint32_t key = A.key[p];
     if (K.batched && key == K.ncells) key += K.sid[p];  // (outside every cell, but in its own scene's grid)
-    cell_walk(tb, lane, todo, xyz3(ps4), key, A.xs, A.start, K, A.nbr, A.nbr_count, A.snb, A.snb_count, skin != 0,
+    cell_walk(tb, A.width, lane, todo, xyz3(ps4), key, A.xs, A.start, K, A.nbr, A.nbr_count, A.snb, A.snb_count, skin != 0,
               A.hand_on != 0, S, hm, ovf);
     // (once for all: an atomic a wavefront took 0.5 ms at 8 million particles)
     if (K.count_overflow && blockIdx.x == 0 && lane == 0)

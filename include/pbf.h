@@ -460,6 +460,10 @@ int pbf_memcpy_device(void* dst, const void* src, uint64_t bytes);  /* device to
  * that took the shared-reciprocal divide / the unwrapped square root, out[4] =
  * divide mismatches among the operands shaped like the passes' own. */
 int pbf_check_arithmetic(uint64_t samples, uint64_t seed, uint64_t* out);
+/* The square root on every float (all 2^32 bit patterns): out[0] = mismatches,
+ * out[1] = patterns that took the unwrapped square root (those of
+ * 2^-96..2^96). */
+int pbf_check_sqrt(uint64_t* out);
 
 /* ---- output ----
  * Append one positions record to `path`, with the content AdiosWriter::write_particles

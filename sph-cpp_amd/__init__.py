@@ -222,6 +222,7 @@ def lib():
     _sig(L, "pbf_warm_model_train", [_P, C.c_uint32, C.c_uint32, C.c_float, C.c_uint64, _F])
     _sig(L, "pbf_warm_model_predict", [_P, _F, C.c_uint64, _F])
     _sig(L, "pbf_check_arithmetic", [C.c_uint64, C.c_uint64, _U64])
+    _sig(L, "pbf_check_sqrt", [_U64])
     _sig(L, "pbf_sync", [_P])
     _sig(L, "pbf_get_stats", [_P, C.POINTER(Stats)])
     _sig(L, "pbf_grid_dims", [_P, _U64])
@@ -623,6 +624,13 @@ def check_arithmetic(samples: int, seed: int = 0) -> dict:
     _check(lib().pbf_check_arithmetic(int(samples), int(seed), out.ctypes.data_as(_U64)))
     return {"divide_mismatches": int(out[0]), "sqrt_mismatches": int(out[1]),
             "divide_fast": int(out[2]), "sqrt_fast": int(out[3]), "divide_mismatches_shaped": int(out[4])}
+
+
+def check_sqrt() -> dict:
+    """pbf_check_sqrt: the library's square root against the plain one for every float."""
+    out = np.zeros(2, dtype=np.uint64)
+    _check(lib().pbf_check_sqrt(out.ctypes.data_as(_U64)))
+    return {"mismatches": int(out[0]), "fast": int(out[1])}
 
 
 NOALLOC_MAX_PAIRS = 1 << 20  # PBF_NOALLOC_MAX_PAIRS

@@ -12,7 +12,9 @@
 // magnitudes over 2^-48 .. 2^48 (both sides of the divide's range test).
 // The instances with the range tests discharged on the host
 // (div3_shared_static, sqrt_corrected) are compared too, on the operands
-// that meet their preconditions.
+// that meet their preconditions.  The square root is compared for every float
+// as well (k_check_sqrt): one in 2^32 rounded the other way would be one too
+// many, and samples would not show it.
 #include "pbf_device.h"
 
 namespace pbf {
@@ -93,6 +95,28 @@ __global__ void k_check_arithmetic(uint64_t samples, uint64_t seed, unsigned lon
   }
 }
 
+// one thread per 2^13 bit patterns
+constexpr uint32_t kSqrtThreads = 1u << 19;
+__global__ void __launch_bounds__(256) k_check_sqrt(unsigned long long* __restrict__ out) {
+  unsigned long long bad = 0, fast = 0;
+  uint32_t u = blockIdx.x * blockDim.x + threadIdx.x;
+  for (uint32_t i = 0; i < (uint32_t)((1ull << 32) / kSqrtThreads); ++i, u += kSqrtThreads) {
+    const float x = __uint_as_float(u), ref = sqrtf(x);
+    const bool f = sqrt_fast(x);
+    fast += f ? 1 : 0;
+    bad += same_bits(sqrt_cr(x), ref) && (!f || same_bits(sqrt_corrected(x), ref)) ? 0 : 1;
+  }
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    bad += __shfl_xor(bad, d, 64);
+    fast += __shfl_xor(fast, d, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    atomicAdd(&out[0], bad);
+    atomicAdd(&out[1], fast);
+  }
+}
+
 }  // namespace pbf
 
 using namespace pbf;
@@ -108,6 +132,21 @@ extern "C" int pbf_check_arithmetic(uint64_t samples, uint64_t seed, uint64_t* o
     rc = check_hip(hipGetLastError(), "check_arithmetic");
   }
   if (!rc) rc = check_hip(hipMemcpy(out, d, 5 * sizeof(unsigned long long), hipMemcpyDeviceToHost), "hipMemcpy");
+  hipFree(d);
+  return rc;
+}
+
+extern "C" int pbf_check_sqrt(uint64_t* out) {
+  if (!out) return set_error(PBF_ERR_ARG, "null argument");
+  unsigned long long* d = nullptr;
+  int rc = check_hip(hipMalloc((void**)&d, 2 * sizeof(unsigned long long)), "hipMalloc");
+  if (rc) return rc;
+  rc = check_hip(hipMemset(d, 0, 2 * sizeof(unsigned long long)), "hipMemset");
+  if (!rc) {
+    hipLaunchKernelGGL(k_check_sqrt, dim3(kSqrtThreads / 256), dim3(256), 0, nullptr, d);
+    rc = check_hip(hipGetLastError(), "check_sqrt");
+  }
+  if (!rc) rc = check_hip(hipMemcpy(out, d, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost), "hipMemcpy");
   hipFree(d);
   return rc;
 }

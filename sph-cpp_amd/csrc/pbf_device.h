@@ -110,8 +110,8 @@ __device__ __forceinline__ f3 div3_shared(f3 a, float b) {
 // operation and four full-rate ones): with y the hardware estimate of
 // 1/sqrt(x), s = x y is within a few ulp of sqrt(x), x - s s is exact (FMA),
 // and s + (x - s s) y / 2 rounds to the nearest (P. Markstein, IBM J. Res.
-// Dev. 34(1), 1990).  Compared with sqrtf on this device for every float in
-// [2^-96, 2^96]: no difference.  The estimate of the root corrected by the
+// Dev. 34(1), 1990).  pbf_check_sqrt compares it with sqrtf on the device for
+// every float in [2^-96, 2^96]: no difference.  The estimate of the root corrected by the
 // signs of two residuals, which it replaces, took one quarter-rate and eight
 // full-rate operations.  Other x take the plain sqrtf, so every result equals
 // sqrtf(x).

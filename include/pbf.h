@@ -476,7 +476,18 @@ int pbf_append_positions_record(pbf_context* ctx, const char* path);
 /* ---- measurement ----
  * Bracket every launch of the kernels named in `names` (comma separated,
  * "" = none) with HIP events on the context stream; pbf_kernel_time returns
- * the accumulated launches and milliseconds of one kernel since enabling. */
+ * the accumulated launches and milliseconds of one kernel since enabling.  A
+ * name that no launch carries counts none.
+ * A step: predict_bin, sort, reorder, fill_neighbors, cell_box, fill_heavy,
+ *   density_lambda, lambda_repair, dp_update (jacobi_persistent in their place),
+ *   surface_tension (in it color, tension), viscosity, vorticity,
+ *   apply_vorticity, viscosity_positions; with no iterations update_velocities.
+ * A solve also: density_features or density_warm_network, warm_dp, warm_retry,
+ *   solve_end.
+ * The passes one by one: forces_predict, bin, sort, reorder, fill_neighbors,
+ *   cell_box, fill_heavy, density, lambda, dp, update_position_stars,
+ *   update_velocities, surface_tension, viscosity, vorticity, apply_vorticity,
+ *   update_positions. */
 int pbf_profile_kernels(pbf_context* ctx, const char* names);
 int pbf_kernel_time(pbf_context* ctx, const char* name, uint64_t* launches, double* total_ms);
 /* Events around a whole region on the context stream. */

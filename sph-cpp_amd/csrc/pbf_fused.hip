@@ -270,10 +270,6 @@ __device__ __forceinline__ unsigned long long fixed_error(float e) {
   return (unsigned long long)(fminf(e, 2147483648.0f) * 4294967296.0f);
 }
 
-// With S.ehist, a wavefront's largest density error goes into a shard of row
-// eslot (atomicMax on the bits of a non-negative float orders like the float)
-// and its fixed-point sum into the same shard of S.esum.  With S.tol >= 0
-// nothing runs once the solve is done.
 // The learned warm start for one wavefront's 64 particles (every lane of the
 // wavefront calls it; fo holds the lane's features, zero past n): the
 // features go through LDS into the B operands of the network, which runs on
@@ -348,6 +344,10 @@ __device__ __forceinline__ void stamp_cells(uint64_t movers, uint32_t p, uint32_
 // calling thread is the one that clears the pass's flags (first): the same
 // bodies run as their own kernels (vb from xcd_block()) and inside the
 // persistent Jacobi kernel (vb from the calling block's share).
+// With S.ehist, a wavefront's largest density error goes into a shard of row
+// eslot (atomicMax on the bits of a non-negative float orders like the float)
+// and its fixed-point sum into the same shard of S.esum.  With S.tol >= 0
+// nothing runs once the solve is done.
 // L: lanes per particle; a block of vb holds blockDim.x / L particles.
 template <int FM, bool FAST, bool SR, int L>
 __device__ __forceinline__ void density_pass(uint32_t vb, bool first, uint32_t n, int it, int eslot,

@@ -16,7 +16,8 @@
 //
 // Lists.  Particles of one cell walk the same 27 cells: a wavefront takes
 // them together, one candidate per lane, and appends every particle's accepted
-// candidates in walk order through ballots (the cell walk, below).  Particles
+// candidates in walk order through ballots (the cell walk, below), or, where
+// few particles share a cell, a lane takes each (sparse_walk).  Particles
 // with very many candidates go to a list that one wavefront each works off,
 // skipping cells and runs of slots that are too far (k_fill_heavy).  With
 // PBF_OPT_LANE_LISTS one lane per particle walks its cells by itself.
@@ -502,8 +503,9 @@ __device__ __forceinline__ bool cell_far(const uint32_t* __restrict__ box, uint3
 // coordinates x + i*s, neighbors.h:171-185), skips itself and accepts
 // d^2 < s^2 while the list has room.  Lists hold sorted slots (list_at).
 //
-// Tiers with identical results: the cell walk, and k_fill_heavy (a wavefront
-// per particle) for those that it hands on; with PBF_OPT_LANE_LISTS one lane per particle
+// Tiers with identical results: the cell walk, with a lane per particle in
+// sparse wavefronts, and k_fill_heavy (a wavefront per particle) for those that
+// it hands on, in scenes of enough particles; with PBF_OPT_LANE_LISTS one lane per particle
 // unless its cells hold more than twice K.heavy_budget candidates and its walk
 // scans K.heavy_budget of them without filling the list (with the overflow
 // count on: more than K.heavy_budget candidates).
@@ -1372,7 +1374,7 @@ RadixPlan radix_plan(uint64_t n, uint32_t key_bits) {
     P.per_group = 1;
     while (P.per_group * P.per_group < P.ntiles) P.per_group *= 2;
   }
-  // (at most 64: 46 of a square root's size, or the prefixed sort's 64)
+  // (at most 32 up to 2,048 tiles, 64 of the prefixed sort's)
   P.ngroups = P.ntiles ? (P.ntiles + P.per_group - 1) / P.per_group : 0u;
   return P;
 }

@@ -30,7 +30,7 @@
 //   counters         u64[C_NUM]  overflow, outside, hacks, hack flags, solve state, ...
 //   ehist, esum      uint32, u64[kMaxSolveSlots+1][kErrShards]  max (float bits) and sum of the
 //                                density errors per solve slot, in shards that their readers combine
-//   cstamp           uint32[C+1] == the iteration's stamp: a particle within two cells was moved
+//   cstamp           uint32[C+2] == the iteration's stamp: a particle within two cells was moved
 //                                by the density fix (cleared with cell_start)
 //   lsum, lsuma      float[n]    multipliers summed over the updates of the last solve
 //                                (carried through the reorder while a warm start may use them)
@@ -259,7 +259,7 @@ struct pbf_context {
   uint32_t *rhist = nullptr, *rsum = nullptr;
   int sorted = 0;  // which of sk, sv the last sort left its result in
   uint32_t* heavy = nullptr;
-  uint32_t* cstamp = nullptr;  // [cells + 1] == dirty_stamp: a particle within two cells was moved
+  uint32_t* cstamp = nullptr;  // [cells + 2] == dirty_stamp: a particle within two cells was moved
   uint32_t* dirty = nullptr;  // == dirty_stamp: the particle or one of its neighbours moved
   uint32_t* mflag = nullptr;  // == dirty_stamp: the density fix moved the particle in that iteration
   uint32_t* cell_start = nullptr;

@@ -54,7 +54,7 @@ __device__ __forceinline__ bool pass_writes() {
 }
 
 // Quads below this many particles, single lanes above, for the reason given at
-// pressure_quads() in pbf_fused.hip: at 131,072 particles the two are within
+// density_lanes() in pbf_fused.hip: at 131,072 particles the two are within
 // 10% of each other on these walks, at 32,768 quads take 60-70% of the time.
 constexpr uint64_t kPassQuads = 131072;
 #define PBF_PASS(c, name, kern, ...)                                                                             \

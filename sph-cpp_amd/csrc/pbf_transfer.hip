@@ -2,20 +2,23 @@
 //
 // They go through a small block of pinned memory of the object: the host
 // copies a chunk while the device moves the others.  Copies straight from and
-// to pageable memory cost more, most of all from 64 KB to 384 KB, which the
-// runtime moves at 2.3 GB/s.  Measured, us for a call that sets / reads an
-// array, its reordering kernel and the wait included (in brackets with the
-// runtime's copies):
-//      12 KB     16 /   15   (22 /   27)
-//     393 KB     35 /   39  (175 /  184)
-//     1.6 MB     78 /  108   (75 /  110)
-//     3.1 MB    121 /  165  (117 /  200)
-//    12.6 MB    400 /  490  (410 /  790)
-//      50 MB   1340 / 1800 (1790 / 3000)
+// to pageable memory cost more, most of all where the runtime takes 100 to 200
+// us for 64 to 400 KB, as it does in some processes.  Measured, us for a call
+// that sets / reads an array, its reordering kernel and the wait included (in
+// brackets with the runtime's copies):
+//      12 KB     14 /   14   (21 /   28)
+//     393 KB     31 /   38   (33 to 175 / 40 to 195)
+//     1.6 MB     70 /   90   (77 /  110)
+//     3.1 MB    125 /  170  (121 /  197)
+//    12.6 MB    337 /  495  (375 /  735)
+//      34 MB    900 /  960 (1000 / 1930)
+//     101 MB   2580 / 2550 (3480 / 5800, into fresh pages 9800)
+// (For some tens of milliseconds after much device memory was given back, the
+// copy engines clear it: copies of either kind then take up to four times as
+// long.)
 // Bound: PCIe (12.6 MB alone take 228 us from pinned memory), the host's copy
 // next to it, and some 15 us a queued copy, which is why chunks are large.  (A
-// kernel that copies instead of the copy engine was no faster: 35 / 34 and
-// 430 / 520 us at 393 KB and 12.6 MB.)
+// kernel that copies instead of the copy engine: 385 us up and 480 down at 12.6 MB.)
 //
 // Memory that the caller has pinned takes no part in this: the copy engine
 // reads and writes it as it is, 257 / 266 us for 12.6 MB against 346 / 515

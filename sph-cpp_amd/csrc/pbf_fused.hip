@@ -132,12 +132,14 @@ __device__ __forceinline__ float density_lambda_one(uint32_t p, uint32_t n, cons
   const int32_t* __restrict__ walk = skin ? snb : nbr;
   const int cnt = skin ? snb_count[p] : nbr_count[p];
   DensitySums s = density_start(K);
+  const bool plain = lost(xp);
   const f3 vp = FEAT ? ld3(v, p) : f3{0.f, 0.f, 0.f};
   // one walk over the list: the entries within h go into the sums, in list
   // order (padding entries read the far row and are never within h).  A
   // near-coincident entry (particles.h:304) ends the walk after its batch, and
-  // the plain walk below redoes the particle with fresh sums.
-  bool hack = false;
+  // the plain walk below redoes the particle with fresh sums; so it does a lost
+  // particle.
+  bool hack = plain;
   uint64_t m0 = 0, m1 = 0;
   const int4* __restrict__ row = list_row(walk, p, K.stride);
   uint32_t q[kBatch];
@@ -215,7 +217,7 @@ __device__ __forceinline__ float density_lambda_group(uint32_t p, const KParams&
   f3 xp = ld3(xs, p);
   const int cnt = skin ? snb_count[p] : nbr_count[p];
   DensitySums s = density_start(K);
-  bool hack = false;
+  bool hack = lost(xp);
   GroupRow<L> row(skin ? snb : nbr, p, K.stride);
   constexpr int kMine = GroupRow<L>::kMine;
   for (int k0 = 0; k0 < cnt && !hack; k0 += GroupRow<L>::kEntries) {
@@ -643,7 +645,7 @@ __device__ __forceinline__ float mean_error_of(const SolveCtl& S, int row, uint3
 // The pressure update's sum over the entries of one particle's list within h
 // (particles.h:355-366), by one lane: under the density pass's mask (entries
 // outside h then gather the particle itself), or with plain every entry of
-// the list tested.
+// the list tested, up to its count.
 template <bool FAST, bool SR>
 __device__ __forceinline__ f3 dp_walk(const int32_t* __restrict__ walk, int cnt, bool plain, uint64_t m0, uint64_t m1,
                                       uint32_t p, f3 xp, float lp, const KParams& K,
@@ -661,7 +663,7 @@ __device__ __forceinline__ f3 dp_walk(const int32_t* __restrict__ walk, int cnt,
     for (int u = 0; u < kBatch; ++u) {
       const f3 d = sub3(xp, xyz(t[u]));
       const float d2 = magsq3(d);
-      if (!((bits >> u) & 1u) || (plain && !within_h(d2, K))) continue;
+      if (!((bits >> u) & 1u) || (plain && (k0 + u >= cnt || !within_h(d2, K)))) continue;
       const float r = nb_sqrt<FAST, SR>(d2);
       acc3(dp, smul3(lp + t[u].w, nb_spiky<FAST, SR>(d, r, K)));
     }
@@ -669,8 +671,8 @@ __device__ __forceinline__ f3 dp_walk(const int32_t* __restrict__ walk, int cnt,
   return dp;
 }
 
-// The same by L lanes.
-template <bool FAST, bool SR, int L>
+// The same by L lanes (PLAIN: entries past the count tested for).
+template <bool FAST, bool SR, int L, bool PLAIN>
 __device__ __forceinline__ f3 dp_walk_group(const int32_t* __restrict__ walk, int cnt, uint32_t p, f3 xp, float lp,
                                            const KParams& K, const float4* __restrict__ xt) {
   f3 dp = {0.f, 0.f, 0.f};
@@ -688,7 +690,7 @@ __device__ __forceinline__ f3 dp_walk_group(const int32_t* __restrict__ walk, in
       const f3 d = sub3(xp, xyz(t[j]));
       const float d2 = magsq3(d);
       f3 term = {0.f, 0.f, 0.f};
-      if (within_h(d2, K)) {
+      if (within_h(d2, K) && (!PLAIN || k0 + (int)lane_in_group<L>() + L * j < cnt)) {
         const float r = nb_sqrt<FAST, SR>(d2);
         term = smul3(lp + t[j].w, nb_spiky<FAST, SR>(d, r, K));
       }
@@ -780,24 +782,24 @@ __device__ __forceinline__ void dp_pass(uint32_t vb, bool first, uint32_t n, int
     if (S.lsum && it == 0 && writes) S.lsum[p] = 0.0f;
     if (track) mv = move2(xyz(t), xs0[p]);
   } else if (p < n) {
-    // a dirty particle (moved by the density fix, or next to one) walks its
-    // whole list; the others walk the list the density pass walked (the skin
-    // list when it could)
-    const bool plain = counters[C_HACK_FLAG + (it & 1)] != 0ull && dirty[p] == stamp;
-    const bool skin = !plain && skin_usable(counters, C_DISP + (it & 1));
-    const int32_t* __restrict__ walk = skin ? snb : nbr;
     // x* and lambda of a particle come in one load (xt.w holds lambda)
     const float4 xp4 = xt[p];
     const f3 xp = xyz(xp4);
+    // a dirty particle (moved by the density fix, or next to one) walks its
+    // whole list, and so does a lost one; the others walk the list the density
+    // pass walked (the skin list when it could)
+    const bool plain = (counters[C_HACK_FLAG + (it & 1)] != 0ull && dirty[p] == stamp) || lost(xp);
+    const bool skin = !plain && skin_usable(counters, C_DISP + (it & 1));
+    const int32_t* __restrict__ walk = skin ? snb : nbr;
     const float lp = xp4.w;
     const int cnt = skin ? snb_count[p] : nbr_count[p];
-    // with no dirty lane in the wavefront every pair within h is one the
+    // with no such lane in the wavefront every pair within h is one the
     // density pass accepted at the same positions (static ranges); the lanes
     // of a group find them by the same test, single lanes by the mask it left
     f3 dp;
     if constexpr (L != 1)
-      dp = (SR && __ballot(plain) == 0ull) ? dp_walk_group<FAST, SR, L>(walk, cnt, p, xp, lp, K, xt)
-                                           : dp_walk_group<FAST, false, L>(walk, cnt, p, xp, lp, K, xt);
+      dp = __ballot(plain) == 0ull ? dp_walk_group<FAST, SR, L, false>(walk, cnt, p, xp, lp, K, xt)
+                                   : dp_walk_group<FAST, false, L, true>(walk, cnt, p, xp, lp, K, xt);
     else {
       const uint64_t m0 = plain ? ~0ull : wmask[p];
       const uint64_t m1 = (plain || K.cap <= 64) ? ~0ull : wmask[n + p];
@@ -952,6 +954,23 @@ __device__ __forceinline__ f3 xsph_term(f3 xp, f3 vp, float4 t, float4 vq, const
   return div3_shared(mul3(sub3(xyz(vq), vp), poly6_in(r, K)), vq.w);
 }
 
+// The first XSPH pass of a lost particle (every lane of its group calls it):
+// its entries within h into the compact row, their number, and their terms.
+__device__ __forceinline__ uint32_t lost_viscosity(const int32_t* __restrict__ list, int cnt, uint32_t p, f3 xp, f3 vp,
+                                                   bool writes, const KParams& K, const float4* __restrict__ xs,
+                                                   const float4* __restrict__ vin, int32_t* __restrict__ out, f3& dv) {
+  uint32_t nc = 0;
+  for (int k = 0; k < cnt; ++k) {
+    const uint32_t at = (uint32_t)list[list_at((uint32_t)k, p, K.stride)] << 4;
+    const float4 t = gather_at(xs, at);
+    if (!within_h(magsq3(sub3(xp, xyz(t))), K)) continue;
+    if (writes) out[(nc & ~3u) * 64u + (nc & 3u)] = (int32_t)at;
+    ++nc;
+    acc3(dv, xsph_term(xp, vp, t, gather_at(vin, at), K));
+  }
+  return nc;
+}
+
 // apply_viscosity (particles.h:436-447), first call: walks the skin or full
 // list and leaves the compact rows of the final positions for the passes that
 // follow.  An accepted entry's place in the row is the number accepted before
@@ -978,8 +997,8 @@ __global__ void __launch_bounds__(kBlock) k_viscosity_first(uint32_t n, KParams 
   const f3 vp = xyz(v4);
   // the skin list holds every entry within h while no particle has moved
   // 0.045 h over the step (skin lists, above)
-  const bool skin = skin_usable(counters, C_DISP_ALL);
-  const int cnt = skin ? snb_count[p] : nbr_count[p];
+  const bool skin = skin_usable(counters, C_DISP_ALL), alone = lost(xp);
+  const int all = skin ? snb_count[p] : nbr_count[p], cnt = alone ? 0 : all;
   GroupRow<L> row(skin ? snb : nbr, p, K.stride);
   constexpr int kMine = GroupRow<L>::kMine;
   int32_t* __restrict__ out = cnb + list_at(0, p, K.stride);
@@ -1010,6 +1029,7 @@ __global__ void __launch_bounds__(kBlock) k_viscosity_first(uint32_t n, KParams 
       group_add3<L>(dv, term);
     }
   }
+  if (__builtin_expect(alone, 0)) nc = lost_viscosity(skin ? snb : nbr, all, p, xp, vp, u == 0u, K, xs, vin, out, dv);
   if (u != 0u) return;
   cnb_count[p] = (int32_t)nc;
   f3 nv = vp;
@@ -1179,6 +1199,14 @@ __global__ void __launch_bounds__(kStageBlock) k_viscosity_first_lane(
     for (int u = 0; u < kBatch; ++u) {
       s_list[nc * kStageBlock + lane] = q[u] << 4;  // a rejected entry is overwritten by the next accepted one
       nc += within_h(magsq3(sub3(xp, xyz(t[u]))), K) ? 1 : 0;
+    }
+  }
+  if (__builtin_expect(lost(xp), 0)) {  // again, up to the count
+    nc = 0;
+    for (int k = 0; k < cnt; ++k) {
+      const uint32_t at = (uint32_t)(skin ? snb : nbr)[list_at((uint32_t)k, p, K.stride)] << 4;
+      s_list[nc * kStageBlock + lane] = at;
+      nc += within_h(magsq3(sub3(xp, xyz(gather_at(xs, at)))), K) ? 1 : 0;
     }
   }
   cnb_count[p] = nc;

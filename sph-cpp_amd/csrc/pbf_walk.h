@@ -34,6 +34,12 @@ __device__ __forceinline__ void load_batch(const int32_t* __restrict__ list, uin
   for (int u = 0; u < kBatch; ++u) q[u] = k0 + u < cnt ? q[u] : p;
 }
 
+// Whether a position has a NaN or an infinity (or a square past the largest
+// float).  The far row is not outside h of such a particle: the distance is a
+// NaN, which within_h keeps.  So its list is taken entry by entry up to its
+// count; the walks below pass over it and their callers do it on their own.
+__device__ __forceinline__ bool lost(f3 x) { return !(magsq3(x) <= 3.402823466e38f); }
+
 // Skin lists (built with the lists, pbf_grid.hip): the entries within
 // 1.1 h of the positions the lists were built from (x*_0), in list order.  A
 // pass may walk the skin list instead of the full one while no particle has
@@ -195,6 +201,20 @@ template <int L, int N, class Data, class Term>
 __device__ __forceinline__ void walk_within(const int32_t* __restrict__ list, int cnt, uint32_t p, f3 xp,
                                             const KParams& K, const float4* __restrict__ pos, Terms<N>& sum,
                                             bool& near, Data data, Term term) {
+  if (__builtin_expect(lost(xp), 0)) {  // (the same for a quad's lanes, each of which takes the whole list)
+    for (int k = 0; k < cnt; ++k) {
+      const uint32_t q = (uint32_t)list[list_at((uint32_t)k, p, K.stride)];
+      const f3 d = sub3(xp, xyz(gather4(pos, q)));
+      const float d2 = magsq3(d);
+      near |= d2 < K.T_hack;
+      if (!within_h(d2, K)) continue;
+      Terms<N> e{};
+      term(d, d2, data(q), e);
+#pragma unroll
+      for (int i = 0; i < N; ++i) sum.a[i] += e.a[i];
+    }
+    return;
+  }
   if constexpr (L != 1) {
     const uint32_t* __restrict__ row = quad_row(list, p, K.stride);
     uint32_t q[2] = {row[0], row[256]};

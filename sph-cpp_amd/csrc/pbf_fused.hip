@@ -882,8 +882,12 @@ __global__ void __launch_bounds__(kBlock) k_warm_dp(uint32_t n, KParams K, const
     boundary(nw, K, p);
     st3(xs, p, nw);
     xsave[p] = xp4;
-    // both x* (kept) and xt (restored on a rejection) count as moves
-    if (track) mv = fmaxf(move2(nw, xs0[p]), move2(xp, xs0[p]));
+    // both x* (kept) and xt (restored on a rejection) count as moves (a NaN
+    // among them too, which a maximum would drop)
+    if (track) {
+      mv = move2(nw, xs0[p]);
+      if (mv < K.disp_lim2) mv = move2(xp, xs0[p]);
+    }
   }
   // slot 0 reads parity 0
   if (track) record_move(mv, counters, C_DISP + 0, K);

@@ -351,3 +351,43 @@ def test_lost_in_the_passes(pbf, scenes, n, cap, value):
         getattr(g, name)()
         f()
         _compare(g, m.state(), name, scratch=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("side", [2, 12, 24, 34, 54])
+def test_nan_multiplier_at_rest(pbf, scenes, side):
+    """Fluid at rest, so that its skin lists serve, and a warm start of zeros
+    with one NaN: the NaN moves count as moves, and the skin lists, which leave
+    out entries that were 1.1 h away, serve no longer."""
+    i = np.arange(side, dtype=F)
+    pos = np.stack(np.meshgrid(i, i, i, indexing="ij"), -1).reshape(-1, 3) * F(0.055) + F(0.03)
+    n = len(pos)
+    vel = np.zeros_like(pos)
+    p = _params(pbf, scenes, n, 60, F(0.055) * side + F(0.03))
+    g = pbf.Particles(p)
+    g.add(pos, pos, vel)
+    g.step(2)
+    m = Model(p, g.positions(), g.velocities())
+    warm = np.zeros(n, F)
+    warm[n // 2] = np.nan
+    g.set_warm_lambdas(warm)
+    g.solve(0.0, 3, pbf.PBF_WARM_GIVEN)
+    info = g.solve_info()
+    m.forces_predict()
+    m.lists(*g.neighbor_lists())
+    m.density()
+    before = m.xs.copy()
+    m.lam = warm
+    m.dps()
+    m.stars()
+    assert np.isnan(m.xs).any()
+    for it in range(info["iterations"]):
+        m.density()
+        m.multipliers()
+        if it == 0 and not info["warm_start_kept"]:
+            m.xs = before
+        elif info["max_error_history"][it] > 0:
+            m.dps()
+            m.stars()
+    m.tail()
+    _compare(g, m.state(), "solve")

@@ -113,13 +113,17 @@ enum Counter {
   C_WARM_KEPT,                 // the warm-start positions were kept (2: the damped retry's, PBF_OPT_WARM_RETRY)
   C_DISP,                      // two flags: some particle has moved too far for the skin lists by the
                                // end of the previous Jacobi iteration (parity of the iteration that reads it)
-  C_SKIN = C_DISP + 2,         // 1: this step's skin lists are built
+  // (a cache line of 128 bytes on: every wavefront reads C_SKIN, and behind the
+  // atomics on C_HEAVY and C_DISP that waited: a pressure update of 256 late
+  // scenes in a batch 485 us with the lines apart and 855 in one)
+  C_SKIN = C_FIRST + 16,       // 1: this step's skin lists are built
   C_DISP_ALL,                  // the same over the whole step so far
   C_TILE,                      // particles that the cell walk set out to list (with PBF_OPT_COUNT_OVERFLOW;
                                // what it handed on is in C_HEAVY)
   C_RETRY,                     // the warm start grew the error at slot 0 and its damped retry was applied
   C_NUM
 };
+static_assert(C_DISP + 2 <= C_SKIN, "counters overlap");
 
 constexpr uint32_t kMaxSolveSlots = PBF_MAX_SOLVE_ITERATIONS;
 // The error of a slot is gathered by atomics of every wavefront: on one

@@ -645,7 +645,7 @@ __device__ __forceinline__ float mean_error_of(const SolveCtl& S, int row, uint3
 // The pressure update's sum over the entries of one particle's list within h
 // (particles.h:355-366), by one lane: under the density pass's mask (entries
 // outside h then gather the particle itself), or with plain every entry of
-// the list tested, up to its count.
+// the list tested.
 template <bool FAST, bool SR>
 __device__ __forceinline__ f3 dp_walk(const int32_t* __restrict__ walk, int cnt, bool plain, uint64_t m0, uint64_t m1,
                                       uint32_t p, f3 xp, float lp, const KParams& K,
@@ -663,7 +663,7 @@ __device__ __forceinline__ f3 dp_walk(const int32_t* __restrict__ walk, int cnt,
     for (int u = 0; u < kBatch; ++u) {
       const f3 d = sub3(xp, xyz(t[u]));
       const float d2 = magsq3(d);
-      if (!((bits >> u) & 1u) || (plain && (k0 + u >= cnt || !within_h(d2, K)))) continue;
+      if (!((bits >> u) & 1u) || (plain && !within_h(d2, K))) continue;
       const float r = nb_sqrt<FAST, SR>(d2);
       acc3(dp, smul3(lp + t[u].w, nb_spiky<FAST, SR>(d, r, K)));
     }
@@ -671,8 +671,26 @@ __device__ __forceinline__ f3 dp_walk(const int32_t* __restrict__ walk, int cnt,
   return dp;
 }
 
-// The same by L lanes (PLAIN: entries past the count tested for).
-template <bool FAST, bool SR, int L, bool PLAIN>
+// The same for a lost particle, entry by entry up to the full list's count
+// (every lane of its group takes all of them).  A walk of its own because a
+// test for the count in dp_walk costs every wavefront with a dirty lane: an
+// update of the collapsed 1M dam break 98 us with it, 92 so.
+template <bool FAST>
+__device__ __forceinline__ f3 lost_update(const int32_t* __restrict__ list, int cnt, uint32_t p, f3 xp, float lp,
+                                          const KParams& K, const float4* __restrict__ xt) {
+  f3 dp = {0.f, 0.f, 0.f};
+  for (int k = 0; k < cnt; ++k) {
+    const float4 t = gather4(xt, (uint32_t)list[list_at((uint32_t)k, p, K.stride)]);
+    const f3 d = sub3(xp, xyz(t));
+    const float d2 = magsq3(d);
+    if (!within_h(d2, K)) continue;
+    acc3(dp, smul3(lp + t.w, nb_spiky<FAST, false>(d, nb_sqrt<FAST, false>(d2), K)));
+  }
+  return dp;
+}
+
+// The same by L lanes.
+template <bool FAST, bool SR, int L>
 __device__ __forceinline__ f3 dp_walk_group(const int32_t* __restrict__ walk, int cnt, uint32_t p, f3 xp, float lp,
                                            const KParams& K, const float4* __restrict__ xt) {
   f3 dp = {0.f, 0.f, 0.f};
@@ -690,7 +708,7 @@ __device__ __forceinline__ f3 dp_walk_group(const int32_t* __restrict__ walk, in
       const f3 d = sub3(xp, xyz(t[j]));
       const float d2 = magsq3(d);
       f3 term = {0.f, 0.f, 0.f};
-      if (within_h(d2, K) && (!PLAIN || k0 + (int)lane_in_group<L>() + L * j < cnt)) {
+      if (within_h(d2, K)) {
         const float r = nb_sqrt<FAST, SR>(d2);
         term = smul3(lp + t[j].w, nb_spiky<FAST, SR>(d, r, K));
       }
@@ -786,20 +804,22 @@ __device__ __forceinline__ void dp_pass(uint32_t vb, bool first, uint32_t n, int
     const float4 xp4 = xt[p];
     const f3 xp = xyz(xp4);
     // a dirty particle (moved by the density fix, or next to one) walks its
-    // whole list, and so does a lost one; the others walk the list the density
-    // pass walked (the skin list when it could)
-    const bool plain = (counters[C_HACK_FLAG + (it & 1)] != 0ull && dirty[p] == stamp) || lost(xp);
+    // whole list; the others walk the list the density pass walked (the skin
+    // list when it could)
+    const bool plain = counters[C_HACK_FLAG + (it & 1)] != 0ull && dirty[p] == stamp;
     const bool skin = !plain && skin_usable(counters, C_DISP + (it & 1));
     const int32_t* __restrict__ walk = skin ? snb : nbr;
     const float lp = xp4.w;
     const int cnt = skin ? snb_count[p] : nbr_count[p];
-    // with no such lane in the wavefront every pair within h is one the
+    // with no dirty lane in the wavefront every pair within h is one the
     // density pass accepted at the same positions (static ranges); the lanes
     // of a group find them by the same test, single lanes by the mask it left
     f3 dp;
-    if constexpr (L != 1)
-      dp = __ballot(plain) == 0ull ? dp_walk_group<FAST, SR, L, false>(walk, cnt, p, xp, lp, K, xt)
-                                   : dp_walk_group<FAST, false, L, true>(walk, cnt, p, xp, lp, K, xt);
+    if (__builtin_expect(lost(xp), 0))
+      dp = lost_update<FAST>(nbr, nbr_count[p], p, xp, lp, K, xt);
+    else if constexpr (L != 1)
+      dp = (SR && __ballot(plain) == 0ull) ? dp_walk_group<FAST, SR, L>(walk, cnt, p, xp, lp, K, xt)
+                                           : dp_walk_group<FAST, false, L>(walk, cnt, p, xp, lp, K, xt);
     else {
       const uint64_t m0 = plain ? ~0ull : wmask[p];
       const uint64_t m1 = (plain || K.cap <= 64) ? ~0ull : wmask[n + p];

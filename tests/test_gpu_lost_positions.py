@@ -232,13 +232,11 @@ def test_the_written_passes_are_the_oracles(pbf, scenes, n, cap):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,cap", SIZES)
-@pytest.mark.parametrize("options", ["none", "full_lists", "persistent"])
-def test_density_fix_to_infinity(pbf, scenes, n, cap, options):
+@pytest.mark.parametrize("options,n,cap", [(o, n, cap) for o, most in (("none", 10**6), ("full_lists", 200000), ("persistent", 20000))
+                                           for n, cap in SIZES if n <= most])
+def test_density_fix_to_infinity(pbf, scenes, options, n, cap):
     """The thrown particles are lost between the density pass and the pressure
     update, which clamps them onto the box (unless they met another one)."""
-    if options == "persistent" and n > 20000 or options == "full_lists" and n > 200000:
-        pytest.skip("covered at the other sizes")
     bits = {"none": 0, "full_lists": pbf.PBF_OPT_FULL_LISTS, "persistent": pbf.PBF_OPT_PERSISTENT}[options]
     pos, vel, side = _thrown(n, cap)
     p = _params(pbf, scenes, n, cap, side, bits)
